@@ -42,7 +42,6 @@ struct Workspace {
   uint8_t* hr = nullptr;
   int32_t* lc = nullptr;
   int32_t* par = nullptr;
-  uint8_t* ppn = nullptr;  // prefix_n of each node's parent (fused build)
   int32_t* edge = nullptr;
   int32_t* offs = nullptr;
   OctNode* nodes = nullptr;
@@ -50,7 +49,7 @@ struct Workspace {
   uint64_t* flags = nullptr;     // flag_cap words
   int32_t* counts = nullptr;     // n_unique[seg_cap], kalloc[seg_cap]
   int32_t* oct_start = nullptr;  // seg_cap + 1
-  int32_t* tables = nullptr;     // seg_start + 4 tile maps, 5 * (seg_cap+1)
+  int32_t* tables = nullptr;     // seg_start + 5 tile maps, 6 * (seg_cap+1)
   float* boxes = nullptr;        // seg_min[seg_cap], seg_range[seg_cap]
   uint32_t* box_mm = nullptr;    // per segment {min, max} while boxes are reduced
   uint32_t* vals_a = nullptr;    // key->point permutation (allocated when enabled): sorted
@@ -65,11 +64,12 @@ struct Plan {
   bool device_boxes = false;  // boxes reduced on the device into ws.boxes
   bool permutation = false;   // point indices carried through sort and unique
   SegView sv{};
-  int32_t tiles_morton = 0, tiles_sort = 0, tiles_scan = 0, tiles_node = 0;
+  int32_t tiles_morton = 0, tiles_sort = 0, tiles_scan = 0, tiles_node = 0, tiles_tree = 0;
   const int32_t* ts_morton = nullptr;
   const int32_t* ts_sort = nullptr;
   const int32_t* ts_scan = nullptr;
   const int32_t* ts_node = nullptr;
+  const int32_t* ts_tree = nullptr;
 };
 
 // Kernels of one build, in launch order (per-kernel event timing).
@@ -255,7 +255,7 @@ int ensure_scratch(ocp_ctx c, int64_t flag_words) {
 
 void free_workspace(Workspace& w) {
   dev_free(w.keys_a); dev_free(w.keys_b); dev_free(w.prefix_n); dev_free(w.hl);
-  dev_free(w.hr); dev_free(w.lc); dev_free(w.par); dev_free(w.ppn); dev_free(w.edge);
+  dev_free(w.hr); dev_free(w.lc); dev_free(w.par); dev_free(w.edge);
   dev_free(w.offs); dev_free(w.nodes); dev_free(w.hist); dev_free(w.flags);
   dev_free(w.counts); dev_free(w.oct_start); dev_free(w.tables); dev_free(w.boxes);
   dev_free(w.box_mm); dev_free(w.vals_a); dev_free(w.vals_b);
@@ -285,14 +285,13 @@ int ensure_workspace(ocp_ctx c, int64_t n, int32_t n_seg, int64_t flag_words) {
   if (grow_n) {
     const int64_t cap = std::max<int64_t>(n, 4096);
     dev_free(w.keys_a); dev_free(w.keys_b); dev_free(w.prefix_n); dev_free(w.hl);
-    dev_free(w.hr); dev_free(w.lc); dev_free(w.par); dev_free(w.ppn); dev_free(w.edge);
+    dev_free(w.hr); dev_free(w.lc); dev_free(w.par); dev_free(w.edge);
     dev_free(w.offs);
     int r = 0;
     if ((r = dev_alloc(c, &w.keys_a, cap)) || (r = dev_alloc(c, &w.keys_b, cap)) ||
         (r = dev_alloc(c, &w.prefix_n, cap)) || (r = dev_alloc(c, &w.hl, cap)) ||
         (r = dev_alloc(c, &w.hr, cap)) || (r = dev_alloc(c, &w.lc, cap)) ||
-        (r = dev_alloc(c, &w.par, cap)) || (r = dev_alloc(c, &w.ppn, cap)) ||
-        (r = dev_alloc(c, &w.edge, cap)) ||
+        (r = dev_alloc(c, &w.par, cap)) || (r = dev_alloc(c, &w.edge, cap)) ||
         (r = dev_alloc(c, &w.offs, cap)))
       return r;
     w.n_cap = cap;
@@ -307,7 +306,7 @@ int ensure_workspace(ocp_ctx c, int64_t n, int32_t n_seg, int64_t flag_words) {
     if ((r = dev_alloc(c, &w.hist, int64_t(cap) * (hist_stride(10) + kCursorWords))) ||
         (r = dev_alloc(c, &w.counts, int64_t(cap) * 2)) ||
         (r = dev_alloc(c, &w.oct_start, int64_t(cap) + 1)) ||
-        (r = dev_alloc(c, &w.tables, 5 * (int64_t(cap) + 1))) ||
+        (r = dev_alloc(c, &w.tables, 6 * (int64_t(cap) + 1))) ||
         (r = dev_alloc(c, &w.boxes, 2 * int64_t(cap))) ||
         (r = dev_alloc(c, &w.box_mm, 2 * int64_t(cap))))
       return r;
@@ -378,6 +377,7 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
   p.tiles_sort = static_cast<int32_t>(cdiv(n, pipe_sort_tile(tt, perm)));
   p.tiles_scan = static_cast<int32_t>(cdiv(n, scan_tile(tt)));
   p.tiles_node = static_cast<int32_t>(cdiv(n, kNodeTile));
+  p.tiles_tree = static_cast<int32_t>(cdiv(n, tree_tile(n)));
   return p;
 }
 
@@ -417,20 +417,22 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   int32_t* d_ts = w.tables + 2 * stride;
   int32_t* d_tc = w.tables + 3 * stride;
   int32_t* d_tn = w.tables + 4 * stride;
+  int32_t* d_tt = w.tables + 5 * stride;
   Plan p;
   p.n_seg = n_seg;
   p.n_total = n;
   p.permutation = perm;
   p.device_boxes = !smin;
   const int stile = pipe_sort_tile(tt, perm);
-  std::vector<int32_t> host(5 * static_cast<size_t>(n_seg + 1));
-  int64_t tm = 0, ts = 0, tc = 0, tn = 0;
+  std::vector<int32_t> host(6 * static_cast<size_t>(n_seg + 1));
+  int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0;
   for (int32_t k = 0; k <= n_seg; ++k) {
     host[k] = offsets[k];
     host[(n_seg + 1) + k] = static_cast<int32_t>(tm);
     host[2 * (n_seg + 1) + k] = static_cast<int32_t>(ts);
     host[3 * (n_seg + 1) + k] = static_cast<int32_t>(tc);
     host[4 * (n_seg + 1) + k] = static_cast<int32_t>(tn);
+    host[5 * (n_seg + 1) + k] = static_cast<int32_t>(ttr);
     if (k < n_seg) {
       const int64_t len = int64_t(offsets[k + 1]) - offsets[k];
       p.max_seg = std::max(p.max_seg, len);
@@ -438,6 +440,7 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
       ts += cdiv(len, stile);
       tc += cdiv(len, scan_tile(tt));
       tn += cdiv(len, kNodeTile);
+      ttr += cdiv(len, tree_tile(n));
     }
   }
   const int tab_key = tune_key(tt) * 2 + (pipe_sort_bits(tt, perm) == 10);
@@ -445,7 +448,7 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
                     c->tab_offsets.size() == static_cast<size_t>(n_seg + 1) &&
                     std::equal(offsets, offsets + n_seg + 1, c->tab_offsets.begin());
   if (!same) {
-    for (int q = 0; q < 5; ++q)
+    for (int q = 0; q < 6; ++q)
       OCP_HIP(c, hipMemcpyAsync(w.tables + q * stride, host.data() + q * (n_seg + 1),
                                 sizeof(int32_t) * (n_seg + 1), hipMemcpyHostToDevice,
                                 c->stream));
@@ -477,10 +480,12 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.tiles_sort = static_cast<int32_t>(ts);
   p.tiles_scan = static_cast<int32_t>(tc);
   p.tiles_node = static_cast<int32_t>(tn);
+  p.tiles_tree = static_cast<int32_t>(ttr);
   p.ts_morton = d_tm;
   p.ts_sort = d_ts;
   p.ts_scan = d_tc;
   p.ts_node = d_tn;
+  p.ts_tree = d_tt;
   *out = p;
   return OCP_OK;
 }
@@ -629,12 +634,12 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
                   p.permutation ? w.vals_b : nullptr); }
   mark(c, 3, capturing);
   { KScope k(c, kKRadixTree, capturing);
-    launch_radix_tree(w.keys_b, w.prefix_n, w.hl, w.hr, w.lc, w.par, w.ppn, p.sv, p.ts_node,
-                      p.tiles_node, n_unique, 0, c->ctrl, s); }
+    launch_radix_pairs(w.keys_b, w.prefix_n, w.hl, w.hr, w.lc, w.par, w.edge, p.sv, p.ts_tree,
+                       p.tiles_tree, tree_tile(p.n_total), n_unique, c->ctrl, s); }
   mark(c, 4, capturing);
   { KScope k(c, kKEdgeScan, capturing);
-    launch_edge_scan(w.prefix_n, w.par, w.ppn, w.edge, w.offs, p.sv, p.ts_scan, p.tiles_scan,
-                     n_unique, 0, w.flags, c->ctrl, kalloc, 0, tt, s); }
+    launch_edge_scan(w.edge, w.offs, p.sv, p.ts_scan, p.tiles_scan, n_unique, 0, w.flags,
+                     c->ctrl, kalloc, tt, s); }
   if (c->order_record && !capturing && c->order_err == hipSuccess)
     c->order_err = hipEventRecord(c->order_record, s);
   mark(c, 5, capturing);
@@ -1079,9 +1084,7 @@ int ocp_k_BuildRadixTree(ocp_ctx c, int32_t n, const uint32_t* codes, uint8_t* p
   if (!codes || !prefix_n || !hl || !hr || !lc || !parent)
     return fail(c, OCP_ERR_INVALID, "null pointer");
   if (n > kMaxPoints) return fail(c, OCP_ERR_CAPACITY, "n > 2^30-1");
-  launch_radix_tree(codes, prefix_n, hl, hr, lc, parent, nullptr, single_view(n + 1, 0.0f, 1.0f),
-                    nullptr, static_cast<int32_t>(cdiv(n, kNodeTile)), nullptr, n, c->ctrl,
-                    c->stream);
+  launch_radix_tree(codes, prefix_n, hl, hr, lc, parent, n, c->ctrl, c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;
 }
@@ -1091,9 +1094,7 @@ int ocp_k_EdgeCount(ocp_ctx c, const uint8_t* prefix_n, const int32_t* parents,
   if (check_ctx(c)) return OCP_ERR_INVALID;
   if (n <= 0) return OCP_OK;
   if (!prefix_n || !parents || !edge_count) return fail(c, OCP_ERR_INVALID, "null pointer");
-  launch_edge_scan(prefix_n, parents, nullptr, edge_count, nullptr, single_view(n, 0.0f, 1.0f),
-                   nullptr, static_cast<int32_t>(cdiv(n, scan_tile(c->tune))), nullptr, n,
-                   nullptr, c->ctrl, nullptr, 1, c->tune, c->stream);
+  launch_edge_count(prefix_n, parents, edge_count, n, c->ctrl, c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;
 }
@@ -1108,10 +1109,8 @@ int ocp_k_PartialSum(ocp_ctx c, const int32_t* data, int64_t first, int64_t last
   const int32_t tiles = static_cast<int32_t>(cdiv(n, scan_tile(c->tune)));
   if (int r = ensure_scratch(c, 2 * int64_t(tiles))) return r;  // tile flags + group sums
   launch_begin(c->ctrl, nullptr, 0, c->stream);
-  launch_edge_scan(nullptr, nullptr, nullptr, const_cast<int32_t*>(data + first), d_first,
-                   single_view(n, 0.0f, 1.0f), nullptr, tiles, nullptr,
-                   static_cast<int32_t>(n), c->s_flags, c->ctrl, nullptr, 2, c->tune,
-                   c->stream);
+  launch_edge_scan(data + first, d_first, single_view(n, 0.0f, 1.0f), nullptr, tiles, nullptr,
+                   static_cast<int32_t>(n), c->s_flags, c->ctrl, nullptr, c->tune, c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;
 }
@@ -1298,7 +1297,7 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
   const int64_t cap = std::max<int64_t>(n, 4096);
   const int64_t seg = std::max<int32_t>(n_seg, 1);
   int64_t b = 2 * 4 * cap          // keys_a, keys_b
-              + 4 * 1 * cap        // prefix_n, hl, hr, parent prefix lengths
+              + 3 * 1 * cap        // prefix_n, hl, hr
               + 4 * 4 * cap        // left child, parent, edge counts, offsets
               + cap * int64_t(sizeof(OctNode)) + 16;  // nodes (K_cap starts at N)
   b += 4 * (seg * (hist_stride(10) + kCursorWords) + 2 * seg + (seg + 1) + 6 * (seg + 1) +

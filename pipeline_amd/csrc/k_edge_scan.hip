@@ -1,123 +1,94 @@
-// Stages 5 + 6: edge count (kernels/05_edge_count.cpp:3-16:
-// e[0] = 0, e[i] = prefix_n[i]/3 - prefix_n[parent[i]]/3) fused with the
-// inclusive scan of kernels/06_partial_sum.cpp:3-15 (the reference GPU path
-// has no scan and round-trips to the host, apps/gpu_demo/main.cu:308-310).
+// Stage 5 (kernels/05_edge_count.cpp:3-16: e[0] = 0, e[i] = prefix_n[i]/3 -
+// prefix_n[parent[i]]/3) for the per-stage entry, and stage 6: the inclusive
+// scan of kernels/06_partial_sum.cpp:3-15 (the reference GPU path has no scan
+// and round-trips to the host, apps/gpu_demo/main.cu:308-310). In the fused
+// build the radix-tree kernel writes the edge counts.
 //
-// Tiles of 256*IPT nodes, one per workgroup, one lookback chain per segment.
-// Each thread handles one node per row of 256 (coalesced loads of prefix_n
-// and, in the fused build, the parent's prefix_n stored by the radix tree;
-// else parent and one gathered byte); rows are scanned with wave64 shuffles,
-// one wave scans the 4*IPT row totals and does the two-level lookback (the
-// tile's group of 64, then the sums of earlier groups). The tiles' maxima of
-// P[i] + e[i] reach the segment's octree slot count with one atomicMax per
-// group of 64 tiles.
-//
-// Modes: 0 = fused, 1 = edge count only, 2 = scan of `edge` only.
+// The scan: tiles of 256*IPT entries, one per workgroup, one lookback chain
+// per segment. A thread takes four consecutive entries per row of 1024 (one
+// 16-byte load and store; the sums of the four are scanned, a quarter of the
+// wave scans of one entry per lane); one wave scans the IPT row totals and
+// does the two-level lookback (the tile's group of 64, then the sums of
+// earlier groups). The tiles' maxima of P[i] + e[i] reach the segment's
+// octree slot count with one atomicMax per group of 64 tiles.
 #include "ocp_internal.hpp"
 
 namespace ocp {
 namespace {
 
+typedef int32_t v4i __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void edge_count_kernel(const uint8_t* __restrict__ prefix_n,
+                                                         const int32_t* __restrict__ parent,
+                                                         int32_t* __restrict__ edge, int32_t n,
+                                                         const uint32_t* __restrict__ ctrl) {
+  if (stopped_any(ctrl)) return;
+  const int32_t i = static_cast<int32_t>(blockIdx.x * 256 + threadIdx.x);
+  if (i >= n) return;
+  int32_t v = 0;
+  if (i > 0)
+    v = static_cast<int32_t>(static_cast<uint32_t>(prefix_n[i]) / 3) -
+        static_cast<int32_t>(static_cast<uint32_t>(prefix_n[parent[i]]) / 3);
+  edge[i] = v;
+}
+
 template <int IPT>
 __global__ __launch_bounds__(256) void edge_scan_kernel(
-    const uint8_t* __restrict__ prefix_all, const int32_t* __restrict__ par_all,
-    const uint8_t* __restrict__ ppn_all, int32_t* __restrict__ edge_all, int32_t* __restrict__ off_all, SegView sv,
-    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ n_unique,
-    int32_t n_brt_host, uint64_t* __restrict__ flags,
-    uint32_t* __restrict__ ctrl, int32_t* __restrict__ kalloc, int mode) {
+    const int32_t* __restrict__ edge_all, int32_t* __restrict__ off_all, SegView sv,
+    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ n_unique, int32_t n_host,
+    uint64_t* __restrict__ flags, uint32_t* __restrict__ ctrl, int32_t* __restrict__ kalloc) {
   constexpr int THREADS = 256;
   constexpr int NW = THREADS / 64;
   constexpr int T = THREADS * IPT;
-  __shared__ uint32_t s_rows[IPT * NW];
+  constexpr int ROWS = IPT / 4;
+  __shared__ uint32_t s_rows[ROWS * NW];
   __shared__ int32_t s_max[NW];
   __shared__ uint32_t s_excl;
 
   const int tid = threadIdx.x;
   const uint32_t w = wave_id();
   const uint32_t lane = lane_id();
-  const bool scan = mode != 1;
   const int32_t t = blockIdx.x;  // in-order dispatch: see lookback_n
   const uint32_t tag = ctrl[kCtrlEpoch] * 8u + kStageScan;
   if (stopped(ctrl, tag)) return;
   const TileRef r = find_tile(tile_start, sv.n_seg, t);
-  const int32_t n = n_unique ? n_unique[r.seg] - 1 : n_brt_host;
+  const int32_t n = n_unique ? n_unique[r.seg] - 1 : n_host;
   const int32_t sb = seg_begin(sv, r.seg);  // loaded with n, before the test
   const int32_t base = r.local * T;
   if (base >= n) return;  // no later tile of this chain waits on it
   const int32_t cnt = min(T, n - base);
-  const uint8_t* pn = prefix_all + sb;
-  int32_t* edge = edge_all + sb;
+  const int32_t* edge = edge_all + sb + base;
+  int32_t* off = off_all + sb + base;
 
-  // Loads first, all in flight together; then the edge counts.
-  int32_t la[IPT];
-  uint32_t lb[IPT];
+  // Loads first, all in flight together (4-byte aligned: a segment or a
+  // caller's range starts anywhere).
+  v4i e[ROWS];
+  if (cnt == T) {
 #pragma unroll
-  for (int k = 0; k < IPT; ++k) {
-    la[k] = 0;
-    lb[k] = 0;
-  }
-  // One loop per source, each a uniform choice, so the loads of a loop are
-  // issued together. The parent's prefix_n is stored beside the node by the
-  // radix tree in the fused build, else gathered through parent[] (never
-  // for node 0, whose edge count is 0).
-  const int32_t i0 = base + tid;
-  if (mode == 2) {
-#pragma unroll
-    for (int k = 0; k < IPT; ++k)
-      if (k * THREADS + tid < cnt) la[k] = edge[i0 + k * THREADS];
-  } else if (ppn_all && cnt == T) {
-#pragma unroll
-    for (int k = 0; k < IPT; ++k) {
-      la[k] = pn[i0 + k * THREADS];
-      lb[k] = ppn_all[sb + i0 + k * THREADS];
-    }
-  } else if (ppn_all) {
-#pragma unroll
-    for (int k = 0; k < IPT; ++k) {
-      if (k * THREADS + tid < cnt) {
-        la[k] = pn[i0 + k * THREADS];
-        lb[k] = ppn_all[sb + i0 + k * THREADS];
-      }
-    }
+    for (int k = 0; k < ROWS; ++k)
+      __builtin_memcpy(&e[k], edge + k * 1024 + tid * 4, 16);
   } else {
-    int32_t par[IPT];
 #pragma unroll
-    for (int k = 0; k < IPT; ++k) {
-      par[k] = 0;
-      if (k * THREADS + tid < cnt) {
-        la[k] = pn[i0 + k * THREADS];
-        if (i0 + k * THREADS > 0) par[k] = par_all[sb + i0 + k * THREADS];
+    for (int k = 0; k < ROWS; ++k) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int32_t idx = k * 1024 + tid * 4 + u;
+        e[k][u] = idx < cnt ? edge[idx] : 0;
       }
     }
-#pragma unroll
-    for (int k = 0; k < IPT; ++k)
-      if (k * THREADS + tid < cnt && i0 + k * THREADS > 0) lb[k] = pn[par[k]];
   }
-  int32_t e[IPT];
+  uint32_t before[ROWS];  // sum of the row's earlier lanes in this wave
 #pragma unroll
-  for (int k = 0; k < IPT; ++k) {
-    const int32_t i = base + k * THREADS + tid;
-    int32_t v = 0;
-    if (k * THREADS + tid < cnt) {
-      if (mode == 2)
-        v = la[k];
-      else if (i > 0)
-        v = static_cast<int32_t>(static_cast<uint32_t>(la[k]) / 3) - static_cast<int32_t>(lb[k] / 3);
-      if (mode != 2) edge[i] = v;
-    }
-    e[k] = v;
-  }
-  if (!scan) return;
-
-  uint32_t incl[IPT];
-#pragma unroll
-  for (int k = 0; k < IPT; ++k) {
-    incl[k] = wave_incl_scan(static_cast<uint32_t>(e[k]));
-    if (lane == 63) s_rows[k * NW + w] = incl[k];
+  for (int k = 0; k < ROWS; ++k) {
+    const uint32_t sum = static_cast<uint32_t>(e[k].x) + static_cast<uint32_t>(e[k].y) +
+                         static_cast<uint32_t>(e[k].z) + static_cast<uint32_t>(e[k].w);
+    const uint32_t incl = wave_incl_scan(sum);
+    before[k] = incl - sum;
+    if (lane == 63) s_rows[k * NW + w] = incl;
   }
   __syncthreads();
   if (w == 0) {
-    const uint32_t total = wave_scan_lds<IPT * NW>(s_rows);
+    const uint32_t total = wave_scan_lds<ROWS * NW>(s_rows);
     if (lane == 0)
       flag_store(&flags[t], flag_pack(tag, kFlagAgg, total));
     bool late = false;
@@ -132,18 +103,32 @@ __global__ __launch_bounds__(256) void edge_scan_kernel(
   }
   __syncthreads();
   const uint32_t excl = s_excl;
-  int32_t* off = off_all + sb;
   int32_t kmax = 1;
-  uint32_t rb[IPT];  // all LDS reads before the stores
+  uint32_t rb[ROWS];  // all LDS reads before the stores
 #pragma unroll
-  for (int k = 0; k < IPT; ++k) rb[k] = s_rows[k * NW + w];
+  for (int k = 0; k < ROWS; ++k) rb[k] = s_rows[k * NW + w];
 #pragma unroll
-  for (int k = 0; k < IPT; ++k) {
-    const int32_t idx = k * THREADS + tid;
-    if (idx < cnt) {
-      const int32_t p = static_cast<int32_t>(excl + rb[k] + incl[k]);
-      off[base + idx] = p;
-      kmax = max(kmax, p + e[k]);
+  for (int k = 0; k < ROWS; ++k) {
+    v4i p;
+    uint32_t run = excl + rb[k] + before[k];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      run += static_cast<uint32_t>(e[k][u]);
+      p[u] = static_cast<int32_t>(run);
+    }
+    const int32_t idx = k * 1024 + tid * 4;
+    if (idx + 4 <= cnt) {
+      __builtin_memcpy(off + idx, &p, 16);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) kmax = max(kmax, p[u] + e[k][u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (idx + u < cnt) {
+          off[idx + u] = p[u];
+          kmax = max(kmax, p[u] + e[k][u]);
+        }
+      }
     }
   }
   if (kalloc) {
@@ -176,31 +161,27 @@ __global__ __launch_bounds__(256) void edge_scan_kernel(
   }
 }
 
-template <int IPT>
-void launch_ipt(const uint8_t* prefix_n, const int32_t* parent, const uint8_t* parent_pn,
-                int32_t* edge, int32_t* offsets, const SegView& sv,
-                const int32_t* tile_start, int32_t total_tiles, const int32_t* n_unique,
-                int32_t n_brt_host, uint64_t* flags, uint32_t* ctrl,
-                int32_t* kalloc, int mode, hipStream_t s) {
-  edge_scan_kernel<IPT><<<total_tiles, 256, 0, s>>>(
-      prefix_n, parent, parent_pn, edge, offsets, sv, tile_start, n_unique, n_brt_host,
-      flags, ctrl, kalloc, mode);
-}
-
 }  // namespace
 
-void launch_edge_scan(const uint8_t* prefix_n, const int32_t* parent,
-                      const uint8_t* parent_pn, int32_t* edge, int32_t* offsets,
-                      const SegView& sv,
-                      const int32_t* tile_start, int32_t total_tiles,
-                      const int32_t* n_unique, int32_t n_brt_host,
-                      uint64_t* flags, uint32_t* ctrl, int32_t* kalloc,
-                      int mode, const TuneTable& tt, hipStream_t s) {
+void launch_edge_count(const uint8_t* prefix_n, const int32_t* parent, int32_t* edge, int32_t n,
+                       const uint32_t* ctrl, hipStream_t s) {
+  if (n <= 0) return;
+  edge_count_kernel<<<(n + 255) / 256, 256, 0, s>>>(prefix_n, parent, edge, n, ctrl);
+}
+
+void launch_edge_scan(const int32_t* edge, int32_t* offsets, const SegView& sv,
+                      const int32_t* tile_start, int32_t total_tiles, const int32_t* n_unique,
+                      int32_t n_host, uint64_t* flags, uint32_t* ctrl, int32_t* kalloc,
+                      const TuneTable& tt, hipStream_t s) {
   if (total_tiles <= 0) return;
+  const auto go = [&](auto kernel) {
+    kernel<<<total_tiles, 256, 0, s>>>(edge, offsets, sv, tile_start, n_unique, n_host, flags,
+                                       ctrl, kalloc);
+  };
   switch (tt.scan_ipt) {
-    case 32: launch_ipt<32>(prefix_n, parent, parent_pn, edge, offsets, sv, tile_start, total_tiles, n_unique, n_brt_host, flags, ctrl, kalloc, mode, s); break;
-    case 8: launch_ipt<8>(prefix_n, parent, parent_pn, edge, offsets, sv, tile_start, total_tiles, n_unique, n_brt_host, flags, ctrl, kalloc, mode, s); break;
-    default: launch_ipt<16>(prefix_n, parent, parent_pn, edge, offsets, sv, tile_start, total_tiles, n_unique, n_brt_host, flags, ctrl, kalloc, mode, s); break;
+    case 32: go(edge_scan_kernel<32>); break;
+    case 8: go(edge_scan_kernel<8>); break;
+    default: go(edge_scan_kernel<16>); break;
   }
 }
 

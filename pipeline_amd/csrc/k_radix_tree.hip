@@ -17,8 +17,12 @@
 // true root split and stores 0 into parent[0] and into the parent entries
 // of the true root's internal children; nodes i >= 1 store plainly. The
 // result equals the sequential reference on zeroed memory without atomics
-// or a zero-fill pass. With the same writes the fused build also stores
-// prefix_n[parent[i]] at parent_pn[i], so the edge count needs no gather.
+// or a zero-fill pass.
+//
+// Two kernels. radix_tree_kernel evaluates the reference's searches as they
+// stand, for any sorted codes a caller passes (repeated ones and codes with
+// bit 31 set included): the per-stage entry. radix_pairs_kernel is the fused
+// build's, whose codes are always strictly increasing 30-bit keys.
 #include "ocp_internal.hpp"
 
 namespace ocp {
@@ -220,24 +224,16 @@ __device__ __forceinline__ bool local_node(const Codes& codes, int32_t i, int32_
 }
 
 __global__ __launch_bounds__(256) void radix_tree_kernel(
-    const uint32_t* __restrict__ codes_all, uint8_t* __restrict__ prefix_all,
-    uint8_t* __restrict__ hl_all, uint8_t* __restrict__ hr_all,
-    int32_t* __restrict__ lc_all, int32_t* __restrict__ par_all,
-    uint8_t* __restrict__ ppn_all, SegView sv,
-    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ n_unique,
-    int32_t n_brt_host, const uint32_t* __restrict__ ctrl) {
+    const uint32_t* __restrict__ codes_g, uint8_t* __restrict__ prefix_n,
+    uint8_t* __restrict__ hl, uint8_t* __restrict__ hr, int32_t* __restrict__ lc,
+    int32_t* __restrict__ parent, int32_t n, const uint32_t* __restrict__ ctrl) {
   static_assert(kLocalMax <= kHalo / 2 + 1, "local searches must stay in the window");
   __shared__ uint32_t s_codes[kNodeTile + 2 * kHalo];
   __shared__ int32_t s_wide[kNodeTile];
   __shared__ uint32_t s_nwide;
-  const TileRef r = find_tile(tile_start, sv.n_seg, xcd_tile(blockIdx.x, gridDim.x));
-  const int32_t n = n_unique ? n_unique[r.seg] - 1 : n_brt_host;
-  const int32_t sb = seg_begin(sv, r.seg);  // loaded with n, before the test
-  const int32_t i0 = r.local * kNodeTile;
+  const int32_t i0 = xcd_tile(blockIdx.x, gridDim.x) * kNodeTile;
   // After a lookback time-out the unique keys are not valid input.
   if (i0 >= n || (ctrl && stopped_any(ctrl))) return;
-  int32_t* parent = par_all + sb;
-  uint8_t* parent_pn = ppn_all ? ppn_all + sb : nullptr;
   if (threadIdx.x == 0) s_nwide = 0;
   // Stage codes [i0 - halo, i0 + kNodeTile + halo) of the n+1 codes.
   const int32_t lo = max(0, i0 - kHalo);
@@ -246,7 +242,7 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
     // every load of the window in flight at once
     constexpr int kRows = (kNodeTile + 2 * kHalo + 255) / 256;
     uint32_t rc[kRows];
-    const uint32_t* src = codes_all + sb + lo + static_cast<int32_t>(threadIdx.x);
+    const uint32_t* src = codes_g + lo + static_cast<int32_t>(threadIdx.x);
     if (hi - lo == kRows * 256) {  // a full window: no per-load guard
 #pragma unroll
       for (int k = 0; k < kRows; ++k) rc[k] = src[k * 256];
@@ -262,22 +258,18 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
     }
   }
   __syncthreads();
-  const Codes codes{codes_all + sb, as_lds<const uint32_t>(s_codes), lo, hi - lo};
+  const Codes codes{codes_g, as_lds<const uint32_t>(s_codes), lo, hi - lo};
 
   auto emit = [&](int32_t node, uint32_t delta_node, int32_t gamma, int32_t j) {
     const bool leaf_l = min(node, j) == gamma;
     const bool leaf_r = max(node, j) == gamma + 1;
-    prefix_all[sb + node] = static_cast<uint8_t>(delta_node);
-    hl_all[sb + node] = leaf_l;
-    hr_all[sb + node] = leaf_r;
-    lc_all[sb + node] = gamma;
+    prefix_n[node] = static_cast<uint8_t>(delta_node);
+    hl[node] = leaf_l;
+    hr[node] = leaf_r;
+    lc[node] = gamma;
     if (node > 0) {
       if (!leaf_l) parent[gamma] = node;
       if (!leaf_r) parent[gamma + 1] = node;
-      if (parent_pn) {
-        if (!leaf_l) parent_pn[gamma] = static_cast<uint8_t>(delta_node);
-        if (!leaf_r) parent_pn[gamma + 1] = static_cast<uint8_t>(delta_node);
-      }
     }
   };
 
@@ -321,30 +313,355 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
         parent[0] = 0;
         if (g0 != 0 && g0 < n) parent[g0] = 0;
         if (g0 + 1 != n && g0 + 1 < n) parent[g0 + 1] = 0;
-        if (parent_pn) {
-          const uint8_t pn0 = static_cast<uint8_t>(o.delta_node);
-          parent_pn[0] = pn0;
-          if (g0 != 0 && g0 < n) parent_pn[g0] = pn0;
-          if (g0 + 1 != n && g0 + 1 < n) parent_pn[g0 + 1] = pn0;
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------- fused build
+// The fused build's keys are strictly increasing 30-bit codes, and there the
+// tree is the Cartesian tree of the adjacent pairs: with b_k = clz(c_k ^
+// c_(k+1)) (the pair's common prefix, plus two), the internal node that splits
+// between keys k and k+1 spans the pairs around k up to the nearest smaller b
+// on either side, L < k < R, so the keys L+1 .. R (two equal values always
+// have a smaller one between them). Its parent is the pair at whichever end
+// holds the larger b; the reference's index for the node is L+1 when that is
+// L (a right child starts its range) and R otherwise. Everything the stage
+// writes follows: prefix_n = b_k - 1, left_child = k, the leaf flags from
+// L+1 == k and R == k+1, the children's parents (nodes k and k+1), and also
+// the edge count of stage 5 (kernels/05_edge_count.cpp:3-16), for the parent's
+// prefix length is max(b_L, b_R) - 1.
+//
+// The pairs' b values of a tile and its halo lie in LDS as bytes, with the
+// minima of 16 and of 256 of them: three levels of 16-byte rows. One row is
+// compared with b_k by four byte-wise subtractions whose top bits four dot
+// products collect into a 16-bit mask; the mask of the pair's own row gives
+// the nearest smaller value on both sides, else the row of row minima names
+// the row to look into, else that of the 256-pair minima. Values outside the
+// segment are 0, below any pair's. An end beyond the window is searched by
+// the wave in the codes themselves, 64 candidates a round trip.
+//
+// Results leave by node index: the records of a tile's own indices through
+// LDS and then as 4-node stores; the others, whose node index lies in another
+// tile, one by one. Every index has one pair, so no entry is stored twice.
+//
+// Node 0 is the reference's short root (see the top of this file): its record
+// comes from its own search, the true root's pair only links its children, and
+// those count their edges from node 0's prefix length.
+//
+// What bounds it: vector instructions, about half of the ~370 per 64 nodes
+// that the searches by code of the kernel above issue. 10M uniform points:
+// 99 -> 66 us, and the edge scan, which reads the counts instead of forming
+// them from two byte arrays, 33 -> 26 us; 2^24 clustered points: 155 -> 99 us
+// and 17 -> 14 us. Tiles of 2048 with a halo of 256, 512 or 1024 pairs: 66.0,
+// 66.4, 68.1 us (98, 99, 101 us clustered).
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef int32_t v4i __attribute__((ext_vector_type(4)));
+typedef uint16_t v2h __attribute__((ext_vector_type(2)));
+
+// Bit p of the result: byte p of the row is below t, where key = t + 127 in
+// every byte (bytes and t at most 31, so no byte borrows from its neighbour).
+__device__ __forceinline__ uint32_t below16(const v4u w, uint32_t key) {
+  const uint32_t hi = 0x80808080u;
+  const uint32_t a = __builtin_amdgcn_udot4(
+      (key - w.y) & hi, 0x80402010u,
+      __builtin_amdgcn_udot4((key - w.x) & hi, 0x08040201u, 0u, false), false);
+  const uint32_t b = __builtin_amdgcn_udot4(
+      (key - w.w) & hi, 0x80402010u,
+      __builtin_amdgcn_udot4((key - w.z) & hi, 0x08040201u, 0u, false), false);
+  return (a >> 7) | (b << 1);
+}
+__device__ __forceinline__ v2h as_halves(uint32_t x) { return __builtin_bit_cast(v2h, x); }
+__device__ __forceinline__ uint32_t min16(const v4u w) {
+  v2h m = as_halves(w.x & 0x00ff00ffu);
+  m = __builtin_elementwise_min(m, as_halves((w.x >> 8) & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves(w.y & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves((w.y >> 8) & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves(w.z & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves((w.z >> 8) & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves(w.w & 0x00ff00ffu));
+  m = __builtin_elementwise_min(m, as_halves((w.w >> 8) & 0x00ff00ffu));
+  return min(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y));
+}
+__device__ __forceinline__ uint32_t third(uint32_t x) { return (x * 11u) >> 5; }  // x / 3, x < 32
+
+// The end of the run of keys around key `from` whose xor with code c is below
+// lim, at least `reach` keys away on the side of d (+1, -1), in [0, m].
+__device__ __forceinline__ int32_t wave_run_end(const uint32_t* __restrict__ codes, uint32_t c,
+                                                uint32_t lim, int32_t from, int32_t d, int32_t m) {
+  const int32_t room = d > 0 ? m - from : from;  // steps that stay in [0, m]
+  const auto in_run = [&](int32_t x) { return (codes[from + x * d] ^ c) < lim; };
+  const int32_t lane = static_cast<int32_t>(lane_id());
+  bool ok = false;
+  if (lane < 30) {
+    const int32_t x = 1 << lane;
+    ok = x <= room && in_run(x);
+  }
+  const int32_t n = __popcll(__ballot(ok));
+  return from + d * wave_max_true(n ? 1 << (n - 1) : 0, min(1 << n, room + 1), in_run);
+}
+
+template <int T, int HALO>
+__global__ __launch_bounds__(256) void radix_pairs_kernel(
+    const uint32_t* __restrict__ codes_all, uint8_t* __restrict__ prefix_all,
+    uint8_t* __restrict__ hl_all, uint8_t* __restrict__ hr_all, int32_t* __restrict__ lc_all,
+    int32_t* __restrict__ par_all, int32_t* __restrict__ edge_all, SegView sv,
+    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ n_unique,
+    const uint32_t* __restrict__ ctrl) {
+  constexpr int W = T + 2 * HALO;
+  constexpr int ROWS = W / 256;
+  static_assert(T % 512 == 0 && T <= 2048 && W % 256 == 0 && W <= 4096, "three levels of 16");
+  __shared__ v4u s_b[W / 16];    // b of the window's pairs, a byte each
+  __shared__ v4u s_b16[16];      // minima of 16
+  __shared__ v4u s_b256;         // minima of 256
+  __shared__ uint32_t s_rec[T];  // records of the tile's node indices
+  __shared__ int32_t s_par[T];
+  constexpr uint32_t kNone = 0xffffffffu;
+
+  const TileRef r = find_tile(tile_start, sv.n_seg, xcd_tile(blockIdx.x, gridDim.x));
+  const int32_t m = n_unique[r.seg] - 1;  // pairs 0 .. m-1 between keys 0 .. m
+  const int32_t sb = seg_begin(sv, r.seg);
+  const int32_t i0 = r.local * T;
+  // After a lookback time-out the unique keys are not valid input.
+  if (i0 >= m || stopped_any(ctrl)) return;
+  const uint32_t* codes = codes_all + sb;
+  uint8_t* prefix = prefix_all + sb;
+  uint8_t* hl = hl_all + sb;
+  uint8_t* hr = hr_all + sb;
+  int32_t* lc = lc_all + sb;
+  int32_t* par = par_all + sb;
+  int32_t* edge = edge_all + sb;
+  const int tid = threadIdx.x;
+  const int32_t wb = i0 - HALO;
+  const uint32_t code_0 = codes[0], code_m = codes[m], code_l = codes[m - 1];
+
+  {
+    // every load of the window in flight at once
+    uint32_t a[ROWS], c[ROWS];
+    if (wb >= 0 && wb + W <= m) {
+      const uint32_t* src = codes + wb + tid;
+#pragma unroll
+      for (int k = 0; k < ROWS; ++k) {
+        a[k] = src[k * 256];
+        c[k] = src[k * 256 + 1];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < ROWS; ++k) {
+        const int32_t g = wb + tid + k * 256;
+        a[k] = 0u;
+        c[k] = 0x80000000u;  // clz 0: outside the segment
+        if (g >= 0 && g < m) {
+          a[k] = codes[g];
+          c[k] = codes[g + 1];
         }
       }
+    }
+    uint8_t* b = reinterpret_cast<uint8_t*>(s_b);
+#pragma unroll
+    for (int k = 0; k < ROWS; ++k)
+      b[tid + k * 256] = static_cast<uint8_t>(__clz(static_cast<int>(a[k] ^ c[k])));
+    for (int k = tid; k < T; k += 256) {
+      s_rec[k] = kNone;
+      s_par[k] = -1;
+    }
+  }
+  __syncthreads();
+  reinterpret_cast<uint8_t*>(s_b16)[tid] =
+      static_cast<uint8_t>(tid < W / 16 ? min16(s_b[tid]) : 31u);
+  __syncthreads();
+  if (tid < 16) reinterpret_cast<uint8_t*>(&s_b256)[tid] = static_cast<uint8_t>(min16(s_b16[tid]));
+  __syncthreads();
+
+  const uint32_t b_root = static_cast<uint32_t>(__clz(static_cast<int>(code_0 ^ code_m)));
+  const uint32_t pn_0 = delta(code_0, code_l);  // node 0's prefix length
+  const uint8_t* b8 = reinterpret_cast<const uint8_t*>(s_b);
+  const v4u row256 = s_b256;
+
+  for (int k = 0; k < T / 256; ++k) {
+    const int32_t p = k * 256 + tid;  // position in the tile
+    const int32_t g = i0 + p;         // the pair
+    const bool live = g < m;
+    const uint32_t q = static_cast<uint32_t>(p + HALO);
+    const uint32_t b = b8[q];
+    // (b + 127 in every byte; a dead lane's b of 0 finds nothing)
+    const uint32_t key = __builtin_amdgcn_perm(0u, b + 127u, 0u);
+    const uint32_t row = q >> 4, grp = q >> 8;
+    const uint32_t m0 = below16(s_b[row], key);
+    const uint32_t m1 = below16(s_b16[grp], key);
+    const uint32_t m2 = below16(row256, key);
+    int32_t end_l = -2, end_r = -2;  // window positions of L and R, -2: not in the window
+    uint32_t hit = m0 & (0xfffeu << (q & 15u)) & 0xffffu;
+    uint32_t at = row;
+    if (hit == 0) {
+      uint32_t gg = grp;
+      uint32_t rr = m1 & (0xfffeu << (row & 15u)) & 0xffffu;
+      if (rr == 0) {
+        const uint32_t g2 = m2 & (0xfffeu << grp) & 0xffffu;
+        if (g2) {
+          gg = static_cast<uint32_t>(__builtin_ctz(g2));
+          rr = below16(s_b16[gg], key);
+        }
+      }
+      if (rr) {
+        at = gg * 16u + static_cast<uint32_t>(__builtin_ctz(rr));
+        hit = below16(s_b[at], key);
+      }
+    }
+    if (hit) end_r = static_cast<int32_t>(at * 16u + static_cast<uint32_t>(__builtin_ctz(hit)));
+    hit = m0 & ((1u << (q & 15u)) - 1u);
+    at = row;
+    if (hit == 0) {
+      uint32_t gg = grp;
+      uint32_t rr = m1 & ((1u << (row & 15u)) - 1u);
+      if (rr == 0) {
+        const uint32_t g2 = m2 & ((1u << grp) - 1u);
+        if (g2) {
+          gg = 31u - static_cast<uint32_t>(__clz(static_cast<int>(g2)));
+          rr = below16(s_b16[gg], key);
+        }
+      }
+      if (rr) {
+        at = gg * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(rr)));
+        hit = below16(s_b[at], key);
+      }
+    }
+    if (hit) end_l = static_cast<int32_t>(at * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(hit))));
+    uint32_t b_l = end_l >= 0 ? b8[end_l] : 0u;
+    uint32_t b_r = end_r >= 0 ? b8[end_r] : 0u;
+    int32_t pl = wb + end_l, pr = wb + end_r;  // the pairs L and R
+    // Ends beyond the window, one at a time by the whole wave. The window's
+    // last key (first key) is then still in the run.
+    for (uint64_t far = __ballot(live && end_r < 0); far; far &= far - 1) {
+      const int src = __builtin_ctzll(far);
+      const int32_t gs = __builtin_amdgcn_readlane(g, src);
+      const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
+      const int32_t j = wave_run_end(codes, codes[gs + 1], lim, wb + W, 1, m);
+      const uint32_t bj = j < m ? clz32(codes[j] ^ codes[j + 1]) : 0u;
+      if (static_cast<int>(lane_id()) == src) {
+        pr = j;
+        b_r = bj;
+      }
+    }
+    for (uint64_t far = __ballot(live && end_l < 0); far; far &= far - 1) {
+      const int src = __builtin_ctzll(far);
+      const int32_t gs = __builtin_amdgcn_readlane(g, src);
+      const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
+      const int32_t j = wave_run_end(codes, codes[gs], lim, wb, -1, m);
+      const uint32_t bj = j > 0 ? clz32(codes[j - 1] ^ codes[j]) : 0u;
+      if (static_cast<int>(lane_id()) == src) {
+        pl = j - 1;
+        b_l = bj;
+      }
+    }
+    if (live) {
+      const uint32_t b_up = max(b_l, b_r);
+      const int32_t node = b_l >= b_r ? pl + 1 : pr;
+      const bool leaf_l = pl + 1 == g;
+      const bool leaf_r = pr == g + 1;
+      const uint32_t pn = b - 1u;
+      const int32_t e = static_cast<int32_t>(third(pn)) -
+                        static_cast<int32_t>(third(b_up == b_root ? pn_0 : b_up - 1u));
+      const uint32_t rec = static_cast<uint32_t>(p) | (pn << 11) | (leaf_l ? 1u << 16 : 0u) |
+                           (leaf_r ? 1u << 17 : 0u) | (static_cast<uint32_t>(e + 16) << 18);
+      const int32_t rel = node - i0;
+      if (b_up == 0) {
+        // the true root: node 0's record is written below
+      } else if (static_cast<uint32_t>(rel) < static_cast<uint32_t>(T)) {
+        s_rec[rel] = rec;
+      } else {
+        prefix[node] = static_cast<uint8_t>(pn);
+        hl[node] = leaf_l;
+        hr[node] = leaf_r;
+        lc[node] = g;
+        edge[node] = e;
+      }
+      if (!leaf_l) s_par[p] = node;
+      if (!leaf_r) {
+        if (p + 1 < T) s_par[p + 1] = node;
+        else par[g + 1] = node;
+      }
+    }
+  }
+  __syncthreads();
+
+  for (int v = tid; v < T / 4; v += 256) {
+    const v4u x = reinterpret_cast<const v4u*>(s_rec)[v];
+    const int32_t n0 = i0 + 4 * v;
+    const auto bytes = [&](uint32_t shift, uint32_t mask) {
+      return ((x.x >> shift) & mask) | (((x.y >> shift) & mask) << 8) |
+             (((x.z >> shift) & mask) << 16) | (((x.w >> shift) & mask) << 24);
+    };
+    if (max(max(x.x, x.y), max(x.z, x.w)) != kNone) {
+      const uint32_t w_pn = bytes(11, 31u), w_hl = bytes(16, 1u), w_hr = bytes(17, 1u);
+      const v4u w_lc = (x & 2047u) + static_cast<uint32_t>(i0);
+      const v4u w_e = ((x >> 18) & 63u) - 16u;
+      __builtin_memcpy(prefix + n0, &w_pn, 4);
+      __builtin_memcpy(hl + n0, &w_hl, 4);
+      __builtin_memcpy(hr + n0, &w_hr, 4);
+      __builtin_memcpy(lc + n0, &w_lc, 16);
+      __builtin_memcpy(edge + n0, &w_e, 16);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t y = x[u];
+        if (y == kNone) continue;
+        prefix[n0 + u] = static_cast<uint8_t>((y >> 11) & 31u);
+        hl[n0 + u] = static_cast<uint8_t>((y >> 16) & 1u);
+        hr[n0 + u] = static_cast<uint8_t>((y >> 17) & 1u);
+        lc[n0 + u] = i0 + static_cast<int32_t>(y & 2047u);
+        edge[n0 + u] = static_cast<int32_t>((y >> 18) & 63u) - 16;
+      }
+    }
+    const v4i w_par = reinterpret_cast<const v4i*>(s_par)[v];
+    if (min(min(w_par.x, w_par.y), min(w_par.z, w_par.w)) >= 0) {
+      __builtin_memcpy(par + n0, &w_par, 16);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (w_par[u] >= 0) par[n0 + u] = w_par[u];
+    }
+  }
+  if (i0 == 0 && wave_id() == 0) {
+    // Node 0: the range [0, m - 1] and its split (04_radix_tree.cpp:63-65,
+    // 94-104): the largest s < m - 1 with a longer common prefix than pn_0.
+    const int32_t s = m < 2 ? 0 : wave_max_true(0, m - 1, [&](int32_t x) {
+      return delta(code_0, codes[x]) > pn_0;
+    });
+    if (lane_id() == 0) {
+      prefix[0] = static_cast<uint8_t>(pn_0);
+      hl[0] = s == 0;
+      hr[0] = s + 1 == m - 1;
+      lc[0] = s;
+      par[0] = 0;
+      edge[0] = 0;
     }
   }
 }
 
 }  // namespace
 
-void launch_radix_tree(const uint32_t* codes, uint8_t* prefix_n,
-                       uint8_t* has_leaf_left, uint8_t* has_leaf_right,
-                       int32_t* left_child, int32_t* parent, uint8_t* parent_pn,
-                       const SegView& sv, const int32_t* tile_start, int32_t total_tiles,
-                       const int32_t* n_unique, int32_t n_brt_host,
+void launch_radix_tree(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_leaf_left,
+                       uint8_t* has_leaf_right, int32_t* left_child, int32_t* parent, int32_t n,
                        const uint32_t* ctrl, hipStream_t s) {
-  if (total_tiles <= 0) return;
+  if (n <= 0) return;
   static_assert(kNodeTile % 256 == 0, "whole node rows per thread");
-  radix_tree_kernel<<<total_tiles, 256, 0, s>>>(
-      codes, prefix_n, has_leaf_left, has_leaf_right, left_child, parent, parent_pn, sv,
-      tile_start, n_unique, n_brt_host, ctrl);
+  radix_tree_kernel<<<(n + kNodeTile - 1) / kNodeTile, 256, 0, s>>>(
+      codes, prefix_n, has_leaf_left, has_leaf_right, left_child, parent, n, ctrl);
+}
+
+void launch_radix_pairs(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_leaf_left,
+                        uint8_t* has_leaf_right, int32_t* left_child, int32_t* parent,
+                        int32_t* edge, const SegView& sv, const int32_t* tile_start,
+                        int32_t total_tiles, int tile, const int32_t* n_unique,
+                        const uint32_t* ctrl, hipStream_t s) {
+  if (total_tiles <= 0) return;
+  const auto go = [&](auto kernel) {
+    kernel<<<total_tiles, 256, 0, s>>>(codes, prefix_n, has_leaf_left, has_leaf_right, left_child,
+                                       parent, edge, sv, tile_start, n_unique, ctrl);
+  };
+  if (tile == 2048) go(radix_pairs_kernel<2048, 512>);
+  else go(radix_pairs_kernel<512, 512>);
 }
 
 }  // namespace ocp

@@ -213,29 +213,35 @@ void launch_unique(const uint32_t* in, uint32_t* out, const SegView& sv,
                    const uint32_t* vin = nullptr, uint32_t* vout = nullptr);
 
 // ---- stage 4 (k_radix_tree.hip)
-// n_brt: per-segment node counts; when n_unique != nullptr the count of
-// segment k is n_unique[k]-1, else n_brt_host (single segment).
-// parent_pn (optional): prefix_n[parent[i]] at i, written with parent[].
+// The per-stage entry: n nodes over n + 1 sorted codes of any value.
 // ctrl (optional): the kernel does nothing once a lookback wait gave up.
-void launch_radix_tree(const uint32_t* codes, uint8_t* prefix_n,
-                       uint8_t* has_leaf_left, uint8_t* has_leaf_right,
-                       int32_t* left_child, int32_t* parent, uint8_t* parent_pn,
-                       const SegView& sv,
-                       const int32_t* tile_start, int32_t total_tiles,
-                       const int32_t* n_unique, int32_t n_brt_host,
+void launch_radix_tree(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_leaf_left,
+                       uint8_t* has_leaf_right, int32_t* left_child, int32_t* parent, int32_t n,
                        const uint32_t* ctrl, hipStream_t s);
+// The fused build: segments of strictly increasing 30-bit codes, n_unique[k]
+// of them in segment k; writes the edge counts of stage 5 as well. Tiles of
+// `tile` = tree_tile(...) nodes per the tile map.
+void launch_radix_pairs(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_leaf_left,
+                        uint8_t* has_leaf_right, int32_t* left_child, int32_t* parent,
+                        int32_t* edge, const SegView& sv, const int32_t* tile_start,
+                        int32_t total_tiles, int tile, const int32_t* n_unique,
+                        const uint32_t* ctrl, hipStream_t s);
+// Nodes per tile of launch_radix_pairs for a build of n points: 2048 once
+// that still gives every CU several workgroups (10M points: 66 us against 74
+// with 512), 512 below (2^20 points: 16.4 us against 19.6).
+inline int tree_tile(int64_t n) { return n >= (int64_t(1) << 21) ? 2048 : 512; }
 
 // ---- stages 5 + 6 (k_edge_scan.hip)
-// mode 0: edge count + inclusive scan fused; 1: edge count only;
-// 2: inclusive scan of `edge` only.
-// parent_pn (optional, fused build): used instead of prefix_n[parent[i]].
-void launch_edge_scan(const uint8_t* prefix_n, const int32_t* parent,
-                      const uint8_t* parent_pn, int32_t* edge, int32_t* offsets,
-                      const SegView& sv,
-                      const int32_t* tile_start, int32_t total_tiles,
-                      const int32_t* n_unique, int32_t n_brt_host,
-                      uint64_t* flags, uint32_t* ctrl, int32_t* kalloc,
-                      int mode, const TuneTable& tt, hipStream_t s);
+// Edge count of one segment of n nodes (the per-stage entry).
+void launch_edge_count(const uint8_t* prefix_n, const int32_t* parent, int32_t* edge, int32_t n,
+                       const uint32_t* ctrl, hipStream_t s);
+// Inclusive scan of `edge` per segment, one lookback chain each. With
+// n_unique, segment k has n_unique[k] - 1 entries and its octree slot count,
+// max(1, max P[i] + e[i]), is folded into kalloc[k]; else n_host entries.
+void launch_edge_scan(const int32_t* edge, int32_t* offsets, const SegView& sv,
+                      const int32_t* tile_start, int32_t total_tiles, const int32_t* n_unique,
+                      int32_t n_host, uint64_t* flags, uint32_t* ctrl, int32_t* kalloc,
+                      const TuneTable& tt, hipStream_t s);
 
 // ---- stage 7 (k_octree.hip)
 struct OctArgs {
