@@ -427,9 +427,8 @@ typedef struct ocp_tune {
                            10 (three passes over the 30-bit keys; builds with
                            the permutation keep 8) */
   int32_t sort10_kpt;   /* keys per thread of a 10-bit pass (8 or 16) */
-  int32_t oct_order;    /* octree work order in a tile: 0 chains by index,
-                           1 by the size of their group walk (faster on
-                           clustered clouds) */
+  int32_t oct_order;    /* 0 or 1, kept for saved tables: one octree kernel
+                           serves both */
   int32_t sort_msd;     /* with sort_bits 10: 0 three LSD passes; 1 one
                            scatter by the top 10-bit digit, then each bucket
                            sorted in LDS by one workgroup; a build with a

@@ -376,7 +376,7 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
   p.tiles_morton = static_cast<int32_t>(cdiv(n, morton_tile(tt)));
   p.tiles_sort = static_cast<int32_t>(cdiv(n, pipe_sort_tile(tt, perm)));
   p.tiles_scan = static_cast<int32_t>(cdiv(n, scan_tile(tt)));
-  p.tiles_node = static_cast<int32_t>(cdiv(n, kNodeTile));
+  p.tiles_node = static_cast<int32_t>(cdiv(n, kOctTile));
   p.tiles_tree = static_cast<int32_t>(cdiv(n, tree_tile(n)));
   return p;
 }
@@ -439,7 +439,7 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
       tm += cdiv(len, morton_tile(tt));
       ts += cdiv(len, stile);
       tc += cdiv(len, scan_tile(tt));
-      tn += cdiv(len, kNodeTile);
+      tn += cdiv(len, kOctTile);
       ttr += cdiv(len, tree_tile(n));
     }
   }
@@ -539,7 +539,7 @@ bool enqueue_octree(ocp_ctx c, const Plan& p, bool capturing) {
     launch_oct_offsets(kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, s); }
   const OctArgs a = pipeline_oct_args(c);
   KScope k(c, kKOctBuild, capturing);
-  return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, c->tune.oct_order != 0, s);
+  return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, s);
 }
 
 void mark(ocp_ctx c, int k, bool capturing) {
@@ -1690,11 +1690,6 @@ int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
         t.morton_grid = grid;
         if (int r = try_cfg(t)) return r;
       }
-    }
-    for (int order : {0, 1}) {
-      ocp_tune t = best;
-      t.oct_order = order;
-      if (int r = try_cfg(t)) return r;
     }
     if (std::memcmp(&start, &best, sizeof(best)) == 0) break;
   }

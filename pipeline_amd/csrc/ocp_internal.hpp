@@ -68,7 +68,7 @@ struct TuneTable {
   int scan_ipt = 16;       // items per thread in unique / edge-scan tiles
   int sort_bits = 8;       // digit width of a build's sort: 8 (4 passes) or 10 (3)
   int sort10_kpt = 8;      // keys per thread of a 10-bit pass (16 waves)
-  int oct_order = 0;       // octree chains in index order (0) or by group size (1)
+  int oct_order = 0;       // 0 or 1, kept for saved tables: one octree kernel serves both
   int sort_msd = 0;        // 10-bit digits: LSD passes (0) or MSD scatter + LDS buckets (1)
 };
 
@@ -92,7 +92,8 @@ inline int pipe_sort_tile(const TuneTable& t, bool perm) {
 constexpr int hist_stride(int bits) { return bits == 10 ? 3 * 1024 : 4 * 256; }
 inline int morton_tile(const TuneTable& t) { return 256 * t.morton_ppt; }
 inline int scan_tile(const TuneTable& t) { return 256 * t.scan_ipt; }
-constexpr int kNodeTile = 256;  // BRT nodes per radix-tree / octree tile
+constexpr int kNodeTile = 256;  // BRT nodes per tile of the per-stage entries
+constexpr int kOctTile = 512;   // ... of the fused build's octree kernel
 
 bool sort_config_supported(int waves, int kpt);
 bool sort10_config_supported(int kpt);
@@ -268,8 +269,7 @@ void launch_oct_root(OctNode* nodes, const uint32_t* codes,
 // Needs every OctArgs array (the fused build has them all); returns false
 // (and launches nothing) when an array it needs is null.
 bool launch_oct_build(const OctArgs& a, const SegView& sv,
-                      const int32_t* tile_start, int32_t total_tiles, bool by_group,
-                      hipStream_t s);
+                      const int32_t* tile_start, int32_t total_tiles, hipStream_t s);
 
 // ---- stage 7, per-stage entry points (k_octree_stage.hip)
 // The make call of the reference signature has no children arrays

@@ -1,7 +1,8 @@
-"""The fused build's radix tree at the edges of its tiles (512 nodes below
-2^21 points, 2048 from there): segment ends at, before and after a tile end
-and a window end, and codes whose nodes reach past the window, all stage
-outputs against the oracle."""
+"""The fused build's radix tree and octree at the edges of their tiles (tree:
+512 nodes below 2^21 points, 2048 from there; octree: 512): segment ends at,
+before and after a tile end and a window end, codes whose nodes reach past the
+window, and tiles with more octree slots than the kernel keeps at once, all
+stage outputs against the oracle."""
 import numpy as np
 import pytest
 
@@ -43,6 +44,18 @@ def test_tile_rule(ctx, n):
                            rng.integers(0, 1 << 30, n - n // 2)])
     pts = _cells(rng.permutation(keys))
     _check_segment(_plain(ctx, pts), 0, oracle.build_plain(pts))
+
+
+@pytest.mark.parametrize("pairs,gap", [(40, 1 << 24), (700, 1 << 20), (5000, 1 << 17)])
+def test_long_chains(ctx, pairs, gap):
+    """Sibling pairs far apart: chains of up to nine slots, so a tile of 512
+    nodes has several times the 320 slots of a round, and chains that start in
+    one tile and cover slots of the next."""
+    base = np.arange(pairs) * gap
+    for extra in ([], [1 << 29], [(1 << 30) - 1]):
+        keys = np.unique(np.concatenate([base, base + 1, np.asarray(extra, np.int64)]))
+        pts = _cells(keys[keys < (1 << 30)])
+        _check_segment(_plain(ctx, pts), 0, oracle.build_plain(pts))
 
 
 def test_batched_odd_starts(ctx):
