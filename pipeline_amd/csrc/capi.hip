@@ -183,6 +183,11 @@ struct ocp_context {
   int tab_tune_key = -1;
   bool have_result = false;
   Plan last_plan;
+  // Pinned host memory: what the last build's offsets kernel reports (see
+  // launch_oct_offsets), then a landing place for small copies back. Current
+  // while no other work that can time out was enqueued after that build.
+  uint32_t* mail = nullptr;
+  bool mail_current = false;
   bool graph_mode = false;
   bool permutation = false;
   // Streaming: the first lookback launch of a build waits for order_wait,
@@ -242,7 +247,10 @@ void clear_graphs(ocp_ctx c) {
   c->graphs.clear();
 }
 
+// For the per-stage entries and sorts: scratch for their waits, whose
+// time-outs the last build's mail does not know.
 int ensure_scratch(ocp_ctx c, int64_t flag_words) {
+  c->mail_current = false;
   if (flag_words > c->s_flag_cap) {
     dev_free(c->s_flags);
     const int64_t cap = std::max<int64_t>(flag_words, 1 << 16);
@@ -536,7 +544,7 @@ bool enqueue_octree(ocp_ctx c, const Plan& p, bool capturing) {
   hipStream_t s = c->stream;
   int32_t* kalloc = w.counts + w.seg_cap;
   { KScope k(c, kKOctOffsets, capturing);
-    launch_oct_offsets(kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, s); }
+    launch_oct_offsets(w.counts, kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, c->mail, s); }
   const OctArgs a = pipeline_oct_args(c);
   KScope k(c, kKOctBuild, capturing);
   return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, s);
@@ -667,6 +675,7 @@ std::string graph_key(const char* kind, const float* pts, int f3, int64_t n,
 int run_plan(ocp_ctx c, const float* pts, int f3, const Plan& p,
              const std::string& key_in) {
   const std::string key = key_in + (p.permutation ? "|perm" : "");
+  c->mail_current = false;
   if (c->graph_mode) {
     auto it = c->graphs.find(key);
     if (it == c->graphs.end()) {
@@ -702,6 +711,7 @@ int run_plan(ocp_ctx c, const float* pts, int f3, const Plan& p,
   }
   c->last_plan = p;
   c->have_result = true;
+  c->mail_current = true;
   return OCP_OK;
 }
 
@@ -712,6 +722,7 @@ int run_plan(ocp_ctx c, const float* pts, int f3, const Plan& p,
 int report_timeout(ocp_ctx c, const uint32_t* hc) {
   if (hc[kCtrlTimeout] == 0) return OCP_OK;
   c->have_result = false;
+  c->mail_current = false;
   launch_fill_u32(c->ctrl + kCtrlTimeout, 0u, 1, c->stream);
   OCP_CHECK_LAUNCH(c);
   OCP_HIP(c, hipStreamSynchronize(c->stream));
@@ -720,11 +731,23 @@ int report_timeout(ocp_ctx c, const uint32_t* hc) {
               "enqueued since the last check is invalid");
 }
 
+// Waits for the stream. *words: the control words as of then, where the
+// build's mail is not current by a copy to the words after it.
+int sync_ctrl(ocp_ctx c, const uint32_t** words) {
+  *words = c->mail;
+  if (!c->mail_current) {
+    *words = c->mail + kMailWords;
+    OCP_HIP(c, hipMemcpyAsync(c->mail + kMailWords, c->ctrl, sizeof(uint32_t) * kCtrlWords,
+                              hipMemcpyDeviceToHost, c->stream));
+  }
+  OCP_HIP(c, hipStreamSynchronize(c->stream));
+  return OCP_OK;
+}
+
 // Synchronises the stream and reports a wait that gave up.
 int sync_and_check(ocp_ctx c) {
-  uint32_t hc[kCtrlWords];
-  OCP_HIP(c, hipMemcpyAsync(hc, c->ctrl, sizeof(hc), hipMemcpyDeviceToHost, c->stream));
-  OCP_HIP(c, hipStreamSynchronize(c->stream));
+  const uint32_t* hc = nullptr;
+  if (int r = sync_ctrl(c, &hc)) return r;
   return report_timeout(c, hc);
 }
 
@@ -732,9 +755,8 @@ int sync_and_check(ocp_ctx c) {
 // stage 7 (its inputs are intact). Synchronises.
 int settle(ocp_ctx c) {
   if (!c->have_result) return fail(c, OCP_ERR_STATE, "no build result (none has run, or it failed)");
-  uint32_t hc[kCtrlWords];
-  OCP_HIP(c, hipMemcpyAsync(hc, c->ctrl, sizeof(hc), hipMemcpyDeviceToHost, c->stream));
-  OCP_HIP(c, hipStreamSynchronize(c->stream));
+  const uint32_t* hc = nullptr;
+  if (int r = sync_ctrl(c, &hc)) return r;
   if (int r = report_timeout(c, hc)) return r;
   if (hc[kCtrlOctOk] == 0) {
     const int64_t need = hc[kCtrlOctTotal];
@@ -745,8 +767,7 @@ int settle(ocp_ctx c) {
       return fail(c, OCP_ERR_INVALID, "octree stage: a stage array is missing");
     }
     OCP_CHECK_LAUNCH(c);
-    OCP_HIP(c, hipMemcpyAsync(hc, c->ctrl, sizeof(hc), hipMemcpyDeviceToHost, c->stream));
-    OCP_HIP(c, hipStreamSynchronize(c->stream));
+    if (int r = sync_ctrl(c, &hc)) return r;
     if (hc[kCtrlOctOk] == 0) return fail(c, OCP_ERR_CAPACITY, "octree node buffer");
   }
   return OCP_OK;
@@ -793,6 +814,9 @@ int ocp_create(ocp_ctx* out, int device, void* stream) {
   }
   if (hipMalloc(reinterpret_cast<void**>(&c->ctrl), sizeof(uint32_t) * kCtrlWords) != hipSuccess ||
       hipMalloc(reinterpret_cast<void**>(&c->s_hist), sizeof(uint32_t) * 1024) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void**>(&c->mail),
+                    sizeof(uint32_t) * (kMailWords + kCtrlWords), hipHostMallocDefault) !=
+          hipSuccess ||
       hipMemsetAsync(c->ctrl, 0, sizeof(uint32_t) * kCtrlWords, c->stream) != hipSuccess) {
     ocp_destroy(c);
     return OCP_ERR_HIP;
@@ -814,6 +838,7 @@ int ocp_destroy(ocp_ctx c) {
   clear_graphs(c);
   free_workspace(c->ws);
   dev_free(c->ctrl);
+  if (c->mail) (void)hipHostFree(c->mail);
   dev_free(c->s_flags);
   dev_free(c->s_hist);
   for (auto& e : c->ev)
@@ -873,6 +898,12 @@ int ocp_memcpy_h2d(ocp_ctx c, void* dst, const void* src, size_t bytes) {
 int ocp_memcpy_d2h(ocp_ctx c, void* dst, const void* src, size_t bytes) {
   if (check_ctx(c)) return OCP_ERR_INVALID;
   if (!bytes) return OCP_OK;
+  if (bytes <= sizeof(uint32_t) * kCtrlWords) {  // a count or two: by way of pinned memory
+    OCP_HIP(c, hipMemcpyAsync(c->mail + kMailWords, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    OCP_HIP(c, hipStreamSynchronize(c->stream));
+    std::memcpy(dst, c->mail + kMailWords, bytes);
+    return OCP_OK;
+  }
   OCP_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
   OCP_HIP(c, hipStreamSynchronize(c->stream));
   return OCP_OK;
@@ -994,6 +1025,7 @@ int ocp_k_SortKeys_static(ocp_ctx c, uint32_t* keys, uint32_t* alt, uint32_t n) 
     return fail(c, OCP_ERR_CAPACITY, "ocp_k_SortKeys_static: too many sort tiles");
   uint8_t* base = (c->device >= 0 && c->device < kMaxDevices) ? g_scratch_ptr[c->device] : nullptr;
   if (!base) return fail(c, OCP_ERR_STATE, "static sort scratch not set up for this device");
+  c->mail_current = false;
   uint32_t* dev_epoch = reinterpret_cast<uint32_t*>(base);
   uint32_t* hist = reinterpret_cast<uint32_t*>(base + kStaticHeaderBytes);
   uint64_t* flags = reinterpret_cast<uint64_t*>(base + kStaticHeaderBytes + kStaticHistBytes);
@@ -1364,6 +1396,12 @@ int ocp_get_counts(ocp_ctx c, int32_t* n_unique, int32_t* n_oct) {
   if (int r = settle(c)) return r;
   const Workspace& w = c->ws;
   const int32_t ns = c->last_plan.n_seg;
+  if (c->mail_current && ns <= kMailSegs) {
+    const size_t bytes = sizeof(int32_t) * static_cast<size_t>(ns);
+    if (n_unique) std::memcpy(n_unique, c->mail + kCtrlWords, bytes);
+    if (n_oct) std::memcpy(n_oct, c->mail + kCtrlWords + kMailSegs, bytes);
+    return OCP_OK;
+  }
   if (n_unique)
     OCP_HIP(c, hipMemcpy(n_unique, w.counts, sizeof(int32_t) * ns, hipMemcpyDeviceToHost));
   if (n_oct)

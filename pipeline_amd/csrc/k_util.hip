@@ -47,10 +47,13 @@ __global__ __launch_bounds__(256) void begin_shared_kernel(uint32_t* ctrl, uint3
 }
 
 // Exclusive scan of the per-segment slot counts into node offsets; one
-// workgroup of 1024 threads walks the segments in chunks.
+// workgroup of 1024 threads walks the segments in chunks. What the host asks
+// for after a build goes straight to its memory: a caller that reads the
+// counts then waits for the stream and reads them there, where each of three
+// copies back (control words, unique keys, slots) cost ~10 us.
 __global__ __launch_bounds__(1024) void oct_offsets_kernel(
-    const int32_t* __restrict__ kalloc, int32_t n_seg,
-    int32_t* __restrict__ oct_start, uint32_t* ctrl, int64_t k_cap) {
+    const int32_t* __restrict__ n_unique, const int32_t* __restrict__ kalloc, int32_t n_seg,
+    int32_t* __restrict__ oct_start, uint32_t* ctrl, int64_t k_cap, uint32_t* __restrict__ mail) {
   __shared__ uint32_t tmp[16];
   int64_t carry = 0;
   for (int32_t c = 0; c < n_seg; c += 1024) {
@@ -58,13 +61,22 @@ __global__ __launch_bounds__(1024) void oct_offsets_kernel(
     const uint32_t v = k < n_seg ? static_cast<uint32_t>(kalloc[k]) : 0u;
     uint32_t total;
     const uint32_t ex = block_excl_scan<1024>(v, tmp, &total);
-    if (k < n_seg) oct_start[k] = static_cast<int32_t>(carry + ex);
+    if (k < n_seg) {
+      oct_start[k] = static_cast<int32_t>(carry + ex);
+      if (n_seg <= kMailSegs) {
+        mail[kCtrlWords + k] = static_cast<uint32_t>(n_unique[k]);
+        mail[kCtrlWords + kMailSegs + k] = v;
+      }
+    }
     carry += total;
   }
   if (threadIdx.x == 0) {
     oct_start[n_seg] = static_cast<int32_t>(carry);
     ctrl[kCtrlOctTotal] = static_cast<uint32_t>(carry);
     ctrl[kCtrlOctOk] = carry <= k_cap ? 1u : 0u;
+    mail[kCtrlOctTotal] = static_cast<uint32_t>(carry);
+    mail[kCtrlOctOk] = carry <= k_cap ? 1u : 0u;
+    mail[kCtrlTimeout] = ctrl[kCtrlTimeout];
   }
 }
 
@@ -156,10 +168,10 @@ void launch_begin_shared(uint32_t* ctrl, uint32_t* dev_epoch, uint32_t* hist, in
   begin_shared_kernel<<<static_cast<int>(blocks), 256, 0, s>>>(ctrl, dev_epoch, hist, n_hist);
 }
 
-void launch_oct_offsets(const int32_t* kalloc, int32_t n_seg,
-                        int32_t* oct_start, uint32_t* ctrl, int64_t k_cap,
+void launch_oct_offsets(const int32_t* n_unique, const int32_t* kalloc, int32_t n_seg,
+                        int32_t* oct_start, uint32_t* ctrl, int64_t k_cap, uint32_t* mail,
                         hipStream_t s) {
-  oct_offsets_kernel<<<1, 1024, 0, s>>>(kalloc, n_seg, oct_start, ctrl, k_cap);
+  oct_offsets_kernel<<<1, 1024, 0, s>>>(n_unique, kalloc, n_seg, oct_start, ctrl, k_cap, mail);
 }
 
 void launch_zero_nodes(OctNode* nodes, const uint32_t* ctrl, int64_t k_cap,

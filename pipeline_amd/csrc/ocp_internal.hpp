@@ -118,8 +118,13 @@ void launch_begin(uint32_t* ctrl, uint32_t* hist, int64_t n_hist,
 // epoch is past both the context's and *dev_epoch, and is stored in both.
 void launch_begin_shared(uint32_t* ctrl, uint32_t* dev_epoch, uint32_t* hist, int64_t n_hist,
                          hipStream_t s);
-void launch_oct_offsets(const int32_t* kalloc, int32_t n_seg,
-                        int32_t* oct_start, uint32_t* ctrl, int64_t k_cap,
+// mail (pinned host memory): the build's time-out mark, slot total and fit
+// flag at their control-word places, then, for at most kMailSegs segments, the
+// counts n_unique and kalloc kMailSegs words apart.
+constexpr int32_t kMailSegs = 4096;
+constexpr int32_t kMailWords = kCtrlWords + 2 * kMailSegs;
+void launch_oct_offsets(const int32_t* n_unique, const int32_t* kalloc, int32_t n_seg,
+                        int32_t* oct_start, uint32_t* ctrl, int64_t k_cap, uint32_t* mail,
                         hipStream_t s);
 void launch_zero_nodes(OctNode* nodes, const uint32_t* ctrl, int64_t k_cap,
                        hipStream_t s);
