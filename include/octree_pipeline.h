@@ -403,8 +403,8 @@ int ocp_get_stage_ms(ocp_ctx ctx, float* ms7);
  * up to max_kernels entries (names are static strings) and the number of
  * kernels a build launches to n_kernels. A build with the MSD sort
  * (ocp_tune.sort_msd) names its sort slots msd_scatter, msd_buckets,
- * msd_lsd_fallback (msd_lsd_skipped when every bucket fit in LDS) and
- * unused. */
+ * msd_lsd_fallback (the digits too large for LDS; msd_lsd_skipped when there
+ * was none) and unused. */
 int ocp_get_kernel_ms(ocp_ctx ctx, float* ms, const char** names,
                       int32_t max_kernels, int32_t* n_kernels);
 /* Time `steps` builds (after `warmup`) of the configured kind on the
@@ -416,7 +416,11 @@ int ocp_time_builds(ocp_ctx ctx, const float* points, int float3,
                     int steps, float* ms_per_build);
 
 /* ------------------------------------------------------------ tuning */
-/* Tile parameters and the sort's digit width (pass count). */
+/* Tile parameters and the sort's digit width (pass count). Until a table is
+ * set (ocp_set_tune, ocp_autotune), a build without the permutation chooses
+ * the sort's form by itself, whatever sort_bits and sort_msd say: sort_msd's
+ * from 16384 points on, the LSD passes for small builds and, for some builds
+ * at a time, where the keys of the last one crowded into few digits. */
 typedef struct ocp_tune {
   int32_t sort_waves;   /* OneSweep tile of 8-bit digits: waves ... */
   int32_t sort_kpt;     /* ... and keys per thread */
@@ -430,11 +434,9 @@ typedef struct ocp_tune {
   int32_t oct_order;    /* 0 or 1, kept for saved tables: one octree kernel
                            serves both */
   int32_t sort_msd;     /* with sort_bits 10: 0 three LSD passes; 1 one
-                           scatter by the top 10-bit digit, then each bucket
-                           sorted in LDS by one workgroup; a build with a
-                           bucket above 16384 keys runs the three LSD passes
-                           after that, one of more than 2048 clouds only
-                           them */
+                           scatter by the top 10-bit digit, then windows of
+                           it sorted in LDS, digits too large for that by a
+                           second scatter (not for more than 2048 clouds) */
 } ocp_tune;
 int ocp_get_tune(ocp_ctx ctx, ocp_tune* out);
 int ocp_set_tune(ocp_ctx ctx, const ocp_tune* in);

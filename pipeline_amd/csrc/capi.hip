@@ -49,27 +49,31 @@ struct Workspace {
   uint64_t* flags = nullptr;     // flag_cap words
   int32_t* counts = nullptr;     // n_unique[seg_cap], kalloc[seg_cap]
   int32_t* oct_start = nullptr;  // seg_cap + 1
-  int32_t* tables = nullptr;     // seg_start + 5 tile maps, 6 * (seg_cap+1)
+  int32_t* tables = nullptr;     // seg_start + 6 tile maps, 7 * (seg_cap+1)
   float* boxes = nullptr;        // seg_min[seg_cap], seg_range[seg_cap]
   uint32_t* box_mm = nullptr;    // per segment {min, max} while boxes are reduced
   uint32_t* vals_a = nullptr;    // key->point permutation (allocated when enabled): sorted
   uint32_t* vals_b = nullptr;    //   point indices, then each unique key's first point
   int64_t vals_cap = 0;
+  MsdLevel2 l2{};                // second level of the MSD sort (allocated when a build takes it)
 };
 
 struct Plan {
+  TuneTable tune;             // the context's, with the sort's form settled
+  bool auto_msd = false;      // the MSD form, by the library's own choice
   int32_t n_seg = 1;
   int64_t n_total = 0;
   int64_t max_seg = 0;        // the largest segment's length
   bool device_boxes = false;  // boxes reduced on the device into ws.boxes
   bool permutation = false;   // point indices carried through sort and unique
   SegView sv{};
-  int32_t tiles_morton = 0, tiles_sort = 0, tiles_scan = 0, tiles_node = 0, tiles_tree = 0;
+  int32_t tiles_morton = 0, tiles_sort = 0, tiles_scan = 0, tiles_node = 0, tiles_tree = 0, tiles_win = 0;
   const int32_t* ts_morton = nullptr;
   const int32_t* ts_sort = nullptr;
   const int32_t* ts_scan = nullptr;
   const int32_t* ts_node = nullptr;
   const int32_t* ts_tree = nullptr;
+  const int32_t* ts_win = nullptr;
 };
 
 // Kernels of one build, in launch order (per-kernel event timing).
@@ -81,7 +85,8 @@ const char* const kKernelNames[kKernelCount] = {
     "begin", "morton_hist", "onesweep_pass0", "onesweep_pass1", "onesweep_pass2",
     "onesweep_pass3", "unique", "radix_tree", "edge_scan", "oct_offsets", "octree"};
 // The sort's kernels when a build takes the MSD form (the last slot unused;
-// the third is named msd_lsd_skipped when every bucket fit in LDS).
+// the third is the second level, named msd_lsd_skipped when every digit fit
+// in LDS).
 const char* const kMsdKernelNames[4] = {"msd_scatter", "msd_buckets", "msd_lsd_fallback",
                                         "unused"};
 
@@ -170,6 +175,11 @@ struct ocp_context {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   TuneTable tune;
+  bool tuned = false;  // a table was set: its sort form is taken as it stands
+  // Builds of about skew_n points to come that take the LSD passes, because the
+  // keys of one like them crowded into few digits.
+  int32_t skew_left = 0;
+  int64_t skew_n = 0;
   std::string err;
   uint32_t* ctrl = nullptr;
   // per-stage scratch
@@ -267,6 +277,8 @@ void free_workspace(Workspace& w) {
   dev_free(w.offs); dev_free(w.nodes); dev_free(w.hist); dev_free(w.flags);
   dev_free(w.counts); dev_free(w.oct_start); dev_free(w.tables); dev_free(w.boxes);
   dev_free(w.box_mm); dev_free(w.vals_a); dev_free(w.vals_b);
+  dev_free(w.l2.big); dev_free(w.l2.tiles); dev_free(w.l2.hist); dev_free(w.l2.cursor);
+  dev_free(w.l2.hist3);
   w = Workspace{};
 }
 
@@ -314,7 +326,7 @@ int ensure_workspace(ocp_ctx c, int64_t n, int32_t n_seg, int64_t flag_words) {
     if ((r = dev_alloc(c, &w.hist, int64_t(cap) * (hist_stride(10) + kCursorWords))) ||
         (r = dev_alloc(c, &w.counts, int64_t(cap) * 2)) ||
         (r = dev_alloc(c, &w.oct_start, int64_t(cap) + 1)) ||
-        (r = dev_alloc(c, &w.tables, 6 * (int64_t(cap) + 1))) ||
+        (r = dev_alloc(c, &w.tables, 7 * (int64_t(cap) + 1))) ||
         (r = dev_alloc(c, &w.boxes, 2 * int64_t(cap))) ||
         (r = dev_alloc(c, &w.box_mm, 2 * int64_t(cap))))
       return r;
@@ -345,6 +357,33 @@ int ensure_perm(ocp_ctx c) {
   return OCP_OK;
 }
 
+// Second-level room of an MSD sort of n keys.
+int ensure_level2(ocp_ctx c, int64_t n, int64_t max_seg) {
+  MsdLevel2 want{};
+  msd_level2_caps(n, max_seg, &want);
+  MsdLevel2& l = c->ws.l2;
+  if (want.max_big <= l.max_big && want.max_tiles <= l.max_tiles && want.max_slots <= l.max_slots)
+    return OCP_OK;
+  want.max_big = std::max(want.max_big, l.max_big);
+  want.max_tiles = std::max(want.max_tiles, l.max_tiles);
+  want.max_slots = std::max(want.max_slots, l.max_slots);
+  OCP_HIP(c, hipStreamSynchronize(c->stream));
+  clear_graphs(c);
+  dev_free(l.big); dev_free(l.tiles); dev_free(l.hist); dev_free(l.cursor); dev_free(l.hist3);
+  l = MsdLevel2{};
+  int r = 0;
+  if ((r = dev_alloc(c, &want.big, want.max_big)) || (r = dev_alloc(c, &want.tiles, want.max_tiles)) ||
+      (r = dev_alloc(c, &want.hist, int64_t(want.max_big) * 1024)) ||
+      (r = dev_alloc(c, &want.cursor, int64_t(want.max_big) * 1024)) ||
+      (r = dev_alloc(c, &want.hist3, int64_t(want.max_slots) * 1024))) {
+    dev_free(want.big); dev_free(want.tiles); dev_free(want.hist); dev_free(want.cursor);
+    dev_free(want.hist3);
+    return r;
+  }
+  l = want;
+  return OCP_OK;
+}
+
 SegView single_view(int64_t n, float mn, float rg) {
   SegView sv{};
   sv.n_seg = 1;
@@ -363,6 +402,39 @@ int tune_key(const TuneTable& t) {
          (t.sort_msd != 0);
 }
 
+// The tile table of a build: the context's, with the library's choice of the
+// sort's form where its caller set no table.
+TuneTable build_tune(const TuneTable& set, bool tuned, int64_t n, int64_t max_seg, int32_t n_seg,
+                     bool perm) {
+  TuneTable t = set;
+  if (!tuned && auto_sort_msd(n, n_seg, perm)) {
+    t.sort_bits = 10;
+    t.sort_msd = 1;
+    t.sort10_kpt = auto_sort10_kpt(max_seg);
+  }
+  return t;
+}
+
+// ... and the form for this build. A large cloud's keys may crowd as they like
+// (see auto_sort_skew).
+TuneTable choose_tune(ocp_ctx c, int64_t n, int64_t max_seg, int32_t n_seg, bool perm) {
+  const TuneTable t = build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm);
+  if (c->tuned || !pipe_sort_msd(t, perm, n_seg) || !auto_sort_skew(max_seg) ||
+      c->skew_left <= 0 || n < c->skew_n / 2 || n > c->skew_n * 2)
+    return t;
+  --c->skew_left;
+  return c->tune;
+}
+
+// After a build of the library's choice: its level-2 tiles tell how many keys
+// lay in digits too large for LDS.
+void note_skew(ocp_ctx c, uint32_t tiles) {
+  const Plan& p = c->last_plan;
+  if (!p.auto_msd || int64_t(tiles) * 8192 * 16 <= p.n_total) return;
+  c->skew_left = kSkewBuilds;
+  c->skew_n = p.n_total;
+}
+
 int64_t flag_words_for(const TuneTable& tt, int64_t n, int32_t n_seg) {
   const int64_t sort_tiles = cdiv(n, sort_tile(tt)) + n_seg;
   const int64_t sort10_tiles = cdiv(n, 1024 * tt.sort10_kpt) + n_seg;
@@ -376,6 +448,7 @@ int64_t flag_words_for(const TuneTable& tt, int64_t n, int32_t n_seg) {
 // Plain plan: one segment, scalar box, no device tables.
 Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
   Plan p;
+  p.tune = tt;
   p.n_seg = 1;
   p.n_total = n;
   p.max_seg = n;
@@ -386,7 +459,19 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
   p.tiles_scan = static_cast<int32_t>(cdiv(n, scan_tile(tt)));
   p.tiles_node = static_cast<int32_t>(cdiv(n, kOctTile));
   p.tiles_tree = static_cast<int32_t>(cdiv(n, tree_tile(n)));
+  p.tiles_win = static_cast<int32_t>(msd_windows(n, n));
   return p;
+}
+
+// ... and the memory it needs.
+int prepare_plain(ocp_ctx c, int64_t n, float mn, float rg, Plan* p) {
+  const TuneTable tt = choose_tune(c, n, n, 1, c->permutation);
+  if (int r = ensure_workspace(c, n, 1, flag_words_for(c->tune, n, 1))) return r;
+  if (pipe_sort_msd(tt, c->permutation, 1))
+    if (int r = ensure_level2(c, n, n)) return r;
+  *p = plain_plan(tt, n, mn, rg, c->permutation);
+  p->auto_msd = !c->tuned && pipe_sort_msd(tt, c->permutation, 1);
+  return OCP_OK;
 }
 
 // Batched plan: validates the table, uploads offsets, boxes and tile maps
@@ -416,8 +501,13 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   std::string why;
   if (int r = validate_batch(offsets, smin, srg, n_seg, &why)) return fail(c, r, why);
   const int64_t n = offsets[n_seg];
-  const TuneTable& tt = c->tune;
-  if (int r = ensure_workspace(c, n, n_seg, flag_words_for(tt, n, n_seg))) return r;
+  int64_t max_seg = 0;
+  for (int32_t k = 0; k < n_seg; ++k)
+    max_seg = std::max<int64_t>(max_seg, int64_t(offsets[k + 1]) - offsets[k]);
+  const TuneTable tt = choose_tune(c, n, max_seg, n_seg, perm);
+  if (int r = ensure_workspace(c, n, n_seg, flag_words_for(c->tune, n, n_seg))) return r;
+  if (pipe_sort_msd(tt, perm, n_seg))
+    if (int r = ensure_level2(c, n, max_seg)) return r;
   Workspace& w = c->ws;
   const int32_t stride = w.seg_cap + 1;
   int32_t* d_start = w.tables;
@@ -426,14 +516,18 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   int32_t* d_tc = w.tables + 3 * stride;
   int32_t* d_tn = w.tables + 4 * stride;
   int32_t* d_tt = w.tables + 5 * stride;
+  int32_t* d_tw = w.tables + 6 * stride;
   Plan p;
+  p.tune = tt;
   p.n_seg = n_seg;
   p.n_total = n;
+  p.max_seg = max_seg;
+  p.auto_msd = !c->tuned && pipe_sort_msd(tt, perm, n_seg);
   p.permutation = perm;
   p.device_boxes = !smin;
   const int stile = pipe_sort_tile(tt, perm);
-  std::vector<int32_t> host(6 * static_cast<size_t>(n_seg + 1));
-  int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0;
+  std::vector<int32_t> host(7 * static_cast<size_t>(n_seg + 1));
+  int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0, tw = 0;
   for (int32_t k = 0; k <= n_seg; ++k) {
     host[k] = offsets[k];
     host[(n_seg + 1) + k] = static_cast<int32_t>(tm);
@@ -441,14 +535,15 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
     host[3 * (n_seg + 1) + k] = static_cast<int32_t>(tc);
     host[4 * (n_seg + 1) + k] = static_cast<int32_t>(tn);
     host[5 * (n_seg + 1) + k] = static_cast<int32_t>(ttr);
+    host[6 * (n_seg + 1) + k] = static_cast<int32_t>(tw);
     if (k < n_seg) {
       const int64_t len = int64_t(offsets[k + 1]) - offsets[k];
-      p.max_seg = std::max(p.max_seg, len);
       tm += cdiv(len, morton_tile(tt));
       ts += cdiv(len, stile);
       tc += cdiv(len, scan_tile(tt));
       tn += cdiv(len, kOctTile);
       ttr += cdiv(len, tree_tile(n));
+      tw += msd_windows(len, max_seg);
     }
   }
   const int tab_key = tune_key(tt) * 2 + (pipe_sort_bits(tt, perm) == 10);
@@ -456,7 +551,7 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
                     c->tab_offsets.size() == static_cast<size_t>(n_seg + 1) &&
                     std::equal(offsets, offsets + n_seg + 1, c->tab_offsets.begin());
   if (!same) {
-    for (int q = 0; q < 6; ++q)
+    for (int q = 0; q < 7; ++q)
       OCP_HIP(c, hipMemcpyAsync(w.tables + q * stride, host.data() + q * (n_seg + 1),
                                 sizeof(int32_t) * (n_seg + 1), hipMemcpyHostToDevice,
                                 c->stream));
@@ -489,11 +584,13 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.tiles_scan = static_cast<int32_t>(tc);
   p.tiles_node = static_cast<int32_t>(tn);
   p.tiles_tree = static_cast<int32_t>(ttr);
+  p.tiles_win = static_cast<int32_t>(tw);
   p.ts_morton = d_tm;
   p.ts_sort = d_ts;
   p.ts_scan = d_tc;
   p.ts_node = d_tn;
   p.ts_tree = d_tt;
+  p.ts_win = d_tw;
   *out = p;
   return OCP_OK;
 }
@@ -560,7 +657,7 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
                       bool capturing) {
   Workspace& w = c->ws;
   hipStream_t s = c->stream;
-  const TuneTable& tt = c->tune;
+  const TuneTable& tt = p.tune;
   int32_t* n_unique = w.counts;
   int32_t* kalloc = w.counts + w.seg_cap;
   // 8-bit digits take four passes over the keys, 10-bit digits three; the
@@ -597,23 +694,16 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
   if (c->order_wait && !capturing && c->order_err == hipSuccess)
     c->order_err = hipStreamWaitEvent(s, c->order_wait, 0);
   if (msd) {
-    // Scatter by the top digit into keys_a, sort each bucket there in LDS;
-    // if a bucket was too large, the counts of the two lower digits and
-    // three LSD passes from the Morton output (left intact in keys_b) sort
-    // into keys_a instead.
+    // Scatter by the top digit into keys_a, sort windows of it there in LDS;
+    // the digits too large for that go through keys_b, whose Morton output
+    // the scatter has read.
     { KScope k(c, kKPass0, capturing);
       launch_msd_scatter(src, dst, p.sv, p.ts_sort, p.tiles_sort, w.hist,
                          w.hist + int64_t(p.n_seg) * hist_stride(10), c->ctrl, tt, s); }
     { KScope k(c, kKPass1, capturing);
-      launch_msd_buckets(dst, p.sv, w.hist, c->ctrl, p.max_seg, s); }
+      launch_msd_windows(dst, p.sv, p.ts_win, p.tiles_win, p.max_seg, w.hist, w.l2, c->ctrl, s); }
     KScope k(c, kKPass2, capturing);
-    launch_msd_low_hist(src, p.sv, p.ts_morton, p.tiles_morton, w.hist, c->ctrl, tt, s);
-    const int32_t* run = reinterpret_cast<const int32_t*>(c->ctrl + kCtrlMsdRun);
-    for (int pass = 0; pass < passes; ++pass) {
-      launch_onesweep_pass(src, dst, p.sv, p.ts_sort, p.tiles_sort, w.hist, w.flags, c->ctrl,
-                           pass, pass != 0, tt, s, bits, run);
-      std::swap(src, dst);
-    }
+    launch_msd_level2(dst, src, w.l2, c->ctrl, s);
   }
   for (int pass = 0; pass < passes && !msd; ++pass) {
     KScope k(c, kKPass0 + pass, capturing);
@@ -741,6 +831,7 @@ int sync_ctrl(ocp_ctx c, const uint32_t** words) {
                               hipMemcpyDeviceToHost, c->stream));
   }
   OCP_HIP(c, hipStreamSynchronize(c->stream));
+  if (c->mail_current) note_skew(c, c->mail[kCtrlMsdTiles]);
   return OCP_OK;
 }
 
@@ -1224,9 +1315,8 @@ int ocp_build(ocp_ctx c, const float* points, int float3, int64_t n, float mn, f
   if (!(rg > 0.0f)) return fail(c, OCP_ERR_INVALID, "range must be > 0");
   if (!float3 && (reinterpret_cast<uintptr_t>(points) & 15u))
     return fail(c, OCP_ERR_INVALID, "float4 input must be 16-byte aligned");
-  const TuneTable& tt = c->tune;
-  if (int r = ensure_workspace(c, n, 1, flag_words_for(tt, n, 1))) return r;
-  Plan p = plain_plan(tt, n, mn, rg, c->permutation);
+  Plan p;
+  if (int r = prepare_plain(c, n, mn, rg, &p)) return r;
   if (int r = ensure_perm(c)) return r;
   c->last.valid = true;
   c->last.batched = false;
@@ -1235,7 +1325,7 @@ int ocp_build(ocp_ctx c, const float* points, int float3, int64_t n, float mn, f
   c->last.n = n;
   c->last.mn = mn;
   c->last.rg = rg;
-  return run_plan(c, points, float3, p, graph_key("plain", points, float3, n, mn, rg, nullptr, tt));
+  return run_plan(c, points, float3, p, graph_key("plain", points, float3, n, mn, rg, nullptr, p.tune));
 }
 
 int ocp_build_autobox(ocp_ctx c, const float* points, int float3, int64_t n) {
@@ -1245,9 +1335,8 @@ int ocp_build_autobox(ocp_ctx c, const float* points, int float3, int64_t n) {
   if (n > kMaxSegPoints) return fail(c, OCP_ERR_CAPACITY, "a single cloud holds at most 2^27 points");
   if (!float3 && (reinterpret_cast<uintptr_t>(points) & 15u))
     return fail(c, OCP_ERR_INVALID, "float4 input must be 16-byte aligned");
-  const TuneTable& tt = c->tune;
-  if (int r = ensure_workspace(c, n, 1, flag_words_for(tt, n, 1))) return r;
-  Plan p = plain_plan(tt, n, 0.0f, 1.0f, c->permutation);
+  Plan p;
+  if (int r = prepare_plain(c, n, 0.0f, 1.0f, &p)) return r;
   p.device_boxes = true;
   p.permutation = c->permutation;
   if (int r = ensure_perm(c)) return r;
@@ -1259,7 +1348,7 @@ int ocp_build_autobox(ocp_ctx c, const float* points, int float3, int64_t n) {
   c->last.float3 = float3;
   c->last.n = n;
   return run_plan(c, points, float3, p,
-                  graph_key("plain-autobox", points, float3, n, 0, 0, nullptr, tt));
+                  graph_key("plain-autobox", points, float3, n, 0, 0, nullptr, p.tune));
 }
 
 int ocp_transform_points(ocp_ctx c, const float* src, float* dst, int float3, int64_t n,
@@ -1300,7 +1389,7 @@ int ocp_build_batched(ocp_ctx c, const float* points, int float3, const int32_t*
   }
   return run_plan(c, points, float3, p,
                   graph_key(smin ? "batch" : "batch-autobox", points, float3, p.n_total, 0, 0,
-                            &c->last.offsets, c->tune));
+                            &c->last.offsets, p.tune));
 }
 
 int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permutation,
@@ -1323,8 +1412,11 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
         (tt.oct_order != 0 && tt.oct_order != 1) || (tt.sort_msd != 0 && tt.sort_msd != 1))
       return OCP_ERR_INVALID;
   }
-  // The allocations of ensure_workspace, alloc_nodes and ensure_perm for a
-  // first build of this shape, plus the context's control words and digit
+  const int32_t clouds = std::max<int32_t>(n_seg, 1);
+  const int64_t flag_words = flag_words_for(tt, n, clouds);
+  tt = build_tune(tt, tune != nullptr, n, n, clouds, permutation != 0);
+  // The allocations of ensure_workspace, alloc_nodes, ensure_level2 and
+  // ensure_perm for a first build of this shape, plus the context's control words and digit
   // counts (ocp_create).
   const int64_t cap = std::max<int64_t>(n, 4096);
   const int64_t seg = std::max<int32_t>(n_seg, 1);
@@ -1332,9 +1424,15 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
               + 3 * 1 * cap        // prefix_n, hl, hr
               + 4 * 4 * cap        // left child, parent, edge counts, offsets
               + cap * int64_t(sizeof(OctNode)) + 16;  // nodes (K_cap starts at N)
-  b += 4 * (seg * (hist_stride(10) + kCursorWords) + 2 * seg + (seg + 1) + 6 * (seg + 1) +
+  b += 4 * (seg * (hist_stride(10) + kCursorWords) + 2 * seg + (seg + 1) + 7 * (seg + 1) +
             4 * seg);
-  b += 8 * std::max<int64_t>(flag_words_for(tt, n, static_cast<int32_t>(seg)), 1 << 16);
+  b += 8 * std::max<int64_t>(flag_words, 1 << 16);
+  if (pipe_sort_msd(tt, permutation != 0, clouds)) {
+    MsdLevel2 l2{};
+    msd_level2_caps(n, n_seg > 1 ? 0 : n, &l2);  // (a batch's largest cloud is not given: the most)
+    b += int64_t(l2.max_big) * (16 + 2 * 4096) + int64_t(l2.max_tiles) * 8 +
+         int64_t(l2.max_slots) * 4096;
+  }
   if (permutation) b += 2 * 4 * cap;
   b += 4 * (kCtrlWords + 1024);
   out->build_bytes = b;
@@ -1570,10 +1668,10 @@ int ocp_get_kernel_ms(ocp_ctx c, float* ms, const char** names, int32_t max_kern
   *n_kernels = kKernelCount;
   if (!c->ev_recorded) return fail(c, OCP_ERR_STATE, "no eager build with stage timing on");
   OCP_HIP(c, hipEventSynchronize(c->ev[6]));
-  // Whether the MSD sort's LSD passes had work (read after the build ended).
+  // Whether the MSD sort's second level had work (read after the build ended).
   uint32_t msd_run = 0;
   if (c->kmsd && names)
-    OCP_HIP(c, hipMemcpy(&msd_run, c->ctrl + kCtrlMsdRun, sizeof(msd_run), hipMemcpyDeviceToHost));
+    OCP_HIP(c, hipMemcpy(&msd_run, c->ctrl + kCtrlMsdTiles, sizeof(msd_run), hipMemcpyDeviceToHost));
   for (int k = 0; k < kKernelCount && k < max_kernels; ++k) {
     if (names)
       names[k] = !(c->kmsd && k >= kKPass0 && k <= kKPass3) ? kKernelNames[k]
@@ -1650,6 +1748,7 @@ int ocp_set_tune(ocp_ctx c, const ocp_tune* in) {
   c->tune.sort10_kpt = in->sort10_kpt;
   c->tune.oct_order = in->oct_order;
   c->tune.sort_msd = in->sort_msd;
+  c->tuned = true;
   clear_graphs(c);
   c->tab_offsets.clear();
   return OCP_OK;

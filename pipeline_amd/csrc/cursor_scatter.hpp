@@ -28,18 +28,16 @@ struct TopDigit10 {
   }
 };
 
-// Digit functor: kBits, kCheap (recomputed from the key rather than staged
-// in LDS), setup(seg, tid, threads) for per-segment LDS tables, and the
-// digit of a key. hist[seg * hstride + d]: the segment's count of digit d;
-// cursor[seg * 2^kBits + d]: zeroed claim counters; tiles_dev (optional):
-// the number of real tiles when the grid is sized for an upper bound. Tiles
-// of THREADS * KPT keys never straddle a segment.
-template <int THREADS, int KPT, class Digit>
-__global__ __launch_bounds__(THREADS) void cursor_scatter_kernel(
-    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, SegView sv,
-    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ tiles_dev,
-    const uint32_t* __restrict__ hist, int64_t hstride, uint32_t* __restrict__ cursor,
-    const uint32_t* __restrict__ ctrl, Digit dig) {
+// A tile's work, one workgroup: the keys in[base, base + cnt) of a segment
+// [sb, sb + len). Digit functor: kBits, kCheap (recomputed from the key rather
+// than staged in LDS) and the digit of a key. hist[d]: the segment's count of
+// digit d; cursor[d]: its zeroed claim counters. extra(digits, keys) runs once
+// the keys are in registers, before they are placed.
+template <int THREADS, int KPT, class Digit, class Extra>
+__device__ __forceinline__ void cursor_scatter_tile(
+    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int32_t sb, int32_t len,
+    int32_t base, int32_t cnt, const uint32_t* __restrict__ hist, uint32_t* __restrict__ cursor,
+    Digit dig, Extra extra) {
   constexpr int RADIX = 1 << Digit::kBits;
   constexpr int T = THREADS * KPT;
   constexpr bool CHEAP = Digit::kCheap;
@@ -50,18 +48,9 @@ __global__ __launch_bounds__(THREADS) void cursor_scatter_kernel(
   __shared__ uint32_t s_run[RADIX];  // tile counts, then the LDS start of each run
   __shared__ int32_t s_gpos[RADIX];  // global slot of a run's LDS slot 0
   __shared__ uint32_t s_tmp[2 * (THREADS / 64)];
-  const int32_t t = static_cast<int32_t>(blockIdx.x);
-  if (tiles_dev && t >= *tiles_dev) return;
-  if (stopped_any(ctrl)) return;
   const int tid = threadIdx.x;
-  const TileRef r = find_tile(tile_start, sv.n_seg, t);
-  const int32_t sb = seg_begin(sv, r.seg);
-  const int32_t len = seg_end(sv, r.seg) - sb;
-  const int32_t base = sb + r.local * T;
-  const int32_t cnt = min(T, sb + len - base);
   if (tid < RADIX) s_run[tid] = 0;
-  dig.setup(r.seg, tid, THREADS);
-  const uint32_t hv = tid < RADIX ? hist[static_cast<int64_t>(r.seg) * hstride + tid] : 0u;
+  const uint32_t hv = tid < RADIX ? hist[tid] : 0u;
   uint32_t keys[KPT];
   const uint32_t* src = in + base + tid;
   if (cnt == T) {
@@ -75,21 +64,21 @@ __global__ __launch_bounds__(THREADS) void cursor_scatter_kernel(
   uint32_t dg[KPT], rank[KPT];
 #pragma unroll
   for (int k = 0; k < KPT; ++k) {
+    dg[k] = 0xffffffffu;
     if (k * THREADS + tid < cnt) {
       dg[k] = dig(keys[k]);
       rank[k] = atomicAdd(&s_run[dg[k]], 1u);
     }
   }
   __syncthreads();
+  extra(hv, dg, keys);
   const uint32_t c = tid < RADIX ? s_run[tid] : 0u;
   uint32_t lstart, gbase;
   block_excl_scan2<THREADS>(c, hv, s_tmp, &lstart, &gbase);
   if (tid < RADIX) {
     int32_t gpos = 0;
     if (c)
-      gpos = sb +
-             static_cast<int32_t>(gbase +
-                                  atomicAdd(&cursor[static_cast<int64_t>(r.seg) * RADIX + tid], c)) -
+      gpos = sb + static_cast<int32_t>(gbase + atomicAdd(&cursor[tid], c)) -
              static_cast<int32_t>(lstart);
     s_run[tid] = lstart;  // (every read of the counts came before the scan's barriers)
     s_gpos[tid] = gpos;
@@ -112,6 +101,38 @@ __global__ __launch_bounds__(THREADS) void cursor_scatter_kernel(
     // launchers' counts do)
     if (static_cast<uint32_t>(p - sb) < static_cast<uint32_t>(len)) out[p] = key;
   }
+}
+
+struct NoExtra {
+  template <int KPT>
+  __device__ __forceinline__ void operator()(uint32_t, const uint32_t (&)[KPT],
+                                             const uint32_t (&)[KPT]) const {}
+};
+
+// One tile per workgroup, tiles of THREADS * KPT keys that never straddle a
+// segment. The functor's setup(seg, tid, threads) fills per-segment LDS
+// tables. hist[seg * hstride + d], cursor[seg * 2^kBits + d]; tiles_dev
+// (optional): the number of real tiles when the grid is sized for an upper
+// bound.
+template <int THREADS, int KPT, class Digit>
+__global__ __launch_bounds__(THREADS) void cursor_scatter_kernel(
+    const uint32_t* __restrict__ in, uint32_t* __restrict__ out, SegView sv,
+    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ tiles_dev,
+    const uint32_t* __restrict__ hist, int64_t hstride, uint32_t* __restrict__ cursor,
+    const uint32_t* __restrict__ ctrl, Digit dig) {
+  constexpr int RADIX = 1 << Digit::kBits;
+  constexpr int T = THREADS * KPT;
+  const int32_t t = static_cast<int32_t>(blockIdx.x);
+  if (tiles_dev && t >= *tiles_dev) return;
+  if (stopped_any(ctrl)) return;
+  const TileRef r = find_tile(tile_start, sv.n_seg, t);
+  const int32_t sb = seg_begin(sv, r.seg);
+  const int32_t len = seg_end(sv, r.seg) - sb;
+  const int32_t base = sb + r.local * T;
+  dig.setup(r.seg, threadIdx.x, THREADS);
+  cursor_scatter_tile<THREADS, KPT>(in, out, sb, len, base, min(T, sb + len - base),
+                                    hist + static_cast<int64_t>(r.seg) * hstride,
+                                    cursor + static_cast<int64_t>(r.seg) * RADIX, dig, NoExtra{});
 }
 
 }  // namespace ocp

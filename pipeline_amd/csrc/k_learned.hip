@@ -409,7 +409,7 @@ __global__ __launch_bounds__(WAVES * 64) void lsort_kernel(uint32_t* __restrict_
   const int32_t lo = bstart[b];
   const int32_t n = bstart[b + 1] - lo;
   if (n <= lo_cap || n > WAVES * 64 * KPT) return;
-  lds_bucket_sort<WAVES, KPT>(keys + lo, n);
+  lds_bucket_sort<WAVES, KPT>(keys + lo, keys + lo, n);
 }
 
 // The last key of each non-empty bucket must not exceed the next key.

@@ -88,27 +88,27 @@ void launch_cfg(const uint32_t* in, uint32_t* out, const SegView& sv,
   const RadixDigit dig{8u * static_cast<uint32_t>(pass)};
   if (stable)
     onesweep_kernel<WAVES, KPT, RadixDigit, true><<<total_tiles, WAVES * 64, 0, s>>>(
-        in, out, sv, tile_start, nullptr, hist, pass, flags, ctrl, stage, dig);
+        in, out, sv, tile_start, hist, pass, flags, ctrl, stage, dig);
   else
     onesweep_kernel<WAVES, KPT, RadixDigit, false><<<total_tiles, WAVES * 64, 0, s>>>(
-        in, out, sv, tile_start, nullptr, hist, pass, flags, ctrl, stage, dig);
+        in, out, sv, tile_start, hist, pass, flags, ctrl, stage, dig);
 }
 
 // 10-bit digits: one thread per digit, so 16 waves per tile.
 // `digit` selects the bits (10 * digit) and the histogram slot; `stage` tags
-// the lookback flags; tiles_dev (optional) is the device-side tile count.
+// the lookback flags.
 template <int KPT>
 void launch_cfg10(const uint32_t* in, uint32_t* out, const SegView& sv,
                   const int32_t* tile_start, int32_t total_tiles, const uint32_t* hist,
                   uint64_t* flags, uint32_t* ctrl, int digit, uint32_t stage, bool stable,
-                  const int32_t* tiles_dev, hipStream_t s) {
+                  hipStream_t s) {
   const RadixDigit10 dig{10u * static_cast<uint32_t>(digit)};
   if (stable)
     onesweep_kernel<16, KPT, RadixDigit10, true><<<total_tiles, 1024, 0, s>>>(
-        in, out, sv, tile_start, tiles_dev, hist, digit, flags, ctrl, stage, dig);
+        in, out, sv, tile_start, hist, digit, flags, ctrl, stage, dig);
   else
     onesweep_kernel<16, KPT, RadixDigit10, false><<<total_tiles, 1024, 0, s>>>(
-        in, out, sv, tile_start, tiles_dev, hist, digit, flags, ctrl, stage, dig);
+        in, out, sv, tile_start, hist, digit, flags, ctrl, stage, dig);
 }
 
 template <int WAVES, int KPT>
@@ -119,7 +119,7 @@ void launch_cfg_kv(const uint32_t* in, uint32_t* out, const uint32_t* vin, uint3
   const uint32_t stage = kStagePass0 + static_cast<uint32_t>(pass);
   const RadixDigit dig{8u * static_cast<uint32_t>(pass)};
   onesweep_kernel<WAVES, KPT, RadixDigit, true, true><<<total_tiles, WAVES * 64, 0, s>>>(
-      in, out, sv, tile_start, nullptr, hist, pass, flags, ctrl, stage, dig, vin, vout);
+      in, out, sv, tile_start, hist, pass, flags, ctrl, stage, dig, vin, vout);
 }
 
 }  // namespace
@@ -158,17 +158,16 @@ void launch_onesweep_pass(const uint32_t* in, uint32_t* out,
                           const SegView& sv, const int32_t* tile_start,
                           int32_t total_tiles, const uint32_t* hist,
                           uint64_t* flags, uint32_t* ctrl, int pass, bool stable,
-                          const TuneTable& tt, hipStream_t s, int bits,
-                          const int32_t* tiles_dev) {
+                          const TuneTable& tt, hipStream_t s, int bits) {
   if (total_tiles <= 0) return;
   if (bits == 10) {
     const uint32_t stage = kStagePass0 + static_cast<uint32_t>(pass);
     if (tt.sort10_kpt == 16)
       launch_cfg10<16>(in, out, sv, tile_start, total_tiles, hist, flags, ctrl, pass, stage,
-                       stable, tiles_dev, s);
+                       stable, s);
     else
       launch_cfg10<8>(in, out, sv, tile_start, total_tiles, hist, flags, ctrl, pass, stage,
-                      stable, tiles_dev, s);
+                      stable, s);
     return;
   }
 #define OCP_SORT_CFG(W, K)                                                   \

@@ -23,7 +23,9 @@ __global__ __launch_bounds__(256) void begin_kernel(uint32_t* ctrl,
   if (tid == 0) {
     ctrl[kCtrlEpoch] = ctrl[kCtrlEpoch] + 1;
     ctrl[kCtrlLearnBad] = 0;
-    ctrl[kCtrlMsdRun] = 0;
+    ctrl[kCtrlMsdBig] = 0;
+    ctrl[kCtrlMsdTiles] = 0;
+    ctrl[kCtrlMsdSlots] = 0;
   }
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
   for (int64_t i = tid; i < n_hist; i += stride) hist[i] = 0;
@@ -77,6 +79,7 @@ __global__ __launch_bounds__(1024) void oct_offsets_kernel(
     mail[kCtrlOctTotal] = static_cast<uint32_t>(carry);
     mail[kCtrlOctOk] = carry <= k_cap ? 1u : 0u;
     mail[kCtrlTimeout] = ctrl[kCtrlTimeout];
+    mail[kCtrlMsdTiles] = ctrl[kCtrlMsdTiles];
   }
 }
 

@@ -16,10 +16,12 @@ enum CtrlSlot : int {
   kCtrlEpoch = 8,      // bumped once per launch group; tags lookback flags
   kCtrlOctTotal = 9,   // total octree slots of the batch
   kCtrlOctOk = 10,     // 1 when the octree fits the node capacity
-  kCtrlMsdRun = 11,    // MSD sort: 0, or 0x7fffffff when the LSD passes must run
+  kCtrlMsdBig = 11,    // MSD sort: digits listed for the second level,
   kCtrlLearnBad = 12,  // learned sort: misordered bucket boundaries
   kCtrlTimeout = 13,   // mark of the launch whose wait gave up (0: none)
   kCtrlWaitLimit = 14, // 0: waits poll up to kSpinLimit times; v > 0: v - 1
+  kCtrlMsdTiles = 15,  // ... their tiles
+  kCtrlMsdSlots = 16,  // ... and the count slots of their long runs
   kCtrlWords = 64,
 };
 
@@ -69,7 +71,7 @@ struct TuneTable {
   int sort_bits = 8;       // digit width of a build's sort: 8 (4 passes) or 10 (3)
   int sort10_kpt = 8;      // keys per thread of a 10-bit pass (16 waves)
   int oct_order = 0;       // 0 or 1, kept for saved tables: one octree kernel serves both
-  int sort_msd = 0;        // 10-bit digits: LSD passes (0) or MSD scatter + LDS buckets (1)
+  int sort_msd = 0;        // 10-bit digits: LSD passes (0) or MSD scatter + LDS windows (1)
 };
 
 inline int sort_tile(const TuneTable& t) { return t.sort_waves * 64 * t.sort_kpt; }
@@ -78,12 +80,31 @@ inline int sort_tile(const TuneTable& t) { return t.sort_waves * 64 * t.sort_kpt
 inline int pipe_sort_bits(const TuneTable& t, bool perm) {
   return (t.sort_bits == 10 && !perm) ? 10 : 8;
 }
-// The MSD form: chosen, 10-bit digits, and few enough segments for one
-// workgroup per (segment, bucket).
-constexpr int32_t kMsdMaxSegments = 2048;  // grid: n_seg * 1024 workgroups of 1024
+// The MSD form: chosen, 10-bit digits, and few enough segments that 1024
+// counts and cursors each are no more than the keys.
+constexpr int32_t kMsdMaxSegments = 2048;
 inline bool pipe_sort_msd(const TuneTable& t, bool perm, int32_t n_seg) {
   return t.sort_msd != 0 && pipe_sort_bits(t, perm) == 10 && n_seg <= kMsdMaxSegments;
 }
+// A build whose caller set no table takes the MSD form by itself, unless it
+// carries the permutation (its passes are stable) or has more clouds than that
+// form takes. Whole builds, four 8-bit passes against it, uniform points:
+// 307,200 114 -> 92 us, 2^20 150 -> 120, 2^22 322 -> 240, 10M 596 -> 475.
+// Below 16,384 points the sort is launches either way.
+inline bool auto_sort_msd(int64_t n, int32_t n_seg, bool perm) {
+  return !perm && n >= 16384 && n_seg <= kMsdMaxSegments;
+}
+// Where many keys crowd into few digits, most of them take the second level:
+// 2^24 clustered points 528 -> 495 us, but 2^20 145 -> 160 and 2^22 232 -> 250.
+// So below 12M points a cloud, a build after which more than a sixteenth of the
+// keys turns out to have gone there (the host learns it with the counts) is
+// followed by kSkewBuilds builds of about its size with the LSD passes, then by
+// another try. The result is the same either way.
+inline bool auto_sort_skew(int64_t max_seg) { return max_seg < 12000000; }
+constexpr int32_t kSkewBuilds = 256;
+// Tiles of 16K keys for the scatter once there are enough of them (10M: 47 ->
+// 39 us), else of 8K.
+inline int auto_sort10_kpt(int64_t max_seg) { return max_seg >= (int64_t(1) << 22) ? 16 : 8; }
 inline int pipe_sort_tile(const TuneTable& t, bool perm) {
   return pipe_sort_bits(t, perm) == 10 ? 1024 * t.sort10_kpt : sort_tile(t);
 }
@@ -166,32 +187,52 @@ void launch_onesweep_pass(const uint32_t* in, uint32_t* out,
                           const SegView& sv, const int32_t* tile_start,
                           int32_t total_tiles, const uint32_t* hist,
                           uint64_t* flags, uint32_t* ctrl, int pass, bool stable,
-                          const TuneTable& tt, hipStream_t s, int bits = 8,
-                          const int32_t* tiles_dev = nullptr);  // (10-bit passes)
+                          const TuneTable& tt, hipStream_t s, int bits = 8);
 // MSD sort of bare 30-bit keys (k_msd.hip): the scatter by the top 10-bit
-// digit (histogram slot 2 of the 10-bit histograms), then one workgroup per
-// (segment, bucket) sorting it in LDS in place; a segment with a bucket too
-// large for LDS raises ctrl[kCtrlMsdRun] instead, which gates the histogram
-// of the two lower digits and the LSD passes that then sort everything
-// again. Grid: n_seg * 1024 workgroups; max_seg (the largest segment's
-// length) picks the LDS capacity.
-void launch_msd_buckets(uint32_t* keys, const SegView& sv, const uint32_t* hist, uint32_t* ctrl,
-                        int64_t max_seg, hipStream_t s);
-// The scatter without a lookback: cursor holds n_seg * 1024 zeroed words
-// (one per bucket), claimed by atomic adds; tiles of 1024 * sort10_kpt keys.
+// digit (histogram slot 2 of the 10-bit histograms) without a lookback (cursor
+// holds n_seg * 1024 zeroed words, claimed by atomic adds; tiles of 1024 *
+// sort10_kpt keys), LDS sorts of windows of msd_window(max_seg) keys of the
+// result, and a second level for the digits too large for LDS.
+struct MsdLevel2 {
+  int4* big;         // listed digits {first key, keys, top digit, first shared slot}
+  int2* tiles;       // second-level tiles {listed digit, tile in it}
+  uint32_t* hist;    // [max_big][1024] counts of bits 10-19
+  uint32_t* cursor;  // [max_big][1024]
+  uint32_t* hist3;   // [max_slots][1024] low-bit counts of long one-prefix runs
+  int32_t max_big, max_tiles, max_slots;
+};
+// Segments of up to 2800 keys a digit on average sort windows in 4096-key
+// workgroups of four waves (four a CU by LDS), larger ones in 12288-key
+// workgroups of eight (two a CU): at 2^20 points 1024 keys a digit, 10M 9800.
+inline bool msd_small(int64_t max_seg) { return max_seg <= 1024 * 2800; }
+// Keys per window; 0: one workgroup per digit, where a digit about fills it.
+inline int32_t msd_window(int64_t max_seg) {
+  return msd_small(max_seg) ? 1024 : max_seg <= 1024 * 6000 ? 4096 : 0;
+}
+inline int64_t msd_windows(int64_t len, int64_t max_seg) {
+  const int32_t w = msd_window(max_seg);
+  return w ? (len + w - 1) / w : (len > 0 ? 1024 : 0);
+}
+// Room for the second level of n keys, whatever they are: listed digits hold
+// more than the LDS capacity each.
+inline void msd_level2_caps(int64_t n, int64_t max_seg, MsdLevel2* l2) {
+  l2->max_big = static_cast<int32_t>(n / (msd_small(max_seg) ? 4096 : 12288) + 1);
+  l2->max_tiles = static_cast<int32_t>(n / 8192 + l2->max_big + 1);
+  l2->max_slots = static_cast<int32_t>(n / 65536 + 1);
+}
 void launch_msd_scatter(const uint32_t* in, uint32_t* out, const SegView& sv,
                         const int32_t* tile_start, int32_t total_tiles, const uint32_t* hist,
                         uint32_t* cursor, const uint32_t* ctrl, const TuneTable& tt,
                         hipStream_t s);
+void launch_msd_windows(uint32_t* keys, const SegView& sv, const int32_t* tile_start,
+                        int32_t total_tiles, int64_t max_seg, const uint32_t* hist,
+                        const MsdLevel2& l2, uint32_t* ctrl, hipStream_t s);
+// `other` is overwritten where digits are listed.
+void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, const uint32_t* ctrl,
+                       hipStream_t s);
 // Cursor words per segment after the segments' histograms (the first sort
 // pass's or the MSD scatter's: one per digit, at most 1024).
 constexpr int kCursorWords = 1024;
-// Digit counts of the two lower 10-bit digits (histogram slots 0 and 1),
-// only when ctrl[kCtrlMsdRun] is set; tiles as the Morton kernel's.
-void launch_msd_low_hist(const uint32_t* keys, const SegView& sv, const int32_t* tile_start,
-                         int32_t total_tiles, uint32_t* hist, const uint32_t* ctrl,
-                         const TuneTable& tt, hipStream_t s);
-
 // First pass of an LSD sort of bare keys (digit key & 255, or key & 1023
 // with bits == 10; any order among equal digits) as a cursor scatter
 // (cursor_scatter.hpp): no lookback; one zeroed cursor per segment and

@@ -74,13 +74,11 @@ struct RadixDigit10 {
 };
 
 // hist: per segment hist_stride(kBits) words; this pass reads the 2^kBits
-// words from slot * 2^kBits of its segment. tiles_dev (optional): the number
-// of real tiles, on device, when the grid is sized for an upper bound.
+// words from slot * 2^kBits of its segment.
 template <int WAVES, int KPT, class Digit, bool STABLE = true, bool KV = false>
 __global__ __launch_bounds__(WAVES * 64) void onesweep_kernel(
     const uint32_t* __restrict__ in, uint32_t* __restrict__ out, SegView sv,
-    const int32_t* __restrict__ tile_start, const int32_t* __restrict__ tiles_dev,
-    const uint32_t* __restrict__ hist, int hist_slot, uint64_t* __restrict__ flags,
+    const int32_t* __restrict__ tile_start, const uint32_t* __restrict__ hist, int hist_slot, uint64_t* __restrict__ flags,
     uint32_t* __restrict__ ctrl, uint32_t stage, Digit dig,
     const uint32_t* __restrict__ vin = nullptr, uint32_t* __restrict__ vout = nullptr) {
   constexpr int THREADS = WAVES * 64;
@@ -101,7 +99,6 @@ __global__ __launch_bounds__(WAVES * 64) void onesweep_kernel(
   __shared__ uint32_t s_trivial;
 
   const int32_t t = blockIdx.x;
-  if (tiles_dev && t >= *tiles_dev) return;
   const uint32_t tag = ctrl[kCtrlEpoch] * 8u + stage;
   if (stopped(ctrl, tag)) return;
   const int tid = threadIdx.x;
