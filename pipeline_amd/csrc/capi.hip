@@ -1525,18 +1525,27 @@ struct TempBuffers {
   }
 };
 
-// Total slots of the last build and each segment's root level (validator
-// and compact form). Settles the build first.
+// Total slots of the last build. Settles it first.
+int build_slots(ocp_ctx c, int64_t* k_total) {
+  if (int r = settle(c)) return r;
+  if (c->mail_current) {
+    *k_total = c->mail[kCtrlOctTotal];
+    return OCP_OK;
+  }
+  uint32_t* got = c->mail + kMailWords;
+  OCP_HIP(c, hipMemcpyAsync(got, c->ws.oct_start + c->last_plan.n_seg, sizeof(int32_t),
+                            hipMemcpyDeviceToHost, c->stream));
+  OCP_HIP(c, hipStreamSynchronize(c->stream));
+  *k_total = *got;
+  return OCP_OK;
+}
+
+// ... and each segment's root level (validator).
 int format_setup(ocp_ctx c, TempBuffers& tb, int64_t* k_total, int32_t** root_level,
                  uint32_t** root_code) {
-  if (int r = settle(c)) return r;
+  if (int r = build_slots(c, k_total)) return r;
   const Workspace& w = c->ws;
   const Plan& p = c->last_plan;
-  int32_t kt = 0;
-  OCP_HIP(c, hipMemcpyAsync(&kt, w.oct_start + p.n_seg, sizeof(int32_t), hipMemcpyDeviceToHost,
-                            c->stream));
-  OCP_HIP(c, hipStreamSynchronize(c->stream));
-  *k_total = kt;
   if (int r = tb.alloc(c, root_level, p.n_seg)) return r;
   if (int r = tb.alloc(c, root_code, p.n_seg)) return r;
   launch_seg_roots(w.keys_b, w.prefix_n, w.counts, p.sv.start, p.n_seg, *root_level, *root_code,
@@ -1580,44 +1589,45 @@ int ocp_compact_octree(ocp_ctx c, ocp_compact_node* nodes, int64_t node_cap, int
                        int64_t child_cap, int64_t* n_nodes, int64_t* n_children) {
   if (check_ctx(c) || !n_nodes || !n_children || node_cap < 0 || child_cap < 0)
     return OCP_ERR_INVALID;
-  TempBuffers tb;
   int64_t kt = 0;
-  int32_t* root_level = nullptr;
-  uint32_t* root_code = nullptr;
-  if (int r = format_setup(c, tb, &kt, &root_level, &root_code)) return r;
+  if (int r = build_slots(c, &kt)) return r;
   const Workspace& w = c->ws;
   const Plan& p = c->last_plan;
-  int32_t* cnt = nullptr;
-  uint32_t* bsum = nullptr;
-  unsigned long long* bad = nullptr;
-  const int64_t nb = compact_scan_blocks(kt);
-  if (int r = tb.alloc(c, &cnt, kt)) return r;
-  if (int r = tb.alloc(c, &bsum, nb + 1)) return r;
-  if (int r = tb.alloc(c, &bad, 1)) return r;
-  OCP_HIP(c, hipMemsetAsync(bad, 0, sizeof(unsigned long long), c->stream));
-  launch_compact_count(w.nodes, w.oct_start, p.n_seg, p.sv.mn, p.sv.rg, p.sv.min1, p.sv.range1,
-                       root_level, kt, cnt, bsum, bad, c->stream);
+  // Room for the pass's flags, and a word that counts what it cannot hold.
+  // (Its waits are reported here, so the build's mail stays the last word.)
+  const bool mail_current = c->mail_current;
+  if (int r = ensure_scratch(c, 2 * compact_tiles(kt) + 1)) return r;
+  c->mail_current = mail_current;
+  auto* bad = reinterpret_cast<unsigned long long*>(c->s_hist);
+  uint32_t* mail = c->mail + kMailWords;
+  mail[0] = mail[1] = mail[2] = 0;
+  // (size queries, and calls whose node array is too small, store nothing)
+  const bool store = nodes && children && node_cap >= kt;
+  launch_begin(c->ctrl, c->s_hist, 2, c->stream);
+  launch_compact(w.nodes, kt, w.oct_start, p.n_seg, p.sv.mn, p.sv.rg, p.sv.min1, p.sv.range1,
+                 p.sv.start, w.counts, w.prefix_n, c->s_flags, c->ctrl, store ? nodes : nullptr,
+                 store ? children : nullptr, child_cap, bad, mail, c->stream);
   OCP_CHECK_LAUNCH(c);
-  uint32_t total = 0;
-  unsigned long long hbad = 0;
-  OCP_HIP(c, hipMemcpyAsync(&total, bsum + nb, sizeof(total), hipMemcpyDeviceToHost, c->stream));
-  OCP_HIP(c, hipMemcpyAsync(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost, c->stream));
   OCP_HIP(c, hipStreamSynchronize(c->stream));
+  if (mail[1]) {
+    c->mail_current = false;
+    return sync_and_check(c);
+  }
+  const int64_t total = mail[0];
   *n_nodes = kt;
   *n_children = total;
-  if (hbad)
+  if (mail[2]) {
+    unsigned long long hbad = 0;
+    OCP_HIP(c, hipMemcpy(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost));
     return fail(c, OCP_ERR_STATE, std::to_string(hbad) +
                                       " octree slots have no exact compact form (corner off "
                                       "its level's grid or cell size not range / 2^k)");
+  }
   if (!nodes || !children) return OCP_OK;  // size query
-  if (node_cap < kt || child_cap < static_cast<int64_t>(total))
+  if (node_cap < kt || child_cap < total)
     return fail(c, OCP_ERR_CAPACITY, "compact octree: output arrays too small (need " +
                                          std::to_string(kt) + " nodes, " +
                                          std::to_string(total) + " children)");
-  launch_compact_write(w.nodes, w.oct_start, p.n_seg, p.sv.mn, p.sv.rg, p.sv.min1, p.sv.range1,
-                       root_level, cnt, nodes, children, c->stream);
-  OCP_CHECK_LAUNCH(c);
-  OCP_HIP(c, hipStreamSynchronize(c->stream));
   return OCP_OK;
 }
 

@@ -233,158 +233,263 @@ struct CompactNode {
 };
 static_assert(sizeof(CompactNode) == 12, "compact node layout");
 
+// depth_of, for the cell sizes of an octree by way of their exponents: a
+// quotient by 2^k lowers the exponent by k and keeps the fraction as long as
+// it stays a normal number.
+__device__ __forceinline__ int32_t depth_fast(float cell, float rg) {
+  const uint32_t c = __float_as_uint(cell), r = __float_as_uint(rg);
+  const int32_t k = static_cast<int32_t>(r >> 23) - static_cast<int32_t>(c >> 23);
+  const bool normal = (c >> 23) - 1u < 254u && (r >> 23) - 1u < 254u;  // positive, finite
+  if (normal && ((c ^ r) & 0x7fffffu) == 0 && k >= 0 && k <= 11) return k;
+  return depth_of(cell, rg);
+}
+
+// axis_value, where one value in sight decodes to c: that value lies within
+// one of (c - min) / range * 1024, so it is the one axis_value finds first.
+__device__ __forceinline__ int32_t axis_fast(float c, int axis, int32_t level, float mn, float rg,
+                                             float inv) {
+  const auto decoded = [&](int32_t q) {  // decode_axis of the value itself
+    return static_cast<float>(q) / 1024.0f * rg + mn;
+  };
+  const float est = (c - mn) * inv;
+  if (est > -1.0f && est < 1024.0f) {
+    const int32_t q = static_cast<int32_t>(rintf(est));
+    const uint32_t grid = (1u << (level_shift(level) / 3u)) - 1u;
+    if (q >= 0 && q <= 1023 && (static_cast<uint32_t>(q) & grid) == 0 &&
+        __float_as_uint(decoded(q)) == __float_as_uint(c) && decoded(q - 1) != c &&
+        decoded(q + 1) != c)
+      return q;
+  }
+  return axis_value(c, axis, level, mn, rg);
+}
+
 // The header of a slot without its first-child index, or false when the
-// slot has no exact compact form.
-__device__ __forceinline__ bool compact_header(const OctNode& nd, float mn, float rg, int32_t rl,
-                                               CompactNode* cn) {
+// slot has no exact compact form. w: the node's 15 words.
+__device__ __forceinline__ bool compact_header(const int32_t (&w)[15], float mn, float rg,
+                                               int32_t rl, CompactNode* cn) {
   *cn = CompactNode{};
-  uint32_t set = 0;
+  uint32_t set = 0, any = 0;
 #pragma unroll
-  for (int q = 0; q < 8; ++q) set |= (nd.children[q] != 0 ? 1u : 0u) << q;
+  for (int q = 0; q < 8; ++q) set |= (w[q] != 0 ? 1u : 0u) << q;
+#pragma unroll
+  for (int q = 0; q < 15; ++q) any |= static_cast<uint32_t>(w[q]);
   cn->child_set = static_cast<uint8_t>(set);
-  if (!any_word(nd)) {
+  if (any == 0) {
     cn->level = 0xff;
     return true;
   }
-  const int32_t depth = depth_of(nd.cell_size, rg);
+  const int32_t depth = depth_fast(__int_as_float(w[12]), rg);
   if (depth < 0 || rl + depth > 14) return false;
-  const uint32_t pre = prefix_of(nd.corner, rl + depth, mn, rg);
-  if (pre == ~0u || __float_as_uint(nd.corner[3]) != __float_as_uint(1.0f) ||
-      static_cast<uint32_t>(nd.child_node_mask) > 255u ||
-      static_cast<uint32_t>(nd.child_leaf_mask) > 255u)
+  const float inv = 1024.0f / rg;
+  uint32_t pre = 0;
+  bool on_grid = true;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int32_t q = axis_fast(__int_as_float(w[8 + a]), a, rl + depth, mn, rg, inv);
+    on_grid &= q >= 0;
+    pre |= split_by_3(static_cast<uint32_t>(q)) << a;
+  }
+  if (!on_grid || w[11] != __float_as_int(1.0f) || static_cast<uint32_t>(w[13]) > 255u ||
+      static_cast<uint32_t>(w[14]) > 255u)
     return false;
   cn->prefix = pre;
   cn->level = static_cast<uint8_t>((rl + depth) | (depth << 4));
-  cn->node_mask = static_cast<uint8_t>(nd.child_node_mask);
-  cn->leaf_mask = static_cast<uint8_t>(nd.child_leaf_mask);
+  cn->node_mask = static_cast<uint8_t>(w[13]);
+  cn->leaf_mask = static_cast<uint8_t>(w[14]);
   return true;
 }
 
-// Pass 1: nonzero children per slot into cnt, and a count of slots with no
-// exact compact form.
-__global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
-    const OctNode* __restrict__ nodes, const int32_t* __restrict__ oct_start, int32_t n_seg,
-    Boxes bx, const int32_t* __restrict__ root_level, int32_t* __restrict__ cnt,
-    unsigned long long* __restrict__ bad) {
-  const int64_t k_total = oct_start[n_seg];
-  uint32_t nbad = 0;
-  for (int64_t g = blockIdx.x * int64_t(kFmtThreads) + threadIdx.x; g < k_total;
-       g += int64_t(gridDim.x) * kFmtThreads) {
-    const OctNode nd = nodes[g];
-    const int32_t seg = seg_of_slot(g, oct_start, n_seg);
-    CompactNode cn;
-    nbad += !compact_header(nd, bx.min_of(seg), bx.range_of(seg), root_level[seg], &cn);
-    cnt[g] = __popc(cn.child_set);
+// A segment's box and root level, as the kernels below need them for a slot.
+struct SegInfo {
+  float mn, rg;
+  int32_t root_level;
+};
+struct SegTables {
+  const int32_t* oct_start;
+  int32_t n_seg;
+  Boxes bx;
+  const int32_t* seg_start;  // or nullptr: one segment
+  const int32_t* n_unique;
+  const uint8_t* prefix_n;
+  __device__ __forceinline__ SegInfo of(int32_t seg) const {
+    const int32_t sb = seg_start ? seg_start[seg] : 0;
+    return {bx.min_of(seg), bx.range_of(seg), n_unique[seg] >= 2 ? prefix_n[sb] / 3 : 0};
   }
-  add_report(bad, 0, nbad);
+};
+
+constexpr int kFmtTile = 512;  // slots per workgroup of the compact and expand kernels
+
+// The compact form in one pass over the nodes: a tile's nodes come through LDS
+// in whole lines, a thread forms the headers of two, the tile's place in the
+// child array comes from the two-level lookback, and headers and children
+// leave through LDS, in whole lines again. nodes or children may be null (the
+// sizes only); children past child_cap are not stored. mail (host memory):
+// [0] the children's total, [1] a wait gave up, [2] slots without an exact
+// form exist (*bad counts them).
+// What bounds it: 60 bytes a slot read and ~28 written; 0.99M slots take
+// 27 us, where two passes over the nodes and three scan launches took 54, and
+// the call 50 us instead of 208.
+__global__ __launch_bounds__(kFmtThreads) void compact_kernel(
+    const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, uint64_t* __restrict__ flags,
+    uint32_t* __restrict__ ctrl, uint32_t* __restrict__ out, int32_t* __restrict__ children,
+    int64_t child_cap, unsigned long long* __restrict__ bad, uint32_t* __restrict__ mail) {
+  constexpr int NPT = kFmtTile / kFmtThreads;
+  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_tmp[kFmtThreads / 64];
+  __shared__ uint32_t s_excl;
+  const uint32_t tag = ctrl[kCtrlEpoch] * 8u + kStageScan;
+  if (stopped(ctrl, tag)) return;
+  const int tid = threadIdx.x;
+  const int32_t t = blockIdx.x;  // in-order dispatch: see lookback_n
+  const int64_t g0 = int64_t(t) * kFmtTile;
+  const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
+  const int32_t words = cnt * 15;
+  const int32_t* src = reinterpret_cast<const int32_t*>(nodes + g0);
+  if (cnt == kFmtTile) {
+    // (a tile starts on a multiple of 16 bytes: 512 nodes are 30,720)
+    constexpr int kVec = kFmtTile * 15 / 4;
+    constexpr int kRows = kVec / kFmtThreads;
+    static_assert(kVec - kRows * kFmtThreads == kFmtThreads / 2, "half a row is left");
+    const int4* v = reinterpret_cast<const int4*>(src) + tid;
+    int4* to = reinterpret_cast<int4*>(s_words) + tid;
+    int4 x[kRows];
+    int4 y = make_int4(0, 0, 0, 0);
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) x[k] = v[k * kFmtThreads];
+    if (tid < kFmtThreads / 2) y = v[kRows * kFmtThreads];
+#pragma unroll
+    for (int k = 0; k < kRows; ++k) to[k * kFmtThreads] = x[k];
+    if (tid < kFmtThreads / 2) to[kRows * kFmtThreads] = y;
+  } else {
+    for (int32_t q = tid; q < words; q += kFmtThreads) s_words[q] = src[q];
+  }
+  // The tile's segment, when one holds all of it.
+  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
+  const bool one = st.oct_start[seg0 + 1] >= g0 + cnt;
+  SegInfo info = st.of(seg0);
+  __syncthreads();
+  // Thread: NPT neighbouring slots, so that its children are neighbours too.
+  CompactNode cn[NPT];
+  int32_t child[NPT][8];
+  uint32_t mine = 0, nbad = 0;
+#pragma unroll
+  for (int u = 0; u < NPT; ++u) {
+    const int32_t l = tid * NPT + u;
+    cn[u] = CompactNode{};
+    if (l >= cnt) continue;
+    int32_t w[15];
+#pragma unroll
+    for (int c = 0; c < 15; ++c) w[c] = s_words[l * 15 + c];
+    if (!one) info = st.of(seg_of_slot(g0 + l, st.oct_start, st.n_seg));
+    nbad += !compact_header(w, info.mn, info.rg, info.root_level, &cn[u]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) child[u][c] = w[c];
+    mine += __popc(cn[u].child_set);
+  }
+  uint32_t total;
+  const uint32_t before = block_excl_scan<kFmtThreads>(mine, s_tmp, &total);
+  if (wave_id() == 0) {
+    if (lane_id() == 0) flag_store(&flags[t], flag_pack(tag, kFlagAgg, total));
+    bool late = false;
+    const uint32_t prev = wave_lookback_groups(flags, flags + gridDim.x, t, 0, total, tag,
+                                               wait_limit(ctrl), &late);
+    if (lane_id() == 0) {
+      if (late) {
+        raise_timeout(ctrl, tag);
+        mail[1] = 1u;
+      }
+      s_excl = prev;
+      if (g0 + cnt == k_total) mail[0] = prev + total;
+    }
+  }
+  if (nbad) {
+    atomicAdd(bad, static_cast<unsigned long long>(nbad));
+    mail[2] = 1u;
+  }
+  __syncthreads();  // (every word of the nodes has been read)
+  if (!out || !children) return;
+  const uint32_t excl = s_excl;
+  uint32_t* s_child = reinterpret_cast<uint32_t*>(s_words);
+  uint32_t* s_head = s_child + kFmtTile * 8;
+  uint32_t o = before;
+#pragma unroll
+  for (int u = 0; u < NPT; ++u) {
+    const int32_t l = tid * NPT + u;
+    if (l >= cnt) continue;
+    cn[u].first_child = excl + o;
+    uint32_t hw[3];
+    __builtin_memcpy(hw, &cn[u], 12);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s_head[l * 3 + c] = hw[c];
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (child[u][c] != 0) s_child[o++] = static_cast<uint32_t>(child[u][c]);
+  }
+  __syncthreads();
+  uint32_t* head = out + g0 * 3;
+  for (int32_t q = tid; q < cnt * 3; q += kFmtThreads) head[q] = s_head[q];
+  for (uint32_t q = tid; q < total; q += kFmtThreads)
+    if (static_cast<int64_t>(excl) + q < child_cap)
+      children[static_cast<int64_t>(excl) + q] = static_cast<int32_t>(s_child[q]);
 }
 
-// Pass 2: headers and children; incl is the inclusive scan of the counts.
-__global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
-    const OctNode* __restrict__ nodes, const int32_t* __restrict__ oct_start, int32_t n_seg,
-    Boxes bx, const int32_t* __restrict__ root_level, const int32_t* __restrict__ incl,
-    CompactNode* __restrict__ out, int32_t* __restrict__ children) {
-  const int64_t k_total = oct_start[n_seg];
-  for (int64_t g = blockIdx.x * int64_t(kFmtThreads) + threadIdx.x; g < k_total;
-       g += int64_t(gridDim.x) * kFmtThreads) {
-    const OctNode nd = nodes[g];
-    const int32_t seg = seg_of_slot(g, oct_start, n_seg);
-    CompactNode cn;
-    (void)compact_header(nd, bx.min_of(seg), bx.range_of(seg), root_level[seg], &cn);
-    int32_t o = incl[g] - __popc(cn.child_set);
-    cn.first_child = static_cast<uint32_t>(o);
-    for (int q = 0; q < 8; ++q)
-      if (nd.children[q] != 0) children[o++] = nd.children[q];
-    out[g] = cn;
-  }
-}
-
-// 60-byte nodes from the compact form. Child indices at or past n_children
-// read as 0.
+// 60-byte nodes from the compact form, a tile's through LDS so that whole
+// lines leave. Child indices at or past n_children read as 0.
+// What bounds it: 60 bytes a slot written and ~28 read; 0.99M slots take 16 us
+// (26 with the 60 bytes stored by each thread for itself).
 __global__ __launch_bounds__(kFmtThreads) void expand_kernel(
     const CompactNode* __restrict__ in, const int32_t* __restrict__ children, int64_t n_children,
     const int32_t* __restrict__ oct_start, int32_t n_seg, Boxes bx, OctNode* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  const int tid = threadIdx.x;
   const int64_t k_total = oct_start[n_seg];
-  for (int64_t g = blockIdx.x * int64_t(kFmtThreads) + threadIdx.x; g < k_total;
-       g += int64_t(gridDim.x) * kFmtThreads) {
-    const CompactNode cn = in[g];
-    OctNode nd{};
-    int64_t o = cn.first_child;
-    for (int q = 0; q < 8; ++q) {
-      if (!((cn.child_set >> q) & 1u)) continue;
-      // a malformed node (offset outside [0, n_children)) reads no memory
-      nd.children[q] = (o >= 0 && o < n_children) ? children[o] : 0;
-      ++o;
-    }
-    if (cn.level != 0xff) {
-      const int32_t seg = seg_of_slot(g, oct_start, n_seg);
+  for (int64_t g0 = int64_t(blockIdx.x) * kFmtTile; g0 < k_total;
+       g0 += int64_t(gridDim.x) * kFmtTile) {
+    const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
+    const int32_t seg0 = seg_of_slot(g0, oct_start, n_seg);
+    const bool one = oct_start[seg0 + 1] >= g0 + cnt;
+#pragma unroll
+    for (int u = 0; u < kFmtTile / kFmtThreads; ++u) {
+      const int32_t l = u * kFmtThreads + tid;
+      if (l >= cnt) continue;
+      const CompactNode cn = in[g0 + l];
+      int32_t* w = s_words + l * 15;
+      int64_t o = cn.first_child;
+      int32_t ch[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        ch[q] = 0;
+        if (!((cn.child_set >> q) & 1u)) continue;
+        // a malformed node (offset outside [0, n_children)) reads no memory
+        if (o < n_children) ch[q] = children[o];
+        ++o;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) w[q] = ch[q];
+      const bool written = cn.level != 0xff;
+      const int32_t seg = one ? seg0 : seg_of_slot(g0 + l, oct_start, n_seg);
       const float mn = bx.min_of(seg), rg = bx.range_of(seg);
-      nd.corner[0] = decode_axis(cn.prefix, 0, mn, rg);
-      nd.corner[1] = decode_axis(cn.prefix, 1, mn, rg);
-      nd.corner[2] = decode_axis(cn.prefix, 2, mn, rg);
-      nd.corner[3] = 1.0f;
       const uint32_t sh = static_cast<uint32_t>(cn.level >> 4) & 31u;
-      nd.cell_size = rg / static_cast<float>(static_cast<int32_t>(1u << sh));
-      nd.child_node_mask = cn.node_mask;
-      nd.child_leaf_mask = cn.leaf_mask;
+      w[8] = written ? __float_as_int(decode_axis(cn.prefix, 0, mn, rg)) : 0;
+      w[9] = written ? __float_as_int(decode_axis(cn.prefix, 1, mn, rg)) : 0;
+      w[10] = written ? __float_as_int(decode_axis(cn.prefix, 2, mn, rg)) : 0;
+      w[11] = written ? __float_as_int(1.0f) : 0;
+      w[12] = written ? __float_as_int(rg / static_cast<float>(static_cast<int32_t>(1u << sh))) : 0;
+      w[13] = written ? cn.node_mask : 0;
+      w[14] = written ? cn.leaf_mask : 0;
     }
-    out[g] = nd;
-  }
-}
-
-// ---- inclusive scan of n int32 counts in place (three launches, no
-// inter-workgroup waits). bsum: n_blocks + 1 words; bsum[n_blocks] = total.
-constexpr int kScanItems = 16;
-constexpr int kScanBlock = kFmtThreads * kScanItems;
-
-__global__ __launch_bounds__(kFmtThreads) void scan_reduce_kernel(const int32_t* __restrict__ a,
-                                                                  int64_t n,
-                                                                  uint32_t* __restrict__ bsum) {
-  __shared__ uint32_t tmp[kFmtThreads / 64];
-  const int64_t b0 = int64_t(blockIdx.x) * kScanBlock;
-  uint32_t s = 0;
-  for (int u = 0; u < kScanItems; ++u) {
-    const int64_t i = b0 + int64_t(u) * kFmtThreads + threadIdx.x;
-    if (i < n) s += static_cast<uint32_t>(a[i]);
-  }
-  uint32_t total;
-  (void)block_excl_scan<kFmtThreads>(s, tmp, &total);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(1024) void scan_blocks_kernel(uint32_t* __restrict__ bsum,
-                                                           int32_t nb) {
-  __shared__ uint32_t tmp[16];
-  uint32_t carry = 0;
-  for (int32_t c = 0; c < nb; c += 1024) {
-    const int32_t k = c + static_cast<int32_t>(threadIdx.x);
-    const uint32_t v = k < nb ? bsum[k] : 0u;
-    uint32_t total;
-    const uint32_t ex = block_excl_scan<1024>(v, tmp, &total);
-    if (k < nb) bsum[k] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) bsum[nb] = carry;
-}
-
-__global__ __launch_bounds__(kFmtThreads) void scan_apply_kernel(int32_t* __restrict__ a,
-                                                                 int64_t n,
-                                                                 const uint32_t* __restrict__ bsum) {
-  __shared__ uint32_t tmp[kFmtThreads / 64];
-  const int64_t t0 = int64_t(blockIdx.x) * kScanBlock + int64_t(threadIdx.x) * kScanItems;
-  uint32_t v[kScanItems];
-  uint32_t s = 0;
-#pragma unroll
-  for (int u = 0; u < kScanItems; ++u) {
-    v[u] = t0 + u < n ? static_cast<uint32_t>(a[t0 + u]) : 0u;
-    s += v[u];
-  }
-  uint32_t total;
-  uint32_t run = bsum[blockIdx.x] + block_excl_scan<kFmtThreads>(s, tmp, &total);
-#pragma unroll
-  for (int u = 0; u < kScanItems; ++u) {
-    run += v[u];
-    if (t0 + u < n) a[t0 + u] = static_cast<int32_t>(run);
+    __syncthreads();
+    int32_t* dst = reinterpret_cast<int32_t*>(out + g0);
+    const int32_t words = cnt * 15;
+    for (int32_t q = tid * 4; q < words; q += kFmtThreads * 4) {
+      if (q + 4 <= words) {
+        const int4 v = *reinterpret_cast<const int4*>(s_words + q);
+        __builtin_memcpy(dst + q, &v, 16);
+      } else {
+        for (int32_t c = q; c < words; ++c) dst[c] = s_words[c];
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -412,33 +517,17 @@ void launch_validate(const OctNode* nodes, const int32_t* edge, const int32_t* o
                                                    root_code, rep);
 }
 
-int64_t compact_scan_blocks(int64_t k_total) { return (k_total + kScanBlock - 1) / kScanBlock; }
+int64_t compact_tiles(int64_t k_total) { return (k_total + kFmtTile - 1) / kFmtTile; }
 
-void launch_compact_count(const OctNode* nodes, const int32_t* oct_start, int32_t n_seg,
-                          const float* smin, const float* srg, float mn1, float rg1,
-                          const int32_t* root_level, int64_t k_total, int32_t* cnt,
-                          uint32_t* bsum, unsigned long long* bad, hipStream_t s) {
-  if (n_seg <= 0) return;
-  const Boxes bx{smin, srg, mn1, rg1};
-  compact_count_kernel<<<kFmtGrid, kFmtThreads, 0, s>>>(nodes, oct_start, n_seg, bx, root_level,
-                                                        cnt, bad);
-  const int64_t nb = compact_scan_blocks(k_total);
-  if (nb > 0)
-    scan_reduce_kernel<<<static_cast<uint32_t>(nb), kFmtThreads, 0, s>>>(cnt, k_total, bsum);
-  scan_blocks_kernel<<<1, 1024, 0, s>>>(bsum, static_cast<int32_t>(nb));
-  if (nb > 0)
-    scan_apply_kernel<<<static_cast<uint32_t>(nb), kFmtThreads, 0, s>>>(cnt, k_total, bsum);
-}
-
-void launch_compact_write(const OctNode* nodes, const int32_t* oct_start, int32_t n_seg,
-                          const float* smin, const float* srg, float mn1, float rg1,
-                          const int32_t* root_level, const int32_t* incl, void* out,
-                          int32_t* children, hipStream_t s) {
-  if (n_seg <= 0) return;
-  const Boxes bx{smin, srg, mn1, rg1};
-  compact_write_kernel<<<kFmtGrid, kFmtThreads, 0, s>>>(nodes, oct_start, n_seg, bx, root_level,
-                                                        incl, static_cast<CompactNode*>(out),
-                                                        children);
+void launch_compact(const OctNode* nodes, int64_t k_total, const int32_t* oct_start, int32_t n_seg,
+                    const float* smin, const float* srg, float mn1, float rg1,
+                    const int32_t* seg_start, const int32_t* n_unique, const uint8_t* prefix_n,
+                    uint64_t* flags, uint32_t* ctrl, void* out, int32_t* children,
+                    int64_t child_cap, unsigned long long* bad, uint32_t* mail, hipStream_t s) {
+  if (n_seg <= 0 || k_total <= 0) return;
+  const SegTables st{oct_start, n_seg, Boxes{smin, srg, mn1, rg1}, seg_start, n_unique, prefix_n};
+  compact_kernel<<<static_cast<uint32_t>(compact_tiles(k_total)), kFmtThreads, 0, s>>>(
+      nodes, k_total, st, flags, ctrl, static_cast<uint32_t*>(out), children, child_cap, bad, mail);
 }
 
 void launch_expand(const void* in, const int32_t* children, int64_t n_children,

@@ -343,18 +343,16 @@ void launch_validate(const OctNode* nodes, const int32_t* edge, const int32_t* o
                      int32_t n_seg, const float* smin, const float* srg, float mn1, float rg1,
                      const int32_t* root_level, const uint32_t* root_code, uint8_t* cov,
                      unsigned long long* rep, hipStream_t s);
-// Scan blocks of the compact pass (bsum holds this + 1 words).
-int64_t compact_scan_blocks(int64_t k_total);
-// cnt[k_total] <- inclusive scan of nonzero children per slot; bsum[nb] =
-// total; *bad += slots without an exact compact form (zeroed beforehand).
-void launch_compact_count(const OctNode* nodes, const int32_t* oct_start, int32_t n_seg,
-                          const float* smin, const float* srg, float mn1, float rg1,
-                          const int32_t* root_level, int64_t k_total, int32_t* cnt,
-                          uint32_t* bsum, unsigned long long* bad, hipStream_t s);
-void launch_compact_write(const OctNode* nodes, const int32_t* oct_start, int32_t n_seg,
-                          const float* smin, const float* srg, float mn1, float rg1,
-                          const int32_t* root_level, const int32_t* incl, void* out,
-                          int32_t* children, hipStream_t s);
+// The compact form of k_total slots in one pass, in the lookback epoch that a
+// launch_begin before it began (flags: 2 * compact_tiles(k_total) words; *bad
+// zeroed). out and children may be null. mail: three words of host memory,
+// zeroed (see compact_kernel).
+int64_t compact_tiles(int64_t k_total);
+void launch_compact(const OctNode* nodes, int64_t k_total, const int32_t* oct_start, int32_t n_seg,
+                    const float* smin, const float* srg, float mn1, float rg1,
+                    const int32_t* seg_start, const int32_t* n_unique, const uint8_t* prefix_n,
+                    uint64_t* flags, uint32_t* ctrl, void* out, int32_t* children,
+                    int64_t child_cap, unsigned long long* bad, uint32_t* mail, hipStream_t s);
 void launch_expand(const void* in, const int32_t* children, int64_t n_children,
                    const int32_t* oct_start, int32_t n_seg, const float* smin, const float* srg,
                    float mn1, float rg1, OctNode* out, hipStream_t s);
