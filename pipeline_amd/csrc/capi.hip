@@ -669,6 +669,22 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
     for (bool& r : c->kran) r = false;
     c->kmsd = msd;
   }
+  if (small_clouds(p.max_seg, p.n_seg, p.permutation) && !c->tuned && !c->stage_timing) {
+    const SmallOut o{w.keys_a, w.keys_b, w.prefix_n, w.hl, w.hr, w.lc, w.par, w.edge, w.offs,
+                     n_unique, kalloc, w.oct_start};
+    const bool single = p.n_seg == 1;
+    launch_small_clouds(pts, f3, p.sv, p.max_seg, p.device_boxes, w.boxes, w.boxes + w.seg_cap, o,
+                        c->ctrl, w.k_cap, single ? c->mail : nullptr, s);
+    if (!single)
+      launch_oct_offsets(n_unique, kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, c->mail, s);
+    const bool ok = launch_oct_build(pipeline_oct_args(c), p.sv, p.ts_node, p.tiles_node, s);
+    // (no wait on another workgroup here; a later frame's lookback launches
+    // still come after those of the frames before this one)
+    if (c->order_wait && !capturing) c->order_err = hipStreamWaitEvent(s, c->order_wait, 0);
+    if (c->order_record && !capturing && c->order_err == hipSuccess)
+      c->order_err = hipEventRecord(c->order_record, s);
+    return ok;
+  }
   mark(c, 0, capturing);
   // Begin also clears the per-segment U and K counts (unique leaves an
   // empty segment's entries untouched).

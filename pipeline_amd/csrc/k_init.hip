@@ -49,15 +49,6 @@ __global__ __launch_bounds__(256) void init_random_kernel(float4* __restrict__ o
   }
 }
 
-// Order-preserving map of a float to an unsigned integer (NaN aside).
-__device__ __forceinline__ uint32_t ord(float f) {
-  const uint32_t u = __float_as_uint(f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float unord(uint32_t u) {
-  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
-}
-
 constexpr int kBoxThreads = 256;
 constexpr int kBoxPts = 8;  // points per thread per step
 
@@ -132,9 +123,7 @@ __global__ __launch_bounds__(kBoxThreads) void box_reduce_kernel(
   if (cur >= 0) flush(cur);
 }
 
-// mm -> (min, range) per cloud: range = max(extent * 1.0001, 1e-3) computed
-// in double and rounded once, extent = max - min in float. An empty cloud
-// gets (0, 1).
+// mm -> (min, range) per cloud; an empty cloud gets (0, 1).
 __global__ __launch_bounds__(256) void box_finalize_kernel(const uint32_t* __restrict__ mm,
                                                            int32_t n_seg, float* __restrict__ mn,
                                                            float* __restrict__ rg) {
@@ -146,10 +135,8 @@ __global__ __launch_bounds__(256) void box_finalize_kernel(const uint32_t* __res
     rg[k] = 1.0f;
     return;
   }
-  const float lo = unord(a);
-  const float ext = unord(b) - lo;
-  mn[k] = lo;
-  rg[k] = static_cast<float>(fmax(static_cast<double>(ext) * 1.0001, 1e-3));
+  mn[k] = unord(a);
+  rg[k] = box_range(mn[k], unord(b));
 }
 
 __global__ void box_init_kernel(uint32_t* __restrict__ mm, int32_t n_seg) {

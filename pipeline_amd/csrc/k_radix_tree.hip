@@ -23,17 +23,11 @@
 // stand, for any sorted codes a caller passes (repeated ones and codes with
 // bit 31 set included): the per-stage entry. radix_pairs_kernel is the fused
 // build's, whose codes are always strictly increasing 30-bit keys.
-#include "ocp_internal.hpp"
+#include "pair_rows.hpp"
 
 namespace ocp {
 namespace {
 
-__device__ __forceinline__ uint32_t clz32(uint32_t x) {
-  return x ? static_cast<uint32_t>(__clz(static_cast<int>(x))) : 32u;
-}
-__device__ __forceinline__ uint32_t delta(uint32_t a, uint32_t b) {
-  return (clz32(a ^ b) - 1u) & 0xffu;
-}
 __device__ __forceinline__ int32_t log2_ceil(uint32_t x) {
   if (x == 0) return 0;
   const int32_t lo = 31 - static_cast<int32_t>(clz32(x));
@@ -355,36 +349,6 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
 // them from two byte arrays, 33 -> 26 us; 2^24 clustered points: 155 -> 99 us
 // and 17 -> 14 us. Tiles of 2048 with a halo of 256, 512 or 1024 pairs: 66.0,
 // 66.4, 68.1 us (98, 99, 101 us clustered).
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-typedef int32_t v4i __attribute__((ext_vector_type(4)));
-typedef uint16_t v2h __attribute__((ext_vector_type(2)));
-
-// Bit p of the result: byte p of the row is below t, where key = t + 127 in
-// every byte (bytes and t at most 31, so no byte borrows from its neighbour).
-__device__ __forceinline__ uint32_t below16(const v4u w, uint32_t key) {
-  const uint32_t hi = 0x80808080u;
-  const uint32_t a = __builtin_amdgcn_udot4(
-      (key - w.y) & hi, 0x80402010u,
-      __builtin_amdgcn_udot4((key - w.x) & hi, 0x08040201u, 0u, false), false);
-  const uint32_t b = __builtin_amdgcn_udot4(
-      (key - w.w) & hi, 0x80402010u,
-      __builtin_amdgcn_udot4((key - w.z) & hi, 0x08040201u, 0u, false), false);
-  return (a >> 7) | (b << 1);
-}
-__device__ __forceinline__ v2h as_halves(uint32_t x) { return __builtin_bit_cast(v2h, x); }
-__device__ __forceinline__ uint32_t min16(const v4u w) {
-  v2h m = as_halves(w.x & 0x00ff00ffu);
-  m = __builtin_elementwise_min(m, as_halves((w.x >> 8) & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves(w.y & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves((w.y >> 8) & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves(w.z & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves((w.z >> 8) & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves(w.w & 0x00ff00ffu));
-  m = __builtin_elementwise_min(m, as_halves((w.w >> 8) & 0x00ff00ffu));
-  return min(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y));
-}
-__device__ __forceinline__ uint32_t third(uint32_t x) { return (x * 11u) >> 5; }  // x / 3, x < 32
-
 // The end of the run of keys around key `from` whose xor with code c is below
 // lim, at least `reach` keys away on the side of d (+1, -1), in [0, m].
 __device__ __forceinline__ int32_t wave_run_end(const uint32_t* __restrict__ codes, uint32_t c,

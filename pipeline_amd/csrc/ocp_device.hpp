@@ -82,6 +82,22 @@ __device__ __forceinline__ float decode_axis(uint32_t code, int axis, float mn,
   return t * rg + mn;
 }
 
+// ---------------------------------------------------------------- boxes
+// Order-preserving map of a float to an unsigned integer (NaN aside).
+__device__ __forceinline__ uint32_t ord(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float unord(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+}
+// A cloud's range from its extremes: max(extent * 1.0001, 1e-3) computed in
+// double and rounded once, extent = max - min in float.
+__device__ __forceinline__ float box_range(float lo, float hi) {
+  const float ext = hi - lo;
+  return static_cast<float>(fmax(static_cast<double>(ext) * 1.0001, 1e-3));
+}
+
 // ---------------------------------------------------------------- scans
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
   const uint32_t l = lane_id();

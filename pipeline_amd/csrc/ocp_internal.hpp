@@ -290,6 +290,36 @@ void launch_edge_scan(const int32_t* edge, int32_t* offsets, const SegView& sv,
                       int32_t n_host, uint64_t* flags, uint32_t* ctrl, int32_t* kalloc,
                       const TuneTable& tt, hipStream_t s);
 
+// ---- stages 1 to 6 of small clouds (k_small.hip), one workgroup each: every
+// output of those stages at the segments' point offsets. mail (for a single
+// segment, else null): the kernel does the offsets kernel's work too.
+constexpr int64_t kSmallCloud = 8192;
+// Up to here because 8192 points' keys, sort and tree take 125 KB of LDS; up to
+// there the kernel is the faster one for one cloud (8192 clustered points 84 us
+// to the general path's 100) as for batches of any length (k_small.hip). Builds
+// with point indices sort pairs, a set tuning table and stage timing name the
+// stages' kernels: these keep the general path.
+inline bool small_clouds(int64_t max_seg, int32_t n_seg, bool perm) {
+  return !perm && max_seg <= kSmallCloud && n_seg >= 1;
+}
+struct SmallOut {
+  uint32_t* sorted;
+  uint32_t* unique;
+  uint8_t* prefix;
+  uint8_t* hl;
+  uint8_t* hr;
+  int32_t* lc;
+  int32_t* par;
+  int32_t* edge;
+  int32_t* offs;
+  int32_t* n_unique;
+  int32_t* kalloc;
+  int32_t* oct_start;
+};
+void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64_t max_seg,
+                         bool device_boxes, float* box_min, float* box_range, const SmallOut& o,
+                         uint32_t* ctrl, int64_t k_cap, uint32_t* mail, hipStream_t s);
+
 // ---- stage 7 (k_octree.hip)
 struct OctArgs {
   OctNode* nodes;            // base of all segments' nodes
