@@ -79,11 +79,8 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
         mx = max(mx, kv[k]);
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      mn = min(mn, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mn), o, 64)));
-      mx = max(mx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mx), o, 64)));
-    }
+    mn = wave_min(mn);
+    mx = wave_max(mx);
     __syncthreads();
     if (lane == 0) {
       atomicMin(&s_mm[0], mn);
@@ -167,7 +164,6 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
     }
     __syncthreads();
   }
-  const uint64_t lt = lanemask_lt();
   uint32_t* wh = s_whist + w * ND;
   // Pass 0 needs no stability (no earlier order to keep), so it is a plain
   // counting sort with LDS atomics over the low P0 bits, one counter per
@@ -223,18 +219,13 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
     for (int k = 0; k < KPT; ++k) {
       if (wbase + k * 64 >= wend) continue;
       const uint32_t d = (kv[k] >> shift) & dmask;
-      uint64_t msk = ~0ull;
+      Differ other;
 #pragma unroll
       for (int bb = 0; bb < P1; ++bb) {
         if (bb >= nb) break;
-        const bool bit = (d >> bb) & 1u;
-        const uint64_t bal = __ballot(bit);
-        msk &= bit ? bal : ~bal;
+        other.bit(d, bb);
       }
-      const uint32_t rank = __popcll(msk & lt);
-      const uint32_t old = wh[d];
-      if (rank == 0) wh[d] = old + __popcll(msk);
-      off[k] = old + rank;
+      off[k] = other.rank(wh, d);
     }
     __syncthreads();
     uint32_t tot[DPT];

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void edge_scan_kernel(
     }
   }
   if (kalloc) {
-    kmax = wave_incl_max(kmax);
+    kmax = wave_max(kmax);
     if (lane == 0) s_max[w] = kmax;
     __syncthreads();
     if (w == 0) {

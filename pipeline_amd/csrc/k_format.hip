@@ -125,8 +125,7 @@ enum Report : int {
 };
 
 __device__ __forceinline__ void add_report(unsigned long long* rep, int field, uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), o, 64));
+  v = wave_sum(v);
   if (lane_id() == 0 && v) atomicAdd(&rep[field], static_cast<unsigned long long>(v));
 }
 

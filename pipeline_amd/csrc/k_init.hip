@@ -67,11 +67,8 @@ __global__ __launch_bounds__(kBoxThreads) void box_reduce_kernel(
   uint32_t vmn = 0xffffffffu, vmx = 0u;
   int32_t cur = -1;
   auto flush = [&](int32_t seg) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      vmn = min(vmn, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vmn), o, 64)));
-      vmx = max(vmx, static_cast<uint32_t>(__shfl_xor(static_cast<int>(vmx), o, 64)));
-    }
+    vmn = wave_min(vmn);
+    vmx = wave_max(vmx);
     if (lane_id() == 0) {
       s_mn[wave_id()] = vmn;
       s_mx[wave_id()] = vmx;

@@ -128,11 +128,8 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
       lo = min(lo, min(a, min(b, c)));
       hi = max(hi, max(a, max(b, c)));
     }
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-      lo = min(lo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), d, 64)));
-      hi = max(hi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), d, 64)));
-    }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
     if (lane_id() == 0) {
       atomicMin(&s_box[0], lo);
       atomicMax(&s_box[1], hi);
@@ -280,7 +277,7 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
       top = max(top, run + e[j]);
     }
   }
-  top = wave_incl_max(top);
+  top = wave_max(top);
   if (lane_id() == 0) atomicMax(&s_max, top);
   __syncthreads();
   for (int32_t i = tid; i < m; i += kThreads) o.offs[sb + i] = s_edge[i];

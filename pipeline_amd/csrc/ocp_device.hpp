@@ -82,6 +82,34 @@ __device__ __forceinline__ float decode_axis(uint32_t code, int axis, float mn,
   return t * rg + mn;
 }
 
+// ---------------------------------------------------------------- multisplit
+// The lanes whose digit differs from this lane's, built up bit by bit: every
+// digit bit is one ballot, whose lanes of the other value are collected by one
+// three-input operation a half.
+struct Differ {
+  uint32_t lo = 0, hi = 0;
+  __device__ __forceinline__ void bit(uint32_t d, int b) {
+    const int32_t t = b == 0 ? -static_cast<int32_t>(d & 1u)
+                             : __builtin_amdgcn_sbfe(static_cast<int32_t>(d), b, 1);
+    const uint64_t set = __builtin_amdgcn_ballot_w64(b == 0 ? (d & 1u) != 0 : t < 0);
+    lo = __builtin_amdgcn_bitop3_b32(lo, t, static_cast<uint32_t>(set), 0xf6);  // lo | (t ^ set)
+    hi = __builtin_amdgcn_bitop3_b32(hi, t, static_cast<uint32_t>(set >> 32), 0xf6);
+  }
+  // A key's rank of its digit in the wave so far, counted in wh[d]: the earlier
+  // rows' keys and this row's lower lanes. The group's first lane adds the row's
+  // keys after every lane has read the counter (LDS takes a wave's operations
+  // in order); an add that returns nothing, so no row waits for the one before.
+  __device__ __forceinline__ uint32_t rank(uint32_t* wh, uint32_t d) const {
+    const uint32_t below =
+        lane_id() - __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    const uint32_t old = wh[d];
+    if (below == 0)
+      __hip_atomic_fetch_add(as_lds<uint32_t>(wh + d), 64u - __popc(lo) - __popc(hi),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return old + below;
+  }
+};
+
 // ---------------------------------------------------------------- boxes
 // Order-preserving map of a float to an unsigned integer (NaN aside).
 __device__ __forceinline__ uint32_t ord(float f) {
@@ -99,42 +127,79 @@ __device__ __forceinline__ float box_range(float lo, float hi) {
 }
 
 // ---------------------------------------------------------------- scans
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  const uint32_t l = lane_id();
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint32_t t = __shfl_up(v, o, kWave);
-    if (l >= static_cast<uint32_t>(o)) v += t;
-  }
+// Data-parallel moves between lanes: a lane's value comes from `SHIFT` lanes
+// below in its row of 16 (0x110 + n), from lane 15 of the row before (0x142) or
+// from lane 31 (0x143), and is `other` where there is none. A scan step is one
+// vector instruction; through LDS (a shuffle) it is a round trip, and a scan of
+// a wave six of them.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ uint32_t lane_move(uint32_t other, uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+      static_cast<int>(other), static_cast<int>(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ uint32_t row_incl_scan(uint32_t v) {  // in each row of 16 lanes
+  v += lane_move<0x111>(0u, v);
+  v += lane_move<0x112>(0u, v);
+  v += lane_move<0x114>(0u, v);
+  v += lane_move<0x118>(0u, v);
   return v;
 }
-__device__ __forceinline__ int32_t wave_incl_max(int32_t v) {
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) v = max(v, __shfl_xor(v, o, kWave));
+// (whole waves only, as everything below)
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  v = row_incl_scan(v);
+  v += lane_move<0x142, 0xa>(0u, v);
+  v += lane_move<0x143, 0xc>(0u, v);
   return v;
+}
+// op over the wave's values, in every lane.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_all(uint32_t v, Op op) {
+  v = op(v, lane_move<0x111>(v, v));
+  v = op(v, lane_move<0x112>(v, v));
+  v = op(v, lane_move<0x114>(v, v));
+  v = op(v, lane_move<0x118>(v, v));
+  v = op(v, lane_move<0x142, 0xa>(v, v));
+  v = op(v, lane_move<0x143, 0xc>(v, v));
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+  return wave_all(v, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  return wave_all(v, [](uint32_t a, uint32_t b) { return max(a, b); });
+}
+__device__ __forceinline__ int32_t wave_max(int32_t v) {
+  return static_cast<int32_t>(wave_all(static_cast<uint32_t>(v), [](uint32_t a, uint32_t b) {
+    return static_cast<uint32_t>(max(static_cast<int32_t>(a), static_cast<int32_t>(b)));
+  }));
+}
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(wave_incl_scan(v)), 63));
+}
+__device__ __forceinline__ uint32_t wave_read(uint32_t v, uint32_t lane) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(lane)));
 }
 
 // Exclusive scan of one value per thread over a block of THREADS threads.
 // `tmp` holds THREADS/64 words of LDS. Ends with a barrier so `tmp` can be
-// reused right away.
+// reused right away. Every wave scans the waves' sums in one row of its lanes.
 template <int THREADS>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* tmp,
                                                     uint32_t* total) {
-  constexpr int NW = THREADS / kWave;
+  constexpr uint32_t NW = THREADS / kWave;
+  static_assert(NW <= 16, "a row of lanes");
   const uint32_t incl = wave_incl_scan(v);
-  const uint32_t w = wave_id();
-  if (lane_id() == kWave - 1) tmp[w] = incl;
+  const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wave_id())));
+  const uint32_t lane = lane_id();
+  if (lane == kWave - 1) tmp[w] = incl;
   __syncthreads();
-  uint32_t off = 0, tot = 0;
-#pragma unroll
-  for (int k = 0; k < NW; ++k) {
-    const uint32_t t = tmp[k];
-    off += (static_cast<uint32_t>(k) < w) ? t : 0u;
-    tot += t;
-  }
+  const uint32_t t = lane < NW ? tmp[lane] : 0u;
+  const uint32_t s = row_incl_scan(t);
   __syncthreads();
-  *total = tot;
-  return off + incl - v;
+  *total = wave_read(s, NW - 1);
+  return wave_read(s - t, w) + incl - v;
 }
 
 // Two exclusive scans at once (one barrier pair): `tmp` holds 2 * THREADS/64
@@ -142,26 +207,22 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* tmp,
 template <int THREADS>
 __device__ __forceinline__ void block_excl_scan2(uint32_t a, uint32_t b, uint32_t* tmp,
                                                  uint32_t* ea, uint32_t* eb) {
-  constexpr int NW = THREADS / kWave;
+  constexpr uint32_t NW = THREADS / kWave;
+  static_assert(NW <= 16, "a row of lanes each");
   const uint32_t ia = wave_incl_scan(a);
   const uint32_t ib = wave_incl_scan(b);
-  const uint32_t w = wave_id();
-  if (lane_id() == kWave - 1) {
+  const uint32_t w = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(wave_id())));
+  const uint32_t lane = lane_id();
+  if (lane == kWave - 1) {
     tmp[w] = ia;
     tmp[NW + w] = ib;
   }
   __syncthreads();
-  uint32_t oa = 0, ob = 0;
-#pragma unroll
-  for (int k = 0; k < NW; ++k) {
-    const uint32_t ta = tmp[k];
-    const uint32_t tb = tmp[NW + k];
-    oa += (static_cast<uint32_t>(k) < w) ? ta : 0u;
-    ob += (static_cast<uint32_t>(k) < w) ? tb : 0u;
-  }
+  const uint32_t t = (lane & 15u) < NW && lane < 32 ? tmp[(lane >> 4) * NW + (lane & 15u)] : 0u;
+  const uint32_t before = row_incl_scan(t) - t;
   __syncthreads();
-  *ea = oa + ia - a;
-  *eb = ob + ib - b;
+  *ea = wave_read(before, w) + ia - a;
+  *eb = wave_read(before, 16 + w) + ib - b;
 }
 
 // Exclusive scan, in place, of R words of LDS by one whole wave (each lane
@@ -186,7 +247,7 @@ __device__ __forceinline__ uint32_t wave_scan_lds(uint32_t* a) {
     if (idx < static_cast<uint32_t>(R)) a[idx] = run;
     run += v[q];
   }
-  return __shfl(incl, kWave - 1, kWave);
+  return wave_read(incl, kWave - 1);
 }
 
 // ---------------------------------------------------------------- lookback
@@ -276,12 +337,7 @@ __device__ __forceinline__ uint32_t wave_sum_flags(const uint64_t* base, int32_t
       __builtin_amdgcn_s_sleep(1);
       continue;
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const uint32_t x = __shfl_xor(c, o, kWave);
-      c = MAX ? max(c, x) : c + x;
-    }
-    return c;
+    return MAX ? wave_max(c) : wave_sum(c);
   }
   *timed_out = true;
   return 0;

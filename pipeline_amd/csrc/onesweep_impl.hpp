@@ -8,7 +8,7 @@
 //      device-scope counter serialises at one atomic per tile).
 //   2. Keys are loaded wave-contiguously (lane-strided, coalesced) and
 //      ranked per wave with a 64-lane multisplit: one ballot per digit bit builds the
-//      mask of lanes holding the same digit; popcount below the lane gives a
+//      mask of lanes holding another digit; the lanes below without them give a
 //      stable rank; the lowest lane bumps the wave's LDS digit counter.
 //   3. The tile's 2^bits digit counts (256, or 1024 for 10-bit digits) are
 //      published at once (aggregate, or inclusive for a segment's first
@@ -19,6 +19,12 @@
 //      a digit is cheap to recompute), then written out with consecutive
 //      threads on consecutive LDS slots, so equal-digit runs go to
 //      consecutive HBM addresses.
+// What bounds a pass: vector instructions (half of its time at 2^24 keys) and how
+// few waves hide the rest. Four operations a digit bit in the multisplit, wave
+// scans without LDS, ranks two a register and digits recomputed rather than kept
+// took it from 120 instructions a row of 64 keys to 85 and from 112 registers to
+// 75, so that a CU holds three 8-wave tiles instead of two: 81 -> 63 us at 2^24
+// keys (128 MB), 18.5 -> 18 us at 1M, where it is round trips.
 // Segments sort independently: each has its own digit histogram and its own
 // lookback chain, and no tile holds keys of two segments.
 //
@@ -119,35 +125,38 @@ __global__ __launch_bounds__(WAVES * 64) void onesweep_kernel(
 
   uint32_t keys[KPT];
   uint32_t dg[KPT];
-  uint32_t off[KPT];
+  uint32_t off[(KPT + 1) / 2];  // ranks in the wave, below 2^16: two a register
   uint32_t vals[KV ? KPT : 1];
-  const int32_t lbase = static_cast<int32_t>(w) * (64 * KPT) + static_cast<int32_t>(lane);
-  const uint32_t* src = in + lbase + base;
+  // (rows at scalar addresses: one register of offsets for all of them)
+  const int32_t wbase = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(w)) * (64 * KPT);
+  const int32_t lbase = wbase + static_cast<int32_t>(lane);
+  const uint32_t* src = in + (wbase + __builtin_amdgcn_readfirstlane(base));
   if constexpr (KV) {
     // Values: given, or the key's index in its segment (the first pass of a
     // build, where the keys are in point order).
-    const uint32_t* vsrc = vin ? vin + lbase + base : nullptr;
+    const uint32_t* vsrc =
+        vin ? vin + (wbase + __builtin_amdgcn_readfirstlane(base)) : nullptr;
 #pragma unroll
     for (int k = 0; k < KPT; ++k) {
       const int32_t idx = lbase + k * 64;
-      vals[k] = vsrc ? (idx < cnt ? vsrc[k * 64] : 0u)
+      vals[k] = vsrc ? (idx < cnt ? (vsrc + k * 64)[lane] : 0u)
                      : static_cast<uint32_t>(base - sb + idx);
     }
   }
   if (cnt == T) {  // every tile but a segment's last: no per-key guards
 #pragma unroll
-    for (int k = 0; k < KPT; ++k) keys[k] = src[k * 64];
+    for (int k = 0; k < KPT; ++k) keys[k] = (src + k * 64)[lane];
 #pragma unroll
     for (int k = 0; k < KPT; ++k) dg[k] = dig(keys[k]);
   } else {
 #pragma unroll
     for (int k = 0; k < KPT; ++k) {
-      const int32_t idx = static_cast<int32_t>(w) * (64 * KPT) + k * 64 + static_cast<int32_t>(lane);
-      keys[k] = idx < cnt ? src[k * 64] : 0xffffffffu;
+      const int32_t idx = lbase + k * 64;
+      keys[k] = idx < cnt ? (src + k * 64)[lane] : 0xffffffffu;
     }
 #pragma unroll
     for (int k = 0; k < KPT; ++k) {
-      const int32_t idx = static_cast<int32_t>(w) * (64 * KPT) + k * 64 + static_cast<int32_t>(lane);
+      const int32_t idx = lbase + k * 64;
       dg[k] = idx < cnt ? dig(keys[k]) : uint32_t(RADIX - 1);  // padding keys rank last
     }
   }
@@ -159,33 +168,28 @@ __global__ __launch_bounds__(WAVES * 64) void onesweep_kernel(
   // segment decides the same way, so none waits on a flag never published.
   if (tid < RADIX && static_cast<int32_t>(hv) == seg_end(sv, r.seg) - sb) s_trivial = 1u;
 
-  // Wave-level multisplit. The read of the digit counter by every lane of a
-  // group happens in the same LDS instruction, before the leader's update.
+  // Wave-level multisplit.
   uint32_t* wh = s_whist + w * RADIX;
   if (STABLE || cnt < T) {
-    const uint64_t lt = lanemask_lt();
 #pragma unroll
     for (int k = 0; k < KPT; ++k) {
-      const uint32_t d = dg[k];
-      uint64_t m = ~0ull;
+      Differ other;
 #pragma unroll
-      for (int b = 0; b < BITS; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t bal = __ballot(bit);
-        m &= bit ? bal : ~bal;
-      }
-      const uint32_t rank = __popcll(m & lt);
-      const uint32_t old = wh[d];
-      if (rank == 0) wh[d] = old + __popcll(m);
-      off[k] = old + rank;
+      for (int b = 0; b < BITS; ++b) other.bit(dg[k], b);
+      const uint32_t r = other.rank(wh, dg[k]);
+      if (k & 1) off[k / 2] |= r << 16;
+      else off[k / 2] = r;
     }
   } else {
     // Each lane takes the next free rank of its digit within the wave.
     lds_ptr<uint32_t> whl = as_lds<uint32_t>(wh);
 #pragma unroll
-    for (int k = 0; k < KPT; ++k)
-      off[k] = __hip_atomic_fetch_add(whl + dg[k], 1u, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (int k = 0; k < KPT; ++k) {
+      const uint32_t r = __hip_atomic_fetch_add(whl + dg[k], 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (k & 1) off[k / 2] |= r << 16;
+      else off[k / 2] = r;
+    }
   }
   __syncthreads();
   if (s_trivial) {
@@ -238,34 +242,41 @@ __global__ __launch_bounds__(WAVES * 64) void onesweep_kernel(
 
 #pragma unroll
   for (int k = 0; k < KPT; ++k) {
-    const uint32_t pos = wh[dg[k]] + off[k];
+    // (a cheap digit is not held across the barriers)
+    const uint32_t d = !CHEAP ? dg[k] : lbase + k * 64 < cnt ? dig(keys[k]) : RADIX - 1u;
+    const uint32_t pos = wh[d] + ((off[k / 2] >> ((k & 1) * 16)) & 0xffffu);
     s_keys[pos] = keys[k];
     if constexpr (KV) s_vals[pos] = vals[k];
-    if constexpr (!CHEAP) s_dig[pos] = static_cast<uint8_t>(dg[k]);
+    if constexpr (!CHEAP) s_dig[pos] = static_cast<uint8_t>(d);
   }
   __syncthreads();
 
   if (cnt == T) {
-    // All LDS reads first, then the stores (a guarded store per iteration
+    // A batch's LDS reads first, then its stores (a guarded store per iteration
     // waits on its two dependent LDS reads before the next begins).
-    uint32_t kv[KPT];
-    uint32_t vv[KV ? KPT : 1];
-    int32_t dst[KPT];
+    constexpr int BATCH = KPT % 8 == 0 ? 8 : KPT % 5 == 0 ? 5 : 4;
+    static_assert(KPT % BATCH == 0, "whole batches");
+#pragma unroll 1
+    for (int p0 = tid; p0 < T; p0 += BATCH * THREADS) {
+      uint32_t kv[BATCH];
+      uint32_t vv[KV ? BATCH : 1];
+      int32_t dst[BATCH];
 #pragma unroll
-    for (int k = 0; k < KPT; ++k) {
-      kv[k] = s_keys[k * THREADS + tid];
-      if constexpr (KV) vv[k] = s_vals[k * THREADS + tid];
-      if constexpr (!CHEAP) dst[k] = s_dig[k * THREADS + tid];
-    }
+      for (int k = 0; k < BATCH; ++k) {
+        kv[k] = s_keys[k * THREADS + p0];
+        if constexpr (KV) vv[k] = s_vals[k * THREADS + p0];
+        if constexpr (!CHEAP) dst[k] = s_dig[k * THREADS + p0];
+      }
 #pragma unroll
-    for (int k = 0; k < KPT; ++k) {
-      if constexpr (CHEAP) dst[k] = static_cast<int32_t>(dig(kv[k]));
-      dst[k] = s_dst[dst[k]] + k * THREADS + tid;
-    }
+      for (int k = 0; k < BATCH; ++k) {
+        if constexpr (CHEAP) dst[k] = static_cast<int32_t>(dig(kv[k]));
+        dst[k] = s_dst[dst[k]] + k * THREADS + p0;
+      }
 #pragma unroll
-    for (int k = 0; k < KPT; ++k) {
-      out[dst[k]] = kv[k];
-      if constexpr (KV) vout[dst[k]] = vv[k];
+      for (int k = 0; k < BATCH; ++k) {
+        out[dst[k]] = kv[k];
+        if constexpr (KV) vout[dst[k]] = vv[k];
+      }
     }
   } else {
 #pragma unroll
