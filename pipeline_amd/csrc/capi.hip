@@ -193,8 +193,8 @@ struct ocp_context {
   int tab_tune_key = -1;
   bool have_result = false;
   Plan last_plan;
-  // Pinned host memory: what the last build's offsets kernel reports (see
-  // launch_oct_offsets), then a landing place for small copies back. Current
+  // Pinned host memory: what the last build's offsets kernel, or for one cloud
+  // its octree kernel, reports (see launch_oct_offsets), then a landing place for small copies back. Current
   // while no other work that can time out was enqueued after that build.
   uint32_t* mail = nullptr;
   bool mail_current = false;
@@ -640,11 +640,17 @@ bool enqueue_octree(ocp_ctx c, const Plan& p, bool capturing) {
   Workspace& w = c->ws;
   hipStream_t s = c->stream;
   int32_t* kalloc = w.counts + w.seg_cap;
-  { KScope k(c, kKOctOffsets, capturing);
-    launch_oct_offsets(w.counts, kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, c->mail, s); }
+  // (an empty cloud has no tile that could do the offsets' work)
+  const bool single = p.n_seg == 1 && p.tiles_node > 0 && oct_single(p.n_total);
+  if (!single) {
+    KScope k(c, kKOctOffsets, capturing);
+    launch_oct_offsets(w.counts, kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, c->mail, s);
+  }
+  const OctSingle one{w.oct_start, c->ctrl, single ? c->mail : nullptr,
+                      static_cast<uint32_t>(std::min<int64_t>(w.k_cap, UINT32_MAX))};
   const OctArgs a = pipeline_oct_args(c);
   KScope k(c, kKOctBuild, capturing);
-  return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, s);
+  return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, one, s);
 }
 
 void mark(ocp_ctx c, int k, bool capturing) {
@@ -671,13 +677,10 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
   }
   if (small_clouds(p.max_seg, p.n_seg, p.permutation) && !c->tuned && !c->stage_timing) {
     const SmallOut o{w.keys_a, w.keys_b, w.prefix_n, w.hl, w.hr, w.lc, w.par, w.edge, w.offs,
-                     n_unique, kalloc, w.oct_start};
-    const bool single = p.n_seg == 1;
+                     n_unique, kalloc};
     launch_small_clouds(pts, f3, p.sv, p.max_seg, p.device_boxes, w.boxes, w.boxes + w.seg_cap, o,
-                        c->ctrl, w.k_cap, single ? c->mail : nullptr, s);
-    if (!single)
-      launch_oct_offsets(n_unique, kalloc, p.n_seg, w.oct_start, c->ctrl, w.k_cap, c->mail, s);
-    const bool ok = launch_oct_build(pipeline_oct_args(c), p.sv, p.ts_node, p.tiles_node, s);
+                        c->ctrl, s);
+    const bool ok = enqueue_octree(c, p, capturing);
     // (no wait on another workgroup here; a later frame's lookback launches
     // still come after those of the frames before this one)
     if (c->order_wait && !capturing) c->order_err = hipStreamWaitEvent(s, c->order_wait, 0);

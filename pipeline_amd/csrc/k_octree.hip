@@ -233,8 +233,9 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
   }
 }
 
+template <bool SINGLE>
 __global__ __launch_bounds__(kThreads) void oct_build_kernel(
-    OctArgs a, SegView sv, const int32_t* __restrict__ tile_start) {
+    OctArgs a, SegView sv, const int32_t* __restrict__ tile_start, OctSingle one) {
   constexpr int T = kOctTile;
   constexpr int NPT = T / kThreads;
   __shared__ u64 s_child[kColWords * kCols];
@@ -250,10 +251,11 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // The segment's scalars are loaded together before any is tested: one
   // round trip instead of one per value.
   // (The launcher guarantees these pointers; the build writes them all.)
-  const uint32_t fits = a.ctrl[kCtrlOctOk];
   const int32_t m_seg = a.n_unique[r.seg] - 1;
-  const int32_t node_base = a.oct_start[r.seg];
   const int32_t k_seg = a.kalloc[r.seg];
+  const uint32_t fits = SINGLE ? (static_cast<uint32_t>(k_seg) <= one.k_cap ? 1u : 0u)
+                               : a.ctrl[kCtrlOctOk];
+  const int32_t node_base = SINGLE ? 0 : a.oct_start[r.seg];
   const int32_t sb = seg_begin(sv, r.seg);
   const float seg_mn = seg_min(sv, r.seg);
   const float seg_rg = seg_range(sv, r.seg);
@@ -263,6 +265,21 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // segment still has its root), the segment has slots and a valid base.
   // After a lookback time-out the inputs are not valid.
   const uint32_t stop = a.ctrl[kCtrlTimeout];
+  if (SINGLE && i0 == 0 && threadIdx.x == 0) {
+    // What the offsets kernel does for several segments (a launch of ~5 us).
+    const uint32_t tiles = a.ctrl[kCtrlMsdTiles];
+    const uint32_t slots = static_cast<uint32_t>(k_seg);
+    one.oct_start[0] = 0;
+    one.oct_start[1] = k_seg;
+    one.ctrl[kCtrlOctTotal] = slots;
+    one.ctrl[kCtrlOctOk] = fits;
+    one.mail[kCtrlOctTotal] = slots;
+    one.mail[kCtrlOctOk] = fits;
+    one.mail[kCtrlTimeout] = stop;
+    one.mail[kCtrlMsdTiles] = tiles;
+    one.mail[kCtrlWords] = static_cast<uint32_t>(m_seg + 1);
+    one.mail[kCtrlWords + kMailSegs] = slots;
+  }
   if (fits == 0 || stop != 0 || (i0 >= m_seg && !(i0 == 0 && m_seg == 0)) || k_seg < 1 ||
       node_base < 0)
     return;
@@ -536,7 +553,7 @@ void launch_oct_root(OctNode* nodes, const uint32_t* codes,
 }
 
 bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_start,
-                      int32_t total_tiles, hipStream_t s) {
+                      int32_t total_tiles, const OctSingle& single, hipStream_t s) {
   // The pushes read every array of the radix tree; the per-segment counts,
   // node bases and the fit flag come from the build.
   if (!a.has_leaf_left || !a.has_leaf_right || !a.left_child || !a.parent || !a.codes ||
@@ -544,7 +561,11 @@ bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_s
       !a.oct_start || !a.kalloc)
     return false;
   if (total_tiles <= 0) return true;
-  oct_build_kernel<<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start);
+  if (single.mail && (sv.n_seg != 1 || !single.oct_start || !single.ctrl)) return false;
+  if (single.mail)
+    oct_build_kernel<true><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
+  else
+    oct_build_kernel<false><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
   return true;
 }
 

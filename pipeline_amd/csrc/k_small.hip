@@ -65,8 +65,7 @@ __device__ __forceinline__ int32_t last_below(const Levels& lv, uint32_t q, uint
 template <int KPT, bool F3>
 __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     const float* __restrict__ pts, SegView sv, bool device_box, float* __restrict__ box_min,
-    float* __restrict__ box_range_out, SmallOut o, uint32_t* __restrict__ ctrl, int64_t k_cap,
-    uint32_t* __restrict__ mail) {
+    float* __restrict__ box_range_out, SmallOut o, uint32_t* __restrict__ ctrl) {
   constexpr int CAP = kThreads * KPT;
   constexpr int ROWS = CAP / 16;
   constexpr int TOP = CAP > 4096 ? 3 : 2;  // the level of one row
@@ -88,7 +87,6 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     if (tid == 0) {
       o.n_unique[seg] = 0;
       o.kalloc[seg] = 0;
-      if (mail) mail[kCtrlTimeout] = ctrl[kCtrlTimeout];
     }
     return;
   }
@@ -282,23 +280,9 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
   __syncthreads();
   for (int32_t i = tid; i < m; i += kThreads) o.offs[sb + i] = s_edge[i];
   if (tid == 0) {
-    const uint32_t slots = u > 0 ? static_cast<uint32_t>(s_max) : 0u;
     o.n_unique[seg] = u;
-    o.kalloc[seg] = static_cast<int32_t>(slots);
-    if (seg == 0) ctrl[kCtrlMsdTiles] = 0u;  // (an earlier build's; the mail's copy too)
-    if (mail) {  // a single segment: what the offsets kernel does for several
-      const uint32_t fits = slots <= k_cap ? 1u : 0u;
-      o.oct_start[0] = 0;
-      o.oct_start[1] = static_cast<int32_t>(slots);
-      ctrl[kCtrlOctTotal] = slots;
-      ctrl[kCtrlOctOk] = fits;
-      mail[kCtrlOctTotal] = slots;
-      mail[kCtrlOctOk] = fits;
-      mail[kCtrlTimeout] = 0u;
-      mail[kCtrlMsdTiles] = 0u;
-      mail[kCtrlWords] = static_cast<uint32_t>(u);
-      mail[kCtrlWords + kMailSegs] = slots;
-    }
+    o.kalloc[seg] = u > 0 ? s_max : 0;
+    if (seg == 0) ctrl[kCtrlMsdTiles] = 0u;  // (an earlier build's)
   }
 }
 
@@ -306,11 +290,10 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
 
 void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64_t max_seg,
                          bool device_boxes, float* box_min, float* box_range, const SmallOut& o,
-                         uint32_t* ctrl, int64_t k_cap, uint32_t* mail, hipStream_t s) {
+                         uint32_t* ctrl, hipStream_t s) {
   if (sv.n_seg <= 0) return;
   const auto go = [&](auto kernel) {
-    kernel<<<sv.n_seg, kThreads, 0, s>>>(pts, sv, device_boxes, box_min, box_range, o, ctrl, k_cap,
-                                         mail);
+    kernel<<<sv.n_seg, kThreads, 0, s>>>(pts, sv, device_boxes, box_min, box_range, o, ctrl);
   };
   if (max_seg <= 4096) {
     if (float3) go(small_cloud_kernel<4, true>);

@@ -291,8 +291,7 @@ void launch_edge_scan(const int32_t* edge, int32_t* offsets, const SegView& sv,
                       const TuneTable& tt, hipStream_t s);
 
 // ---- stages 1 to 6 of small clouds (k_small.hip), one workgroup each: every
-// output of those stages at the segments' point offsets. mail (for a single
-// segment, else null): the kernel does the offsets kernel's work too.
+// output of those stages at the segments' point offsets.
 constexpr int64_t kSmallCloud = 8192;
 // Up to here because 8192 points' keys, sort and tree take 125 KB of LDS; up to
 // there the kernel is the faster one for one cloud (8192 clustered points 84 us
@@ -314,11 +313,10 @@ struct SmallOut {
   int32_t* offs;
   int32_t* n_unique;
   int32_t* kalloc;
-  int32_t* oct_start;
 };
 void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64_t max_seg,
                          bool device_boxes, float* box_min, float* box_range, const SmallOut& o,
-                         uint32_t* ctrl, int64_t k_cap, uint32_t* mail, hipStream_t s);
+                         uint32_t* ctrl, hipStream_t s);
 
 // ---- stage 7 (k_octree.hip)
 struct OctArgs {
@@ -344,8 +342,19 @@ void launch_oct_root(OctNode* nodes, const uint32_t* codes,
 // The fused make + link + root pass: writes every slot, zero gaps included.
 // Needs every OctArgs array (the fused build has them all); returns false
 // (and launches nothing) when an array it needs is null.
-bool launch_oct_build(const OctArgs& a, const SegView& sv,
-                      const int32_t* tile_start, int32_t total_tiles, hipStream_t s);
+// single (one segment with points): the kernel does the offsets kernel's work
+// as well, which there is two comparisons. Eight frames of 1M points in a stream
+// 715 -> 680 us without that launch, 307,200 points 85 -> 81, 6M 287 -> 283; 10M
+// points took 437 us with it and 439 without, so from 2^23 on it is launched.
+inline bool oct_single(int64_t n) { return n < (int64_t(1) << 23); }
+struct OctSingle {
+  int32_t* oct_start;
+  uint32_t* ctrl;
+  uint32_t* mail;  // null: the offsets kernel has run
+  uint32_t k_cap;
+};
+bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_start,
+                      int32_t total_tiles, const OctSingle& single, hipStream_t s);
 
 // ---- stage 7, per-stage entry points (k_octree_stage.hip)
 // The make call of the reference signature has no children arrays
