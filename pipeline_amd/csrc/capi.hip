@@ -1298,11 +1298,7 @@ int ocp_k_MakeOctNodes(ocp_ctx c, ocp_oct_node* nodes, const int32_t* offs,
   if (n >= kMaxSegPoints) return fail(c, OCP_ERR_CAPACITY, "N >= 2^27");
   const OctArgs a = stage_oct_args(nodes, offs, counts, codes, pn, nullptr, nullptr, par,
                                    nullptr, n, n_alloc);
-  const SegView sv = single_view(n + 1, mn, rg);
-  const int32_t tiles = static_cast<int32_t>(cdiv(n, kNodeTile));
-  // No children arrays in this call: the push-style kernels.
-  launch_oct_scatter(a, sv, nullptr, tiles, 1, c->stream);
-  launch_oct_finalize(a, sv, nullptr, tiles, 1 | 4, c->stream);
+  launch_oct_make(a, single_view(n + 1, mn, rg), c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;
 }
@@ -1317,10 +1313,7 @@ int ocp_k_LinkLeafNodes(ocp_ctx c, ocp_oct_node* nodes, const int32_t* offs,
     return fail(c, OCP_ERR_INVALID, "null pointer");
   if (n >= kMaxSegPoints) return fail(c, OCP_ERR_CAPACITY, "N >= 2^27");
   const OctArgs a = stage_oct_args(nodes, offs, counts, codes, pn, hl, hr, par, lc, n, n_alloc);
-  const SegView sv = single_view(n + 1, 0.0f, 1.0f);
-  const int32_t tiles = static_cast<int32_t>(cdiv(n, kNodeTile));
-  launch_oct_scatter(a, sv, nullptr, tiles, 2 | 4, c->stream);
-  launch_oct_finalize(a, sv, nullptr, tiles, 2, c->stream);
+  launch_oct_link(a, single_view(n + 1, 0.0f, 1.0f), c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;
 }

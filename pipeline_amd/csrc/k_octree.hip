@@ -1,4 +1,4 @@
-// Stage 7 of the fused build: octree nodes from the radix tree -
+// Stage 7: octree nodes from the radix tree -
 // ProcessOctNode and ProcessLinkLeaf of include/shared/oct.h:24-134, driven
 // by kernels/07_octree.cpp:5-57 - with the sequential (ascending index)
 // semantics of the reference CPU path, in one pass.
@@ -51,6 +51,12 @@
 //  3. One thread per slot assembles the node in its column's place, and the
 //     tile's nodes leave as consecutive 16-byte stores.
 // A tile with more slots than columns takes them in several rounds.
+//
+// The per-stage entries (k_MakeOctNodes, k_LinkLeafNodes: include/cuda/kernels/
+// 07_octree.cuh:7-28) are the same kernel doing one half of the pushes into
+// nodes that it reads and writes whole. Make has no children arrays: see
+// oct_far_kernel. For 2M points make takes 52 us and link 33; a scatter of order
+// keys by global atomics and a kernel that resolved them took 117 and 187.
 //
 // What bounds it: 10M uniform points take 174 us, of which the walks of the
 // listed children (a chain of up to four dependent loads that one wave of the
@@ -177,6 +183,7 @@ struct SubNode {
   int32_t x, lc;
   uint32_t flags;  // level | has_leaf_left << 8 | has_leaf_right << 9
 };
+template <bool MAKE>
 __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& cols, int32_t x,
                                               uint32_t slot) {
   SubNode cur, s0{}, s1{}, s2{};  // s0..s2: pending, s0 on top
@@ -188,7 +195,8 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
     const int32_t level = third(b.pn[x]);
     cur = {x, b.lc[x],
            static_cast<uint32_t>(level) | (b.hl[x] ? 256u : 0u) | (b.hr[x] ? 512u : 0u)};
-    if (e > 0) cols.put_make(slot, child_of(code, level - e + 1), make_key(x, e - 1), p + e - 1);
+    if (MAKE && e > 0)
+      cols.put_make(slot, child_of(code, level - e + 1), make_key(x, e - 1), p + e - 1);
     if (e != 0) return;
   }
   while (true) {
@@ -215,7 +223,7 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
       if (at.flags & (256u << side)) {
         cols.put(slot, child_of(code[side], level + 1), link_key(at.x, side), ch);
       } else if (e[side] > 0) {
-        cols.put_make(slot, child_of(code[side], lv - e[side] + 1), make_key(ch, e[side] - 1),
+        if (MAKE) cols.put_make(slot, child_of(code[side], lv - e[side] + 1), make_key(ch, e[side] - 1),
                       p[side] + e[side] - 1);
       } else if (e[side] == 0 && pending < 3) {
         s2 = s1;
@@ -233,11 +241,16 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
   }
 }
 
-template <bool SINGLE>
+// What a launch does: the whole stage, or one of its two per-stage entries on
+// nodes that the caller prepared.
+enum OctPhase { kWhole, kMakePhase, kLinkPhase };
+
+template <bool SINGLE, OctPhase PHASE>
 __global__ __launch_bounds__(kThreads) void oct_build_kernel(
     OctArgs a, SegView sv, const int32_t* __restrict__ tile_start, OctSingle one) {
   constexpr int T = kOctTile;
   constexpr int NPT = T / kThreads;
+  constexpr bool MAKE = PHASE != kLinkPhase, LINK = PHASE != kMakePhase;
   __shared__ u64 s_child[kColWords * kCols];
   __shared__ u64 s_owner[kCols];
   // A node's step of a walk up: kHead | slot where the walk ends (a chain's
@@ -251,11 +264,12 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // The segment's scalars are loaded together before any is tested: one
   // round trip instead of one per value.
   // (The launcher guarantees these pointers; the build writes them all.)
-  const int32_t m_seg = a.n_unique[r.seg] - 1;
-  const int32_t k_seg = a.kalloc[r.seg];
-  const uint32_t fits = SINGLE ? (static_cast<uint32_t>(k_seg) <= one.k_cap ? 1u : 0u)
-                               : a.ctrl[kCtrlOctOk];
-  const int32_t node_base = SINGLE ? 0 : a.oct_start[r.seg];
+  const int32_t m_seg = PHASE == kWhole ? a.n_unique[r.seg] - 1 : a.n_brt_host;
+  const int32_t k_seg = PHASE == kWhole ? a.kalloc[r.seg] : a.k_host;
+  const uint32_t fits = PHASE != kWhole ? 1u
+                        : SINGLE        ? (static_cast<uint32_t>(k_seg) <= one.k_cap ? 1u : 0u)
+                                        : a.ctrl[kCtrlOctOk];
+  const int32_t node_base = SINGLE || PHASE != kWhole ? 0 : a.oct_start[r.seg];
   const int32_t sb = seg_begin(sv, r.seg);
   const float seg_mn = seg_min(sv, r.seg);
   const float seg_rg = seg_range(sv, r.seg);
@@ -264,7 +278,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // loads after it back): the nodes fit, the tile has nodes (a single-key
   // segment still has its root), the segment has slots and a valid base.
   // After a lookback time-out the inputs are not valid.
-  const uint32_t stop = a.ctrl[kCtrlTimeout];
+  const uint32_t stop = PHASE == kWhole ? a.ctrl[kCtrlTimeout] : 0u;
   if (SINGLE && i0 == 0 && threadIdx.x == 0) {
     // What the offsets kernel does for several segments (a launch of ~5 us).
     const uint32_t tiles = a.ctrl[kCtrlMsdTiles];
@@ -301,8 +315,15 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   const int tid = threadIdx.x;
   // The slots of the tile.
   const int32_t i_end = min(i0 + T, b.m);
-  const int32_t p_before = i0 > 0 ? b.p[i0 - 1] : -1;
-  const int32_t s_end = i_end >= b.m ? b.k : b.p[i_end - 1] + 1;
+  int32_t p_before = i0 > 0 ? b.p[i0 - 1] : -1;
+  int32_t s_end = i_end >= b.m ? b.k : b.p[i_end - 1] + 1;
+  if constexpr (PHASE != kWhole) {
+    // The caller's slots bound every access, and those past the last chain
+    // stay as they are.
+    if (i_end >= b.m) s_end = b.p[b.m - 1] + kMaxEdge;
+    p_before = max(p_before, -1);
+    s_end = min(s_end, b.k);
+  }
   const int32_t root_level = b.m >= 1 ? third(b.pn[0]) : 0;
 
   if (p_before + 1 >= s_end) return;  // a tile without slots
@@ -326,12 +347,14 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
         const int32_t i = i0 + u * kThreads + tid;
         p[u] = b.p[i];
         e[u] = b.e[i];
-        lc[u] = b.lc[i];
         par[u] = b.par[i];
         code[u] = b.codes[i];
         pn[u] = b.pn[i];
-        hl[u] = b.hl[i];
-        hr[u] = b.hr[i];
+        if constexpr (LINK) {
+          lc[u] = b.lc[i];
+          hl[u] = b.hl[i];
+          hr[u] = b.hr[i];
+        }
       }
     } else {
 #pragma unroll
@@ -344,11 +367,13 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
         if (i < b.m) {
           p[u] = b.p[i];
           e[u] = b.e[i];
-          lc[u] = b.lc[i];
           par[u] = b.par[i];
           pn[u] = b.pn[i];
-          hl[u] = b.hl[i];
-          hr[u] = b.hr[i];
+          if constexpr (LINK) {
+            lc[u] = b.lc[i];
+            hl[u] = b.hl[i];
+            hr[u] = b.hr[i];
+          }
         }
         if (i <= b.m) code[u] = b.codes[i];
       }
@@ -360,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
     }
     int32_t back_e = 0, back_p = 0;
     const int32_t back_q = i0 - 1 - static_cast<int32_t>(lane_id());
-    const bool back_wave = wave_id() == kThreads / 64 - 1 && i0 > 0;
+    const bool back_wave = MAKE && wave_id() == kThreads / 64 - 1 && i0 > 0;
     if (back_wave && back_q >= 1) {
       back_e = b.e[back_q];
       back_p = b.p[back_q];
@@ -401,7 +426,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
         }
       }
       const uint32_t slot = (e[u] > 0 || i == 0) ? static_cast<uint32_t>(p[u]) : up;
-      if (slot != kNoSlot) {
+      if (LINK && slot != kNoSlot) {
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
           const int32_t ch = lc[u] + side;
@@ -418,7 +443,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
           }
         }
       }
-      if (e[u] > 0) {
+      if (MAKE && e[u] > 0) {
         if (up != kNoSlot)
           cols.put_make(up, child_of(code[u], level - e[u] + 1), make_key(i, e[u] - 1),
                         p[u] + e[u] - 1);
@@ -444,7 +469,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
         }
       }
     }
-    if (i0 == 0 && wave_id() == 1 && b.m >= 1) {
+    if (LINK && i0 == 0 && wave_id() == 1 && b.m >= 1) {
       // The true root's internal children, the nodes whose parent entry is 0:
       // the split of [0, m] (04_radix_tree.cpp:94-104 with d = +1, l = n).
       const uint32_t c0 = b.codes[0];
@@ -465,10 +490,12 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
       }
     }
     __syncthreads();
-    const uint32_t n_out = min(s_nout, static_cast<uint32_t>(kMaxOutside));
-    if (static_cast<uint32_t>(tid) < n_out)
-      push_subgroup(b, cols, static_cast<int32_t>(s_out[tid].x), s_out[tid].y);
-    __syncthreads();
+    if constexpr (LINK) {
+      const uint32_t n_out = min(s_nout, static_cast<uint32_t>(kMaxOutside));
+      if (static_cast<uint32_t>(tid) < n_out)
+        push_subgroup<MAKE>(b, cols, static_cast<int32_t>(s_out[tid].x), s_out[tid].y);
+      __syncthreads();
+    }
 
     // The nodes, a slot per thread, each in its column's place.
     for (int t = tid; t < cols.n; t += kThreads) {
@@ -476,12 +503,34 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
       const u64 own = s_owner[t];
       int32_t* col = reinterpret_cast<int32_t*>(s_child + t * kColWords);
       int32_t w[15];
+      if constexpr (PHASE == kWhole) {
 #pragma unroll
-      for (int c = 0; c < 8; ++c) w[c] = col[2 * c];
-      w[13] = col[16];
-      w[14] = 0;
-      w[8] = w[9] = w[10] = w[11] = w[12] = 0;
-      if (own != 0 || s == 0) {
+        for (int c = 0; c < 8; ++c) w[c] = col[2 * c];
+        w[13] = col[16];
+        w[14] = 0;
+        w[8] = w[9] = w[10] = w[11] = w[12] = 0;
+      } else {
+        __builtin_memcpy(w, b.nodes + s, sizeof(w));
+        int32_t links = 0;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const uint32_t key = static_cast<uint32_t>(col[2 * c + 1]);
+          if constexpr (MAKE) {
+            // (a zeroed node's word holds at most the key of a chain whose walk
+            // left its tile)
+            const uint32_t far = static_cast<uint32_t>(w[c]);
+            w[c] = col[2 * c];
+            if (far > key) w[c] = b.p[(far - 1u) >> 4] + static_cast<int32_t>((far - 1u) & 15u);
+            if (far) links |= 1 << c;
+          } else if (key) {
+            w[c] = col[2 * c];
+            links |= 1 << c;
+          }
+        }
+        if constexpr (MAKE) w[13] |= links | col[16];
+        else w[14] &= ~links;
+      }
+      if (MAKE && (own != 0 || s == 0) && (PHASE == kWhole || s != 0)) {
         // Corner and cell size of the chain's step (oct.h:44-57, 76-88); slot
         // 0 is the root of apps/cpu_demo/main.cpp:125-132. Other slots no
         // chain covers stay zero.
@@ -528,6 +577,31 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   }
 }
 
+// The make call alone has no children arrays to walk down from a slot's owner,
+// so the top link of a chain whose walk up leaves its tile comes from below: the
+// walk in global memory, and the order key into the child's word of the zeroed
+// node, kept by an atomic max. The make phase turns it into the link.
+__global__ __launch_bounds__(256) void oct_far_kernel(OctArgs a) {
+  const int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x);
+  if (i < 1 || i >= a.n_brt_host) return;
+  const int32_t e = a.edge[i];
+  int32_t h = a.parent[i];
+  if (e <= 0) return;
+  bool far = false;
+  for (int hop = 0; hop < 32; ++hop) {
+    far |= (h ^ i) >= kOctTile;  // (another tile: the numbers differ above its bits)
+    if (a.edge[h] > 0 || h == 0) break;
+    h = a.parent[h];
+  }
+  if (!far) return;
+  const int32_t slot = a.offsets[h];
+  if (slot < 0 || slot >= a.k_host) return;
+  const int32_t level = a.prefix_n[i] / 3;
+  atomicMax(reinterpret_cast<uint32_t*>(
+                &a.nodes[slot].children[child_of(a.codes[i], level - e + 1)]),
+            make_key(i, e - 1));
+}
+
 // Root node of apps/cpu_demo/main.cpp:125-132 alone (the per-stage entry
 // point that stands in for that host code).
 __global__ void oct_root_kernel(OctNode* nodes, const uint32_t* codes,
@@ -563,10 +637,21 @@ bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_s
   if (total_tiles <= 0) return true;
   if (single.mail && (sv.n_seg != 1 || !single.oct_start || !single.ctrl)) return false;
   if (single.mail)
-    oct_build_kernel<true><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
+    oct_build_kernel<true, kWhole><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
   else
-    oct_build_kernel<false><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
+    oct_build_kernel<false, kWhole><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
   return true;
+}
+
+void launch_oct_make(const OctArgs& a, const SegView& sv, hipStream_t s) {
+  oct_far_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
+  oct_build_kernel<false, kMakePhase>
+      <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
+}
+
+void launch_oct_link(const OctArgs& a, const SegView& sv, hipStream_t s) {
+  oct_build_kernel<false, kLinkPhase>
+      <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
 }
 
 }  // namespace ocp

@@ -113,8 +113,8 @@ inline int pipe_sort_tile(const TuneTable& t, bool perm) {
 constexpr int hist_stride(int bits) { return bits == 10 ? 3 * 1024 : 4 * 256; }
 inline int morton_tile(const TuneTable& t) { return 256 * t.morton_ppt; }
 inline int scan_tile(const TuneTable& t) { return 256 * t.scan_ipt; }
-constexpr int kNodeTile = 256;  // BRT nodes per tile of the per-stage entries
-constexpr int kOctTile = 512;   // ... of the fused build's octree kernel
+constexpr int kNodeTile = 256;  // BRT nodes per tile of the per-stage radix tree
+constexpr int kOctTile = 512;   // ... of the octree kernel
 
 bool sort_config_supported(int waves, int kpt);
 bool sort10_config_supported(int kpt);
@@ -356,18 +356,11 @@ struct OctSingle {
 bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_start,
                       int32_t total_tiles, const OctSingle& single, hipStream_t s);
 
-// ---- stage 7, per-stage entry points (k_octree_stage.hip)
-// The make call of the reference signature has no children arrays
-// (has_leaf_*, left_child may be null with phases/resolve bit 1 only).
-// phase bits: 1 = make writes, 2 = link writes, 4 = leaf-mask AND-NOT
-void launch_oct_scatter(const OctArgs& a, const SegView& sv,
-                        const int32_t* tile_start, int32_t total_tiles,
-                        int phases, hipStream_t s);
-// resolve bits: 1 = resolve make keys, 2 = resolve link keys,
-//               4 = write corners and cell sizes, 8 = write the root node
-void launch_oct_finalize(const OctArgs& a, const SegView& sv,
-                         const int32_t* tile_start, int32_t total_tiles,
-                         int resolve, hipStream_t s);
+// The per-stage entries: the same kernel on n_brt_host nodes and k_host slots,
+// doing the make writes (without the children arrays, which may be null) or the
+// link writes, into nodes that the caller prepared.
+void launch_oct_make(const OctArgs& a, const SegView& sv, hipStream_t s);
+void launch_oct_link(const OctArgs& a, const SegView& sv, hipStream_t s);
 
 // ---- node formats and validator (k_format.hip). Node counts come from
 // oct_start[n_seg] on the device; boxes are per segment (smin/srg) or the
