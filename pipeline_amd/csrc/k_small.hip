@@ -286,7 +286,23 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
   }
 }
 
+// The keys-only sort entry for few keys: one launch instead of six.
+template <int WAVES, int KPT, int P0, int BINS>
+__global__ __launch_bounds__(WAVES * 64) void small_sort_kernel(uint32_t* __restrict__ keys,
+                                                               int32_t n,
+                                                               const uint32_t* __restrict__ ctrl) {
+  if (stopped_any(ctrl)) return;
+  lds_bucket_sort<WAVES, KPT, P0, 8, BINS>(keys, keys, n);
+}
+
 }  // namespace
+
+void launch_small_sort(uint32_t* keys, int32_t n, const uint32_t* ctrl, hipStream_t s) {
+  if (n <= 4096)
+    small_sort_kernel<16, 4, 12, 13><<<1, 1024, 0, s>>>(keys, n, ctrl);
+  else
+    small_sort_kernel<16, 16, 12, 13><<<1, 1024, 0, s>>>(keys, n, ctrl);
+}
 
 void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64_t max_seg,
                          bool device_boxes, float* box_min, float* box_range, const SmallOut& o,

@@ -318,6 +318,13 @@ void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64
                          bool device_boxes, float* box_min, float* box_range, const SmallOut& o,
                          uint32_t* ctrl, hipStream_t s);
 
+// Sort of at most kSmallSort keys in place by one workgroup: what LDS holds, and
+// up to there faster than the six launches of the passes, for spread keys (2000:
+// 52 -> 20 us, 16,384: 54 -> 33) as for those that take the radix passes (16,384
+// clustered ones: 55 -> 50).
+constexpr uint32_t kSmallSort = 16384;
+void launch_small_sort(uint32_t* keys, int32_t n, const uint32_t* ctrl, hipStream_t s);
+
 // ---- stage 7 (k_octree.hip)
 struct OctArgs {
   OctNode* nodes;            // base of all segments' nodes

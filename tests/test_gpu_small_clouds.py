@@ -35,6 +35,22 @@ def test_sizes(ctx, n):
         _both_ways(ctx, pts, oracle.build_plain(pts))
 
 
+@pytest.mark.parametrize("n", [2, 3, 63, 1023, 4095, 4096, 4097, 9999, 16383, 16384, 16385,
+                               (1 << 20) - 1, 1 << 20])
+def test_key_sort_sizes(ctx, n):
+    """The sort entry around what one workgroup takes and where its first pass
+    changes form: spread, crowded, equal and full 32-bit keys."""
+    rng = np.random.default_rng(n)
+    for keys in (rng.integers(0, 1 << 30, n), rng.integers(0, 1 << 32, n),
+                 rng.integers(0, 50, n) + (rng.integers(0, 3, n) << 28), np.full(n, 0xffffffff)):
+        keys = keys.astype(np.uint32)
+        a, b = ctx.upload(keys), ctx.empty(n, np.uint32)
+        ctx.k_SortKeys(a, b, n)
+        np.testing.assert_array_equal(a.to_host(), np.sort(keys))
+        a.free()
+        b.free()
+
+
 @pytest.mark.parametrize("u", [511, 2049, 4096, 8192])
 def test_code_patterns(ctx, u):
     """Consecutive codes, powers of two apart, far pairs, and a crowd of codes
