@@ -48,26 +48,29 @@
 //     one thread per listed child walks that part of the group downwards in
 //     global memory. Such a node spans a tile end, and the nodes spanning one
 //     are nested with different prefix lengths, so at most 124 are listed.
-//  3. One thread per slot assembles the node in its column's place, and the
+//  3. One thread per slot assembles the node, packs it over the columns, and the
 //     tile's nodes leave as consecutive 16-byte stores.
 // A tile with more slots than columns takes them in several rounds.
 //
 // The per-stage entries (k_MakeOctNodes, k_LinkLeafNodes: include/cuda/kernels/
 // 07_octree.cuh:7-28) are the same kernel doing one half of the pushes into
 // nodes that it reads and writes whole. Make has no children arrays: see
-// oct_far_kernel. For 2M points make takes 52 us and link 33; a scatter of order
+// oct_far_kernel. For 2M points make takes 46 us and link 30; a scatter of order
 // keys by global atomics and a kernel that resolved them took 117 and 187.
 //
-// What bounds it: 10M uniform points take 174 us, of which the walks of the
-// listed children (a chain of up to four dependent loads that one wave of the
-// tile makes while the others wait) are 41 us and the node stores, 280 MB, 34;
-// 24 bytes a node read and 60 a slot written are 104 us at the rate of a large
-// copy. The owner-computes form this replaces, a lane per chain that walked
-// its group down, read its neighbours' chains and resolved keys into values,
-// issued 1587 vector instructions a wave and took 250 us (99 -> 69 us at 2^24
-// clustered points). 512 nodes a tile and two per thread, for the walks cost
-// the same for any tile: 256 nodes, one per thread, and stores of 60 bytes a
-// lane took 244 us; two per thread in 512-thread workgroups 212 us.
+// What bounds it: how many tiles share a CU while each waits for its loads, its
+// barriers and the walks of its listed children (a chain of up to four dependent
+// loads that one wave makes while the others wait). 10M uniform points take
+// 152 us, 2^24 clustered ones 59; 24 bytes a node read and 60 a slot written are
+// 104 us of the former at the rate of a large copy. 312 columns of 64 bytes are
+// what lets six tiles share a CU's LDS, as 60 registers do; with 80 bytes a
+// column (an own word for the mask) and nodes finished where their column lay,
+// five did, in 174 us and 67. Four tiles by registers took 188; 256 columns, with
+// which more tiles need a second round, 155 and 68. One wave walking the listed
+// children while three push was slower (182), and so were 256 nodes a tile, one
+// per thread, and stores of 60 bytes a lane (244), two per thread in 512-thread
+// workgroups (212), and a lane per chain that walked its group down, read its
+// neighbours' chains and resolved keys into values (250).
 //
 // Edge counts are at most 10 (prefix lengths are at most 31 for 30-bit
 // codes), so a chain spans at most 10 slots.
@@ -78,10 +81,14 @@ namespace {
 
 constexpr int32_t kMaxEdge = 10;
 constexpr int kThreads = 256;
-constexpr int kCols = 320;      // slots per round; a tile of 512 nodes has ~240
+constexpr int kCols = 312;      // slots per round; a tile of 512 nodes has ~240
 constexpr int kCodeHalo = 32;   // codes staged on either side of a tile
 constexpr int kMaxOutside = 128;
-constexpr uint32_t kHead = 0x80000000u;
+// A node's step of a walk up, 16 bits: kHead + slot of the tile where the walk
+// ends (a chain's first slot, node 0's slot 0), else the parent's place in the
+// tile, kOutside if it has none.
+constexpr uint32_t kHead = 0x8000u;
+constexpr uint32_t kOutside = 0x4000u;
 constexpr uint32_t kNoSlot = 0xffffffffu;
 
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
@@ -125,21 +132,25 @@ __device__ __forceinline__ uint32_t link_key(int32_t node, int side) {
 
 typedef unsigned long long u64;
 
-// The columns of the slots [base, base + n), n <= kCols: nine 8-byte words a
-// slot, the last writer of each child index (order key << 32 | value, 0: none)
-// and the child-node mask. An odd number of them, so that the pushes of a wave
-// spread over the LDS banks. The finished node takes the column's place.
-constexpr int kColWords = 9;
+// The columns of the slots [base, base + n), n <= kCols: eight 8-byte words a
+// slot, the last writer of each child index (order key << 32 | value, 0: none),
+// turned by one every four slots so that one child index of many slots spreads
+// over the LDS banks. The finished nodes take the columns' place.
+constexpr int kColWords = 8;
+__device__ __forceinline__ uint32_t col_word(uint32_t r, uint32_t which) {
+  return r * kColWords + ((which + (r >> 2)) & 7u);
+}
 struct Columns {
   lds_ptr<u64> child;
-  lds_ptr<u64> owner;  // chain + 1 << 34 | level << 30 | code, 0: no chain
+  lds_ptr<u64> owner;     // chain + 1 << 34 | level << 30 | code, 0: no chain
+  lds_ptr<uint32_t> mask;  // child-node masks, a byte each
   int32_t base;
   int32_t n;
   __device__ __forceinline__ void put(uint32_t slot, uint32_t which, uint32_t key,
                                       int32_t value) const {
     const uint32_t r = slot - static_cast<uint32_t>(base);
     if (r < static_cast<uint32_t>(n))
-      __hip_atomic_fetch_max(child + r * kColWords + which,
+      __hip_atomic_fetch_max(child + col_word(r, which),
                              (static_cast<u64>(key) << 32) | static_cast<uint32_t>(value),
                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
@@ -149,7 +160,7 @@ struct Columns {
     const uint32_t r = slot - static_cast<uint32_t>(base);
     if (r >= static_cast<uint32_t>(n)) return;
     put(slot, which, key, value);
-    __hip_atomic_fetch_or((lds_ptr<uint32_t>)(child + r * kColWords + 8), 1u << which,
+    __hip_atomic_fetch_or(mask + (r >> 2), 1u << ((r & 3u) * 8u + which),
                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
   // Chain i: the slots p .. p + e - 1 with their geometry, and its step links
@@ -251,13 +262,13 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   constexpr int T = kOctTile;
   constexpr int NPT = T / kThreads;
   constexpr bool MAKE = PHASE != kLinkPhase, LINK = PHASE != kMakePhase;
-  __shared__ u64 s_child[kColWords * kCols];
+  __shared__ __attribute__((aligned(16))) u64 s_child[kColWords * kCols];
   __shared__ u64 s_owner[kCols];
-  // A node's step of a walk up: kHead | slot where the walk ends (a chain's
-  // first slot, node 0's slot 0), else the node's parent.
-  __shared__ uint32_t s_walk[T];
+  __shared__ uint32_t s_mask[kCols / 4];
+  __shared__ uint16_t s_walk[T];
   __shared__ uint32_t s_code[T + 2 * kCodeHalo];
-  __shared__ uint2 s_out[kMaxOutside];  // listed children {node, slot}
+  __shared__ int32_t s_out[kMaxOutside];  // listed children ...
+  __shared__ uint16_t s_out_slot[kMaxOutside];  // ... and their slots of the tile
   __shared__ uint32_t s_nout;
 
   const TileRef r = find_tile(tile_start, sv.n_seg, xcd_tile(blockIdx.x, gridDim.x));
@@ -312,7 +323,6 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   b.mn = seg_mn;
   b.rg = seg_rg;
 
-  const int tid = threadIdx.x;
   // The slots of the tile.
   const int32_t i_end = min(i0 + T, b.m);
   int32_t p_before = i0 > 0 ? b.p[i0 - 1] : -1;
@@ -331,9 +341,14 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   Columns cols;
   cols.child = as_lds<u64>(s_child);
   cols.owner = as_lds<u64>(s_owner);
+  cols.mask = as_lds<uint32_t>(s_mask);
+  const int32_t slot_0 = p_before + 1;
 
-  for (cols.base = p_before + 1; cols.base < s_end; cols.base += kCols) {
+  for (cols.base = slot_0; cols.base < s_end; cols.base += kCols) {
     cols.n = min(kCols, s_end - cols.base);
+    // (opaque: the compiler would keep every address of a round for the next)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     // (loaded in every round, of which a tile rarely has a second, so that
     // they hold no register beyond the pushes)
     // This thread's nodes, and for the last wave one of the 64 nodes before the
@@ -390,14 +405,19 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
       back_e = b.e[back_q];
       back_p = b.p[back_q];
     }
-    for (int q = tid; q < kColWords * kCols; q += kThreads) s_child[q] = 0;
+    for (int q = tid; q < kColWords * kCols / 2; q += kThreads)
+      reinterpret_cast<v4i*>(s_child)[q] = v4i{0, 0, 0, 0};
     for (int q = tid; q < kCols; q += kThreads) s_owner[q] = 0;
+    static_assert(kCols % 4 == 0 && kCols / 4 <= kThreads, "masks");
+    if (tid < kCols / 4) s_mask[tid] = 0;
 #pragma unroll
     for (int u = 0; u < NPT; ++u) {
       const int32_t i = i0 + u * kThreads + tid;
       const bool head = i < b.m && (e[u] > 0 || i == 0);
-      s_walk[u * kThreads + tid] =
-          head ? kHead | static_cast<uint32_t>(p[u]) : static_cast<uint32_t>(par[u]);
+      const uint32_t up = static_cast<uint32_t>(par[u] - i0);
+      s_walk[u * kThreads + tid] = static_cast<uint16_t>(
+          head ? kHead | (static_cast<uint32_t>(p[u] - slot_0) & 0x3fffu)
+               : min(up, kOutside));
       s_code[kCodeHalo + u * kThreads + tid] = code[u];
     }
     if (tid < kCodeHalo) s_code[tid] = code_halo;
@@ -414,16 +434,9 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
       // where it leaves the tile.
       uint32_t up = kNoSlot;
       if (i > 0) {
-        uint32_t h = static_cast<uint32_t>(par[u]);
-        for (int hop = 0; hop < 8; ++hop) {
-          const uint32_t rel = h - static_cast<uint32_t>(i0);
-          if (rel >= static_cast<uint32_t>(T)) break;
-          h = s_walk[rel];
-          if (h & kHead) {
-            up = h & ~kHead;
-            break;
-          }
-        }
+        uint32_t h = min(static_cast<uint32_t>(par[u] - i0), kOutside);
+        for (int hop = 0; hop < 8 && h < static_cast<uint32_t>(T); ++hop) h = s_walk[h];
+        if (h - kHead <= 0x3fffu) up = static_cast<uint32_t>(slot_0) + (h - kHead);
       }
       const uint32_t slot = (e[u] > 0 || i == 0) ? static_cast<uint32_t>(p[u]) : up;
       if (LINK && slot != kNoSlot) {
@@ -439,7 +452,10 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
             // (node 0 is the short-range root: its group grows through the
             // true root's children below, not through its own)
             const uint32_t at = atomicAdd(&s_nout, 1u);
-            if (at < kMaxOutside) s_out[at] = make_uint2(static_cast<uint32_t>(ch), slot);
+            if (at < kMaxOutside) {
+              s_out[at] = ch;
+              s_out_slot[at] = static_cast<uint16_t>(slot - static_cast<uint32_t>(slot_0));
+            }
           }
         }
       }
@@ -486,91 +502,105 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
       const int32_t y = lo + lane;
       if (lane < 2 && y >= T && y < b.m) {
         const uint32_t at = atomicAdd(&s_nout, 1u);
-        if (at < kMaxOutside) s_out[at] = make_uint2(static_cast<uint32_t>(y), 0u);
+        if (at < kMaxOutside) {
+          s_out[at] = y;
+          s_out_slot[at] = 0;
+        }
       }
     }
     __syncthreads();
     if constexpr (LINK) {
       const uint32_t n_out = min(s_nout, static_cast<uint32_t>(kMaxOutside));
       if (static_cast<uint32_t>(tid) < n_out)
-        push_subgroup<MAKE>(b, cols, static_cast<int32_t>(s_out[tid].x), s_out[tid].y);
+        push_subgroup<MAKE>(b, cols, s_out[tid],
+                            static_cast<uint32_t>(slot_0) + s_out_slot[tid]);
       __syncthreads();
     }
 
-    // The nodes, a slot per thread, each in its column's place.
-    for (int t = tid; t < cols.n; t += kThreads) {
-      const int32_t s = cols.base + t;
-      const u64 own = s_owner[t];
-      int32_t* col = reinterpret_cast<int32_t*>(s_child + t * kColWords);
-      int32_t w[15];
-      if constexpr (PHASE == kWhole) {
+    // The nodes, a slot per thread, packed over the columns: those of a turn are
+    // read before its nodes overwrite them, and a node is shorter than a column.
+    // (two calls, not a loop: nearly every tile has one turn, and in a loop 10M
+    // points took 166 us, not 162)
+    const auto turn = [&](int t) {
+      const bool live = t < cols.n;
+      int32_t nd[15];
+      if (live) {
+        const int32_t s = cols.base + t;
+        const u64 own = s_owner[t];
+        const uint32_t kids = (s_mask[t >> 2] >> ((t & 3) * 8)) & 255u;
+        if constexpr (PHASE == kWhole) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) w[c] = col[2 * c];
-        w[13] = col[16];
-        w[14] = 0;
-        w[8] = w[9] = w[10] = w[11] = w[12] = 0;
-      } else {
-        __builtin_memcpy(w, b.nodes + s, sizeof(w));
-        int32_t links = 0;
+          for (int c = 0; c < 8; ++c) nd[c] = static_cast<int32_t>(s_child[col_word(t, c)]);
+          nd[13] = static_cast<int32_t>(kids);
+          nd[14] = 0;
+          nd[8] = nd[9] = nd[10] = nd[11] = nd[12] = 0;
+        } else {
+          __builtin_memcpy(nd, b.nodes + s, sizeof(nd));
+          int32_t links = 0;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          const uint32_t key = static_cast<uint32_t>(col[2 * c + 1]);
-          if constexpr (MAKE) {
-            // (a zeroed node's word holds at most the key of a chain whose walk
-            // left its tile)
-            const uint32_t far = static_cast<uint32_t>(w[c]);
-            w[c] = col[2 * c];
-            if (far > key) w[c] = b.p[(far - 1u) >> 4] + static_cast<int32_t>((far - 1u) & 15u);
-            if (far) links |= 1 << c;
-          } else if (key) {
-            w[c] = col[2 * c];
-            links |= 1 << c;
+          for (int c = 0; c < 8; ++c) {
+            const u64 last = s_child[col_word(t, c)];
+            const uint32_t key = static_cast<uint32_t>(last >> 32);
+            if constexpr (MAKE) {
+              // (a zeroed node's word holds at most the key of a chain whose walk
+              // left its tile)
+              const uint32_t far = static_cast<uint32_t>(nd[c]);
+              nd[c] = static_cast<int32_t>(last);
+              if (far > key) nd[c] = b.p[(far - 1u) >> 4] + static_cast<int32_t>((far - 1u) & 15u);
+              if (far) links |= 1 << c;
+            } else if (key) {
+              nd[c] = static_cast<int32_t>(last);
+              links |= 1 << c;
+            }
           }
+          if constexpr (MAKE) nd[13] |= links | static_cast<int32_t>(kids);
+          else nd[14] &= ~links;
         }
-        if constexpr (MAKE) w[13] |= links | col[16];
-        else w[14] &= ~links;
+        if (MAKE && (own != 0 || s == 0) && (PHASE == kWhole || s != 0)) {
+          // Corner and cell size of the chain's step (oct.h:44-57, 76-88); slot
+          // 0 is the root of apps/cpu_demo/main.cpp:125-132. Other slots no
+          // chain covers stay zero.
+          const int32_t lv = s == 0 ? root_level : static_cast<int32_t>((own >> 30) & 15u);
+          const uint32_t cd = s == 0 ? b.codes[0] : static_cast<uint32_t>(own) & 0x3fffffffu;
+          const uint32_t shift = static_cast<uint32_t>(kMortonBits - 3 * lv) & 31u;
+          const uint32_t corner = (cd >> shift) << shift;
+          nd[8] = __float_as_int(decode_axis(corner, 0, b.mn, b.rg));
+          nd[9] = __float_as_int(decode_axis(corner, 1, b.mn, b.rg));
+          nd[10] = __float_as_int(decode_axis(corner, 2, b.mn, b.rg));
+          nd[11] = __float_as_int(1.0f);
+          const uint32_t sh = static_cast<uint32_t>(lv - root_level) & 31u;
+          nd[12] = __float_as_int(b.rg / static_cast<float>(static_cast<int32_t>(1u << sh)));
+        }
       }
-      if (MAKE && (own != 0 || s == 0) && (PHASE == kWhole || s != 0)) {
-        // Corner and cell size of the chain's step (oct.h:44-57, 76-88); slot
-        // 0 is the root of apps/cpu_demo/main.cpp:125-132. Other slots no
-        // chain covers stay zero.
-        const int32_t lv = s == 0 ? root_level : static_cast<int32_t>((own >> 30) & 15u);
-        const uint32_t cd = s == 0 ? b.codes[0] : static_cast<uint32_t>(own) & 0x3fffffffu;
-        const uint32_t shift = static_cast<uint32_t>(kMortonBits - 3 * lv) & 31u;
-        const uint32_t corner = (cd >> shift) << shift;
-        w[8] = __float_as_int(decode_axis(corner, 0, b.mn, b.rg));
-        w[9] = __float_as_int(decode_axis(corner, 1, b.mn, b.rg));
-        w[10] = __float_as_int(decode_axis(corner, 2, b.mn, b.rg));
-        w[11] = __float_as_int(1.0f);
-        const uint32_t sh = static_cast<uint32_t>(lv - root_level) & 31u;
-        w[12] = __float_as_int(b.rg / static_cast<float>(static_cast<int32_t>(1u << sh)));
-      }
+      __syncthreads();
+      if (live) {
 #pragma unroll
-      for (int c = 0; c < 15; ++c) col[c] = w[c];
-    }
+        for (int c = 0; c < 15; ++c) reinterpret_cast<int32_t*>(s_child)[t * 15 + c] = nd[c];
+      }
+    };
+    static_assert(kCols <= 2 * kThreads, "two turns");
+    turn(tid);
+    if (cols.n > kThreads) turn(tid + kThreads);
     __syncthreads();
     // Out in whole lines: consecutive lanes store consecutive 16 bytes.
     int32_t* dst = reinterpret_cast<int32_t*>(b.nodes + cols.base);
     const int32_t words = cols.n * 15;
-    const int32_t* s_node = reinterpret_cast<const int32_t*>(s_child);
-    for (int32_t q = tid * 4; q < words; q += kThreads * 4) {
-      int32_t x[4];
-      uint32_t node = static_cast<uint32_t>(q) / 15u, c = static_cast<uint32_t>(q) % 15u;
+    // (all LDS reads in flight together; those past the last node are not stored)
+    constexpr int OUT = (kCols * 15 + kThreads * 4 - 1) / (kThreads * 4);
+    constexpr int LAST = kCols * kColWords / 2 - 1;  // in 16 bytes
+    v4i x[OUT];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        // (past the last node: its column's unused words or the next column's)
-        x[u] = s_node[min(node, static_cast<uint32_t>(kCols - 1)) * (2 * kColWords) + c];
-        if (++c == 15u) {
-          c = 0;
-          ++node;
-        }
-      }
+    for (int k = 0; k < OUT; ++k)
+      x[k] = reinterpret_cast<const v4i*>(s_child)[min(k * kThreads + tid, LAST)];
+#pragma unroll
+    for (int k = 0; k < OUT; ++k) {
+      const int32_t q = (k * kThreads + tid) * 4;
       if (q + 4 <= words) {
-        __builtin_memcpy(dst + q, x, 16);
+        __builtin_memcpy(dst + q, &x[k], 16);
       } else {
 #pragma unroll
         for (int u = 0; u < 4; ++u)
-          if (q + u < words) dst[q + u] = x[u];
+          if (q + u < words) dst[q + u] = x[k][u];
       }
     }
     __syncthreads();
