@@ -329,9 +329,11 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
 // The pairs' b values of a tile and its halo lie in LDS as bytes, with the
 // minima of 16 and of 256 of them: three levels of 16-byte rows. One row is
 // compared with b_k by four byte-wise subtractions whose top bits four dot
-// products collect into a 16-bit mask; the mask of the pair's own row gives
-// the nearest smaller value on both sides, else the row of row minima names
-// the row to look into, else that of the 256-pair minima. Values outside the
+// products collect into a 16-bit mask. The masks of the pair's own row and of the
+// one nearer to it give the nearest smaller value on both sides of five pairs in
+// six; the others are listed and searched a full wave at a time: their own row,
+// else the row of row minima names the row to look into, else that of the
+// 256-pair minima. Values outside the
 // segment are 0, below any pair's. An end beyond the window is searched by
 // the wave in the codes themselves, 64 candidates a round trip.
 //
@@ -343,12 +345,12 @@ __global__ __launch_bounds__(256) void radix_tree_kernel(
 // comes from its own search, the true root's pair only links its children, and
 // those count their edges from node 0's prefix length.
 //
-// What bounds it: vector instructions, about half of the ~370 per 64 nodes
-// that the searches by code of the kernel above issue. 10M uniform points:
-// 99 -> 66 us, and the edge scan, which reads the counts instead of forming
-// them from two byte arrays, 33 -> 26 us; 2^24 clustered points: 155 -> 99 us
-// and 17 -> 14 us. Tiles of 2048 with a halo of 256, 512 or 1024 pairs: 66.0,
-// 66.4, 68.1 us (98, 99, 101 us clustered).
+// What bounds it: vector instructions and stores. 10M uniform points take 55 us
+// (the 190 MB it moves 37 at the rate of a large copy), 2^24 clustered ones 31;
+// searching every pair at all three levels, because some lane of a wave needs
+// each, 66 and 37; the searches by code of the kernel above 99 us, with an edge
+// scan of 33 us that formed the counts it now reads (22). The halo is 512 pairs
+// for tiles of 2048 and 256 for those of 512 (2^20 points 17.3 us with 512, 16.8).
 // The end of the run of keys around key `from` whose xor with code c is below
 // lim, at least `reach` keys away on the side of d (+1, -1), in [0, m].
 __device__ __forceinline__ int32_t wave_run_end(const uint32_t* __restrict__ codes, uint32_t c,
@@ -380,6 +382,7 @@ __global__ __launch_bounds__(256) void radix_pairs_kernel(
   __shared__ v4u s_b256;         // minima of 256
   __shared__ uint32_t s_rec[T];  // records of the tile's node indices
   __shared__ int32_t s_par[T];
+  __shared__ uint16_t s_list[4][128];
   constexpr uint32_t kNone = 0xffffffffu;
 
   const TileRef r = find_tile(tile_start, sv.n_seg, xcd_tile(blockIdx.x, gridDim.x));
@@ -442,109 +445,146 @@ __global__ __launch_bounds__(256) void radix_pairs_kernel(
   const uint8_t* b8 = reinterpret_cast<const uint8_t*>(s_b);
   const v4u row256 = s_b256;
 
+  // What a pair's two ends give.
+  const auto emit = [&](int32_t p, uint32_t b, int32_t pl, int32_t pr, uint32_t b_l,
+                        uint32_t b_r) {
+    const int32_t g = i0 + p;
+    const uint32_t b_up = max(b_l, b_r);
+    const int32_t node = b_l >= b_r ? pl + 1 : pr;
+    const bool leaf_l = pl + 1 == g;
+    const bool leaf_r = pr == g + 1;
+    const uint32_t pn = b - 1u;
+    const int32_t e = static_cast<int32_t>(third(pn)) -
+                      static_cast<int32_t>(third(b_up == b_root ? pn_0 : b_up - 1u));
+    const uint32_t rec = static_cast<uint32_t>(p) | (pn << 11) | (leaf_l ? 1u << 16 : 0u) |
+                         (leaf_r ? 1u << 17 : 0u) | (static_cast<uint32_t>(e + 16) << 18);
+    const int32_t rel = node - i0;
+    if (b_up == 0) {
+      // the true root: node 0's record is written below
+    } else if (static_cast<uint32_t>(rel) < static_cast<uint32_t>(T)) {
+      s_rec[rel] = rec;
+    } else {
+      prefix[node] = static_cast<uint8_t>(pn);
+      hl[node] = leaf_l;
+      hr[node] = leaf_r;
+      lc[node] = g;
+      edge[node] = e;
+    }
+    if (!leaf_l) s_par[p] = node;
+    if (!leaf_r) {
+      if (p + 1 < T) s_par[p + 1] = node;
+      else par[g + 1] = node;
+    }
+  };
+  // Most ends lie within eight pairs: every pair is compared with the two rows
+  // nearest to it; those for which that is not enough are listed.
+  uint32_t listed = 0;
+  uint16_t* list = s_list[wave_id()];
+  const int32_t lane = static_cast<int32_t>(lane_id());
+#pragma unroll 1
   for (int k = 0; k < T / 256; ++k) {
-    const int32_t p = k * 256 + tid;  // position in the tile
-    const int32_t g = i0 + p;         // the pair
-    const bool live = g < m;
-    const uint32_t q = static_cast<uint32_t>(p + HALO);
-    const uint32_t b = b8[q];
-    // (b + 127 in every byte; a dead lane's b of 0 finds nothing)
-    const uint32_t key = __builtin_amdgcn_perm(0u, b + 127u, 0u);
-    const uint32_t row = q >> 4, grp = q >> 8;
-    const uint32_t m0 = below16(s_b[row], key);
-    const uint32_t m1 = below16(s_b16[grp], key);
-    const uint32_t m2 = below16(row256, key);
-    int32_t end_l = -2, end_r = -2;  // window positions of L and R, -2: not in the window
-    uint32_t hit = m0 & (0xfffeu << (q & 15u)) & 0xffffu;
-    uint32_t at = row;
-    if (hit == 0) {
-      uint32_t gg = grp;
-      uint32_t rr = m1 & (0xfffeu << (row & 15u)) & 0xffffu;
-      if (rr == 0) {
-        const uint32_t g2 = m2 & (0xfffeu << grp) & 0xffffu;
-        if (g2) {
-          gg = static_cast<uint32_t>(__builtin_ctz(g2));
-          rr = below16(s_b16[gg], key);
+    {
+      const int32_t p = k * 256 + tid;  // place in the tile
+      const bool live = i0 + p < m;
+      const uint32_t q = static_cast<uint32_t>(p + HALO);
+      const uint32_t b = b8[q];
+      const uint32_t key = __builtin_amdgcn_perm(0u, b + 127u, 0u);
+      const uint32_t row = (q - 8u) >> 4;
+      const uint32_t pos = q - row * 16u;
+      const uint32_t hits = below16(s_b[row], key) | (below16(s_b[row + 1], key) << 16);
+      const uint32_t to_r = hits & (0xfffffffeu << pos), to_l = hits & ((1u << pos) - 1u);
+      const bool found = to_r != 0 && to_l != 0;
+      if (live && found) {
+        const int32_t end_r = static_cast<int32_t>(row * 16u) + __builtin_ctz(to_r);
+        const int32_t end_l =
+            static_cast<int32_t>(row * 16u) + 31 - __clz(static_cast<int>(to_l));
+        emit(p, b, wb + end_l, wb + end_r, b8[end_l], b8[end_r]);
+      }
+      const uint64_t more = __ballot(live && !found);
+      if ((more >> lane) & 1u)
+        list[listed + static_cast<uint32_t>(__popcll(more & lanemask_lt()))] =
+            static_cast<uint16_t>(p);
+      listed += static_cast<uint32_t>(__popcll(more));
+    }
+    while (listed >= (k == T / 256 - 1 ? 1u : 64u)) {
+      const uint32_t batch = min(listed, 64u);
+      listed -= batch;
+      const bool live = static_cast<uint32_t>(lane) < batch;
+      const int32_t p = live ? list[listed + lane] : 0;
+      const int32_t g = i0 + p;  // the pair
+      const uint32_t q = static_cast<uint32_t>(p + HALO);
+      const uint32_t b = b8[q];
+      // (b + 127 in every byte; a dead lane's b of 0 finds nothing)
+      const uint32_t key = __builtin_amdgcn_perm(0u, b + 127u, 0u);
+      const uint32_t row = q >> 4, grp = q >> 8;
+      const uint32_t m0 = below16(s_b[row], key);
+      const uint32_t m1 = below16(s_b16[grp], key);
+      const uint32_t m2 = below16(row256, key);
+      int32_t end_l = -2, end_r = -2;  // window positions of L and R, -2: not in the window
+      uint32_t hit = m0 & (0xfffeu << (q & 15u)) & 0xffffu;
+      uint32_t at = row;
+      if (hit == 0) {
+        uint32_t gg = grp;
+        uint32_t rr = m1 & (0xfffeu << (row & 15u)) & 0xffffu;
+        if (rr == 0) {
+          const uint32_t g2 = m2 & (0xfffeu << grp) & 0xffffu;
+          if (g2) {
+            gg = static_cast<uint32_t>(__builtin_ctz(g2));
+            rr = below16(s_b16[gg], key);
+          }
+        }
+        if (rr) {
+          at = gg * 16u + static_cast<uint32_t>(__builtin_ctz(rr));
+          hit = below16(s_b[at], key);
         }
       }
-      if (rr) {
-        at = gg * 16u + static_cast<uint32_t>(__builtin_ctz(rr));
-        hit = below16(s_b[at], key);
-      }
-    }
-    if (hit) end_r = static_cast<int32_t>(at * 16u + static_cast<uint32_t>(__builtin_ctz(hit)));
-    hit = m0 & ((1u << (q & 15u)) - 1u);
-    at = row;
-    if (hit == 0) {
-      uint32_t gg = grp;
-      uint32_t rr = m1 & ((1u << (row & 15u)) - 1u);
-      if (rr == 0) {
-        const uint32_t g2 = m2 & ((1u << grp) - 1u);
-        if (g2) {
-          gg = 31u - static_cast<uint32_t>(__clz(static_cast<int>(g2)));
-          rr = below16(s_b16[gg], key);
+      if (hit) end_r = static_cast<int32_t>(at * 16u + static_cast<uint32_t>(__builtin_ctz(hit)));
+      hit = m0 & ((1u << (q & 15u)) - 1u);
+      at = row;
+      if (hit == 0) {
+        uint32_t gg = grp;
+        uint32_t rr = m1 & ((1u << (row & 15u)) - 1u);
+        if (rr == 0) {
+          const uint32_t g2 = m2 & ((1u << grp) - 1u);
+          if (g2) {
+            gg = 31u - static_cast<uint32_t>(__clz(static_cast<int>(g2)));
+            rr = below16(s_b16[gg], key);
+          }
+        }
+        if (rr) {
+          at = gg * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(rr)));
+          hit = below16(s_b[at], key);
         }
       }
-      if (rr) {
-        at = gg * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(rr)));
-        hit = below16(s_b[at], key);
+      if (hit) end_l = static_cast<int32_t>(at * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(hit))));
+      uint32_t b_l = end_l >= 0 ? b8[end_l] : 0u;
+      uint32_t b_r = end_r >= 0 ? b8[end_r] : 0u;
+      int32_t pl = wb + end_l, pr = wb + end_r;  // the pairs L and R
+      // Ends beyond the window, one at a time by the whole wave. The window's
+      // last key (first key) is then still in the run.
+      for (uint64_t far = __ballot(live && end_r < 0); far; far &= far - 1) {
+        const int src = __builtin_ctzll(far);
+        const int32_t gs = __builtin_amdgcn_readlane(g, src);
+        const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
+        const int32_t j = wave_run_end(codes, codes[gs + 1], lim, wb + W, 1, m);
+        const uint32_t bj = j < m ? clz32(codes[j] ^ codes[j + 1]) : 0u;
+        if (static_cast<int>(lane_id()) == src) {
+          pr = j;
+          b_r = bj;
+        }
       }
-    }
-    if (hit) end_l = static_cast<int32_t>(at * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(hit))));
-    uint32_t b_l = end_l >= 0 ? b8[end_l] : 0u;
-    uint32_t b_r = end_r >= 0 ? b8[end_r] : 0u;
-    int32_t pl = wb + end_l, pr = wb + end_r;  // the pairs L and R
-    // Ends beyond the window, one at a time by the whole wave. The window's
-    // last key (first key) is then still in the run.
-    for (uint64_t far = __ballot(live && end_r < 0); far; far &= far - 1) {
-      const int src = __builtin_ctzll(far);
-      const int32_t gs = __builtin_amdgcn_readlane(g, src);
-      const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
-      const int32_t j = wave_run_end(codes, codes[gs + 1], lim, wb + W, 1, m);
-      const uint32_t bj = j < m ? clz32(codes[j] ^ codes[j + 1]) : 0u;
-      if (static_cast<int>(lane_id()) == src) {
-        pr = j;
-        b_r = bj;
+      for (uint64_t far = __ballot(live && end_l < 0); far; far &= far - 1) {
+        const int src = __builtin_ctzll(far);
+        const int32_t gs = __builtin_amdgcn_readlane(g, src);
+        const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
+        const int32_t j = wave_run_end(codes, codes[gs], lim, wb, -1, m);
+        const uint32_t bj = j > 0 ? clz32(codes[j - 1] ^ codes[j]) : 0u;
+        if (static_cast<int>(lane_id()) == src) {
+          pl = j - 1;
+          b_l = bj;
+        }
       }
-    }
-    for (uint64_t far = __ballot(live && end_l < 0); far; far &= far - 1) {
-      const int src = __builtin_ctzll(far);
-      const int32_t gs = __builtin_amdgcn_readlane(g, src);
-      const uint32_t lim = 1u << (32u - __builtin_amdgcn_readlane(b, src));
-      const int32_t j = wave_run_end(codes, codes[gs], lim, wb, -1, m);
-      const uint32_t bj = j > 0 ? clz32(codes[j - 1] ^ codes[j]) : 0u;
-      if (static_cast<int>(lane_id()) == src) {
-        pl = j - 1;
-        b_l = bj;
-      }
-    }
-    if (live) {
-      const uint32_t b_up = max(b_l, b_r);
-      const int32_t node = b_l >= b_r ? pl + 1 : pr;
-      const bool leaf_l = pl + 1 == g;
-      const bool leaf_r = pr == g + 1;
-      const uint32_t pn = b - 1u;
-      const int32_t e = static_cast<int32_t>(third(pn)) -
-                        static_cast<int32_t>(third(b_up == b_root ? pn_0 : b_up - 1u));
-      const uint32_t rec = static_cast<uint32_t>(p) | (pn << 11) | (leaf_l ? 1u << 16 : 0u) |
-                           (leaf_r ? 1u << 17 : 0u) | (static_cast<uint32_t>(e + 16) << 18);
-      const int32_t rel = node - i0;
-      if (b_up == 0) {
-        // the true root: node 0's record is written below
-      } else if (static_cast<uint32_t>(rel) < static_cast<uint32_t>(T)) {
-        s_rec[rel] = rec;
-      } else {
-        prefix[node] = static_cast<uint8_t>(pn);
-        hl[node] = leaf_l;
-        hr[node] = leaf_r;
-        lc[node] = g;
-        edge[node] = e;
-      }
-      if (!leaf_l) s_par[p] = node;
-      if (!leaf_r) {
-        if (p + 1 < T) s_par[p + 1] = node;
-        else par[g + 1] = node;
-      }
+      if (live) emit(p, b, pl, pr, b_l, b_r);
     }
   }
   __syncthreads();
@@ -625,7 +665,7 @@ void launch_radix_pairs(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_l
                                        parent, edge, sv, tile_start, n_unique, ctrl);
   };
   if (tile == 2048) go(radix_pairs_kernel<2048, 512>);
-  else go(radix_pairs_kernel<512, 512>);
+  else go(radix_pairs_kernel<512, 256>);
 }
 
 }  // namespace ocp

@@ -274,8 +274,9 @@ void launch_radix_pairs(const uint32_t* codes, uint8_t* prefix_n, uint8_t* has_l
                         int32_t total_tiles, int tile, const int32_t* n_unique,
                         const uint32_t* ctrl, hipStream_t s);
 // Nodes per tile of launch_radix_pairs for a build of n points: 2048 once
-// that still gives every CU several workgroups (10M points: 66 us against 74
-// with 512), 512 below (2^20 points: 16.4 us against 19.6).
+// that still gives every CU several workgroups (10M points, before the listed
+// search: 66 us against 74 with 512), 512 below (2^20 points: 16.4 us against
+// 19.6).
 inline int tree_tile(int64_t n) { return n >= (int64_t(1) << 21) ? 2048 : 512; }
 
 // ---- stages 5 + 6 (k_edge_scan.hip)
