@@ -648,7 +648,8 @@ bool enqueue_octree(ocp_ctx c, const Plan& p, bool capturing) {
   }
   const OctSingle one{w.oct_start, c->ctrl, single ? c->mail : nullptr,
                       static_cast<uint32_t>(std::min<int64_t>(w.k_cap, UINT32_MAX))};
-  const OctArgs a = pipeline_oct_args(c);
+  OctArgs a = pipeline_oct_args(c);
+  a.stream_nodes = oct_stream(p.n_total);
   KScope k(c, kKOctBuild, capturing);
   return launch_oct_build(a, p.sv, p.ts_node, p.tiles_node, one, s);
 }

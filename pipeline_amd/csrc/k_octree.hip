@@ -61,8 +61,9 @@
 // What bounds it: how many tiles share a CU while each waits for its loads, its
 // barriers and the walks of its listed children (a chain of up to four dependent
 // loads that one wave makes while the others wait). 10M uniform points take
-// 152 us, 2^24 clustered ones 59; 24 bytes a node read and 60 a slot written are
-// 104 us of the former at the rate of a large copy. 312 columns of 64 bytes are
+// 135 us, 2^24 clustered ones 57; 24 bytes a node read and 60 a slot written are
+// 104 us of the former at the rate of a large copy. Before the nodes of builds
+// that size were stored past the caches (oct_stream), 152 us and 59. 312 columns of 64 bytes are
 // what lets six tiles share a CU's LDS, as 60 registers do; with 80 bytes a
 // column (an own word for the mask) and nodes finished where their column lay,
 // five did, in 174 us and 67. Four tiles by registers took 188; 256 columns, with
@@ -92,6 +93,7 @@ constexpr uint32_t kOutside = 0x4000u;
 constexpr uint32_t kNoSlot = 0xffffffffu;
 
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
+typedef int32_t v4i_any __attribute__((ext_vector_type(4), aligned(4)));
 
 struct SegBind {
   OctNode* nodes;
@@ -252,9 +254,10 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
   }
 }
 
-// What a launch does: the whole stage, or one of its two per-stage entries on
-// nodes that the caller prepared.
-enum OctPhase { kWhole, kMakePhase, kLinkPhase };
+// What a launch does: the whole stage (storing its nodes past the caches or not:
+// a template, for as a branch the two stores are merged into an ordinary one), or
+// one of its two per-stage entries on nodes that the caller prepared.
+enum OctPhase { kWhole, kWholeStreamed, kMakePhase, kLinkPhase };
 
 template <bool SINGLE, OctPhase PHASE>
 __global__ __launch_bounds__(kThreads) void oct_build_kernel(
@@ -262,6 +265,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   constexpr int T = kOctTile;
   constexpr int NPT = T / kThreads;
   constexpr bool MAKE = PHASE != kLinkPhase, LINK = PHASE != kMakePhase;
+  constexpr bool WHOLE = PHASE == kWhole || PHASE == kWholeStreamed;
   __shared__ __attribute__((aligned(16))) u64 s_child[kColWords * kCols];
   __shared__ u64 s_owner[kCols];
   __shared__ uint32_t s_mask[kCols / 4];
@@ -275,12 +279,12 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // The segment's scalars are loaded together before any is tested: one
   // round trip instead of one per value.
   // (The launcher guarantees these pointers; the build writes them all.)
-  const int32_t m_seg = PHASE == kWhole ? a.n_unique[r.seg] - 1 : a.n_brt_host;
-  const int32_t k_seg = PHASE == kWhole ? a.kalloc[r.seg] : a.k_host;
-  const uint32_t fits = PHASE != kWhole ? 1u
+  const int32_t m_seg = WHOLE ? a.n_unique[r.seg] - 1 : a.n_brt_host;
+  const int32_t k_seg = WHOLE ? a.kalloc[r.seg] : a.k_host;
+  const uint32_t fits = !WHOLE ? 1u
                         : SINGLE        ? (static_cast<uint32_t>(k_seg) <= one.k_cap ? 1u : 0u)
                                         : a.ctrl[kCtrlOctOk];
-  const int32_t node_base = SINGLE || PHASE != kWhole ? 0 : a.oct_start[r.seg];
+  const int32_t node_base = SINGLE || !WHOLE ? 0 : a.oct_start[r.seg];
   const int32_t sb = seg_begin(sv, r.seg);
   const float seg_mn = seg_min(sv, r.seg);
   const float seg_rg = seg_range(sv, r.seg);
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   // loads after it back): the nodes fit, the tile has nodes (a single-key
   // segment still has its root), the segment has slots and a valid base.
   // After a lookback time-out the inputs are not valid.
-  const uint32_t stop = PHASE == kWhole ? a.ctrl[kCtrlTimeout] : 0u;
+  const uint32_t stop = WHOLE ? a.ctrl[kCtrlTimeout] : 0u;
   if (SINGLE && i0 == 0 && threadIdx.x == 0) {
     // What the offsets kernel does for several segments (a launch of ~5 us).
     const uint32_t tiles = a.ctrl[kCtrlMsdTiles];
@@ -327,7 +331,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   const int32_t i_end = min(i0 + T, b.m);
   int32_t p_before = i0 > 0 ? b.p[i0 - 1] : -1;
   int32_t s_end = i_end >= b.m ? b.k : b.p[i_end - 1] + 1;
-  if constexpr (PHASE != kWhole) {
+  if constexpr (!WHOLE) {
     // The caller's slots bound every access, and those past the last chain
     // stay as they are.
     if (i_end >= b.m) s_end = b.p[b.m - 1] + kMaxEdge;
@@ -528,7 +532,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
         const int32_t s = cols.base + t;
         const u64 own = s_owner[t];
         const uint32_t kids = (s_mask[t >> 2] >> ((t & 3) * 8)) & 255u;
-        if constexpr (PHASE == kWhole) {
+        if constexpr (WHOLE) {
 #pragma unroll
           for (int c = 0; c < 8; ++c) nd[c] = static_cast<int32_t>(s_child[col_word(t, c)]);
           nd[13] = static_cast<int32_t>(kids);
@@ -556,7 +560,7 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
           if constexpr (MAKE) nd[13] |= links | static_cast<int32_t>(kids);
           else nd[14] &= ~links;
         }
-        if (MAKE && (own != 0 || s == 0) && (PHASE == kWhole || s != 0)) {
+        if (MAKE && (own != 0 || s == 0) && (WHOLE || s != 0)) {
           // Corner and cell size of the chain's step (oct.h:44-57, 76-88); slot
           // 0 is the root of apps/cpu_demo/main.cpp:125-132. Other slots no
           // chain covers stay zero.
@@ -596,7 +600,11 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
     for (int k = 0; k < OUT; ++k) {
       const int32_t q = (k * kThreads + tid) * 4;
       if (q + 4 <= words) {
-        __builtin_memcpy(dst + q, &x[k], 16);
+        if constexpr (PHASE == kWholeStreamed)
+          __builtin_nontemporal_store(static_cast<v4i_any>(x[k]),
+                                      reinterpret_cast<v4i_any*>(dst + q));
+        else
+          __builtin_memcpy(dst + q, &x[k], 16);
       } else {
 #pragma unroll
         for (int u = 0; u < 4; ++u)
@@ -666,10 +674,13 @@ bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_s
     return false;
   if (total_tiles <= 0) return true;
   if (single.mail && (sv.n_seg != 1 || !single.oct_start || !single.ctrl)) return false;
-  if (single.mail)
-    oct_build_kernel<true, kWhole><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
-  else
-    oct_build_kernel<false, kWhole><<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
+  const auto go = [&](auto kernel) {
+    kernel<<<total_tiles, kThreads, 0, s>>>(a, sv, tile_start, single);
+  };
+  if (single.mail && a.stream_nodes) go(oct_build_kernel<true, kWholeStreamed>);
+  else if (single.mail) go(oct_build_kernel<true, kWhole>);
+  else if (a.stream_nodes) go(oct_build_kernel<false, kWholeStreamed>);
+  else go(oct_build_kernel<false, kWhole>);
   return true;
 }
 

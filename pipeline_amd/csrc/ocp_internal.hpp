@@ -343,7 +343,15 @@ struct OctArgs {
   const int32_t* offsets;
   const int32_t* n_unique;  // per segment (nullptr: n_brt_host + 1)
   int32_t n_brt_host;
+  bool stream_nodes;  // nodes past the caches (oct_stream)
 };
+// Whether a build of n points stores its nodes past the caches: once they and
+// the arrays they are made from outgrow the 256 MB behind the L2s, where they
+// only push out what is still to be read (octree of 10M points 151 -> 135 us,
+// builds of 8M 335 -> 303, of 4M 207 -> 203); nodes of smaller builds are still
+// there for whoever reads them next (compact form of 1M points 35 us, 40 when
+// they are not).
+inline bool oct_stream(int64_t n) { return n >= (int64_t(1) << 22); }
 void launch_oct_root(OctNode* nodes, const uint32_t* codes,
                      const uint8_t* prefix_n, int32_t n_brt, float mn,
                      float rg, hipStream_t s);
