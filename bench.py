@@ -70,8 +70,8 @@ def kernel_bytes(name: str, n: int, u: int, k: int, float4: bool = True) -> floa
         "msd_buckets": 8 * n,                   # every bucket read and written once
         "msd_lsd_fallback": 28 * n,             # lower-digit counts + three passes
         "unique": 4 * n + 4 * u,                # sorted read + unique write
-        "radix_tree": 4 * u + 11 * m,           # codes read; 1+1+1+4+4 written
-        "edge_scan": 14 * m,                    # 1+4+1 read; 4+4 written
+        "radix_tree": 4 * u + 15 * m,           # codes read; 1+1+1+4+4+4 written
+        "edge_scan": 8 * m,                     # 4 read; 4 written
         "octree": 24 * m + 60 * k,              # BRT reads + one 60-B node per slot
     }
     return float(table.get(name, 0.0))

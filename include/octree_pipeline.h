@@ -125,7 +125,8 @@ int ocp_k_DigitBinning(ocp_ctx ctx, const uint32_t* global_histogram,
 /* Replaces k_SimpleRadixSort(keys, keys_alt, n)
  * (include/kernels/02_sort.hpp:7) and the reference's DispatchSortKernels
  * (apps/gpu_demo/main.cu:63-125): histogram + 4 passes
- * keys -> alt -> keys -> alt -> keys; the sorted keys end in `keys`. */
+ * keys -> alt -> keys -> alt -> keys; the sorted keys end in `keys`. Up to
+ * 16,384 keys are sorted in place by one kernel, which leaves keys_alt alone. */
 int ocp_k_SortKeys(ocp_ctx ctx, uint32_t* keys, uint32_t* keys_alt,
                    uint32_t n);
 
