@@ -415,15 +415,21 @@ TuneTable build_tune(const TuneTable& set, bool tuned, int64_t n, int64_t max_se
   return t;
 }
 
-// ... and the form for this build. A large cloud's keys may crowd as they like
-// (see auto_sort_skew).
+// ... and the LSD table that stands in for it where keys crowd (auto_sort_skew).
+TuneTable crowd_tune(const TuneTable& set, bool tuned, int64_t n, int32_t n_seg) {
+  TuneTable t = set;
+  if (!tuned && crowd_sort10(n, n_seg)) t.sort_bits = 10;
+  return t;
+}
+
+// The form for this build. A large cloud's keys may crowd as they like.
 TuneTable choose_tune(ocp_ctx c, int64_t n, int64_t max_seg, int32_t n_seg, bool perm) {
   const TuneTable t = build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm);
   if (c->tuned || !pipe_sort_msd(t, perm, n_seg) || !auto_sort_skew(max_seg) ||
       c->skew_left <= 0 || n < c->skew_n / 2 || n > c->skew_n * 2)
     return t;
   --c->skew_left;
-  return c->tune;
+  return crowd_tune(c->tune, c->tuned, n, n_seg);
 }
 
 // After a build of the library's choice: its level-2 tiles tell how many keys
@@ -466,8 +472,11 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
 // ... and the memory it needs.
 int prepare_plain(ocp_ctx c, int64_t n, float mn, float rg, Plan* p) {
   const TuneTable tt = choose_tune(c, n, n, 1, c->permutation);
-  if (int r = ensure_workspace(c, n, 1, flag_words_for(c->tune, n, 1))) return r;
-  if (pipe_sort_msd(tt, c->permutation, 1))
+  // (for either form of the sort: which one a later build of this size takes
+  // does not change the memory)
+  if (int r = ensure_workspace(c, n, 1, flag_words_for(crowd_tune(c->tune, c->tuned, n, 1), n, 1)))
+    return r;
+  if (pipe_sort_msd(build_tune(c->tune, c->tuned, n, n, 1, c->permutation), c->permutation, 1))
     if (int r = ensure_level2(c, n, n)) return r;
   *p = plain_plan(tt, n, mn, rg, c->permutation);
   p->auto_msd = !c->tuned && pipe_sort_msd(tt, c->permutation, 1);
@@ -505,8 +514,10 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   for (int32_t k = 0; k < n_seg; ++k)
     max_seg = std::max<int64_t>(max_seg, int64_t(offsets[k + 1]) - offsets[k]);
   const TuneTable tt = choose_tune(c, n, max_seg, n_seg, perm);
-  if (int r = ensure_workspace(c, n, n_seg, flag_words_for(c->tune, n, n_seg))) return r;
-  if (pipe_sort_msd(tt, perm, n_seg))
+  if (int r = ensure_workspace(
+          c, n, n_seg, flag_words_for(crowd_tune(c->tune, c->tuned, n, n_seg), n, n_seg)))
+    return r;
+  if (pipe_sort_msd(build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm), perm, n_seg))
     if (int r = ensure_level2(c, n, max_seg)) return r;
   Workspace& w = c->ws;
   const int32_t stride = w.seg_cap + 1;
@@ -1442,7 +1453,8 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
       return OCP_ERR_INVALID;
   }
   const int32_t clouds = std::max<int32_t>(n_seg, 1);
-  const int64_t flag_words = flag_words_for(tt, n, clouds);
+  const int64_t flag_words =
+      flag_words_for(crowd_tune(tt, tune != nullptr, n, clouds), n, clouds);
   tt = build_tune(tt, tune != nullptr, n, n, clouds, permutation != 0);
   // The allocations of ensure_workspace, alloc_nodes, ensure_level2 and
   // ensure_perm for a first build of this shape, plus the context's control words and digit
@@ -1463,7 +1475,7 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
          int64_t(l2.max_slots) * 4096;
   }
   if (permutation) b += 2 * 4 * cap;
-  b += 4 * (kCtrlWords + 1024);
+  b += 4 * (kCtrlWords + 1024 + 256);
   out->build_bytes = b;
   const int64_t sort_tiles = cdiv(n, sort_tile(tt));
   const int64_t scan_tiles = cdiv(n, scan_tile(tt));

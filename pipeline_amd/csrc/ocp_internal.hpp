@@ -95,13 +95,18 @@ inline bool auto_sort_msd(int64_t n, int32_t n_seg, bool perm) {
   return !perm && n >= 16384 && n_seg <= kMsdMaxSegments;
 }
 // Where many keys crowd into few digits, most of them take the second level:
-// 2^24 clustered points 528 -> 495 us, but 2^20 145 -> 160 and 2^22 232 -> 250.
+// 2^24 clustered points 528 -> 495 us, but 2^20 133 -> 147 and 10M 315 -> 341.
 // So below 12M points a cloud, a build after which more than a sixteenth of the
 // keys turns out to have gone there (the host learns it with the counts) is
-// followed by kSkewBuilds builds of about its size with the LSD passes, then by
+// followed by kSkewBuilds builds of about its size with LSD passes, then by
 // another try. The result is the same either way.
 inline bool auto_sort_skew(int64_t max_seg) { return max_seg < 12000000; }
 constexpr int32_t kSkewBuilds = 256;
+// Those passes' digits, for one cloud: three passes of 10 bits while the tiles'
+// 1024 runs stay in the caches, else four of 8. Clustered points, four passes
+// against three: 307,200 105 -> 98 us, 2^20 133 -> 126, 2^21 166 -> 151, but 2^22
+// 208 -> 212 and 10M 315 -> 347.
+inline bool crowd_sort10(int64_t n, int32_t n_seg) { return n_seg <= 1 && n < 3000000; }
 // Tiles of 16K keys for the scatter once there are enough of them (10M: 47 ->
 // 39 us), else of 8K.
 inline int auto_sort10_kpt(int64_t max_seg) { return max_seg >= (int64_t(1) << 22) ? 16 : 8; }

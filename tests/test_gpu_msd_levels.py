@@ -85,3 +85,16 @@ def test_batch_of_every_kind():
         for k, p in enumerate(pts):
             if p.shape[0]:
                 _check_segment(out, k, oracle.build_plain(p))
+
+
+@pytest.mark.parametrize("n", [20_000, 300_000, 2_999_999, 3_000_000])
+def test_builds_after_crowded_keys(n):
+    """Once the counts of a build have told that its keys crowd, the next of
+    about its size take LSD passes; 3M points is the line between their widths."""
+    rng = np.random.default_rng(n)
+    sets = [_cells((700 << 20) + rng.integers(0, 1 << 20, m)) for m in (n, n, n - n // 3)]
+    with pipeline_amd.Context(0) as ctx:
+        for pts in sets:
+            d = ctx.upload(pts)
+            ctx.build(d, pts.shape[0], 0.0, 1024.0)
+            _check_segment(ctx.fetch(), 0, oracle.build_plain(pts))
