@@ -235,12 +235,19 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     if (!leaf_r) o.par[sb + g + 1] = node;
   }
   if (wave_id() == 0 && m > 0) {
-    // Node 0: the range [0, m - 1] and the last s in it with a longer prefix.
-    int32_t s = 0;
-    for (int32_t c = 0; c < m - 1; c += 64) {
-      const int32_t at = c + static_cast<int32_t>(lane_id());
-      s += __popcll(__ballot(at > 0 && at < m - 1 && delta(code_0, s_key[at]) > pn_0));
+    // Node 0: the range [0, m - 1] and the last s in it with a longer prefix
+    // (prefixes with code_0 only get shorter: 64 probes of the rest at a time).
+    int32_t lo = 1, hi = m - 1;  // the first that has none is in [lo, hi]
+    while (lo < hi) {
+      const int32_t step = (hi - lo + 63) >> 6;
+      const int32_t at = lo + static_cast<int32_t>(lane_id()) * step;
+      const int32_t has =
+          __popcll(__ballot(at < hi && delta(code_0, s_key[min(at, m)]) > pn_0));
+      if (has == 0) break;
+      hi = min(hi, lo + has * step);
+      lo += (has - 1) * step + 1;
     }
+    const int32_t s = max(lo - 1, 0);
     if (lane_id() == 0) {
       o.prefix[sb] = static_cast<uint8_t>(pn_0);
       o.hl[sb] = s == 0;
