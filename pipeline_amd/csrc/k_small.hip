@@ -6,10 +6,10 @@
 // A build of such a cloud moves next to nothing: it is launches and the round
 // trips inside them, nine kernels of 4 to 11 us each. One workgroup keeps every
 // array in LDS and needs neither the begin kernel nor a lookback. A build and
-// its counts, us, the stages' kernels -> this one: 700 uniform points 85 -> 32,
-// 4096 89 -> 47 (clustered 95 -> 60), 8192 92 -> 65 (clustered 100 -> 84); in
-// batches, a workgroup per cloud: 64 x 4096 108 -> 59, 512 x 4096 199 -> 120,
-// 2000 x 8192 909 -> 709.
+// its counts, us, the stages' kernels -> this one: 700 uniform points 85 -> 27,
+// 4096 89 -> 36 (clustered 95 -> 48), 8192 92 -> 49 (clustered 100 -> 66); in
+// batches, a workgroup per cloud: 64 x 4096 108 -> 47, 512 x 4096 199 -> 87,
+// 2000 x 8192 909 -> 545.
 #include "bucket_sort.hpp"
 #include "pair_rows.hpp"
 
@@ -18,48 +18,50 @@ namespace {
 
 constexpr int kThreads = 1024;
 
-// Rows of 16 pairs' common prefixes, and of the minima of 16, 256 and 4096.
-struct Levels {
-  const v4u* row[4];
-};
+// Which pairs' common prefix is below b, for each b: a row of 64-bit words a
+// value (a word more than it has, so that one word's values lie in different
+// banks), and which words of it are not zero. A pair's nearest ones below its own
+// are then a few bit operations on one or two words on either side. (Against
+// walks over rows of 16 bytes and their minima, which took 19,000 of 8192 points'
+// 81,000 cycles a side: 4096 points 40.4 -> 36.8 us, 8192 56.7 -> 49.5.)
+template <int WORDS>
+struct Below {
+  static constexpr int kStride = WORDS + 1;
+  uint64_t low[32 * kStride];
+  uint64_t any[32][WORDS / 64];
 
-// The nearest position right of q (left of it) whose value is below the row
-// key's, or -1. The last level is one row.
-template <int TOP>
-__device__ __forceinline__ int32_t next_below(const Levels& lv, uint32_t q, uint32_t key) {
-  uint32_t at = q;
-#pragma unroll
-  for (int l = 0; l <= TOP; ++l) {
-    const uint32_t hit = below16(lv.row[l][at >> 4], key) & (0xfffeu << (at & 15u)) & 0xffffu;
-    if (hit) {
-      at = (at & ~15u) + static_cast<uint32_t>(__builtin_ctz(hit));
-#pragma unroll
-      for (int d = TOP - 1; d >= 0; --d)
-        if (d < l) at = at * 16u + static_cast<uint32_t>(__builtin_ctz(below16(lv.row[d][at], key)));
-      return static_cast<int32_t>(at);
+  // The nearest position right of g; there is one.
+  __device__ __forceinline__ int32_t next(int32_t g, uint32_t b, uint64_t word) const {
+    uint32_t w = static_cast<uint32_t>(g) >> 6;
+    uint64_t hit = word & (~1ull << (g & 63));
+    if (!hit) {
+      uint64_t rest = any[b][w >> 6] & (~1ull << (w & 63u));
+      if (WORDS > 64 && !rest && w < 64u) {
+        rest = any[b][WORDS / 64 - 1];
+        w = 64u;
+      }
+      w = (w & ~63u) + static_cast<uint32_t>(__builtin_ctzll(rest));
+      hit = low[b * kStride + w];
     }
-    at >>= 4;
+    return static_cast<int32_t>(w * 64u) + __builtin_ctzll(hit);
   }
-  return -1;
-}
-template <int TOP>
-__device__ __forceinline__ int32_t last_below(const Levels& lv, uint32_t q, uint32_t key) {
-  uint32_t at = q;
-#pragma unroll
-  for (int l = 0; l <= TOP; ++l) {
-    const uint32_t hit = below16(lv.row[l][at >> 4], key) & ((1u << (at & 15u)) - 1u);
-    if (hit) {
-      at = (at & ~15u) + 31u - static_cast<uint32_t>(__clz(static_cast<int>(hit)));
-#pragma unroll
-      for (int d = TOP - 1; d >= 0; --d)
-        if (d < l)
-          at = at * 16u + 31u - static_cast<uint32_t>(__clz(static_cast<int>(below16(lv.row[d][at], key))));
-      return static_cast<int32_t>(at);
+  // The nearest left of g, or -1.
+  __device__ __forceinline__ int32_t last(int32_t g, uint32_t b, uint64_t word) const {
+    uint32_t w = static_cast<uint32_t>(g) >> 6;
+    uint64_t hit = word & ((1ull << (g & 63)) - 1ull);
+    if (!hit) {
+      uint64_t rest = any[b][w >> 6] & ((1ull << (w & 63u)) - 1ull);
+      if (WORDS > 64 && !rest && w >= 64u) {
+        rest = any[b][0];
+        w = 0u;
+      }
+      if (!rest) return -1;
+      w = (w & ~63u) + 63u - static_cast<uint32_t>(__builtin_clzll(rest));
+      hit = low[b * kStride + w];
     }
-    at >>= 4;
+    return static_cast<int32_t>(w * 64u) + 63 - __builtin_clzll(hit);
   }
-  return -1;
-}
+};
 
 // One workgroup per segment of at most 1024 * KPT points.
 template <int KPT, bool F3>
@@ -67,14 +69,12 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     const float* __restrict__ pts, SegView sv, bool device_box, float* __restrict__ box_min,
     float* __restrict__ box_range_out, SmallOut o, uint32_t* __restrict__ ctrl) {
   constexpr int CAP = kThreads * KPT;
-  constexpr int ROWS = CAP / 16;
-  constexpr int TOP = CAP > 4096 ? 3 : 2;  // the level of one row
+  constexpr int WORDS = CAP / 64;
+  static_assert(WORDS == 64 || WORDS == 128, "one or two words say which words of a row count");
   __shared__ __attribute__((aligned(16))) uint32_t s_key[CAP];  // codes, sorted, then unique
-  __shared__ v4u s_b[ROWS];
-  __shared__ v4u s_b16[ROWS / 16];
-  __shared__ v4u s_b256[TOP > 2 ? ROWS / 256 : 1];
-  __shared__ v4u s_b4096;
-  __shared__ int32_t s_edge[CAP];
+  __shared__ uint8_t s_b[CAP];  // the pairs' common prefixes
+  __shared__ Below<WORDS> s_below;
+  __shared__ int8_t s_edge[CAP];  // (at most 10 levels)
   __shared__ uint32_t s_tmp[kThreads / 64];
   __shared__ uint32_t s_box[2];
   __shared__ int32_t s_max;
@@ -90,6 +90,8 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     }
     return;
   }
+
+  for (int i = tid; i < 32 * (WORDS + 1); i += kThreads) s_below.low[i] = 0u;
 
   // ---- points, box, codes
   float x[KPT], y[KPT], z[KPT];
@@ -181,44 +183,55 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
   const int32_t m = u - 1;  // pairs
   for (int32_t i = tid; i < u; i += kThreads) o.unique[sb + i] = s_key[i];
 
-  // ---- radix tree (k_radix_tree.hip): the pairs' common prefixes and minima
-  uint8_t* b8 = reinterpret_cast<uint8_t*>(s_b);
+  // ---- radix tree (k_radix_tree.hip): the pairs' common prefixes, where each
+  // value is, then where any below it is. The position after the last pair
+  // holds 0: every pair has a lower one on its right.
 #pragma unroll
   for (int k = 0; k < KPT; ++k) {
     const int32_t i = k * kThreads + tid;
-    b8[i] = static_cast<uint8_t>(i < m ? clz32(s_key[i] ^ s_key[i + 1]) : 0u);
+    if (i > m) continue;
+    const uint32_t b = i < m ? clz32(s_key[i] ^ s_key[i + 1]) : 0u;
+    s_b[i] = static_cast<uint8_t>(b);
+    atomicOr(reinterpret_cast<uint32_t*>(&s_below.low[b * (WORDS + 1) + (i >> 6)]) + ((i >> 5) & 1),
+             1u << (i & 31));
   }
   __syncthreads();
-  if (tid < ROWS) reinterpret_cast<uint8_t*>(s_b16)[tid] = static_cast<uint8_t>(min16(s_b[tid]));
-  __syncthreads();
-  if constexpr (TOP > 2) {
-    if (tid < ROWS / 16)
-      reinterpret_cast<uint8_t*>(s_b256)[tid] = static_cast<uint8_t>(min16(s_b16[tid]));
+  {
+    const int v0 = 2 * static_cast<int>(wave_id());  // 16 waves, two values each
+    uint64_t even[WORDS / 64], odd[WORDS / 64];
+#pragma unroll
+    for (int c = 0; c < WORDS / 64; ++c) {
+      const uint64_t* at = s_below.low + c * 64 + static_cast<int>(lane_id());
+      even[c] = 0u;
+#pragma unroll 4
+      for (int v = 0; v < v0; ++v) even[c] |= at[v * (WORDS + 1)];
+      odd[c] = even[c] | at[v0 * (WORDS + 1)];
+    }
     __syncthreads();
-    if (tid < 16)
-      reinterpret_cast<uint8_t*>(&s_b4096)[tid] =
-          static_cast<uint8_t>(tid < ROWS / 256 ? min16(s_b256[tid]) : 31u);
-  } else {
-    if (tid < 16)
-      reinterpret_cast<uint8_t*>(s_b256)[tid] =
-          static_cast<uint8_t>(tid < ROWS / 16 ? min16(s_b16[tid]) : 31u);
+#pragma unroll
+    for (int c = 0; c < WORDS / 64; ++c) {
+      uint64_t* at = s_below.low + c * 64 + static_cast<int>(lane_id());
+      at[v0 * (WORDS + 1)] = even[c];
+      at[(v0 + 1) * (WORDS + 1)] = odd[c];
+      const uint64_t any_even = __ballot(even[c] != 0u), any_odd = __ballot(odd[c] != 0u);
+      if (lane_id() == 0) {
+        s_below.any[v0][c] = any_even;
+        s_below.any[v0 + 1][c] = any_odd;
+      }
+    }
   }
   __syncthreads();
-  const Levels lv{{s_b, s_b16, s_b256, &s_b4096}};
   const uint32_t code_0 = s_key[0];
   const uint32_t b_root = m > 0 ? clz32(code_0 ^ s_key[m]) : 0u;
   const uint32_t pn_0 = m > 0 ? delta(code_0, s_key[m - 1]) : 0u;  // node 0's prefix length
 #pragma unroll 1
   for (int32_t g = tid; g < m; g += kThreads) {
-    const uint32_t b = b8[g];
-    const uint32_t rk = __builtin_amdgcn_perm(0u, b + 127u, 0u);
-    // (the position after the last pair holds 0, so the right end is found;
-    // the last pair of a full array ends at m)
-    int32_t r = next_below<TOP>(lv, static_cast<uint32_t>(g), rk);
-    const int32_t l = last_below<TOP>(lv, static_cast<uint32_t>(g), rk);
-    if (r < 0) r = m;
-    const uint32_t b_l = l >= 0 ? b8[l] : 0u;
-    const uint32_t b_r = r < m ? b8[r] : 0u;
+    const uint32_t b = s_b[g];
+    const uint64_t word = s_below.low[b * (WORDS + 1) + (static_cast<uint32_t>(g) >> 6)];
+    const int32_t r = s_below.next(g, b, word);
+    const int32_t l = s_below.last(g, b, word);
+    const uint32_t b_l = l >= 0 ? s_b[l] : 0u;
+    const uint32_t b_r = s_b[r];
     const uint32_t b_up = max(b_l, b_r);
     const int32_t node = b_l >= b_r ? l + 1 : r;
     const bool leaf_l = l + 1 == g, leaf_r = r == g + 1;
@@ -229,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
       o.hl[sb + node] = leaf_l;
       o.hr[sb + node] = leaf_r;
       o.lc[sb + node] = g;
-      s_edge[node] = e;
+      s_edge[node] = static_cast<int8_t>(e);
     }
     if (!leaf_l) o.par[sb + g] = node;
     if (!leaf_r) o.par[sb + g + 1] = node;
@@ -260,6 +273,8 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
   __syncthreads();
 
   // ---- edge counts, their inclusive scan, the octree's slots
+  static_assert(sizeof(s_below.low) >= sizeof(int32_t) * CAP, "the scan takes the rows' place");
+  int32_t* s_run = reinterpret_cast<int32_t*>(s_below.low);
   int32_t e[KPT];
   int32_t sum = 0;
 #pragma unroll
@@ -278,14 +293,14 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
     const int32_t i = tid * KPT + j;
     run += e[j];
     if (i < m) {
-      s_edge[i] = run;
+      s_run[i] = run;
       top = max(top, run + e[j]);
     }
   }
   top = wave_max(top);
   if (lane_id() == 0) atomicMax(&s_max, top);
   __syncthreads();
-  for (int32_t i = tid; i < m; i += kThreads) o.offs[sb + i] = s_edge[i];
+  for (int32_t i = tid; i < m; i += kThreads) o.offs[sb + i] = s_run[i];
   if (tid == 0) {
     o.n_unique[seg] = u;
     o.kalloc[seg] = u > 0 ? s_max : 0;
