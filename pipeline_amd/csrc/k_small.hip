@@ -7,7 +7,7 @@
 // trips inside them, nine kernels of 4 to 11 us each. One workgroup keeps every
 // array in LDS and needs neither the begin kernel nor a lookback. A build and
 // its counts, us, the stages' kernels -> this one: 700 uniform points 85 -> 27,
-// 4096 89 -> 36 (clustered 95 -> 48), 8192 92 -> 49 (clustered 100 -> 66); in
+// 4096 89 -> 36 (clustered 95 -> 48), 8192 92 -> 49 (clustered 100 -> 63); in
 // batches, a workgroup per cloud: 64 x 4096 108 -> 47, 512 x 4096 199 -> 87,
 // 2000 x 8192 909 -> 545.
 #include "bucket_sort.hpp"
@@ -154,8 +154,12 @@ __global__ __launch_bounds__(kThreads) void small_cloud_kernel(
   if (tid == 0) s_max = 1;
   __syncthreads();
 
-  // ---- sort (the span is found from the keys: a small cloud may lie anywhere)
-  if (n > 1) lds_bucket_sort<kThreads / 64, KPT, 12, 8, 13>(s_key, s_key, n);
+  // ---- sort (the span is found from the keys: a small cloud may lie anywhere).
+  // Crowded keys take stable passes after the first 12 bits: where one workgroup
+  // fits a CU anyway, of 9 bits, two for 30 bits and not three (8192 clustered
+  // points 65.7 -> 63.4 us a build; at 4096 points the counters would cost the
+  // second workgroup).
+  if (n > 1) lds_bucket_sort<kThreads / 64, KPT, 12, (KPT > 4 ? 9 : 8), 13>(s_key, s_key, n);
   __syncthreads();
 
   // ---- unique: thread t holds keys t*KPT .. t*KPT + KPT-1
