@@ -192,6 +192,7 @@ struct ocp_context {
   std::vector<float> tab_min, tab_rg;
   int tab_tune_key = -1;
   bool have_result = false;
+  uint32_t oct_calls = 0;  // make and link calls so far, as their mark in the control words
   Plan last_plan;
   // Pinned host memory: what the last build's offsets kernel, or for one cloud
   // its octree kernel, reports (see launch_oct_offsets), then a landing place for small copies back. Current
@@ -1297,11 +1298,14 @@ int ocp_k_InitOctNodes(ocp_ctx c, ocp_oct_node* nodes, int32_t n_alloc, const ui
   return OCP_OK;
 }
 
-static OctArgs stage_oct_args(ocp_oct_node* nodes, const int32_t* offs, const int32_t* counts,
-                              const uint32_t* codes, const uint8_t* pn, const uint8_t* hl,
-                              const uint8_t* hr, const int32_t* par, const int32_t* lc,
-                              int32_t n, int32_t n_alloc) {
+static OctArgs stage_oct_args(ocp_ctx c, ocp_oct_node* nodes, const int32_t* offs,
+                              const int32_t* counts, const uint32_t* codes, const uint8_t* pn,
+                              const uint8_t* hl, const uint8_t* hr, const int32_t* par,
+                              const int32_t* lc, int32_t n, int32_t n_alloc) {
   OctArgs a{};
+  a.form = c->ctrl + kCtrlOctForm;
+  if (++c->oct_calls == 0) c->oct_calls = 1;  // (0: the word of a new context)
+  a.form_id = c->oct_calls;
   a.nodes = reinterpret_cast<OctNode*>(nodes);
   a.k_host = n_alloc;
   a.codes = codes;
@@ -1324,7 +1328,7 @@ int ocp_k_MakeOctNodes(ocp_ctx c, ocp_oct_node* nodes, const int32_t* offs,
   if (!nodes || !offs || !counts || !codes || !pn || !par)
     return fail(c, OCP_ERR_INVALID, "null pointer");
   if (n >= kMaxSegPoints) return fail(c, OCP_ERR_CAPACITY, "N >= 2^27");
-  const OctArgs a = stage_oct_args(nodes, offs, counts, codes, pn, nullptr, nullptr, par,
+  const OctArgs a = stage_oct_args(c, nodes, offs, counts, codes, pn, nullptr, nullptr, par,
                                    nullptr, n, n_alloc);
   launch_oct_make(a, single_view(n + 1, mn, rg), c->stream);
   OCP_CHECK_LAUNCH(c);
@@ -1340,7 +1344,7 @@ int ocp_k_LinkLeafNodes(ocp_ctx c, ocp_oct_node* nodes, const int32_t* offs,
   if (!nodes || !offs || !counts || !codes || !hl || !hr || !pn || !par || !lc)
     return fail(c, OCP_ERR_INVALID, "null pointer");
   if (n >= kMaxSegPoints) return fail(c, OCP_ERR_CAPACITY, "N >= 2^27");
-  const OctArgs a = stage_oct_args(nodes, offs, counts, codes, pn, hl, hr, par, lc, n, n_alloc);
+  const OctArgs a = stage_oct_args(c, nodes, offs, counts, codes, pn, hl, hr, par, lc, n, n_alloc);
   launch_oct_link(a, single_view(n + 1, 0.0f, 1.0f), c->stream);
   OCP_CHECK_LAUNCH(c);
   return OCP_OK;

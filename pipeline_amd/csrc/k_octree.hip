@@ -54,9 +54,13 @@
 //
 // The per-stage entries (k_MakeOctNodes, k_LinkLeafNodes: include/cuda/kernels/
 // 07_octree.cuh:7-28) are the same kernel doing one half of the pushes into
-// nodes that it reads and writes whole. Make has no children arrays: see
-// oct_far_kernel. For 2M points make takes 46 us and link 30; a scatter of order
-// keys by global atomics and a kernel that resolved them took 117 and 187.
+// nodes that it reads and writes whole, where a kernel before it has found the
+// caller's arrays to be what a build's are (tiled_form); for any others, as
+// offsets that are not the inclusive scan, it scatters order keys by global
+// atomics and a kernel after it resolves them. Make has no children arrays: see
+// make_check_kernel. For 2M points make takes 16 us of check, 31 of the tiled
+// kernel and 5 of the idle resolve, link 5, 31 and 5; the scatter and the resolve
+// took 117 and 187 for every array.
 //
 // What bounds it: how many tiles share a CU while each waits for its loads, its
 // barriers and the walks of its listed children (a chain of up to four dependent
@@ -254,6 +258,67 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
   }
 }
 
+// The writes of node i as order keys in the child words of the nodes, kept by an
+// atomic max: the per-stage entries' path for arrays of any form, finished by
+// resolve_kernel.
+__device__ __forceinline__ void put_word(const OctArgs& a, int32_t slot, uint32_t which,
+                                         uint32_t key) {
+  if (slot >= 0 && slot < a.k_host)
+    atomicMax(reinterpret_cast<uint32_t*>(&a.nodes[slot].children[which]), key);
+}
+__device__ __forceinline__ void put_make_word(const OctArgs& a, int32_t slot, uint32_t which,
+                                              uint32_t key) {
+  if (slot < 0 || slot >= a.k_host) return;
+  put_word(a, slot, which, key);
+  atomicOr(&a.nodes[slot].child_node_mask, 1 << which);
+}
+// The node that the walk of oct.h:61-73 from node i's parent ends at (at most
+// 31 hops; node 0 is its own parent). at(h): the nodes on the way. A hop's two
+// loads are in flight together.
+template <class At>
+__device__ __forceinline__ int32_t make_head(const OctArgs& a, int32_t i, At at) {
+  int32_t h = a.parent[i];
+  for (int hop = 0; hop < 31; ++hop) {
+    at(h);
+    const int32_t e = a.edge[h], up = a.parent[h];
+    if (e != 0 || up == h) break;
+    h = up;
+  }
+  return h;
+}
+template <bool MAKE>
+__device__ __forceinline__ void scatter_node(const OctArgs& a, int32_t i) {
+  if (i >= a.n_brt_host) return;
+  if constexpr (MAKE) {
+    const int32_t e = a.edge[i];
+    if (i == 0 || e <= 0) return;
+    const int32_t p = a.offsets[i];
+    const int32_t level = a.prefix_n[i] / 3;
+    const uint32_t code = a.codes[i];
+    for (int32_t j = 0; j < e - 1; ++j)
+      put_make_word(a, p + j + 1, child_of(code, level - j), make_key(i, j));
+    put_make_word(a, a.offsets[make_head(a, i, [](int32_t) {})], child_of(code, level - e + 1),
+                  make_key(i, e - 1));
+  } else {
+    int32_t head = -1;
+    for (int side = 0; side < 2; ++side) {
+      if (!(side == 0 ? a.has_leaf_left[i] : a.has_leaf_right[i])) continue;
+      if (head < 0) {
+        // oct.h:111-113, stopped at node 0 and after 64 hops
+        head = i;
+        for (int hop = 0; hop < 64 && a.edge[head] == 0 && head != 0; ++hop)
+          head = a.parent[head];
+      }
+      const int32_t slot = a.offsets[head];
+      const uint32_t which =
+          child_of(a.codes[a.left_child[i] + side], a.prefix_n[i] / 3 + 1);
+      put_word(a, slot, which, link_key(i, side));
+      if (slot >= 0 && slot < a.k_host)
+        atomicAnd(&a.nodes[slot].child_leaf_mask, ~(1 << which));
+    }
+  }
+}
+
 // What a launch does: the whole stage (storing its nodes past the caches or not:
 // a template, for as a branch the two stores are merged into an ordinary one), or
 // one of its two per-stage entries on nodes that the caller prepared.
@@ -276,6 +341,13 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   __shared__ uint32_t s_nout;
 
   const TileRef r = find_tile(tile_start, sv.n_seg, xcd_tile(blockIdx.x, gridDim.x));
+  if constexpr (!WHOLE) {
+    if (*a.form == a.form_id) {  // (arrays of another form than a build's)
+      for (int u = 0; u < NPT; ++u)
+        scatter_node<MAKE>(a, r.local * T + u * kThreads + static_cast<int32_t>(threadIdx.x));
+      return;
+    }
+  }
   // The segment's scalars are loaded together before any is tested: one
   // round trip instead of one per value.
   // (The launcher guarantees these pointers; the build writes them all.)
@@ -615,29 +687,105 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   }
 }
 
+// Whether node i's entries are those of a build, as the tiled kernel takes them:
+// offsets that are the inclusive scan of the counts, counts of at most ten.
+__device__ __forceinline__ bool tiled_form(const OctArgs& a, int32_t i) {
+  const int32_t e = a.edge[i], p = a.offsets[i];
+  if (i == 0) return e == 0 && p == 0;
+  return e >= 0 && e <= kMaxEdge &&
+         static_cast<uint32_t>(p) - static_cast<uint32_t>(a.offsets[i - 1]) ==
+             static_cast<uint32_t>(e);
+}
+
+// Before the make phase: one thread per node looks its entries over; *form
+// becomes form_id where they are not a build's. (Any other value, an earlier
+// call's among them, means that they are, so the word needs no clearing.)
 // The make call alone has no children arrays to walk down from a slot's owner,
 // so the top link of a chain whose walk up leaves its tile comes from below: the
 // walk in global memory, and the order key into the child's word of the zeroed
-// node, kept by an atomic max. The make phase turns it into the link.
-__global__ __launch_bounds__(256) void oct_far_kernel(OctArgs a) {
+// node, kept by an atomic max, where the scatter of the other form would put it
+// too. The make phase turns it into the link.
+__global__ __launch_bounds__(256) void make_check_kernel(OctArgs a) {
   const int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x);
-  if (i < 1 || i >= a.n_brt_host) return;
+  if (i >= a.n_brt_host) return;
+  if (!tiled_form(a, i)) *a.form = a.form_id;
   const int32_t e = a.edge[i];
-  int32_t h = a.parent[i];
-  if (e <= 0) return;
+  if (i < 1 || e <= 0) return;
   bool far = false;
-  for (int hop = 0; hop < 32; ++hop) {
-    far |= (h ^ i) >= kOctTile;  // (another tile: the numbers differ above its bits)
-    if (a.edge[h] > 0 || h == 0) break;
-    h = a.parent[h];
-  }
+  const int32_t h = make_head(a, i, [&](int32_t at) {
+    far |= (at ^ i) >= kOctTile;  // (another tile: the numbers differ above its bits)
+  });
   if (!far) return;
-  const int32_t slot = a.offsets[h];
-  if (slot < 0 || slot >= a.k_host) return;
-  const int32_t level = a.prefix_n[i] / 3;
-  atomicMax(reinterpret_cast<uint32_t*>(
-                &a.nodes[slot].children[child_of(a.codes[i], level - e + 1)]),
-            make_key(i, e - 1));
+  put_word(a, a.offsets[h], child_of(a.codes[i], a.prefix_n[i] / 3 - e + 1), make_key(i, e - 1));
+}
+
+__global__ __launch_bounds__(256) void link_check_kernel(OctArgs a) {
+  const int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x);
+  if (i < a.n_brt_host && !tiled_form(a, i)) *a.form = a.form_id;
+}
+
+// After a scatter of order keys: the keys of the slots of chain i become the
+// values that they stand for, and a make call's slots get their corner and cell
+// size. Chain i owns slot P[i]+j when no later chain covers it; every slot that
+// receives a child write is covered by a chain or is the root slot 0.
+template <bool MAKE>
+__device__ __forceinline__ void resolve_children(const OctArgs& a, int32_t slot) {
+  int32_t* ch = a.nodes[slot].children;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const uint32_t v = static_cast<uint32_t>(ch[c]);
+    if (v == 0 || (v >> 31) == (MAKE ? 1u : 0u)) continue;
+    if constexpr (MAKE) {
+      ch[c] = a.offsets[(v - 1u) >> 4] + static_cast<int32_t>((v - 1u) & 15u);
+    } else {
+      const uint32_t q = v & 0x7fffffffu;
+      ch[c] = a.left_child[q >> 1] + static_cast<int32_t>(q & 1u);
+    }
+  }
+}
+template <bool MAKE>
+__global__ __launch_bounds__(1024) void resolve_kernel(OctArgs a, float mn, float rg) {
+  if (*a.form != a.form_id) return;
+  const int32_t m = a.n_brt_host;
+  for (int32_t i = blockIdx.x * 1024 + static_cast<int32_t>(threadIdx.x); i < m;
+       i += static_cast<int32_t>(gridDim.x) * 1024) {
+    if (i == 0) {
+      resolve_children<MAKE>(a, 0);
+      continue;
+    }
+    const int32_t e = a.edge[i];
+    if (e <= 0) continue;
+    const int32_t p = a.offsets[i];
+    const int32_t last = p + e - 1;
+    uint32_t owned = e >= 32 ? ~0u : (1u << e) - 1u;
+    for (int32_t k = i + 1; k < m && owned; ++k) {
+      const int32_t pk = a.offsets[k];
+      if (pk > last) break;
+      const int32_t ek = a.edge[k];
+      if (ek <= 0) continue;
+      const int32_t lo = max(pk, p) - p, hi = min(pk + ek - 1, last) - p;
+      for (int32_t q = lo; q <= min(hi, 31); ++q) owned &= ~(1u << q);
+    }
+    const int32_t root_level = a.prefix_n[0] / 3, level = a.prefix_n[i] / 3;
+    const uint32_t code = a.codes[i];
+    for (int32_t j = 0; j < e && j < 32; ++j) {
+      const int32_t slot = p + j;
+      // (slot 0 is the root's)
+      if (!((owned >> j) & 1u) || slot <= 0 || slot >= a.k_host) continue;
+      if constexpr (MAKE) {
+        OctNode* nd = a.nodes + slot;
+        const uint32_t shift = static_cast<uint32_t>(kMortonBits - 3 * (level - j)) & 31u;
+        const uint32_t corner = (code >> shift) << shift;
+        nd->corner[0] = decode_axis(corner, 0, mn, rg);
+        nd->corner[1] = decode_axis(corner, 1, mn, rg);
+        nd->corner[2] = decode_axis(corner, 2, mn, rg);
+        nd->corner[3] = 1.0f;
+        const uint32_t sh = static_cast<uint32_t>(level - j - root_level) & 31u;
+        nd->cell_size = rg / static_cast<float>(static_cast<int32_t>(1u << sh));
+      }
+      resolve_children<MAKE>(a, slot);
+    }
+  }
 }
 
 // Root node of apps/cpu_demo/main.cpp:125-132 alone (the per-stage entry
@@ -684,15 +832,27 @@ bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_s
   return true;
 }
 
+namespace {
+// (a grid that fills the chip; it returns at once for a build's arrays)
+template <bool MAKE>
+void launch_resolve(const OctArgs& a, const SegView& sv, hipStream_t s) {
+  const int32_t blocks = (a.n_brt_host + 1023) / 1024;
+  resolve_kernel<MAKE><<<blocks < 256 ? blocks : 256, 1024, 0, s>>>(a, sv.min1, sv.range1);
+}
+}  // namespace
+
 void launch_oct_make(const OctArgs& a, const SegView& sv, hipStream_t s) {
-  oct_far_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
+  make_check_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
   oct_build_kernel<false, kMakePhase>
       <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
+  launch_resolve<true>(a, sv, s);
 }
 
 void launch_oct_link(const OctArgs& a, const SegView& sv, hipStream_t s) {
+  link_check_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
   oct_build_kernel<false, kLinkPhase>
       <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
+  launch_resolve<false>(a, sv, s);
 }
 
 }  // namespace ocp

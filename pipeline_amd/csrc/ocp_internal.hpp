@@ -22,6 +22,7 @@ enum CtrlSlot : int {
   kCtrlWaitLimit = 14, // 0: waits poll up to kSpinLimit times; v > 0: v - 1
   kCtrlMsdTiles = 15,  // ... their tiles
   kCtrlMsdSlots = 16,  // ... and the count slots of their long runs
+  kCtrlOctForm = 17,   // last make or link call whose arrays were not a build's
   kCtrlWords = 64,
 };
 
@@ -349,6 +350,10 @@ struct OctArgs {
   const int32_t* n_unique;  // per segment (nullptr: n_brt_host + 1)
   int32_t n_brt_host;
   bool stream_nodes;  // nodes past the caches (oct_stream)
+  // Per-stage entries: *form == form_id once a kernel of this call has found
+  // arrays that are not a build's.
+  uint32_t* form;
+  uint32_t form_id;
 };
 // Whether a build of n points stores its nodes past the caches: once they and
 // the arrays they are made from outgrow the 256 MB behind the L2s, where they
@@ -377,9 +382,10 @@ struct OctSingle {
 bool launch_oct_build(const OctArgs& a, const SegView& sv, const int32_t* tile_start,
                       int32_t total_tiles, const OctSingle& single, hipStream_t s);
 
-// The per-stage entries: the same kernel on n_brt_host nodes and k_host slots,
-// doing the make writes (without the children arrays, which may be null) or the
-// link writes, into nodes that the caller prepared.
+// The per-stage entries: the make writes (without the children arrays, which may
+// be null) or the link writes of n_brt_host nodes, into the k_host nodes that the
+// caller prepared. The same kernel where the arrays have a build's form, which a
+// kernel before it checks; else a scatter and a kernel that resolves it.
 void launch_oct_make(const OctArgs& a, const SegView& sv, hipStream_t s);
 void launch_oct_link(const OctArgs& a, const SegView& sv, hipStream_t s);
 
