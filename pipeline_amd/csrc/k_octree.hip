@@ -55,12 +55,12 @@
 // The per-stage entries (k_MakeOctNodes, k_LinkLeafNodes: include/cuda/kernels/
 // 07_octree.cuh:7-28) are the same kernel doing one half of the pushes into
 // nodes that it reads and writes whole, where a kernel before it has found the
-// caller's arrays to be what a build's are (tiled_form); for any others, as
-// offsets that are not the inclusive scan, it scatters order keys by global
-// atomics and a kernel after it resolves them. Make has no children arrays: see
-// make_check_kernel. For 2M points make takes 16 us of check, 31 of the tiled
-// kernel and 5 of the idle resolve, link 5, 31 and 5; the scatter and the resolve
-// took 117 and 187 for every array.
+// caller's arrays to be what a build's are (check_kernel); for any others, as
+// offsets that are not the inclusive scan or codes that repeat, it scatters order
+// keys by global atomics and a kernel after it resolves them. Make has no children
+// arrays: see check_kernel. For 2M points make takes 17 us of check, 30 of the
+// tiled kernel and 5 of the idle resolve, link 14, 30 and 5; the scatter and the
+// resolve took 117 and 187 when they served every array.
 //
 // What bounds it: how many tiles share a CU while each waits for its loads, its
 // barriers and the walks of its listed children (a chain of up to four dependent
@@ -195,7 +195,8 @@ struct Columns {
 // of their loads in flight together, so the chain of dependent loads is one
 // per e == 0 node. Such nodes are at most three levels deep: prefix lengths
 // grow strictly down the tree and one octree level spans three of them, so
-// three pending ones suffice.
+// three pending ones suffice and seven steps are the most.
+constexpr int kMaxSteps = 16;
 struct SubNode {
   int32_t x, lc;
   uint32_t flags;  // level | has_leaf_left << 8 | has_leaf_right << 9
@@ -216,7 +217,7 @@ __device__ __forceinline__ void push_subgroup(const SegBind& b, const Columns& c
       cols.put_make(slot, child_of(code, level - e + 1), make_key(x, e - 1), p + e - 1);
     if (e != 0) return;
   }
-  while (true) {
+  for (int step = 0; step < kMaxSteps; ++step) {
     int32_t e[2], p[2], lc[2];
     uint32_t code[2];
     uint8_t pn[2], hl[2], hr[2];
@@ -273,13 +274,10 @@ __device__ __forceinline__ void put_make_word(const OctArgs& a, int32_t slot, ui
   atomicOr(&a.nodes[slot].child_node_mask, 1 << which);
 }
 // The node that the walk of oct.h:61-73 from node i's parent ends at (at most
-// 31 hops; node 0 is its own parent). at(h): the nodes on the way. A hop's two
-// loads are in flight together.
-template <class At>
-__device__ __forceinline__ int32_t make_head(const OctArgs& a, int32_t i, At at) {
+// 31 hops; node 0 is its own parent). A hop's two loads are in flight together.
+__device__ __forceinline__ int32_t make_head(const OctArgs& a, int32_t i) {
   int32_t h = a.parent[i];
   for (int hop = 0; hop < 31; ++hop) {
-    at(h);
     const int32_t e = a.edge[h], up = a.parent[h];
     if (e != 0 || up == h) break;
     h = up;
@@ -297,7 +295,7 @@ __device__ __forceinline__ void scatter_node(const OctArgs& a, int32_t i) {
     const uint32_t code = a.codes[i];
     for (int32_t j = 0; j < e - 1; ++j)
       put_make_word(a, p + j + 1, child_of(code, level - j), make_key(i, j));
-    put_make_word(a, a.offsets[make_head(a, i, [](int32_t) {})], child_of(code, level - e + 1),
+    put_make_word(a, a.offsets[make_head(a, i)], child_of(code, level - e + 1),
                   make_key(i, e - 1));
   } else {
     int32_t head = -1;
@@ -687,41 +685,193 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
   }
 }
 
-// Whether node i's entries are those of a build, as the tiled kernel takes them:
-// offsets that are the inclusive scan of the counts, counts of at most ten.
-__device__ __forceinline__ bool tiled_form(const OctArgs& a, int32_t i) {
-  const int32_t e = a.edge[i], p = a.offsets[i];
-  if (i == 0) return e == 0 && p == 0;
-  return e >= 0 && e <= kMaxEdge &&
-         static_cast<uint32_t>(p) - static_cast<uint32_t>(a.offsets[i - 1]) ==
-             static_cast<uint32_t>(e);
-}
-
-// Before the make phase: one thread per node looks its entries over; *form
-// becomes form_id where they are not a build's. (Any other value, an earlier
-// call's among them, means that they are, so the word needs no clearing.)
+// Before the phase of a per-stage entry: whether the caller's arrays are those
+// of a build, as the tiled kernel takes them; *form becomes form_id where they are
+// not. (Any other value, an earlier call's among them, means that they are, so the
+// word needs no clearing.) A build's are: offsets that are the inclusive scan of
+// the counts, counts of at most ten that are the levels between a node and its
+// parent, codes that increase, prefix lengths that grow down the tree (or the
+// parent is node 0), and, for the link phase, children and parents that name each
+// other, where node 0 stands for the true root. Over repeated codes two nodes of
+// one level can be each other's child, and a child be node m.
+//
+// A tile's nodes find their parents and children in LDS; those with one elsewhere
+// are listed and looked up in memory by full waves. What bounds it is the reading
+// of every array (link of 2M points: 23 bytes a node, 14 us; 19 when every node
+// gathered its neighbours from memory, 16 with tiles of 1024).
+//
 // The make call alone has no children arrays to walk down from a slot's owner,
 // so the top link of a chain whose walk up leaves its tile comes from below: the
 // walk in global memory, and the order key into the child's word of the zeroed
-// node, kept by an atomic max, where the scatter of the other form would put it
-// too. The make phase turns it into the link.
-__global__ __launch_bounds__(256) void make_check_kernel(OctArgs a) {
-  const int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x);
-  if (i >= a.n_brt_host) return;
-  if (!tiled_form(a, i)) *a.form = a.form_id;
-  const int32_t e = a.edge[i];
-  if (i < 1 || e <= 0) return;
-  bool far = false;
-  const int32_t h = make_head(a, i, [&](int32_t at) {
-    far |= (at ^ i) >= kOctTile;  // (another tile: the numbers differ above its bits)
-  });
-  if (!far) return;
-  put_word(a, a.offsets[h], child_of(a.codes[i], a.prefix_n[i] / 3 - e + 1), make_key(i, e - 1));
-}
-
-__global__ __launch_bounds__(256) void link_check_kernel(OctArgs a) {
-  const int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x);
-  if (i < a.n_brt_host && !tiled_form(a, i)) *a.form = a.form_id;
+// node, kept by an atomic max, where the scatter of other arrays would put it too.
+// The make phase turns it into the link.
+constexpr int kCheckTile = 512;
+constexpr uint32_t kCheckList = 512;  // of each kind; a build's tile has at most 124 (see 2.)
+template <bool LINK>
+__global__ __launch_bounds__(kThreads) void check_kernel(OctArgs a) {
+  constexpr int T = kCheckTile;
+  constexpr int NPT = T / kThreads;
+  __shared__ int32_t s_par[T];
+  __shared__ uint8_t s_pn[T];
+  __shared__ uint8_t s_chain[T];  // make: the count is not 0
+  __shared__ uint8_t s_named[T];  // link: by its parent, as a child
+  __shared__ uint16_t s_up[kCheckList], s_down[kCheckList];  // nodes; places of children's parents
+  __shared__ uint32_t s_n[2];
+  const int tid = threadIdx.x;
+  const int32_t m = a.n_brt_host;
+  const int32_t i0 = static_cast<int32_t>(blockIdx.x) * T;
+  // (neighbouring nodes, so that one load takes a thread's)
+  const int l0 = tid * NPT;
+  const int32_t at0 = i0 + l0;
+  int32_t e[NPT], p[NPT], lc[NPT], par[NPT], p_before = 0;
+  uint32_t code[NPT], before = 0, next = 0;
+  uint8_t pn[NPT], hl[NPT], hr[NPT];
+  if (i0 + T <= m) {
+    __builtin_memcpy(e, a.edge + at0, sizeof(e));
+    __builtin_memcpy(p, a.offsets + at0, sizeof(p));
+    __builtin_memcpy(par, a.parent + at0, sizeof(par));
+    __builtin_memcpy(code, a.codes + at0, sizeof(code));
+    __builtin_memcpy(pn, a.prefix_n + at0, sizeof(pn));
+    if constexpr (LINK) {
+      __builtin_memcpy(lc, a.left_child + at0, sizeof(lc));
+      __builtin_memcpy(hl, a.has_leaf_left + at0, sizeof(hl));
+      __builtin_memcpy(hr, a.has_leaf_right + at0, sizeof(hr));
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < NPT; ++u) {
+      const int32_t i = at0 + u;
+      e[u] = p[u] = lc[u] = par[u] = 0;
+      code[u] = 0;
+      pn[u] = hl[u] = hr[u] = 0;
+      if (LINK && i == m) code[u] = a.codes[m];
+      if (i >= m) continue;
+      e[u] = a.edge[i];
+      p[u] = a.offsets[i];
+      par[u] = a.parent[i];
+      code[u] = a.codes[i];
+      pn[u] = a.prefix_n[i];
+      if constexpr (LINK) {
+        lc[u] = a.left_child[i];
+        hl[u] = a.has_leaf_left[i];
+        hr[u] = a.has_leaf_right[i];
+      }
+    }
+  }
+  if (at0 > 0 && at0 < m) {
+    p_before = a.offsets[at0 - 1];
+    before = a.codes[at0 - 1];
+  }
+  if (LINK && at0 + NPT <= m) next = a.codes[at0 + NPT];
+  const uint32_t pn_0 = a.prefix_n[0];
+  uint32_t root = 0;
+  if constexpr (LINK) root = delta(a.codes[0], a.codes[m]);
+#pragma unroll
+  for (int u = 0; u < NPT; ++u) {
+    const int l = l0 + u;
+    s_par[l] = par[u];
+    s_pn[l] = pn[u];
+    if constexpr (LINK) s_named[l] = 0;
+    else s_chain[l] = e[u] != 0;
+  }
+  if (tid < 2) s_n[tid] = 0;
+  __syncthreads();
+  const auto in_tile = [&](int32_t q) { return static_cast<uint32_t>(q - i0) < static_cast<uint32_t>(T); };
+  const auto is_node = [&](int32_t q) { return static_cast<uint32_t>(q) < static_cast<uint32_t>(m); };
+  bool ok = true;
+  // (a full list: not a build's)
+  const auto push = [&](uint16_t* list, int which, uint32_t l) {
+    const uint32_t at = atomicAdd(&s_n[which], 1u);
+    if (at < kCheckList) list[at] = static_cast<uint16_t>(l);
+    else ok = false;
+  };
+#pragma unroll
+  for (int u = 0; u < NPT; ++u) {
+    const int32_t i = at0 + u;
+    const uint32_t l = static_cast<uint32_t>(l0 + u);
+    const uint32_t code_l = u ? code[u - 1] : before, code_r = u + 1 < NPT ? code[u + 1] : next;
+    if (i >= m) continue;
+    if constexpr (LINK) ok = ok && code[u] < code_r && is_node(lc[u]);
+    if (i == 0) {
+      ok = ok && e[u] == 0 && p[u] == 0;
+      continue;
+    }
+    const int32_t up = par[u];
+    ok = ok && e[u] >= 0 && e[u] <= kMaxEdge &&
+         static_cast<uint32_t>(p[u]) - static_cast<uint32_t>(u ? p[u - 1] : p_before) ==
+             static_cast<uint32_t>(e[u]) &&
+         code_l < code[u] && is_node(up);
+    if (up == 0 || in_tile(up)) {
+      const uint32_t pn_up = up == 0 ? pn_0 : s_pn[up - i0];
+      ok = ok && static_cast<int32_t>(pn[u] / 3u) - static_cast<int32_t>(pn_up / 3u) == e[u] &&
+           (up == 0 || pn_up < pn[u]);
+    } else if (is_node(up)) {
+      push(s_up, 0, l);
+    }
+    if constexpr (LINK) {
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        if (side == 0 ? hl[u] != 0 : hr[u] != 0) continue;
+        const int32_t ch = lc[u] + side;
+        if (ch <= 0 || !is_node(ch)) {
+          ok = false;
+        } else if (!in_tile(ch)) {
+          push(s_down, 1, l * 2u + static_cast<uint32_t>(side));
+        } else if (s_par[ch - i0] == i) {
+          s_named[ch - i0] = 1;
+        } else {
+          ok = false;
+        }
+      }
+      // The true root's children lie on either side of the pair of codes with the
+      // shortest common prefix.
+      const bool of_root = delta(code[u], code_r) == root || delta(code_l, code[u]) == root;
+      ok = ok && of_root == (up == 0);
+    } else if (e[u] > 0 && is_node(up)) {
+      bool far = false;  // out of the octree kernel's tile: the numbers differ above its bits
+      int32_t h = up;
+      for (int hop = 0; hop < 31; ++hop) {
+        far |= (h ^ i) >= kOctTile;
+        if (!in_tile(h) || s_chain[h - i0] != 0) break;
+        const int32_t next_up = s_par[h - i0];
+        if (next_up == h) break;
+        h = next_up;
+      }
+      if (far) push(s_down, 1, l);
+    }
+  }
+  __syncthreads();
+  if constexpr (LINK) {
+    // (a parent in the tile has named its children there)
+#pragma unroll
+    for (int u = 0; u < NPT; ++u)
+      if (at0 + u < m && at0 + u > 0 && par[u] != 0 && in_tile(par[u]) && !s_named[l0 + u]) ok = false;
+  }
+  for (uint32_t q = tid; q < min(s_n[0], kCheckList); q += kThreads) {
+    const uint32_t l = s_up[q];
+    const int32_t i = i0 + static_cast<int32_t>(l), up = s_par[l];
+    const uint32_t own = s_pn[l], pn_up = a.prefix_n[up];
+    ok = ok && static_cast<int32_t>(own / 3u) - static_cast<int32_t>(pn_up / 3u) == a.edge[i] &&
+         pn_up < own;
+    if constexpr (LINK) {
+      const int32_t at = a.left_child[up];
+      const bool leaf_l = a.has_leaf_left[up], leaf_r = a.has_leaf_right[up];
+      ok = ok && (i == at ? !leaf_l : i == at + 1 && !leaf_r);
+    }
+  }
+  for (uint32_t q = tid; q < min(s_n[1], kCheckList); q += kThreads) {
+    const uint32_t l = s_down[q];
+    if constexpr (LINK) {
+      const int32_t i = i0 + static_cast<int32_t>(l >> 1);
+      ok = ok && a.parent[a.left_child[i] + static_cast<int32_t>(l & 1u)] == i;
+    } else {
+      const int32_t i = i0 + static_cast<int32_t>(l);
+      const int32_t n_new = a.edge[i];
+      put_word(a, a.offsets[make_head(a, i)], child_of(a.codes[i], s_pn[l] / 3 - n_new + 1),
+               make_key(i, n_new - 1));
+    }
+  }
+  if (!ok) *a.form = a.form_id;
 }
 
 // After a scatter of order keys: the keys of the slots of chain i become the
@@ -842,14 +992,14 @@ void launch_resolve(const OctArgs& a, const SegView& sv, hipStream_t s) {
 }  // namespace
 
 void launch_oct_make(const OctArgs& a, const SegView& sv, hipStream_t s) {
-  make_check_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
+  check_kernel<false><<<(a.n_brt_host + kCheckTile - 1) / kCheckTile, kThreads, 0, s>>>(a);
   oct_build_kernel<false, kMakePhase>
       <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
   launch_resolve<true>(a, sv, s);
 }
 
 void launch_oct_link(const OctArgs& a, const SegView& sv, hipStream_t s) {
-  link_check_kernel<<<(a.n_brt_host + 255) / 256, 256, 0, s>>>(a);
+  check_kernel<true><<<(a.n_brt_host + kCheckTile - 1) / kCheckTile, kThreads, 0, s>>>(a);
   oct_build_kernel<false, kLinkPhase>
       <<<(a.n_brt_host + kOctTile - 1) / kOctTile, kThreads, 0, s>>>(a, sv, nullptr, OctSingle{});
   launch_resolve<false>(a, sv, s);

@@ -57,3 +57,25 @@ def test_offsets_of_any_form(ctx, form, u):
         used = max(1, int((p + e).max()))
         for k in (used, used + 90, max(1, used - used // 5)):
             _check(ctx, codes, tree, e, p, k)
+
+
+def _repeated(kind, u):
+    """Sorted codes with repeats."""
+    base = _codes(u, "uniform")
+    mid = base[base.size // 2]
+    return {"one code": lambda: np.full(u, mid), "one pair": lambda: np.append(base, mid),
+            "twice": lambda: np.repeat(base[:u // 2 + 1], 2),
+            "run": lambda: np.append(base, np.full(700, mid))}[kind]()
+
+
+@pytest.mark.parametrize("kind", ["one code", "one pair", "twice", "run"])
+@pytest.mark.parametrize("u", [513, 1400, 5400])
+def test_repeated_codes(ctx, kind, u):
+    """The tree over codes that repeat, which its entry takes: chains by the
+    inclusive scan, children that are no node, nodes that name each other."""
+    codes = np.sort(_repeated(kind, u)).astype(np.uint32)
+    tree = oracle.build_radix_tree(codes)
+    e = oracle.edge_count(tree["prefix_n"], tree["parent"])
+    p = oracle.partial_sum(e)
+    assert e.min() >= 0 and p[0] == 0
+    _check(ctx, codes, tree, e, p, max(1, int((p + e).max())))
