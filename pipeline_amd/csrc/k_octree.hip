@@ -56,11 +56,11 @@
 // 07_octree.cuh:7-28) are the same kernel doing one half of the pushes into
 // nodes that it reads and writes whole, where a kernel before it has found the
 // caller's arrays to be what a build's are (check_kernel); for any others, as
-// offsets that are not the inclusive scan or codes that repeat, it scatters order
-// keys by global atomics and a kernel after it resolves them. Make has no children
-// arrays: see check_kernel. For 2M points make takes 17 us of check, 30 of the
-// tiled kernel and 5 of the idle resolve, link 14, 30 and 5; the scatter and the
-// resolve took 117 and 187 when they served every array.
+// offsets that are not the inclusive scan, or codes that repeat or have more than
+// 30 bits, it scatters order keys by global atomics and a kernel after it resolves
+// them. Make has no children arrays: see check_kernel. For 2M points make takes 17
+// us of check, 30 of the tiled kernel and 5 of the idle resolve, link 15, 30 and 5;
+// the scatter and the resolve took 117 and 187 when they served every array.
 //
 // What bounds it: how many tiles share a CU while each waits for its loads, its
 // barriers and the walks of its listed children (a chain of up to four dependent
@@ -85,6 +85,8 @@ namespace ocp {
 namespace {
 
 constexpr int32_t kMaxEdge = 10;
+constexpr uint32_t kMaxPrefix = 31;                // of 30-bit codes (a node of one code)
+constexpr uint32_t kCodeEnd = 1u << kMortonBits;  // what an owner word and third() hold
 constexpr int kThreads = 256;
 constexpr int kCols = 312;      // slots per round; a tile of 512 nodes has ~240
 constexpr int kCodeHalo = 32;   // codes staged on either side of a tile
@@ -690,8 +692,8 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
 // not. (Any other value, an earlier call's among them, means that they are, so the
 // word needs no clearing.) A build's are: offsets that are the inclusive scan of
 // the counts, counts of at most ten that are the levels between a node and its
-// parent, codes that increase, prefix lengths that grow down the tree (or the
-// parent is node 0), and, for the link phase, children and parents that name each
+// parent, codes of 30 bits that increase, prefix lengths of such codes that grow
+// down the tree (or the parent is node 0), and, for the link phase, children and parents that name each
 // other, where node 0 stands for the true root. Over repeated codes two nodes of
 // one level can be each other's child, and a child be node m.
 //
@@ -791,7 +793,8 @@ __global__ __launch_bounds__(kThreads) void check_kernel(OctArgs a) {
     const uint32_t l = static_cast<uint32_t>(l0 + u);
     const uint32_t code_l = u ? code[u - 1] : before, code_r = u + 1 < NPT ? code[u + 1] : next;
     if (i >= m) continue;
-    if constexpr (LINK) ok = ok && code[u] < code_r && is_node(lc[u]);
+    ok = ok && code[u] < kCodeEnd && pn[u] <= kMaxPrefix;
+    if constexpr (LINK) ok = ok && code[u] < code_r && code_r < kCodeEnd && is_node(lc[u]);
     if (i == 0) {
       ok = ok && e[u] == 0 && p[u] == 0;
       continue;
@@ -886,7 +889,11 @@ __device__ __forceinline__ void resolve_children(const OctArgs& a, int32_t slot)
     const uint32_t v = static_cast<uint32_t>(ch[c]);
     if (v == 0 || (v >> 31) == (MAKE ? 1u : 0u)) continue;
     if constexpr (MAKE) {
-      ch[c] = a.offsets[(v - 1u) >> 4] + static_cast<int32_t>((v - 1u) & 15u);
+      // (a chain of more than 16 steps, over codes that differ in bit 31, can run
+      // into the next numbers: nothing is read past the arrays)
+      const uint32_t i = (v - 1u) >> 4;
+      if (i < static_cast<uint32_t>(a.n_brt_host))
+        ch[c] = a.offsets[i] + static_cast<int32_t>((v - 1u) & 15u);
     } else {
       const uint32_t q = v & 0x7fffffffu;
       ch[c] = a.left_child[q >> 1] + static_cast<int32_t>(q & 1u);

@@ -79,3 +79,16 @@ def test_repeated_codes(ctx, kind, u):
     p = oracle.partial_sum(e)
     assert e.min() >= 0 and p[0] == 0
     _check(ctx, codes, tree, e, p, max(1, int((p + e).max())))
+
+
+@pytest.mark.parametrize("bits", ["30", "30 or not", "31"])
+@pytest.mark.parametrize("u", [3, 513, 3000])
+def test_codes_of_more_than_30_bits(ctx, bits, u):
+    base = _codes(u, "uniform").astype(np.uint64)
+    some = np.random.default_rng(u).integers(0, 2, base.size).astype(np.uint64)
+    top = {"30": 1 << 30, "30 or not": some << np.uint64(30), "31": 1 << 31}[bits]
+    codes = np.sort(base + top).astype(np.uint32)
+    tree = oracle.build_radix_tree(codes)
+    e = oracle.edge_count(tree["prefix_n"], tree["parent"])
+    p = oracle.partial_sum(e)
+    _check(ctx, codes, tree, e, p, max(1, int((p + e).max())))
