@@ -466,11 +466,11 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
             hr[u] = b.hr[i];
           }
         }
-        if (i <= b.m) code[u] = b.codes[i];
+        if (LINK ? i <= b.m : i < b.m) code[u] = b.codes[i];  // (make: as many codes as nodes)
       }
     }
     uint32_t code_halo = 0;
-    if (tid < 2 * kCodeHalo) {
+    if (LINK && tid < 2 * kCodeHalo) {
       const int32_t g = tid < kCodeHalo ? i0 - kCodeHalo + tid : i0 + T + tid - kCodeHalo;
       if (g >= 0 && g <= b.m) code_halo = b.codes[g];
     }
