@@ -201,6 +201,9 @@ struct ocp_context {
   bool mail_current = false;
   bool graph_mode = false;
   bool permutation = false;
+  uint32_t* fmt = nullptr;  // counts or flags of the compact form's tiles
+  int64_t fmt_cap = 0;
+  bool in_pipeline = false;  // a slot of an ocp_pipeline
   // Streaming: the first lookback launch of a build waits for order_wait,
   // and order_record is recorded after its last one (eager builds only).
   hipEvent_t order_wait = nullptr;
@@ -269,6 +272,19 @@ int ensure_scratch(ocp_ctx c, int64_t flag_words) {
     OCP_HIP(c, hipMemsetAsync(c->s_flags, 0, sizeof(uint64_t) * cap, c->stream));
     c->s_flag_cap = cap;
   }
+  return OCP_OK;
+}
+
+// For the compact form, its own: captured per-stage calls keep the scratch above.
+int ensure_fmt(ocp_ctx c, int64_t words) {
+  if (words <= c->fmt_cap) return OCP_OK;
+  dev_free(c->fmt);
+  c->fmt_cap = 0;
+  const int64_t cap = std::max<int64_t>(words, 1 << 14);
+  if (int r = dev_alloc(c, &c->fmt, cap)) return r;
+  launch_fill_u32(c->fmt, 0u, cap, c->stream);  // (no flag of an earlier owner)
+  OCP_CHECK_LAUNCH(c);
+  c->fmt_cap = cap;
   return OCP_OK;
 }
 
@@ -964,6 +980,7 @@ int ocp_destroy(ocp_ctx c) {
   if (c->mail) (void)hipHostFree(c->mail);
   dev_free(c->s_flags);
   dev_free(c->s_hist);
+  dev_free(c->fmt);
   for (auto& e : c->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : c->kev)
@@ -1638,36 +1655,44 @@ int ocp_compact_octree(ocp_ctx c, ocp_compact_node* nodes, int64_t node_cap, int
   if (int r = build_slots(c, &kt)) return r;
   const Workspace& w = c->ws;
   const Plan& p = c->last_plan;
-  // Room for the pass's flags, and a word that counts what it cannot hold.
-  // (Its waits are reported here, so the build's mail stays the last word.)
-  const bool mail_current = c->mail_current;
-  if (int r = ensure_scratch(c, 2 * compact_tiles(kt) + 1)) return r;
-  c->mail_current = mail_current;
-  auto* bad = reinterpret_cast<unsigned long long*>(c->s_hist);
-  uint32_t* mail = c->mail + kMailWords;
-  mail[0] = mail[1] = mail[2] = 0;
   // (size queries, and calls whose node array is too small, store nothing)
   const bool store = nodes && children && node_cap >= kt;
-  launch_begin(c->ctrl, c->s_hist, 2, c->stream);
-  launch_compact(w.nodes, kt, w.oct_start, p.n_seg, p.sv.mn, p.sv.rg, p.sv.min1, p.sv.range1,
-                 p.sv.start, w.counts, w.prefix_n, c->s_flags, c->ctrl, store ? nodes : nullptr,
-                 store ? children : nullptr, child_cap, bad, mail, c->stream);
-  OCP_CHECK_LAUNCH(c);
-  OCP_HIP(c, hipStreamSynchronize(c->stream));
-  if (mail[1]) {
-    c->mail_current = false;
-    return sync_and_check(c);
+  const CompactSource src{w.nodes, kt, w.oct_start, p.n_seg, p.sv.mn, p.sv.rg, p.sv.min1,
+                          p.sv.range1, p.sv.start, w.counts, w.prefix_n};
+  uint32_t* mail = c->mail + kMailWords;
+  mail[0] = mail[1] = mail[2] = 0;
+  uint64_t hbad = 0;
+  if (c->in_pipeline) {
+    if (int r = ensure_fmt(c, compact_words(kt))) return r;
+    launch_compact_no_wait(src, c->fmt, store ? nodes : nullptr, children, child_cap, mail,
+                           c->stream);
+    OCP_CHECK_LAUNCH(c);
+    OCP_HIP(c, hipStreamSynchronize(c->stream));
+    hbad = mail[2];
+  } else {
+    // Room for the pass's flags, and a word that counts what has no such form.
+    // (Its waits are reported here, so the build's mail stays the last word.)
+    if (int r = ensure_fmt(c, 2 * (2 * compact_tiles(kt) + 1))) return r;
+    auto* flags = reinterpret_cast<uint64_t*>(c->fmt) + 1;
+    auto* bad = reinterpret_cast<unsigned long long*>(c->fmt);
+    launch_begin(c->ctrl, c->fmt, 2, c->stream);
+    launch_compact(src, flags, c->ctrl, store ? nodes : nullptr, store ? children : nullptr,
+                   child_cap, bad, mail, c->stream);
+    OCP_CHECK_LAUNCH(c);
+    OCP_HIP(c, hipStreamSynchronize(c->stream));
+    if (mail[1]) {
+      c->mail_current = false;
+      return sync_and_check(c);
+    }
+    if (mail[2]) OCP_HIP(c, hipMemcpy(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost));
   }
   const int64_t total = mail[0];
   *n_nodes = kt;
   *n_children = total;
-  if (mail[2]) {
-    unsigned long long hbad = 0;
-    OCP_HIP(c, hipMemcpy(&hbad, bad, sizeof(hbad), hipMemcpyDeviceToHost));
+  if (hbad)
     return fail(c, OCP_ERR_STATE, std::to_string(hbad) +
                                       " octree slots have no exact compact form (corner off "
                                       "its level's grid or cell size not range / 2^k)");
-  }
   if (!nodes || !children) return OCP_OK;  // size query
   if (node_cap < kt || child_cap < total)
     return fail(c, OCP_ERR_CAPACITY, "compact octree: output arrays too small (need " +
@@ -2318,7 +2343,8 @@ int ocp_sort_learned(ocp_ctx c, uint32_t* keys, uint32_t* alt, uint32_t n,
 // kernels run in order on its slot's stream, so slots overlap: one frame's
 // upload (a DMA engine) and Morton, radix-tree and octree kernels run beside
 // another's. Lookback launches (sort passes, unique, edge scan) of two frames
-// never overlap: each build's first one waits on the previous frame's last.
+// never overlap: each build's first one waits on the previous frame's last. The
+// compact form of a slot's octree, which no event orders, has no such launch.
 struct ocp_pipeline {
   int device = 0;
   int64_t max_points = 0;
@@ -2380,6 +2406,7 @@ int ocp_ppl_create(ocp_ppl* out, int device, int32_t depth, int64_t max_points) 
       ocp_ppl_destroy(p);
       return r;
     }
+    p->slots[i]->in_pipeline = true;
     if (hipEventCreateWithFlags(&p->scan_done[i], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&p->upload_done[i], hipEventDisableTiming) != hipSuccess ||
         (bytes && (hipHostMalloc(reinterpret_cast<void**>(&p->host[i]), bytes,

@@ -317,35 +317,15 @@ struct SegTables {
 };
 
 constexpr int kFmtTile = 512;  // slots per workgroup of the compact and expand kernels
+constexpr int kFmtPer = kFmtTile / kFmtThreads;
 
-// The compact form in one pass over the nodes: a tile's nodes come through LDS
-// in whole lines, a thread forms the headers of two, the tile's place in the
-// child array comes from the two-level lookback, and headers and children
-// leave through LDS, in whole lines again. nodes or children may be null (the
-// sizes only); children past child_cap are not stored. mail (host memory):
-// [0] the children's total, [1] a wait gave up, [2] slots without an exact
-// form exist (*bad counts them).
-// What bounds it: 60 bytes a slot read and ~28 written; 0.99M slots take
-// 27 us, where two passes over the nodes and three scan launches took 54, and
-// the call 50 us instead of 208.
-__global__ __launch_bounds__(kFmtThreads) void compact_kernel(
-    const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, uint64_t* __restrict__ flags,
-    uint32_t* __restrict__ ctrl, uint32_t* __restrict__ out, int32_t* __restrict__ children,
-    int64_t child_cap, unsigned long long* __restrict__ bad, uint32_t* __restrict__ mail) {
-  constexpr int NPT = kFmtTile / kFmtThreads;
-  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
-  __shared__ uint32_t s_tmp[kFmtThreads / 64];
-  __shared__ uint32_t s_excl;
-  const uint32_t tag = ctrl[kCtrlEpoch] * 8u + kStageScan;
-  if (stopped(ctrl, tag)) return;
+// A tile's nodes into LDS in whole lines (a tile starts on a multiple of 16
+// bytes: 512 nodes are 30,720).
+__device__ __forceinline__ void load_tile(const OctNode* __restrict__ nodes, int64_t g0,
+                                          int32_t cnt, int32_t* s_words) {
   const int tid = threadIdx.x;
-  const int32_t t = blockIdx.x;  // in-order dispatch: see lookback_n
-  const int64_t g0 = int64_t(t) * kFmtTile;
-  const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
-  const int32_t words = cnt * 15;
   const int32_t* src = reinterpret_cast<const int32_t*>(nodes + g0);
   if (cnt == kFmtTile) {
-    // (a tile starts on a multiple of 16 bytes: 512 nodes are 30,720)
     constexpr int kVec = kFmtTile * 15 / 4;
     constexpr int kRows = kVec / kFmtThreads;
     static_assert(kVec - kRows * kFmtThreads == kFmtThreads / 2, "half a row is left");
@@ -360,33 +340,97 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
     for (int k = 0; k < kRows; ++k) to[k * kFmtThreads] = x[k];
     if (tid < kFmtThreads / 2) to[kRows * kFmtThreads] = y;
   } else {
-    for (int32_t q = tid; q < words; q += kFmtThreads) s_words[q] = src[q];
+    for (int32_t q = tid; q < cnt * 15; q += kFmtThreads) s_words[q] = src[q];
   }
-  // The tile's segment, when one holds all of it.
-  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
-  const bool one = st.oct_start[seg0 + 1] >= g0 + cnt;
-  SegInfo info = st.of(seg0);
-  __syncthreads();
-  // Thread: NPT neighbouring slots, so that its children are neighbours too.
-  CompactNode cn[NPT];
-  int32_t child[NPT][8];
-  uint32_t mine = 0, nbad = 0;
+}
+
+// The headers of a thread's neighbouring slots, from the tile in LDS (loaded
+// by the caller, who also passes the barrier after it).
+struct TileSlots {
+  CompactNode cn[kFmtPer];
+  int32_t child[kFmtPer][8];
+  uint32_t children = 0, bad = 0;
+  __device__ __forceinline__ void form(const int32_t* s_words, int64_t g0, int32_t cnt,
+                                       const SegTables& st, int32_t seg0, SegInfo info) {
+    // (one segment holds the whole tile, as a rule)
+    const bool one = st.oct_start[seg0 + 1] >= g0 + cnt;
 #pragma unroll
-  for (int u = 0; u < NPT; ++u) {
-    const int32_t l = tid * NPT + u;
-    cn[u] = CompactNode{};
+    for (int u = 0; u < kFmtPer; ++u) {
+      const int32_t l = static_cast<int32_t>(threadIdx.x) * kFmtPer + u;
+      cn[u] = CompactNode{};
+      if (l >= cnt) continue;
+      int32_t w[15];
+#pragma unroll
+      for (int c = 0; c < 15; ++c) w[c] = s_words[l * 15 + c];
+      if (!one) info = st.of(seg_of_slot(g0 + l, st.oct_start, st.n_seg));
+      bad += !compact_header(w, info.mn, info.rg, info.root_level, &cn[u]);
+#pragma unroll
+      for (int c = 0; c < 8; ++c) child[u][c] = w[c];
+      children += __popc(cn[u].child_set);
+    }
+  }
+};
+
+// A tile's headers and children through LDS (whose nodes every thread has read),
+// to leave in whole lines. excl, before: the children before the tile and, in it,
+// before the thread's slots. Children past child_cap are not stored.
+__device__ __forceinline__ void store_tile(TileSlots& slots, int32_t* s_words, int64_t g0,
+                                           int32_t cnt, uint32_t excl, uint32_t before,
+                                           uint32_t total, uint32_t* __restrict__ out,
+                                           int32_t* __restrict__ children, int64_t child_cap) {
+  const int tid = threadIdx.x;
+  uint32_t* s_child = reinterpret_cast<uint32_t*>(s_words);
+  uint32_t* s_head = s_child + kFmtTile * 8;
+  uint32_t o = before;
+#pragma unroll
+  for (int u = 0; u < kFmtPer; ++u) {
+    const int32_t l = tid * kFmtPer + u;
     if (l >= cnt) continue;
-    int32_t w[15];
+    slots.cn[u].first_child = excl + o;
+    uint32_t hw[3];
+    __builtin_memcpy(hw, &slots.cn[u], 12);
 #pragma unroll
-    for (int c = 0; c < 15; ++c) w[c] = s_words[l * 15 + c];
-    if (!one) info = st.of(seg_of_slot(g0 + l, st.oct_start, st.n_seg));
-    nbad += !compact_header(w, info.mn, info.rg, info.root_level, &cn[u]);
+    for (int c = 0; c < 3; ++c) s_head[l * 3 + c] = hw[c];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) child[u][c] = w[c];
-    mine += __popc(cn[u].child_set);
+    for (int c = 0; c < 8; ++c)
+      if (slots.child[u][c] != 0) s_child[o++] = static_cast<uint32_t>(slots.child[u][c]);
   }
+  __syncthreads();
+  uint32_t* head = out + g0 * 3;
+  for (int32_t q = tid; q < cnt * 3; q += kFmtThreads) head[q] = s_head[q];
+  for (uint32_t q = tid; q < total; q += kFmtThreads)
+    if (static_cast<int64_t>(excl) + q < child_cap)
+      children[static_cast<int64_t>(excl) + q] = static_cast<int32_t>(s_child[q]);
+}
+
+// The compact form in one pass over the nodes: a tile's place in the child array
+// comes from the two-level lookback. out and children may be null (the sizes
+// only); children past child_cap are not stored. mail (host memory): [0] the
+// children's total, [1] a wait gave up, [2] slots without an exact form exist
+// (*bad counts them).
+// What bounds it: 60 bytes a slot read and ~28 written; 0.99M slots take
+// 27 us, where two passes over the nodes and three scan launches took 54, and
+// the call 45 us instead of 208.
+__global__ __launch_bounds__(kFmtThreads) void compact_kernel(
+    const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, uint64_t* __restrict__ flags,
+    uint32_t* __restrict__ ctrl, uint32_t* __restrict__ out, int32_t* __restrict__ children,
+    int64_t child_cap, unsigned long long* __restrict__ bad, uint32_t* __restrict__ mail) {
+  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_tmp[kFmtThreads / 64];
+  __shared__ uint32_t s_excl;
+  const uint32_t tag = ctrl[kCtrlEpoch] * 8u + kStageScan;
+  if (stopped(ctrl, tag)) return;
+  const int32_t t = blockIdx.x;  // in-order dispatch: see lookback_n
+  const int64_t g0 = int64_t(t) * kFmtTile;
+  const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
+  load_tile(nodes, g0, cnt, s_words);
+  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
+  const SegInfo info = st.of(seg0);
+  __syncthreads();
+  TileSlots slots;
+  slots.form(s_words, g0, cnt, st, seg0, info);
   uint32_t total;
-  const uint32_t before = block_excl_scan<kFmtThreads>(mine, s_tmp, &total);
+  const uint32_t before = block_excl_scan<kFmtThreads>(slots.children, s_tmp, &total);
   if (wave_id() == 0) {
     if (lane_id() == 0) flag_store(&flags[t], flag_pack(tag, kFlagAgg, total));
     bool late = false;
@@ -401,35 +445,113 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
       if (g0 + cnt == k_total) mail[0] = prev + total;
     }
   }
-  if (nbad) {
-    atomicAdd(bad, static_cast<unsigned long long>(nbad));
+  if (slots.bad) {
+    atomicAdd(bad, static_cast<unsigned long long>(slots.bad));
     mail[2] = 1u;
   }
   __syncthreads();  // (every word of the nodes has been read)
   if (!out || !children) return;
-  const uint32_t excl = s_excl;
-  uint32_t* s_child = reinterpret_cast<uint32_t*>(s_words);
-  uint32_t* s_head = s_child + kFmtTile * 8;
-  uint32_t o = before;
+  store_tile(slots, s_words, g0, cnt, s_excl, before, total, out, children, child_cap);
+}
+
+// The compact form in two passes over the nodes, whose tiles wait for nothing, for
+// a pipeline's slots: launches with waits of two frames may not overlap, and this
+// one is outside their order. Tiles form at most kCompactGroups groups of
+// neighbours, a workgroup each in the first pass: tile_children[t], and per group
+// {children, slots without an exact form}. The second pass sums the groups before
+// its own and its group's tiles before its own.
+// What bounds them: 60 bytes a slot read twice and ~28 written; 0.99M slots take
+// 16 and 24 us, the call 54 where the one pass takes 45.
+constexpr int32_t kCompactGroups = 2048;
+__host__ __device__ __forceinline__ int32_t tiles_per_group(int32_t tiles) {
+  return (tiles + kCompactGroups - 1) / kCompactGroups;
+}
+__global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
+    const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, int32_t tiles,
+    uint2* __restrict__ groups, uint32_t* __restrict__ tile_children) {
+  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_tmp[2 * (kFmtThreads / 64)];
+  const int32_t per = tiles_per_group(tiles);
+  const int32_t t0 = static_cast<int32_t>(blockIdx.x) * per;
+  uint2 sum = make_uint2(0u, 0u);
+  for (int32_t t = t0; t < min(t0 + per, tiles); ++t) {
+    const int64_t g0 = int64_t(t) * kFmtTile;
+    const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
+    const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
+    const SegInfo info = st.of(seg0);
+    load_tile(nodes, g0, cnt, s_words);
+    __syncthreads();
+    TileSlots slots;
+    slots.form(s_words, g0, cnt, st, seg0, info);
+    const uint32_t c = wave_sum(slots.children), b = wave_sum(slots.bad);
+    if (lane_id() == 0) {
+      s_tmp[2 * wave_id()] = c;
+      s_tmp[2 * wave_id() + 1] = b;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t n = 0;
 #pragma unroll
-  for (int u = 0; u < NPT; ++u) {
-    const int32_t l = tid * NPT + u;
-    if (l >= cnt) continue;
-    cn[u].first_child = excl + o;
-    uint32_t hw[3];
-    __builtin_memcpy(hw, &cn[u], 12);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) s_head[l * 3 + c] = hw[c];
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      if (child[u][c] != 0) s_child[o++] = static_cast<uint32_t>(child[u][c]);
+      for (int w = 0; w < kFmtThreads / 64; ++w) {
+        n += s_tmp[2 * w];
+        sum.y += s_tmp[2 * w + 1];
+      }
+      tile_children[t] = n;
+      sum.x += n;
+    }
+  }
+  if (threadIdx.x == 0) groups[blockIdx.x] = sum;
+}
+
+// mail (host memory): [0] the children's total, [2] the number of slots without
+// an exact form. A grid of one with out null: these alone. Children past
+// child_cap are not stored.
+__global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
+    const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, int32_t tiles,
+    const uint2* __restrict__ groups, const uint32_t* __restrict__ tile_children,
+    uint32_t* __restrict__ out, int32_t* __restrict__ children, int64_t child_cap,
+    uint32_t* __restrict__ mail) {
+  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_tmp[kFmtThreads / 64];
+  __shared__ uint32_t s_sum[3];  // children before the tile, all children, bad slots
+  const int tid = threadIdx.x;
+  const int32_t t = blockIdx.x;
+  const int64_t g0 = int64_t(t) * kFmtTile;
+  const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
+  if (tid < 3) s_sum[tid] = 0;
+  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
+  const SegInfo info = st.of(seg0);
+  const int32_t per = tiles_per_group(tiles);
+  const int32_t own = t / per, n_groups = (tiles + per - 1) / per;
+  uint32_t before = 0, all = 0, bad = 0;
+  for (int32_t q = tid; q < n_groups; q += kFmtThreads) {
+    const uint2 g = groups[q];
+    all += g.x;
+    bad += g.y;
+    if (q < own) before += g.x;
+  }
+  for (int32_t q = own * per + tid; q < t; q += kFmtThreads) before += tile_children[q];
+  if (out) load_tile(nodes, g0, cnt, s_words);
+  __syncthreads();
+  before = wave_sum(before);
+  all = wave_sum(all);
+  bad = wave_sum(bad);
+  if (lane_id() == 0) {
+    atomicAdd(&s_sum[0], before);
+    atomicAdd(&s_sum[1], all);
+    atomicAdd(&s_sum[2], bad);
   }
   __syncthreads();
-  uint32_t* head = out + g0 * 3;
-  for (int32_t q = tid; q < cnt * 3; q += kFmtThreads) head[q] = s_head[q];
-  for (uint32_t q = tid; q < total; q += kFmtThreads)
-    if (static_cast<int64_t>(excl) + q < child_cap)
-      children[static_cast<int64_t>(excl) + q] = static_cast<int32_t>(s_child[q]);
+  if (t == 0 && tid == 0) {
+    mail[0] = s_sum[1];
+    mail[2] = s_sum[2];
+  }
+  if (!out) return;
+  TileSlots slots;
+  slots.form(s_words, g0, cnt, st, seg0, info);
+  uint32_t total;
+  const uint32_t first = block_excl_scan<kFmtThreads>(slots.children, s_tmp, &total);
+  store_tile(slots, s_words, g0, cnt, s_sum[0], first, total, out, children, child_cap);
 }
 
 // 60-byte nodes from the compact form, a tile's through LDS so that whole
@@ -518,15 +640,35 @@ void launch_validate(const OctNode* nodes, const int32_t* edge, const int32_t* o
 
 int64_t compact_tiles(int64_t k_total) { return (k_total + kFmtTile - 1) / kFmtTile; }
 
-void launch_compact(const OctNode* nodes, int64_t k_total, const int32_t* oct_start, int32_t n_seg,
-                    const float* smin, const float* srg, float mn1, float rg1,
-                    const int32_t* seg_start, const int32_t* n_unique, const uint8_t* prefix_n,
-                    uint64_t* flags, uint32_t* ctrl, void* out, int32_t* children,
-                    int64_t child_cap, unsigned long long* bad, uint32_t* mail, hipStream_t s) {
-  if (n_seg <= 0 || k_total <= 0) return;
-  const SegTables st{oct_start, n_seg, Boxes{smin, srg, mn1, rg1}, seg_start, n_unique, prefix_n};
-  compact_kernel<<<static_cast<uint32_t>(compact_tiles(k_total)), kFmtThreads, 0, s>>>(
-      nodes, k_total, st, flags, ctrl, static_cast<uint32_t*>(out), children, child_cap, bad, mail);
+static SegTables seg_tables(const CompactSource& c) {
+  return {c.oct_start, c.n_seg, Boxes{c.smin, c.srg, c.mn1, c.rg1}, c.seg_start, c.n_unique,
+          c.prefix_n};
+}
+
+void launch_compact(const CompactSource& c, uint64_t* flags, uint32_t* ctrl, void* out,
+                    int32_t* children, int64_t child_cap, unsigned long long* bad, uint32_t* mail,
+                    hipStream_t s) {
+  if (c.n_seg <= 0 || c.k_total <= 0) return;
+  compact_kernel<<<static_cast<uint32_t>(compact_tiles(c.k_total)), kFmtThreads, 0, s>>>(
+      c.nodes, c.k_total, seg_tables(c), flags, ctrl, static_cast<uint32_t*>(out), children,
+      child_cap, bad, mail);
+}
+
+int64_t compact_words(int64_t k_total) { return 2 * kCompactGroups + compact_tiles(k_total); }
+
+void launch_compact_no_wait(const CompactSource& c, uint32_t* words, void* out, int32_t* children,
+                            int64_t child_cap, uint32_t* mail, hipStream_t s) {
+  if (c.n_seg <= 0 || c.k_total <= 0) return;
+  const SegTables st = seg_tables(c);
+  const int32_t tiles = static_cast<int32_t>(compact_tiles(c.k_total));
+  const int32_t per = tiles_per_group(tiles);
+  uint2* groups = reinterpret_cast<uint2*>(words);
+  uint32_t* tile_children = words + 2 * kCompactGroups;
+  compact_count_kernel<<<(tiles + per - 1) / per, kFmtThreads, 0, s>>>(c.nodes, c.k_total, st,
+                                                                      tiles, groups, tile_children);
+  compact_write_kernel<<<out ? tiles : 1, kFmtThreads, 0, s>>>(
+      c.nodes, c.k_total, st, tiles, groups, tile_children, static_cast<uint32_t*>(out), children,
+      child_cap, mail);
 }
 
 void launch_expand(const void* in, const int32_t* children, int64_t n_children,

@@ -402,16 +402,31 @@ void launch_validate(const OctNode* nodes, const int32_t* edge, const int32_t* o
                      int32_t n_seg, const float* smin, const float* srg, float mn1, float rg1,
                      const int32_t* root_level, const uint32_t* root_code, uint8_t* cov,
                      unsigned long long* rep, hipStream_t s);
-// The compact form of k_total slots in one pass, in the lookback epoch that a
-// launch_begin before it began (flags: 2 * compact_tiles(k_total) words; *bad
-// zeroed). out and children may be null. mail: three words of host memory,
-// zeroed (see compact_kernel).
+// What the compact form is made from: k_total slots of a build.
+struct CompactSource {
+  const OctNode* nodes;
+  int64_t k_total;
+  const int32_t* oct_start;
+  int32_t n_seg;
+  const float* smin;
+  const float* srg;
+  float mn1, rg1;
+  const int32_t* seg_start;
+  const int32_t* n_unique;
+  const uint8_t* prefix_n;
+};
 int64_t compact_tiles(int64_t k_total);
-void launch_compact(const OctNode* nodes, int64_t k_total, const int32_t* oct_start, int32_t n_seg,
-                    const float* smin, const float* srg, float mn1, float rg1,
-                    const int32_t* seg_start, const int32_t* n_unique, const uint8_t* prefix_n,
-                    uint64_t* flags, uint32_t* ctrl, void* out, int32_t* children,
-                    int64_t child_cap, unsigned long long* bad, uint32_t* mail, hipStream_t s);
+// In one pass, in the lookback epoch that a launch_begin before it began (flags:
+// 2 * compact_tiles(k_total) words; *bad zeroed). out and children may be null.
+// mail: three words of host memory, zeroed (see compact_kernel).
+void launch_compact(const CompactSource& c, uint64_t* flags, uint32_t* ctrl, void* out,
+                    int32_t* children, int64_t child_cap, unsigned long long* bad, uint32_t* mail,
+                    hipStream_t s);
+// In two, without waits between workgroups (words: compact_words(k_total)); with
+// out null the sizes only.
+int64_t compact_words(int64_t k_total);
+void launch_compact_no_wait(const CompactSource& c, uint32_t* words, void* out, int32_t* children,
+                            int64_t child_cap, uint32_t* mail, hipStream_t s);
 void launch_expand(const void* in, const int32_t* children, int64_t n_children,
                    const int32_t* oct_start, int32_t n_seg, const float* smin, const float* srg,
                    float mn1, float rg1, OctNode* out, hipStream_t s);
