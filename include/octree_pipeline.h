@@ -374,8 +374,9 @@ typedef struct ocp_compact_node {
  * device arrays. With nodes or children NULL, only writes the sizes
  * (n_nodes = K total, n_children). OCP_ERR_CAPACITY when a cap is below
  * them; OCP_ERR_STATE when a slot has no exact compact form (not the case
- * for the pipeline's own output); the arrays, never written past their caps,
- * are then not complete. Synchronises. */
+ * for the pipeline's own output in a box that is not far from the origin for
+ * its size). A refused call stores nothing, unless the caller has changed
+ * the build's nodes itself. Synchronises. */
 int ocp_compact_octree(ocp_ctx ctx, ocp_compact_node* nodes, int64_t node_cap,
                        int32_t* children, int64_t child_cap, int64_t* n_nodes,
                        int64_t* n_children);

@@ -65,6 +65,7 @@ struct Plan {
   int64_t n_total = 0;
   int64_t max_seg = 0;        // the largest segment's length
   bool device_boxes = false;  // boxes reduced on the device into ws.boxes
+  bool exact_boxes = false;   // see box_exact
   bool permutation = false;   // point indices carried through sort and unique
   SegView sv{};
   int32_t tiles_morton = 0, tiles_sort = 0, tiles_scan = 0, tiles_node = 0, tiles_tree = 0, tiles_win = 0;
@@ -401,6 +402,13 @@ int ensure_level2(ocp_ctx c, int64_t n, int64_t max_seg) {
   return OCP_OK;
 }
 
+// Whether every corner that a build decodes in this box has an exact compact form
+// for sure: 1024 times its rounding against the range stays below one cell, and
+// the range's binary fractions are normal numbers.
+bool box_exact(float mn, float rg) {
+  return rg > 1e-30f && rg < 1e30f && std::fabs(mn) < 8192.0f * rg;
+}
+
 SegView single_view(int64_t n, float mn, float rg) {
   SegView sv{};
   sv.n_seg = 1;
@@ -477,6 +485,7 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
   p.max_seg = n;
   p.permutation = perm;
   p.sv = single_view(n, mn, rg);
+  p.exact_boxes = box_exact(mn, rg);
   p.tiles_morton = static_cast<int32_t>(cdiv(n, morton_tile(tt)));
   p.tiles_sort = static_cast<int32_t>(cdiv(n, pipe_sort_tile(tt, perm)));
   p.tiles_scan = static_cast<int32_t>(cdiv(n, scan_tile(tt)));
@@ -553,6 +562,8 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.auto_msd = !c->tuned && pipe_sort_msd(tt, perm, n_seg);
   p.permutation = perm;
   p.device_boxes = !smin;
+  p.exact_boxes = smin != nullptr;
+  for (int32_t k = 0; k < n_seg && p.exact_boxes; ++k) p.exact_boxes = box_exact(smin[k], srg[k]);
   const int stile = pipe_sort_tile(tt, perm);
   std::vector<int32_t> host(7 * static_cast<size_t>(n_seg + 1));
   int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0, tw = 0;
@@ -1399,6 +1410,7 @@ int ocp_build_autobox(ocp_ctx c, const float* points, int float3, int64_t n) {
   Plan p;
   if (int r = prepare_plain(c, n, 0.0f, 1.0f, &p)) return r;
   p.device_boxes = true;
+  p.exact_boxes = false;
   p.permutation = c->permutation;
   if (int r = ensure_perm(c)) return r;
   p.sv.mn = c->ws.boxes;
@@ -1662,7 +1674,13 @@ int ocp_compact_octree(ocp_ctx c, ocp_compact_node* nodes, int64_t node_cap, int
   uint32_t* mail = c->mail + kMailWords;
   mail[0] = mail[1] = mail[2] = 0;
   uint64_t hbad = 0;
-  if (c->in_pipeline) {
+  // One pass where nothing can be refused any more: boxes in which every slot of a
+  // build has its form, and more room than its links need (a cloud's chains link
+  // fewer times than it has slots, and it has a leaf per unique key, two more at its
+  // quirk root). Else the tiles' counts come first, and the second pass stores
+  // nothing where they refuse.
+  const bool sure = p.exact_boxes && child_cap >= kt + p.n_total + 32 * int64_t(p.n_seg);
+  if (c->in_pipeline || (store && !sure)) {
     if (int r = ensure_fmt(c, compact_words(kt))) return r;
     launch_compact_no_wait(src, c->fmt, store ? nodes : nullptr, children, child_cap, mail,
                            c->stream);

@@ -454,9 +454,10 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
   store_tile(slots, s_words, g0, cnt, s_excl, before, total, out, children, child_cap);
 }
 
-// The compact form in two passes over the nodes, whose tiles wait for nothing, for
-// a pipeline's slots: launches with waits of two frames may not overlap, and this
-// one is outside their order. Tiles form at most kCompactGroups groups of
+// The compact form in two passes over the nodes, whose tiles wait for nothing. For
+// a pipeline's slots, as launches with waits of two frames may not overlap, and
+// this one is outside their order; and for calls that may yet be refused, as the
+// second pass knows all counts before it stores. Tiles form at most kCompactGroups groups of
 // neighbours, a workgroup each in the first pass: tile_children[t], and per group
 // {children, slots without an exact form}. The second pass sums the groups before
 // its own and its group's tiles before its own.
@@ -504,8 +505,8 @@ __global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
 }
 
 // mail (host memory): [0] the children's total, [2] the number of slots without
-// an exact form. A grid of one with out null: these alone. Children past
-// child_cap are not stored.
+// an exact form. A grid of one with out null: these alone. Where there are such
+// slots, or more children than child_cap, nothing is stored.
 __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
     const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, int32_t tiles,
     const uint2* __restrict__ groups, const uint32_t* __restrict__ tile_children,
@@ -546,7 +547,7 @@ __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
     mail[0] = s_sum[1];
     mail[2] = s_sum[2];
   }
-  if (!out) return;
+  if (!out || s_sum[2] != 0 || static_cast<int64_t>(s_sum[1]) > child_cap) return;
   TileSlots slots;
   slots.form(s_words, g0, cnt, st, seg0, info);
   uint32_t total;
