@@ -419,11 +419,13 @@ int ocp_time_builds(ocp_ctx ctx, const float* points, int float3,
                     int steps, float* ms_per_build);
 
 /* ------------------------------------------------------------ tuning */
-/* Tile parameters and the sort's digit width (pass count). Until a table is
- * set (ocp_set_tune, ocp_autotune), a build without the permutation chooses
- * the sort's form by itself, whatever sort_bits and sort_msd say: sort_msd's
- * from 16384 points on, the LSD passes for small builds and, for some builds
- * at a time, where the keys of the last one crowded into few digits. */
+/* Tile parameters and the sort's digit width (pass count). Under the default
+ * table, which a new context has (whatever its oct_order), a build without the
+ * permutation chooses the sort's form by itself, whatever sort_bits and
+ * sort_msd say: sort_msd's from 16384 points on, the LSD passes for small
+ * builds and, for some builds at a time, where the keys of the last one
+ * crowded into few digits; clouds of at most 8192 points take one kernel for
+ * all stages before the octree. Setting that table again goes back to this. */
 typedef struct ocp_tune {
   int32_t sort_waves;   /* OneSweep tile of 8-bit digits: waves ... */
   int32_t sort_kpt;     /* ... and keys per thread */
@@ -444,9 +446,10 @@ typedef struct ocp_tune {
 int ocp_get_tune(ocp_ctx ctx, ocp_tune* out);
 int ocp_set_tune(ocp_ctx ctx, const ocp_tune* in);
 /* Time the supported configurations on the given workload (plain when
- * n_seg == 0, else batched) by two rounds of coordinate descent, each
- * configuration's time the best of three runs of `reps` builds, and keep
- * the fastest; writes the choice. */
+ * n_seg == 0, else batched) by two rounds of coordinate descent, and the
+ * library's own choice, each one's time the best of three runs of `reps`
+ * builds, and keep the fastest; writes the choice (the library's own: the
+ * default table). */
 int ocp_autotune(ocp_ctx ctx, const float* points, int float3, int64_t n,
                  const int32_t* seg_offsets, const float* seg_min,
                  const float* seg_range, int32_t n_seg, int reps,

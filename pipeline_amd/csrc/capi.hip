@@ -176,7 +176,7 @@ struct ocp_context {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   TuneTable tune;
-  bool tuned = false;  // a table was set: its sort form is taken as it stands
+  bool tuned = false;  // a table other than the default was set: its sort form stands
   // Builds of about skew_n points to come that take the LSD passes, because the
   // keys of one like them crowded into few digits.
   int32_t skew_left = 0;
@@ -425,6 +425,17 @@ int tune_key(const TuneTable& t) {
   const int k = ((t.sort_waves * 64 + t.sort_kpt) * 64 + t.morton_ppt) * 64 + t.scan_ipt;
   return (((k * 2 + (t.sort_bits == 10)) * 32 + t.sort10_kpt) * 2 + (t.oct_order != 0)) * 2 +
          (t.sort_msd != 0);
+}
+
+// The table that a new context starts with stands for the library's choice, so
+// that a table read and set again leaves a context as it was. (oct_order changes
+// nothing.)
+bool default_tune(const TuneTable& t) {
+  const TuneTable d;
+  return t.sort_waves == d.sort_waves && t.sort_kpt == d.sort_kpt &&
+         t.morton_ppt == d.morton_ppt && t.morton_grid == d.morton_grid &&
+         t.scan_ipt == d.scan_ipt && t.sort_bits == d.sort_bits &&
+         t.sort10_kpt == d.sort10_kpt && t.sort_msd == d.sort_msd;
 }
 
 // The tile table of a build: the context's, with the library's choice of the
@@ -1486,9 +1497,9 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
       return OCP_ERR_INVALID;
   }
   const int32_t clouds = std::max<int32_t>(n_seg, 1);
-  const int64_t flag_words =
-      flag_words_for(crowd_tune(tt, tune != nullptr, n, clouds), n, clouds);
-  tt = build_tune(tt, tune != nullptr, n, n, clouds, permutation != 0);
+  const bool tuned = !default_tune(tt);
+  const int64_t flag_words = flag_words_for(crowd_tune(tt, tuned, n, clouds), n, clouds);
+  tt = build_tune(tt, tuned, n, n, clouds, permutation != 0);
   // The allocations of ensure_workspace, alloc_nodes, ensure_level2 and
   // ensure_perm for a first build of this shape, plus the context's control words and digit
   // counts (ocp_create).
@@ -1813,22 +1824,26 @@ int ocp_time_builds(ocp_ctx c, const float* points, int float3, const int32_t* o
 }
 
 // ---------------------------------------------------------------- tuning
+static void fill_tune(const TuneTable& t, ocp_tune* out) {
+  out->sort_waves = t.sort_waves;
+  out->sort_kpt = t.sort_kpt;
+  out->morton_ppt = t.morton_ppt;
+  out->morton_grid = t.morton_grid;
+  out->scan_ipt = t.scan_ipt;
+  out->sort_bits = t.sort_bits;
+  out->sort10_kpt = t.sort10_kpt;
+  out->oct_order = t.oct_order;
+  out->sort_msd = t.sort_msd;
+}
+
 int ocp_get_tune(ocp_ctx c, ocp_tune* out) {
   if (check_ctx(c) || !out) return OCP_ERR_INVALID;
-  out->sort_waves = c->tune.sort_waves;
-  out->sort_kpt = c->tune.sort_kpt;
-  out->morton_ppt = c->tune.morton_ppt;
-  out->morton_grid = c->tune.morton_grid;
-  out->scan_ipt = c->tune.scan_ipt;
-  out->sort_bits = c->tune.sort_bits;
-  out->sort10_kpt = c->tune.sort10_kpt;
-  out->oct_order = c->tune.oct_order;
-  out->sort_msd = c->tune.sort_msd;
+  fill_tune(c->tune, out);
   return OCP_OK;
 }
 
-int ocp_set_tune(ocp_ctx c, const ocp_tune* in) {
-  if (check_ctx(c) || !in) return OCP_ERR_INVALID;
+// explicit_form: the table's sort form stands, also the default table's.
+static int set_table(ocp_ctx c, const ocp_tune* in, bool explicit_form) {
   const bool sort_ok = sort_config_supported(in->sort_waves, in->sort_kpt) ||
                        (in->sort_waves == 8 && in->sort_kpt == 15);
   if (!sort_ok || !morton_config_supported(in->morton_ppt) ||
@@ -1846,10 +1861,15 @@ int ocp_set_tune(ocp_ctx c, const ocp_tune* in) {
   c->tune.sort10_kpt = in->sort10_kpt;
   c->tune.oct_order = in->oct_order;
   c->tune.sort_msd = in->sort_msd;
-  c->tuned = true;
+  c->tuned = explicit_form || !default_tune(c->tune);
   clear_graphs(c);
   c->tab_offsets.clear();
   return OCP_OK;
+}
+
+int ocp_set_tune(ocp_ctx c, const ocp_tune* in) {
+  if (check_ctx(c) || !in) return OCP_ERR_INVALID;
+  return set_table(c, in, false);
 }
 
 int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
@@ -1861,8 +1881,8 @@ int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
   const int32_t* offs = n_seg == 0 ? plain_off.data() : offsets;
   // A configuration's time: the best of three runs of `reps` builds (the
   // choices differ by fractions of a percent, about the spread of one run).
-  auto time_cfg = [&](const ocp_tune& t, float* ms) -> int {
-    if (int r = ocp_set_tune(c, &t)) return r;
+  auto time_cfg = [&](const ocp_tune& t, bool explicit_form, float* ms) -> int {
+    if (int r = set_table(c, &t, explicit_form)) return r;
     float best_run = 0;
     for (int run = 0; run < 3; ++run) {
       float m = 0;
@@ -1877,7 +1897,7 @@ int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
   ocp_tune best;
   ocp_get_tune(c, &best);
   float best_ms = 0;
-  if (int r = time_cfg(best, &best_ms)) return r;
+  if (int r = time_cfg(best, true, &best_ms)) return r;
   // Coordinate descent, two rounds: sort tile of 8-bit digits, then the
   // pass count (four 8-bit passes, three 10-bit ones, or the MSD form: one
   // 10-bit scatter and LDS bucket sorts; two tile sizes each),
@@ -1888,7 +1908,7 @@ int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
   const int sort_cfgs[][2] = {{8, 15}, {4, 16}, {4, 24}, {8, 8}, {8, 12}, {8, 16}, {16, 8}};
   auto try_cfg = [&](const ocp_tune& t) -> int {
     float ms;
-    if (int r = time_cfg(t, &ms)) return r;
+    if (int r = time_cfg(t, true, &ms)) return r;
     if (ms < best_ms) {
       best_ms = ms;
       best = t;
@@ -1928,7 +1948,14 @@ int ocp_autotune(ocp_ctx c, const float* points, int float3, int64_t n,
     }
     if (std::memcmp(&start, &best, sizeof(best)) == 0) break;
   }
-  if (int r = ocp_set_tune(c, &best)) return r;
+  // The library's own choice, which no table gives (the small clouds' kernel, the
+  // sort's form by what the keys were like): the default table stands for it.
+  ocp_tune none{};
+  fill_tune(TuneTable{}, &none);
+  float none_ms = 0;
+  if (int r = time_cfg(none, false, &none_ms)) return r;
+  if (none_ms <= best_ms) best = none;
+  else if (int r = set_table(c, &best, true)) return r;
   if (chosen) *chosen = best;
   return OCP_OK;
 }
