@@ -114,14 +114,14 @@ __device__ __forceinline__ int span_bits(uint32_t n, int low) {
   return low + (n > 1 ? 32 - __clz(static_cast<int>(n - 1)) : 0);
 }
 
-// First level: window `local` of a segment (with window == 0 the digit of that
-// number), sorted in place. A digit above CAP is listed for the
+// First level: window `local` of a segment (of a long one the digit of that
+// number, see msd_window), sorted in place. A digit above CAP is listed for the
 // second level, with its counts and cursors cleared.
 // (four waves a SIMD: what the LDS of the larger workgroups allows)
 template <int WAVES, int KPT, int P1, int BINS>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) void msd_window_kernel(
     uint32_t* __restrict__ keys, SegView sv, const int32_t* __restrict__ tile_start,
-    int32_t window, const uint32_t* __restrict__ hist, MsdLevel2 l2, uint32_t* __restrict__ ctrl) {
+    const uint32_t* __restrict__ hist, MsdLevel2 l2, uint32_t* __restrict__ ctrl) {
   constexpr int THREADS = WAVES * 64;
   constexpr uint32_t CAP = THREADS * KPT;
   __shared__ int32_t s_big[3];
@@ -129,6 +129,7 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(4)))
   const TileRef r = find_tile(tile_start, sv.n_seg, static_cast<int32_t>(blockIdx.x));
   const int32_t sb = seg_begin(sv, r.seg);
   const int32_t len = seg_end(sv, r.seg) - sb;
+  const int32_t window = msd_window(WAVES == 4, len);
   const uint32_t wlo = static_cast<uint32_t>(r.local) * static_cast<uint32_t>(window);
   uint32_t cnt[kRadix / THREADS];
   const Window w = find_window<THREADS>(
@@ -398,13 +399,13 @@ void launch_msd_windows(uint32_t* keys, const SegView& sv, const int32_t* tile_s
                         int32_t total_tiles, int64_t max_seg, const uint32_t* hist,
                         const MsdLevel2& l2, uint32_t* ctrl, hipStream_t s) {
   if (total_tiles <= 0) return;
-  const int32_t window = msd_window(max_seg);
+  // (four waves a workgroup: the windows of small segments)
   if (msd_small(max_seg))
-    msd_window_kernel<4, 16, 10, 12><<<total_tiles, 256, 0, s>>>(keys, sv, tile_start, window, hist,
-                                                             l2, ctrl);
+    msd_window_kernel<4, 16, 10, 12><<<total_tiles, 256, 0, s>>>(keys, sv, tile_start, hist, l2,
+                                                             ctrl);
   else
-    msd_window_kernel<8, 24, 9, 13><<<total_tiles, 512, 0, s>>>(keys, sv, tile_start, window, hist,
-                                                            l2, ctrl);
+    msd_window_kernel<8, 24, 9, 13><<<total_tiles, 512, 0, s>>>(keys, sv, tile_start, hist, l2,
+                                                            ctrl);
 }
 
 void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, const uint32_t* ctrl,

@@ -197,7 +197,7 @@ void launch_onesweep_pass(const uint32_t* in, uint32_t* out,
 // MSD sort of bare 30-bit keys (k_msd.hip): the scatter by the top 10-bit
 // digit (histogram slot 2 of the 10-bit histograms) without a lookback (cursor
 // holds n_seg * 1024 zeroed words, claimed by atomic adds; tiles of 1024 *
-// sort10_kpt keys), LDS sorts of windows of msd_window(max_seg) keys of the
+// sort10_kpt keys), LDS sorts of windows of msd_window(...) keys of the
 // result, and a second level for the digits too large for LDS.
 struct MsdLevel2 {
   int4* big;         // listed digits {first key, keys, top digit, first shared slot}
@@ -211,13 +211,16 @@ struct MsdLevel2 {
 // workgroups of four waves (four a CU by LDS), larger ones in 12288-key
 // workgroups of eight (two a CU): at 2^20 points 1024 keys a digit, 10M 9800.
 inline bool msd_small(int64_t max_seg) { return max_seg <= 1024 * 2800; }
-// Keys per window; 0: one workgroup per digit, where a digit about fills it.
-inline int32_t msd_window(int64_t max_seg) {
-  return msd_small(max_seg) ? 1024 : max_seg <= 1024 * 6000 ? 4096 : 0;
+// Keys per window of a segment of len keys; 0: one workgroup per digit, where a
+// digit about fills it. By the segment, not the batch's largest: with the latter a
+// batch of one cloud of 6.2M points and 2000 of 100 launched two million
+// workgroups (7,970 us a build, now 352).
+__host__ __device__ inline int32_t msd_window(bool small, int64_t len) {
+  return small ? 1024 : len <= 1024 * 6000 ? 4096 : 0;
 }
 inline int64_t msd_windows(int64_t len, int64_t max_seg) {
-  const int32_t w = msd_window(max_seg);
-  return w ? (len + w - 1) / w : (len > 0 ? 1024 : 0);
+  const int32_t w = msd_window(msd_small(max_seg), len);
+  return w ? (len + w - 1) / w : 1024;
 }
 // Room for the second level of n keys, whatever they are: listed digits hold
 // more than the LDS capacity each.
