@@ -773,7 +773,7 @@ bool enqueue_pipeline(ocp_ctx c, const float* pts, bool f3, const Plan& p,
     { KScope k(c, kKPass1, capturing);
       launch_msd_windows(dst, p.sv, p.ts_win, p.tiles_win, p.max_seg, w.hist, w.l2, c->ctrl, s); }
     KScope k(c, kKPass2, capturing);
-    launch_msd_level2(dst, src, w.l2, c->ctrl, s);
+    launch_msd_level2(dst, src, w.l2, p.n_total, p.max_seg, c->ctrl, s);
   }
   for (int pass = 0; pass < passes && !msd; ++pass) {
     KScope k(c, kKPass0 + pass, capturing);

@@ -408,16 +408,21 @@ void launch_msd_windows(uint32_t* keys, const SegView& sv, const int32_t* tile_s
                                                             ctrl);
 }
 
-void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, const uint32_t* ctrl,
-                       hipStream_t s) {
+void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, int64_t n,
+                       int64_t max_seg, const uint32_t* ctrl, hipStream_t s) {
+  // Tiles that this build can list; the room may be that of a longer one before it
+  // (20,000 points after a build of 30M: 70 us by the room, 60 as before it).
+  MsdLevel2 need{};
+  msd_level2_caps(n, max_seg, &need);
+  const int32_t tiles = std::min(need.max_tiles, l2.max_tiles);
   // Counting takes a grid that fills the chip once, whose workgroups take every
   // grid-th tile; the scatter and the LDS sorts one tile each (in a loop the
   // compiler keeps a tile's addresses, and one scatter shares a CU instead of two:
   // 2^24 clustered points 457 -> 446 us).
-  const uint32_t grid = static_cast<uint32_t>(std::max(1, std::min(l2.max_tiles, 768)));
+  const uint32_t grid = static_cast<uint32_t>(std::max(1, std::min(tiles, 768)));
   msd_l2_hist_kernel<<<grid, 512, 0, s>>>(keys, l2, ctrl);
-  msd_l2_scatter_kernel<<<static_cast<uint32_t>(l2.max_tiles), 1024, 0, s>>>(keys, other, l2, ctrl);
-  msd_l2_window_kernel<<<static_cast<uint32_t>(l2.max_tiles), 512, 0, s>>>(other, keys, l2, ctrl);
+  msd_l2_scatter_kernel<<<static_cast<uint32_t>(tiles), 1024, 0, s>>>(keys, other, l2, ctrl);
+  msd_l2_window_kernel<<<static_cast<uint32_t>(tiles), 512, 0, s>>>(other, keys, l2, ctrl);
 }
 
 }  // namespace ocp

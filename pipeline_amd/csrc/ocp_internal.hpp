@@ -236,9 +236,10 @@ void launch_msd_scatter(const uint32_t* in, uint32_t* out, const SegView& sv,
 void launch_msd_windows(uint32_t* keys, const SegView& sv, const int32_t* tile_start,
                         int32_t total_tiles, int64_t max_seg, const uint32_t* hist,
                         const MsdLevel2& l2, uint32_t* ctrl, hipStream_t s);
-// `other` is overwritten where digits are listed.
-void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, const uint32_t* ctrl,
-                       hipStream_t s);
+// `other` is overwritten where digits are listed. The grids are what n keys of
+// segments of at most max_seg can need, however much room l2 has by now.
+void launch_msd_level2(uint32_t* keys, uint32_t* other, const MsdLevel2& l2, int64_t n,
+                       int64_t max_seg, const uint32_t* ctrl, hipStream_t s);
 // Cursor words per segment after the segments' histograms (the first sort
 // pass's or the MSD scatter's: one per digit, at most 1024).
 constexpr int kCursorWords = 1024;

@@ -44,3 +44,21 @@ def test_short_clouds_cost_little():
         batch = ctx.time_builds(d, seg_offsets=offs, seg_min=box[0], seg_range=box[1], warmup=3,
                                 steps=10)
         assert batch < 4 * alone, (batch, alone)
+
+
+def test_small_build_after_a_large_one():
+    """What a context has room for must not cost the builds that need little."""
+    n, large = 20_000, 100_000_000
+    with pipeline_amd.Context(0) as ctx:
+        d = ctx.empty((large, 4), np.float32)
+        ctx.k_InitRandomVec4(d, large, 0.0, 1024.0, 1)
+
+        def best():
+            return min(ctx.time_builds(d, n=n, warmup=10, steps=50) for _ in range(5))
+        before = best()
+        ctx.build(d, large, 0.0, 1024.0)
+        ctx.synchronize()
+        after = best()
+        assert after < 1.25 * before, (before, after)
+        ctx.build(d, n, 0.0, 1024.0)
+        _check_segment(ctx.fetch(), 0, oracle.build_plain(d.to_host(n * 4).reshape(n, 4)))
