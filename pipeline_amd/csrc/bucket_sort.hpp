@@ -24,8 +24,32 @@ namespace ocp {
 // 47 us); keys that crowd into few parts take the radix passes. More than 16
 // in a part (32, 64) cost clustered clouds 30-130% of their windows' time.
 constexpr uint32_t kBinMax = 16;
+
+// Adds `unit` to a digit's counter in LDS and returns what it was. Adds of one wave
+// to one counter are made one after the other; with SHARED the lanes that have the
+// first lane's digit are added at once, where there are several.
+template <bool SHARED>
+__device__ __forceinline__ uint32_t count_digit(uint32_t* counter, uint32_t digit, uint32_t unit) {
+  if constexpr (SHARED) {
+    const uint32_t first = static_cast<uint32_t>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(digit)));
+    const uint64_t same = __ballot(digit == first);
+    const uint32_t n = static_cast<uint32_t>(__popcll(same));
+    if (n >= 8u && digit == first) {
+      const uint32_t rank = static_cast<uint32_t>(__popcll(same & lanemask_lt()));
+      uint32_t old = 0;
+      if (rank == 0) old = atomicAdd(counter, n * unit);
+      old = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(old)));
+      return old + rank * unit;
+    }
+  }
+  return atomicAdd(counter, unit);
+}
+
+// SHARED (see count_digit): for keys of which many may be equal, or equal in the
+// bits that a pass looks at.
 template <int WAVES, int KPT, int P0 = (WAVES >= 16 ? 12 : WAVES == 8 ? 11 : 10), int P1 = 8,
-          int BINS = 0>
+          int BINS = 0, bool SHARED = false>
 __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g, int32_t n,
                                                 uint32_t base = 0, int span = 0) {
   constexpr int THREADS = WAVES * 64;
@@ -113,7 +137,7 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
       const int32_t idx = wbase + k * 64 + static_cast<int32_t>(lane);
       if (idx < wend) {
         const uint32_t b = kv[k] >> low, sh = (b & 1u) * 16u;
-        at[k] = (atomicAdd(&s_whist[b >> 1], 1u << sh) >> sh) & 0xffffu;
+        at[k] = (count_digit<SHARED>(&s_whist[b >> 1], b, 1u << sh) >> sh) & 0xffffu;
         crowded |= at[k] >= kBinMax;
       }
     }
@@ -177,7 +201,8 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
     for (int k = 0; k < KPT; ++k) {
       if (wbase + k * 64 >= wend) continue;
       const int32_t idx = wbase + k * 64 + static_cast<int32_t>(lane);
-      if (idx < wend) atomicAdd(&s_whist[kv[k] & (NB - 1u)], 1u);
+      const uint32_t d = kv[k] & (NB - 1u);
+      if (idx < wend) (void)count_digit<SHARED>(&s_whist[d], d, 1u);
     }
     __syncthreads();
     uint32_t cc[PER];
@@ -199,7 +224,8 @@ __device__ __forceinline__ void lds_bucket_sort(const uint32_t* src, uint32_t* g
     for (int k = 0; k < KPT; ++k) {
       if (wbase + k * 64 >= wend) continue;
       const int32_t idx = wbase + k * 64 + static_cast<int32_t>(lane);
-      if (idx < wend) s_keys[atomicAdd(&s_whist[kv[k] & (NB - 1u)], 1u)] = kv[k];
+      const uint32_t d = kv[k] & (NB - 1u);
+      if (idx < wend) s_keys[count_digit<SHARED>(&s_whist[d], d, 1u)] = kv[k];
     }
     const int32_t pad_end = (n + 63) & ~63;  // <= CAP
     for (int i = n + tid; i < pad_end; i += THREADS) s_keys[i] = 0xffffffffu;

@@ -331,8 +331,8 @@ void launch_small_clouds(const float* pts, bool float3, const SegView& sv, int64
 
 // Sort of at most kSmallSort keys in place by one workgroup: what LDS holds, and
 // up to there faster than the six launches of the passes, for spread keys (2000:
-// 52 -> 20 us, 16,384: 54 -> 33) as for those that take the radix passes (16,384
-// clustered ones: 55 -> 50).
+// 41 -> 8 us, 16,384: 46 -> 19) as for those that take its radix passes (16,384
+// clustered ones 46 -> 36, of a few values in the top bits 44 -> 41).
 constexpr uint32_t kSmallSort = 16384;
 void launch_small_sort(uint32_t* keys, int32_t n, const uint32_t* ctrl, hipStream_t s);
 
