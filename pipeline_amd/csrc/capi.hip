@@ -30,6 +30,8 @@ struct DevBuf {
   int64_t n = 0;
 };
 
+constexpr int kBatchTables = 8;  // point offsets and tile maps of a batch
+
 struct Workspace {
   int64_t n_cap = 0;
   int32_t seg_cap = 0;
@@ -49,7 +51,7 @@ struct Workspace {
   uint64_t* flags = nullptr;     // flag_cap words
   int32_t* counts = nullptr;     // n_unique[seg_cap], kalloc[seg_cap]
   int32_t* oct_start = nullptr;  // seg_cap + 1
-  int32_t* tables = nullptr;     // seg_start + 6 tile maps, 7 * (seg_cap+1)
+  int32_t* tables = nullptr;     // seg_start + 7 tile maps, kBatchTables * (seg_cap+1)
   float* boxes = nullptr;        // seg_min[seg_cap], seg_range[seg_cap]
   uint32_t* box_mm = nullptr;    // per segment {min, max} while boxes are reduced
   uint32_t* vals_a = nullptr;    // key->point permutation (allocated when enabled): sorted
@@ -344,7 +346,7 @@ int ensure_workspace(ocp_ctx c, int64_t n, int32_t n_seg, int64_t flag_words) {
     if ((r = dev_alloc(c, &w.hist, int64_t(cap) * (hist_stride(10) + kCursorWords))) ||
         (r = dev_alloc(c, &w.counts, int64_t(cap) * 2)) ||
         (r = dev_alloc(c, &w.oct_start, int64_t(cap) + 1)) ||
-        (r = dev_alloc(c, &w.tables, 7 * (int64_t(cap) + 1))) ||
+        (r = dev_alloc(c, &w.tables, kBatchTables * (int64_t(cap) + 1))) ||
         (r = dev_alloc(c, &w.boxes, 2 * int64_t(cap))) ||
         (r = dev_alloc(c, &w.box_mm, 2 * int64_t(cap))))
       return r;
@@ -458,14 +460,14 @@ TuneTable crowd_tune(const TuneTable& set, bool tuned, int64_t n, int32_t n_seg)
   return t;
 }
 
-// The form for this build. A large cloud's keys may crowd as they like.
-TuneTable choose_tune(ocp_ctx c, int64_t n, int64_t max_seg, int32_t n_seg, bool perm) {
-  const TuneTable t = build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm);
-  if (c->tuned || !pipe_sort_msd(t, perm, n_seg) || !auto_sort_skew(max_seg) ||
+// Whether this build takes that one. A large cloud's keys may crowd as they like.
+bool take_crowd(ocp_ctx c, const TuneTable& own, int64_t n, int64_t max_seg, int32_t n_seg,
+                bool perm) {
+  if (c->tuned || !pipe_sort_msd(own, perm, n_seg) || !auto_sort_skew(max_seg) ||
       c->skew_left <= 0 || n < c->skew_n / 2 || n > c->skew_n * 2)
-    return t;
+    return false;
   --c->skew_left;
-  return crowd_tune(c->tune, c->tuned, n, n_seg);
+  return true;
 }
 
 // After a build of the library's choice: its level-2 tiles tell how many keys
@@ -508,12 +510,13 @@ Plan plain_plan(const TuneTable& tt, int64_t n, float mn, float rg, bool perm) {
 
 // ... and the memory it needs.
 int prepare_plain(ocp_ctx c, int64_t n, float mn, float rg, Plan* p) {
-  const TuneTable tt = choose_tune(c, n, n, 1, c->permutation);
+  const TuneTable own = build_tune(c->tune, c->tuned, n, n, 1, c->permutation);
+  const TuneTable crowd = crowd_tune(c->tune, c->tuned, n, 1);
+  const TuneTable& tt = take_crowd(c, own, n, n, 1, c->permutation) ? crowd : own;
   // (for either form of the sort: which one a later build of this size takes
   // does not change the memory)
-  if (int r = ensure_workspace(c, n, 1, flag_words_for(crowd_tune(c->tune, c->tuned, n, 1), n, 1)))
-    return r;
-  if (pipe_sort_msd(build_tune(c->tune, c->tuned, n, n, 1, c->permutation), c->permutation, 1))
+  if (int r = ensure_workspace(c, n, 1, flag_words_for(crowd, n, 1))) return r;
+  if (pipe_sort_msd(own, c->permutation, 1))
     if (int r = ensure_level2(c, n, n)) return r;
   *p = plain_plan(tt, n, mn, rg, c->permutation);
   p->auto_msd = !c->tuned && pipe_sort_msd(tt, c->permutation, 1);
@@ -550,14 +553,15 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   int64_t max_seg = 0;
   for (int32_t k = 0; k < n_seg; ++k)
     max_seg = std::max<int64_t>(max_seg, int64_t(offsets[k + 1]) - offsets[k]);
-  const TuneTable tt = choose_tune(c, n, max_seg, n_seg, perm);
-  if (int r = ensure_workspace(
-          c, n, n_seg, flag_words_for(crowd_tune(c->tune, c->tuned, n, n_seg), n, n_seg)))
-    return r;
-  if (pipe_sort_msd(build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm), perm, n_seg))
+  const TuneTable own = build_tune(c->tune, c->tuned, n, max_seg, n_seg, perm);
+  const TuneTable crowd = crowd_tune(c->tune, c->tuned, n, n_seg);
+  const bool crowded = take_crowd(c, own, n, max_seg, n_seg, perm);
+  const TuneTable& tt = crowded ? crowd : own;
+  if (int r = ensure_workspace(c, n, n_seg, flag_words_for(crowd, n, n_seg))) return r;
+  if (pipe_sort_msd(own, perm, n_seg))
     if (int r = ensure_level2(c, n, max_seg)) return r;
   Workspace& w = c->ws;
-  const int32_t stride = w.seg_cap + 1;
+  const int32_t stride = n_seg + 1;  // (one copy brings them all)
   int32_t* d_start = w.tables;
   int32_t* d_tm = w.tables + stride;
   int32_t* d_ts = w.tables + 2 * stride;
@@ -565,6 +569,7 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   int32_t* d_tn = w.tables + 4 * stride;
   int32_t* d_tt = w.tables + 5 * stride;
   int32_t* d_tw = w.tables + 6 * stride;
+  int32_t* d_tx = w.tables + 7 * stride;
   Plan p;
   p.tune = tt;
   p.n_seg = n_seg;
@@ -575,9 +580,12 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.device_boxes = !smin;
   p.exact_boxes = smin != nullptr;
   for (int32_t k = 0; k < n_seg && p.exact_boxes; ++k) p.exact_boxes = box_exact(smin[k], srg[k]);
-  const int stile = pipe_sort_tile(tt, perm);
-  std::vector<int32_t> host(7 * static_cast<size_t>(n_seg + 1));
-  int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0, tw = 0;
+  // Sort tiles of either form, so that the tables do not change with the form: a
+  // caller's captured build reads them where they were, and a captured call that
+  // changes form uploads nothing.
+  const int stile = pipe_sort_tile(own, perm), xtile = pipe_sort_tile(crowd, perm);
+  std::vector<int32_t> host(kBatchTables * static_cast<size_t>(n_seg + 1));
+  int64_t tm = 0, ts = 0, tc = 0, tn = 0, ttr = 0, tw = 0, tx = 0;
   for (int32_t k = 0; k <= n_seg; ++k) {
     host[k] = offsets[k];
     host[(n_seg + 1) + k] = static_cast<int32_t>(tm);
@@ -586,25 +594,26 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
     host[4 * (n_seg + 1) + k] = static_cast<int32_t>(tn);
     host[5 * (n_seg + 1) + k] = static_cast<int32_t>(ttr);
     host[6 * (n_seg + 1) + k] = static_cast<int32_t>(tw);
+    host[7 * (n_seg + 1) + k] = static_cast<int32_t>(tx);
     if (k < n_seg) {
       const int64_t len = int64_t(offsets[k + 1]) - offsets[k];
       tm += cdiv(len, morton_tile(tt));
       ts += cdiv(len, stile);
+      tx += cdiv(len, xtile);
       tc += cdiv(len, scan_tile(tt));
       tn += cdiv(len, kOctTile);
       ttr += cdiv(len, tree_tile(n));
       tw += msd_windows(len, max_seg);
     }
   }
-  const int tab_key = tune_key(tt) * 2 + (pipe_sort_bits(tt, perm) == 10);
+  // (own, crowd and the tiles follow from these and the offsets)
+  const int tab_key = tune_key(own) * 2 + (pipe_sort_bits(own, perm) == 10);
   const bool same = c->tab_tune_key == tab_key &&
                     c->tab_offsets.size() == static_cast<size_t>(n_seg + 1) &&
                     std::equal(offsets, offsets + n_seg + 1, c->tab_offsets.begin());
   if (!same) {
-    for (int q = 0; q < 7; ++q)
-      OCP_HIP(c, hipMemcpyAsync(w.tables + q * stride, host.data() + q * (n_seg + 1),
-                                sizeof(int32_t) * (n_seg + 1), hipMemcpyHostToDevice,
-                                c->stream));
+    OCP_HIP(c, hipMemcpyAsync(w.tables, host.data(), sizeof(int32_t) * host.size(),
+                              hipMemcpyHostToDevice, c->stream));
     c->tab_offsets.assign(offsets, offsets + n_seg + 1);
     c->tab_tune_key = tab_key;
     c->tab_min.clear();
@@ -630,13 +639,13 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.sv.min1 = 0.0f;
   p.sv.range1 = 1.0f;
   p.tiles_morton = static_cast<int32_t>(tm);
-  p.tiles_sort = static_cast<int32_t>(ts);
+  p.tiles_sort = static_cast<int32_t>(crowded ? tx : ts);
   p.tiles_scan = static_cast<int32_t>(tc);
   p.tiles_node = static_cast<int32_t>(tn);
   p.tiles_tree = static_cast<int32_t>(ttr);
   p.tiles_win = static_cast<int32_t>(tw);
   p.ts_morton = d_tm;
-  p.ts_sort = d_ts;
+  p.ts_sort = crowded ? d_tx : d_ts;
   p.ts_scan = d_tc;
   p.ts_node = d_tn;
   p.ts_tree = d_tt;
@@ -1509,7 +1518,7 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
               + 3 * 1 * cap        // prefix_n, hl, hr
               + 4 * 4 * cap        // left child, parent, edge counts, offsets
               + cap * int64_t(sizeof(OctNode)) + 16;  // nodes (K_cap starts at N)
-  b += 4 * (seg * (hist_stride(10) + kCursorWords) + 2 * seg + (seg + 1) + 7 * (seg + 1) +
+  b += 4 * (seg * (hist_stride(10) + kCursorWords) + 2 * seg + (seg + 1) + kBatchTables * (seg + 1) +
             4 * seg);
   b += 8 * std::max<int64_t>(flag_words, 1 << 16);
   if (pipe_sort_msd(tt, permutation != 0, clouds)) {
