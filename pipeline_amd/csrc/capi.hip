@@ -895,6 +895,7 @@ int report_timeout(ocp_ctx c, const uint32_t* hc) {
   launch_fill_u32(c->ctrl + kCtrlTimeout, 0u, 1, c->stream);
   OCP_CHECK_LAUNCH(c);
   OCP_HIP(c, hipStreamSynchronize(c->stream));
+  c->mail[kCtrlTimeout] = 0;
   return fail(c, OCP_ERR_STATE,
               "a lookback wait gave up (wait limit reached); the result of the work "
               "enqueued since the last check is invalid");
@@ -991,6 +992,10 @@ int ocp_create(ocp_ctx* out, int device, void* stream) {
     ocp_destroy(c);
     return OCP_ERR_HIP;
   }
+  c->mail[kCtrlTimeout] = 0;
+  const uint64_t at = reinterpret_cast<uint64_t>(c->mail + kCtrlTimeout);
+  launch_fill_u32(c->ctrl + kCtrlMailAt, static_cast<uint32_t>(at), 1, c->stream);
+  launch_fill_u32(c->ctrl + kCtrlMailAt + 1, static_cast<uint32_t>(at >> 32), 1, c->stream);
   std::string why;
   if (int r = scratch_init(device, c->stream, &why)) {
     ocp_destroy(c);

@@ -23,6 +23,7 @@ enum CtrlSlot : int {
   kCtrlMsdTiles = 15,  // ... their tiles
   kCtrlMsdSlots = 16,  // ... and the count slots of their long runs
   kCtrlOctForm = 17,   // last make or link call whose arrays were not a build's
+  kCtrlMailAt = 18,    // (two words) where the host reads of a time-out
   kCtrlWords = 64,
 };
 
@@ -46,8 +47,14 @@ __device__ __forceinline__ bool stopped(const uint32_t* ctrl, uint32_t tag) {
   const uint32_t v = ctrl[kCtrlTimeout];
   return v != 0u && v != timeout_mark(tag);
 }
+// The host's own word is told as well: what it last heard of a build would not
+// show the time-out of a launch replayed from a caller's graph since.
 __device__ __forceinline__ void raise_timeout(uint32_t* ctrl, uint32_t tag) {
   ctrl[kCtrlTimeout] = timeout_mark(tag);
+  const uint64_t at = static_cast<uint64_t>(ctrl[kCtrlMailAt]) |
+                      (static_cast<uint64_t>(ctrl[kCtrlMailAt + 1]) << 32);
+  __hip_atomic_store(reinterpret_cast<uint32_t*>(at), timeout_mark(tag), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // Kernels without waits stop on any mark.
 __device__ __forceinline__ bool stopped_any(const uint32_t* ctrl) {

@@ -81,3 +81,30 @@ def test_batch_whose_sort_changes_its_form():
                 check()
                 build()
                 check()
+
+
+def test_replayed_time_out_is_reported():
+    """A wait that gives up in a replay, after a build whose report was good."""
+    rng = np.random.default_rng(3)
+    keys = rng.integers(0, 1 << 30, 300_000, dtype=np.uint32)
+    pts = _cells(rng.integers(0, 1 << 30, 20_000))
+    with _Capture() as cap:
+        ctx = cap.ctx
+        d, alt, p = ctx.upload(keys), ctx.empty(keys.size, np.uint32), ctx.upload(pts)
+        ctx.k_SortKeys(d, alt, keys.size)
+        ctx.synchronize()
+        replay = cap.record(lambda: ctx.k_SortKeys(d, alt, keys.size))
+        for limit in (-1, 0, -1):
+            d.copy_from(keys)
+            ctx.set_wait_limit(-1)
+            ctx.build(p, pts.shape[0], 0.0, 1024.0)
+            ctx.synchronize()
+            ctx.set_wait_limit(limit)
+            replay()
+            if limit == 0:
+                with pytest.raises(pipeline_amd.OcpError, match="wait gave up"):
+                    ctx.synchronize()
+            else:
+                ctx.synchronize()
+                np.testing.assert_array_equal(d.to_host(), np.sort(keys))
+                ctx.counts(1)
