@@ -1791,10 +1791,9 @@ int ocp_get_kernel_ms(ocp_ctx c, float* ms, const char** names, int32_t max_kern
   *n_kernels = kKernelCount;
   if (!c->ev_recorded) return fail(c, OCP_ERR_STATE, "no eager build with stage timing on");
   OCP_HIP(c, hipEventSynchronize(c->ev[6]));
-  // Whether the MSD sort's second level had work (read after the build ended).
-  uint32_t msd_run = 0;
-  if (c->kmsd && names)
-    OCP_HIP(c, hipMemcpy(&msd_run, c->ctrl + kCtrlMsdTiles, sizeof(msd_run), hipMemcpyDeviceToHost));
+  // Whether the MSD sort's second level had work, as the build reported (the control
+  // word is cleared by what comes after it).
+  const uint32_t msd_run = c->mail[kCtrlMsdTiles];
   for (int k = 0; k < kKernelCount && k < max_kernels; ++k) {
     if (names)
       names[k] = !(c->kmsd && k >= kKPass0 && k <= kKPass3) ? kKernelNames[k]
