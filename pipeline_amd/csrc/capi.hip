@@ -987,22 +987,27 @@ int ocp_create(ocp_ctx* out, int device, void* stream) {
       hipMalloc(reinterpret_cast<void**>(&c->s_hist), sizeof(uint32_t) * (1024 + 256)) != hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->mail),
                     sizeof(uint32_t) * (kMailWords + kCtrlWords), hipHostMallocDefault) !=
-          hipSuccess ||
-      hipMemsetAsync(c->ctrl, 0, sizeof(uint32_t) * kCtrlWords, c->stream) != hipSuccess) {
+          hipSuccess) {
     ocp_destroy(c);
     return OCP_ERR_HIP;
   }
-  c->mail[kCtrlTimeout] = 0;
+  // The control words, by way of the landing place behind the mail.
+  uint32_t* first = c->mail + kMailWords;
   const uint64_t at = reinterpret_cast<uint64_t>(c->mail + kCtrlTimeout);
-  launch_fill_u32(c->ctrl + kCtrlMailAt, static_cast<uint32_t>(at), 1, c->stream);
-  launch_fill_u32(c->ctrl + kCtrlMailAt + 1, static_cast<uint32_t>(at >> 32), 1, c->stream);
+  std::memset(first, 0, sizeof(uint32_t) * kCtrlWords);
+  first[kCtrlMailAt] = static_cast<uint32_t>(at);
+  first[kCtrlMailAt + 1] = static_cast<uint32_t>(at >> 32);
+  c->mail[kCtrlTimeout] = 0;
+  if (hipMemcpyAsync(c->ctrl, first, sizeof(uint32_t) * kCtrlWords, hipMemcpyHostToDevice,
+                     c->stream) != hipSuccess) {
+    ocp_destroy(c);
+    return OCP_ERR_HIP;
+  }
   std::string why;
   if (int r = scratch_init(device, c->stream, &why)) {
     ocp_destroy(c);
     return r;
   }
-  for (auto& e : c->ev) (void)hipEventCreate(&e);
-  for (auto& e : c->kev) (void)hipEventCreate(&e);
   *out = c;
   return OCP_OK;
 }
@@ -1772,6 +1777,12 @@ int ocp_set_cold_timing(ocp_ctx c, int64_t flush_bytes) {
 
 int ocp_set_stage_timing(ocp_ctx c, int enable) {
   if (check_ctx(c)) return OCP_ERR_INVALID;
+  if (enable) {  // (the events of contexts that never time a build are never made)
+    for (auto& e : c->ev)
+      if (!e) OCP_HIP(c, hipEventCreate(&e));
+    for (auto& e : c->kev)
+      if (!e) OCP_HIP(c, hipEventCreate(&e));
+  }
   c->stage_timing = enable != 0;
   return OCP_OK;
 }
