@@ -68,7 +68,8 @@ def kernel_bytes(name: str, n: int, u: int, k: int, float4: bool = True) -> floa
         "onesweep_pass3": 8 * n,
         "msd_scatter": 8 * n,                   # MSD sort: scatter by the top digit
         "msd_buckets": 8 * n,                   # every bucket read and written once
-        "msd_lsd_fallback": 28 * n,             # lower-digit counts + three passes
+        # (msd_lsd_fallback, the second level, handles the keys of the digits too
+        # large for LDS only: its bytes follow from the keys, not from n)
         "unique": 4 * n + 4 * u,                # sorted read + unique write
         "radix_tree": 4 * u + 15 * m,           # codes read; 1+1+1+4+4+4 written
         "edge_scan": 8 * m,                     # 4 read; 4 written
