@@ -901,11 +901,11 @@ __device__ __forceinline__ void resolve_children(const OctArgs& a, int32_t slot)
   }
 }
 template <bool MAKE>
-__global__ __launch_bounds__(1024) void resolve_kernel(OctArgs a, float mn, float rg) {
+__global__ __launch_bounds__(256) void resolve_kernel(OctArgs a, float mn, float rg) {
   if (*a.form != a.form_id) return;
   const int32_t m = a.n_brt_host;
-  for (int32_t i = blockIdx.x * 1024 + static_cast<int32_t>(threadIdx.x); i < m;
-       i += static_cast<int32_t>(gridDim.x) * 1024) {
+  for (int32_t i = blockIdx.x * 256 + static_cast<int32_t>(threadIdx.x); i < m;
+       i += static_cast<int32_t>(gridDim.x) * 256) {
     if (i == 0) {
       resolve_children<MAKE>(a, 0);
       continue;
@@ -993,8 +993,8 @@ namespace {
 // (a grid that fills the chip; it returns at once for a build's arrays)
 template <bool MAKE>
 void launch_resolve(const OctArgs& a, const SegView& sv, hipStream_t s) {
-  const int32_t blocks = (a.n_brt_host + 1023) / 1024;
-  resolve_kernel<MAKE><<<blocks < 256 ? blocks : 256, 1024, 0, s>>>(a, sv.min1, sv.range1);
+  const int32_t blocks = (a.n_brt_host + 255) / 256;
+  resolve_kernel<MAKE><<<blocks < 2048 ? blocks : 2048, 256, 0, s>>>(a, sv.min1, sv.range1);
 }
 }  // namespace
 
