@@ -58,9 +58,10 @@
 // caller's arrays to be what a build's are (check_kernel); for any others, as
 // offsets that are not the inclusive scan, or codes that repeat or have more than
 // 30 bits, it scatters order keys by global atomics and a kernel after it resolves
-// them. Make has no children arrays: see check_kernel. For 2M points make takes 17
-// us of check, 30 of the tiled kernel and 5 of the idle resolve, link 15, 30 and 5;
-// the scatter and the resolve took 117 and 187 when they served every array.
+// them. Make has no children arrays: see check_kernel. For 2M points make takes 16
+// us of check, 30 of the tiled kernel and 5 of the idle resolve, link 13, 30 and 5;
+// for arrays of another form they take 131 and 197 us (117 and 182 when the scatter
+// and the resolve, without a check, served every array).
 //
 // What bounds it: how many tiles share a CU while each waits for its loads, its
 // barriers and the walks of its listed children (a chain of up to four dependent
@@ -699,8 +700,9 @@ __global__ __launch_bounds__(kThreads) void oct_build_kernel(
 //
 // A tile's nodes find their parents and children in LDS; those with one elsewhere
 // are listed and looked up in memory by full waves. What bounds it is the reading
-// of every array (link of 2M points: 23 bytes a node, 14 us; 19 when every node
-// gathered its neighbours from memory, 16 with tiles of 1024).
+// of every array (link: 23 bytes a node) and its tests. Link of 2M points: 19 us
+// when every node gathered its neighbours from memory, 15 with branches between the
+// tests (16 with tiles of 1024), 13.
 //
 // The make call alone has no children arrays to walk down from a slot's owner,
 // so the top link of a chain whose walk up leaves its tile comes from below: the
@@ -780,57 +782,52 @@ __global__ __launch_bounds__(kThreads) void check_kernel(OctArgs a) {
   __syncthreads();
   const auto in_tile = [&](int32_t q) { return static_cast<uint32_t>(q - i0) < static_cast<uint32_t>(T); };
   const auto is_node = [&](int32_t q) { return static_cast<uint32_t>(q) < static_cast<uint32_t>(m); };
-  bool ok = true;
+  // (all tests of a node without branches: its few loads and LDS reads are bounded
+  // by selects, and most of what this kernel takes is instructions)
+  bool bad = false;
   // (a full list: not a build's)
   const auto push = [&](uint16_t* list, int which, uint32_t l) {
     const uint32_t at = atomicAdd(&s_n[which], 1u);
     if (at < kCheckList) list[at] = static_cast<uint16_t>(l);
-    else ok = false;
+    else bad = true;
   };
 #pragma unroll
   for (int u = 0; u < NPT; ++u) {
     const int32_t i = at0 + u;
     const uint32_t l = static_cast<uint32_t>(l0 + u);
     const uint32_t code_l = u ? code[u - 1] : before, code_r = u + 1 < NPT ? code[u + 1] : next;
-    if (i >= m) continue;
-    ok = ok && code[u] < kCodeEnd && pn[u] <= kMaxPrefix;
-    if constexpr (LINK) ok = ok && code[u] < code_r && code_r < kCodeEnd && is_node(lc[u]);
-    if (i == 0) {
-      ok = ok && e[u] == 0 && p[u] == 0;
-      continue;
-    }
+    const bool live = i < m, inner = live & (i != 0);
     const int32_t up = par[u];
-    ok = ok && e[u] >= 0 && e[u] <= kMaxEdge &&
-         static_cast<uint32_t>(p[u]) - static_cast<uint32_t>(u ? p[u - 1] : p_before) ==
-             static_cast<uint32_t>(e[u]) &&
-         code_l < code[u] && is_node(up);
-    if (up == 0 || in_tile(up)) {
-      const uint32_t pn_up = up == 0 ? pn_0 : s_pn[up - i0];
-      ok = ok && static_cast<int32_t>(pn[u] / 3u) - static_cast<int32_t>(pn_up / 3u) == e[u] &&
-           (up == 0 || pn_up < pn[u]);
-    } else if (is_node(up)) {
-      push(s_up, 0, l);
-    }
+    bad |= live & ((code[u] >= kCodeEnd) | (pn[u] > kMaxPrefix));
+    if constexpr (LINK) bad |= live & ((code[u] >= code_r) | (code_r >= kCodeEnd) | !is_node(lc[u]));
+    bad |= live & (i == 0) & ((e[u] | p[u]) != 0);
+    bad |= inner & ((static_cast<uint32_t>(e[u]) > static_cast<uint32_t>(kMaxEdge)) |
+                    (static_cast<uint32_t>(p[u]) - static_cast<uint32_t>(u ? p[u - 1] : p_before) !=
+                     static_cast<uint32_t>(e[u])) |
+                    (code_l >= code[u]) | !is_node(up));
+    const bool near = (up == 0) | in_tile(up);
+    const uint32_t own = pn[u];
+    const uint32_t pn_up = up == 0 ? pn_0 : s_pn[in_tile(up) ? up - i0 : 0];
+    bad |= inner & near &
+           ((third(own) - third(pn_up) != e[u]) | (pn_up > kMaxPrefix) |
+            ((up != 0) & (pn_up >= own)));
+    if (inner & !near & is_node(up)) push(s_up, 0, l);
     if constexpr (LINK) {
 #pragma unroll
       for (int side = 0; side < 2; ++side) {
-        if (side == 0 ? hl[u] != 0 : hr[u] != 0) continue;
+        const bool inside = inner & ((side == 0 ? hl[u] : hr[u]) == 0);
         const int32_t ch = lc[u] + side;
-        if (ch <= 0 || !is_node(ch)) {
-          ok = false;
-        } else if (!in_tile(ch)) {
-          push(s_down, 1, l * 2u + static_cast<uint32_t>(side));
-        } else if (s_par[ch - i0] == i) {
-          s_named[ch - i0] = 1;
-        } else {
-          ok = false;
-        }
+        const bool node = is_node(ch) & (ch != 0), here = in_tile(ch);
+        const bool named = s_par[here ? ch - i0 : 0] == i;
+        bad |= inside & (!node | (here & !named));
+        if (inside & here & named) s_named[ch - i0] = 1;
+        if (inside & node & !here) push(s_down, 1, l * 2u + static_cast<uint32_t>(side));
       }
       // The true root's children lie on either side of the pair of codes with the
       // shortest common prefix.
-      const bool of_root = delta(code[u], code_r) == root || delta(code_l, code[u]) == root;
-      ok = ok && of_root == (up == 0);
-    } else if (e[u] > 0 && is_node(up)) {
+      const bool of_root = (delta(code[u], code_r) == root) | (delta(code_l, code[u]) == root);
+      bad |= inner & (of_root != (up == 0));
+    } else if (inner & (e[u] > 0) & is_node(up)) {
       bool far = false;  // out of the octree kernel's tile: the numbers differ above its bits
       int32_t h = up;
       for (int hop = 0; hop < 31; ++hop) {
@@ -848,25 +845,25 @@ __global__ __launch_bounds__(kThreads) void check_kernel(OctArgs a) {
     // (a parent in the tile has named its children there)
 #pragma unroll
     for (int u = 0; u < NPT; ++u)
-      if (at0 + u < m && at0 + u > 0 && par[u] != 0 && in_tile(par[u]) && !s_named[l0 + u]) ok = false;
+      bad |= (at0 + u < m) & (at0 + u > 0) & (par[u] != 0) & in_tile(par[u]) &
+             (s_named[l0 + u] == 0);
   }
   for (uint32_t q = tid; q < min(s_n[0], kCheckList); q += kThreads) {
     const uint32_t l = s_up[q];
     const int32_t i = i0 + static_cast<int32_t>(l), up = s_par[l];
     const uint32_t own = s_pn[l], pn_up = a.prefix_n[up];
-    ok = ok && static_cast<int32_t>(own / 3u) - static_cast<int32_t>(pn_up / 3u) == a.edge[i] &&
-         pn_up < own;
+    bad |= (third(own) - third(pn_up) != a.edge[i]) | (pn_up >= own);
     if constexpr (LINK) {
       const int32_t at = a.left_child[up];
       const bool leaf_l = a.has_leaf_left[up], leaf_r = a.has_leaf_right[up];
-      ok = ok && (i == at ? !leaf_l : i == at + 1 && !leaf_r);
+      bad |= !(i == at ? !leaf_l : (i == at + 1) & !leaf_r);
     }
   }
   for (uint32_t q = tid; q < min(s_n[1], kCheckList); q += kThreads) {
     const uint32_t l = s_down[q];
     if constexpr (LINK) {
       const int32_t i = i0 + static_cast<int32_t>(l >> 1);
-      ok = ok && a.parent[a.left_child[i] + static_cast<int32_t>(l & 1u)] == i;
+      bad |= a.parent[a.left_child[i] + static_cast<int32_t>(l & 1u)] != i;
     } else {
       const int32_t i = i0 + static_cast<int32_t>(l);
       const int32_t n_new = a.edge[i];
@@ -874,7 +871,7 @@ __global__ __launch_bounds__(kThreads) void check_kernel(OctArgs a) {
                make_key(i, n_new - 1));
     }
   }
-  if (!ok) *a.form = a.form_id;
+  if (bad) *a.form = a.form_id;
 }
 
 // After a scatter of order keys: the keys of the slots of chain i become the
