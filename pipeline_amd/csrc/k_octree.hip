@@ -121,15 +121,6 @@ struct SegBind {
 __device__ __forceinline__ uint32_t child_of(uint32_t code, int32_t level) {
   return (code >> (static_cast<uint32_t>(kMortonBits - 3 * level) & 31u)) & 7u;
 }
-__device__ __forceinline__ uint32_t delta(uint32_t a, uint32_t b) {
-  const uint32_t x = a ^ b;
-  return ((x ? static_cast<uint32_t>(__clz(static_cast<int>(x))) : 32u) - 1u) & 0xffu;
-}
-// (a byte: prefix lengths are at most 31)
-__device__ __forceinline__ int32_t third(uint32_t x) {
-  return static_cast<int32_t>((x * 11u) >> 5);
-}
-
 // Order of the sequential program: make writes by (chain, step), every link
 // write after every make write, links by (node, side).
 __device__ __forceinline__ uint32_t make_key(int32_t chain, int32_t step) {

@@ -514,7 +514,7 @@ __global__ __launch_bounds__(256) void radix_pairs_kernel(
       const int32_t g = i0 + p;  // the pair
       const uint32_t q = static_cast<uint32_t>(p + HALO);
       const uint32_t b = b8[q];
-      // (b + 127 in every byte; a dead lane's b of 0 finds nothing)
+      // (b + 127 in every byte; a dead lane looks for the first pair's, to no end)
       const uint32_t key = __builtin_amdgcn_perm(0u, b + 127u, 0u);
       const uint32_t row = q >> 4, grp = q >> 8;
       const uint32_t m0 = below16(s_b[row], key);

@@ -11,7 +11,6 @@
 // batches, a workgroup per cloud: 64 x 4096 108 -> 47, 512 x 4096 199 -> 87,
 // 2000 x 8192 909 -> 545.
 #include "bucket_sort.hpp"
-#include "pair_rows.hpp"
 
 namespace ocp {
 namespace {

@@ -82,6 +82,19 @@ __device__ __forceinline__ float decode_axis(uint32_t code, int axis, float mn,
   return t * rg + mn;
 }
 
+// ---------------------------------------------------------------- common prefixes
+__device__ __forceinline__ uint32_t clz32(uint32_t x) {
+  return x ? static_cast<uint32_t>(__clz(static_cast<int>(x))) : 32u;
+}
+// The reference's prefix length of two codes, a byte (04_radix_tree.cpp:16-37).
+__device__ __forceinline__ uint32_t delta(uint32_t a, uint32_t b) {
+  return (clz32(a ^ b) - 1u) & 0xffu;
+}
+// The octree level of a prefix length below 32, which those of 30-bit codes are.
+__device__ __forceinline__ int32_t third(uint32_t x) {
+  return static_cast<int32_t>((x * 11u) >> 5);
+}
+
 // ---------------------------------------------------------------- multisplit
 // The lanes whose digit differs from this lane's, built up bit by bit: every
 // digit bit is one ballot, whose lanes of the other value are collected by one

@@ -1,18 +1,11 @@
 // Rows of sixteen small values as bytes, and the comparison of a whole row with
 // one value: what the radix tree's search for the nearest smaller common
-// prefix (k_radix_tree.hip) is made of. Shared with the small clouds' kernel.
+// prefix (k_radix_tree.hip) is made of.
 #pragma once
 
 #include "ocp_internal.hpp"
 
 namespace ocp {
-
-__device__ __forceinline__ uint32_t clz32(uint32_t x) {
-  return x ? static_cast<uint32_t>(__clz(static_cast<int>(x))) : 32u;
-}
-__device__ __forceinline__ uint32_t delta(uint32_t a, uint32_t b) {
-  return (clz32(a ^ b) - 1u) & 0xffu;
-}
 
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
@@ -42,6 +35,5 @@ __device__ __forceinline__ uint32_t min16(const v4u w) {
   m = __builtin_elementwise_min(m, as_halves((w.w >> 8) & 0x00ff00ffu));
   return min(static_cast<uint32_t>(m.x), static_cast<uint32_t>(m.y));
 }
-__device__ __forceinline__ uint32_t third(uint32_t x) { return (x * 11u) >> 5; }  // x / 3, x < 32
 
 }  // namespace ocp
