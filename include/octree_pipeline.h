@@ -194,7 +194,10 @@ int ocp_k_InitOctNodes(ocp_ctx ctx, ocp_oct_node* nodes, int32_t n_alloc,
 /* Replaces gpu::k_MakeOctNodes (include/cuda/kernels/07_octree.cuh:7-17) and
  * k_MakeOctNodes (include/kernels/07_octree.hpp:5-14). N = number of BRT
  * nodes; n_alloc = number of node slots (max(1, max_i P[i]+e[i])), which
- * bounds every write. Expects nodes prepared by ocp_k_InitOctNodes. */
+ * bounds every write. Expects nodes prepared by ocp_k_InitOctNodes. The arrays
+ * may be any the reference takes, offsets of another layout than
+ * ocp_k_PartialSum's, repeated codes and codes above 30 bits among them; those
+ * that the stages here give for unique Morton codes take half the time. */
 int ocp_k_MakeOctNodes(ocp_ctx ctx, ocp_oct_node* oct_nodes,
                        const int32_t* node_offsets,
                        const int32_t* rt_node_counts, const uint32_t* codes,
@@ -202,7 +205,8 @@ int ocp_k_MakeOctNodes(ocp_ctx ctx, ocp_oct_node* oct_nodes,
                        float min_coord, float range, int32_t N,
                        int32_t n_alloc);
 /* Replaces gpu::k_LinkLeafNodes (include/cuda/kernels/07_octree.cuh:19-28)
- * and k_LinkLeafNodes (include/kernels/07_octree.hpp:16-25). */
+ * and k_LinkLeafNodes (include/kernels/07_octree.hpp:16-25). As for the make
+ * call. */
 int ocp_k_LinkLeafNodes(ocp_ctx ctx, ocp_oct_node* nodes,
                         const int32_t* node_offsets,
                         const int32_t* rt_node_counts, const uint32_t* codes,
@@ -327,7 +331,8 @@ int ocp_ppl_submit(ocp_ppl ppl, int32_t slot, const float* points, int float3,
                    int64_t n, float min_coord, float range);
 /* Waits for the slot's frame; reports its errors as ocp_synchronize does. */
 int ocp_ppl_wait(ocp_ppl ppl, int32_t slot);
-/* The slot's context: its results, validator and compact form. */
+/* The slot's context: its results, validator and compact form (which waits for
+ * nothing that another slot runs). */
 int ocp_ppl_context(ocp_ppl ppl, int32_t slot, ocp_ctx* ctx);
 
 /* ------------------------------------------------------------ octree checks

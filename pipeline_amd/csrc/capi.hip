@@ -198,8 +198,9 @@ struct ocp_context {
   uint32_t oct_calls = 0;  // make and link calls so far, as their mark in the control words
   Plan last_plan;
   // Pinned host memory: what the last build's offsets kernel, or for one cloud
-  // its octree kernel, reports (see launch_oct_offsets), then a landing place for small copies back. Current
-  // while no other work that can time out was enqueued after that build.
+  // its octree kernel, reports (see launch_oct_offsets), then a landing place for
+  // small copies back. Current while no other work that can time out was enqueued
+  // after that build.
   uint32_t* mail = nullptr;
   bool mail_current = false;
   bool graph_mode = false;
@@ -1520,8 +1521,8 @@ int ocp_workspace_size(const ocp_tune* tune, int64_t n, int32_t n_seg, int permu
   const int64_t flag_words = flag_words_for(crowd_tune(tt, tuned, n, clouds), n, clouds);
   tt = build_tune(tt, tuned, n, n, clouds, permutation != 0);
   // The allocations of ensure_workspace, alloc_nodes, ensure_level2 and
-  // ensure_perm for a first build of this shape, plus the context's control words and digit
-  // counts (ocp_create).
+  // ensure_perm for a first build of this shape, plus the context's control words
+  // and digit counts (ocp_create).
   const int64_t cap = std::max<int64_t>(n, 4096);
   const int64_t seg = std::max<int32_t>(n_seg, 1);
   int64_t b = 2 * 4 * cap          // keys_a, keys_b

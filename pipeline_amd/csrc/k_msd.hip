@@ -17,12 +17,13 @@
 // No kernel waits for another workgroup, and the passes over memory are two
 // for keys of ordinary digits and four (a read of them, two scatters, the
 // windows) for the others, against four passes and their lookbacks. At 10M
-// uniform points: scatter 38 us, windows 47 (58 before the binning of
-// bucket_sort.hpp), the idle second level 14, against 39 + 3 x 55 us for four
-// 8-bit passes; 2^24 clustered points, most of whose keys take the second
-// level: 48 + 30 + 27 + 58 + 97 us against 284. The LDS sorts bound it: 2 (8)
-// waves a SIMD by LDS, and their chain of barriers. Figures of whole builds are
-// given at the rule that takes this form, beside auto_sort_msd.
+// uniform points: scatter 35 us, windows 44 (58 before the binning of
+// bucket_sort.hpp), the idle second level 14, against 38 + 3 x 45 us for four
+// 8-bit passes; 2^24 clustered points, most of whose keys take the second level:
+// scatter 38, windows 27, then counts 28, scatter 36 and windows 104 us, against
+// 250. The LDS sorts bound it: 2 (8) waves a SIMD by LDS, and their chain of
+// barriers. Figures of whole builds are given at the rule that takes this form,
+// beside auto_sort_msd.
 #include "bucket_sort.hpp"
 #include "cursor_scatter.hpp"
 

@@ -311,11 +311,11 @@ void launch_edge_scan(const int32_t* edge, int32_t* offsets, const SegView& sv,
 // ---- stages 1 to 6 of small clouds (k_small.hip), one workgroup each: every
 // output of those stages at the segments' point offsets.
 constexpr int64_t kSmallCloud = 8192;
-// Up to here because 8192 points' keys, sort and tree take 125 KB of LDS; up to
-// there the kernel is the faster one for one cloud (8192 clustered points 84 us
-// to the general path's 100) as for batches of any length (k_small.hip). Builds
-// with point indices sort pairs, a set tuning table and stage timing name the
-// stages' kernels: these keep the general path.
+// Up to here because 8192 points' keys, sort and tree take 147 KB of the 160 KB of
+// LDS; up to there the kernel is the faster one for one cloud (8192 clustered
+// points 63 us to the general path's 100) as for batches of any length
+// (k_small.hip). Builds with point indices sort pairs, a table other than the
+// default and stage timing name the stages' kernels: these keep the general path.
 inline bool small_clouds(int64_t max_seg, int32_t n_seg, bool perm) {
   return !perm && max_seg <= kSmallCloud && n_seg >= 1;
 }
