@@ -193,6 +193,7 @@ struct ocp_context {
   // batch tables currently on device
   std::vector<int32_t> tab_offsets;
   std::vector<float> tab_min, tab_rg;
+  bool tab_exact = false;  // box_exact for all of them
   int tab_tune_key = -1;
   bool have_result = false;
   uint32_t oct_calls = 0;  // make and link calls so far, as their mark in the control words
@@ -579,8 +580,6 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
   p.auto_msd = !c->tuned && pipe_sort_msd(tt, perm, n_seg);
   p.permutation = perm;
   p.device_boxes = !smin;
-  p.exact_boxes = smin != nullptr;
-  for (int32_t k = 0; k < n_seg && p.exact_boxes; ++k) p.exact_boxes = box_exact(smin[k], srg[k]);
   // Sort tiles of either form, so that the tables do not change with the form: a
   // caller's captured build reads them where they were, and a captured call that
   // changes form uploads nothing.
@@ -631,7 +630,10 @@ int batched_plan(ocp_ctx c, const int32_t* offsets, const float* smin,
     OCP_HIP(c, hipStreamSynchronize(c->stream));  // host arrays may go away
     c->tab_min.assign(smin, smin + n_seg);
     c->tab_rg.assign(srg, srg + n_seg);
+    c->tab_exact = true;
+    for (int32_t k = 0; k < n_seg; ++k) c->tab_exact &= box_exact(smin[k], srg[k]);
   }
+  p.exact_boxes = !dev_boxes && c->tab_exact;
   p.sv.n_seg = n_seg;
   p.sv.start = d_start;
   p.sv.mn = w.boxes;
