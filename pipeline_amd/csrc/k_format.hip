@@ -319,67 +319,49 @@ struct SegTables {
 constexpr int kFmtTile = 512;  // slots per workgroup of the compact and expand kernels
 constexpr int kFmtPer = kFmtTile / kFmtThreads;
 
-// A tile's nodes into LDS in whole lines (a tile starts on a multiple of 16
-// bytes: 512 nodes are 30,720).
-__device__ __forceinline__ void load_tile(const OctNode* __restrict__ nodes, int64_t g0,
-                                          int32_t cnt, int32_t* s_words) {
-  const int tid = threadIdx.x;
-  const int32_t* src = reinterpret_cast<const int32_t*>(nodes + g0);
-  if (cnt == kFmtTile) {
-    constexpr int kVec = kFmtTile * 15 / 4;
-    constexpr int kRows = kVec / kFmtThreads;
-    static_assert(kVec - kRows * kFmtThreads == kFmtThreads / 2, "half a row is left");
-    const int4* v = reinterpret_cast<const int4*>(src) + tid;
-    int4* to = reinterpret_cast<int4*>(s_words) + tid;
-    int4 x[kRows];
-    int4 y = make_int4(0, 0, 0, 0);
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) x[k] = v[k * kFmtThreads];
-    if (tid < kFmtThreads / 2) y = v[kRows * kFmtThreads];
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) to[k * kFmtThreads] = x[k];
-    if (tid < kFmtThreads / 2) to[kRows * kFmtThreads] = y;
-  } else {
-    for (int32_t q = tid; q < cnt * 15; q += kFmtThreads) s_words[q] = src[q];
-  }
-}
-
-// The headers of a thread's neighbouring slots, from the tile in LDS (loaded
-// by the caller, who also passes the barrier after it).
+// The headers of a thread's neighbouring slots, whose 120 bytes it loads for
+// itself: a wave's are consecutive, and the caches pass every line on once.
 struct TileSlots {
   CompactNode cn[kFmtPer];
   int32_t child[kFmtPer][8];
   uint32_t children = 0, bad = 0;
-  __device__ __forceinline__ void form(const int32_t* s_words, int64_t g0, int32_t cnt,
-                                       const SegTables& st, int32_t seg0, SegInfo info) {
+  __device__ __forceinline__ void form(const OctNode* __restrict__ nodes, int64_t g0, int32_t cnt,
+                                       const SegTables& st) {
+    const int32_t l0 = static_cast<int32_t>(threadIdx.x) * kFmtPer;
+    int32_t w[kFmtPer][15];
+    if (l0 + kFmtPer <= cnt) {
+      __builtin_memcpy(w, nodes + g0 + l0, sizeof(w));
+    } else {
+#pragma unroll
+      for (int u = 0; u < kFmtPer; ++u)
+        if (l0 + u < cnt) __builtin_memcpy(w[u], nodes + g0 + l0 + u, sizeof(w[u]));
+    }
     // (one segment holds the whole tile, as a rule)
+    const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
     const bool one = st.oct_start[seg0 + 1] >= g0 + cnt;
+    SegInfo info = st.of(seg0);
 #pragma unroll
     for (int u = 0; u < kFmtPer; ++u) {
-      const int32_t l = static_cast<int32_t>(threadIdx.x) * kFmtPer + u;
+      const int32_t l = l0 + u;
       cn[u] = CompactNode{};
       if (l >= cnt) continue;
-      int32_t w[15];
-#pragma unroll
-      for (int c = 0; c < 15; ++c) w[c] = s_words[l * 15 + c];
       if (!one) info = st.of(seg_of_slot(g0 + l, st.oct_start, st.n_seg));
-      bad += !compact_header(w, info.mn, info.rg, info.root_level, &cn[u]);
+      bad += !compact_header(w[u], info.mn, info.rg, info.root_level, &cn[u]);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) child[u][c] = w[c];
+      for (int c = 0; c < 8; ++c) child[u][c] = w[u][c];
       children += __popc(cn[u].child_set);
     }
   }
 };
 
-// A tile's headers and children through LDS (whose nodes every thread has read),
-// to leave in whole lines. excl, before: the children before the tile and, in it,
+// A tile's headers and children through LDS, to leave in whole lines. excl, before: the children before the tile and, in it,
 // before the thread's slots. Children past child_cap are not stored.
-__device__ __forceinline__ void store_tile(TileSlots& slots, int32_t* s_words, int64_t g0,
+constexpr int kFmtWords = kFmtTile * 11;  // eight children and a header of three words a slot
+__device__ __forceinline__ void store_tile(TileSlots& slots, uint32_t* s_child, int64_t g0,
                                            int32_t cnt, uint32_t excl, uint32_t before,
                                            uint32_t total, uint32_t* __restrict__ out,
                                            int32_t* __restrict__ children, int64_t child_cap) {
   const int tid = threadIdx.x;
-  uint32_t* s_child = reinterpret_cast<uint32_t*>(s_words);
   uint32_t* s_head = s_child + kFmtTile * 8;
   uint32_t o = before;
 #pragma unroll
@@ -409,13 +391,13 @@ __device__ __forceinline__ void store_tile(TileSlots& slots, int32_t* s_words, i
 // children's total, [1] a wait gave up, [2] slots without an exact form exist
 // (*bad counts them).
 // What bounds it: 60 bytes a slot read and ~28 written; 0.99M slots take
-// 27 us, where two passes over the nodes and three scan launches took 54, and
-// the call 45 us instead of 208.
+// 25 us (27 with the nodes staged through LDS), where two passes over the nodes
+// and three scan launches took 54, and the call 43 us instead of 208.
 __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
     const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, uint64_t* __restrict__ flags,
     uint32_t* __restrict__ ctrl, uint32_t* __restrict__ out, int32_t* __restrict__ children,
     int64_t child_cap, unsigned long long* __restrict__ bad, uint32_t* __restrict__ mail) {
-  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_words[kFmtWords];
   __shared__ uint32_t s_tmp[kFmtThreads / 64];
   __shared__ uint32_t s_excl;
   const uint32_t tag = ctrl[kCtrlEpoch] * 8u + kStageScan;
@@ -423,12 +405,8 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
   const int32_t t = blockIdx.x;  // in-order dispatch: see lookback_n
   const int64_t g0 = int64_t(t) * kFmtTile;
   const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
-  load_tile(nodes, g0, cnt, s_words);
-  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
-  const SegInfo info = st.of(seg0);
-  __syncthreads();
   TileSlots slots;
-  slots.form(s_words, g0, cnt, st, seg0, info);
+  slots.form(nodes, g0, cnt, st);
   uint32_t total;
   const uint32_t before = block_excl_scan<kFmtThreads>(slots.children, s_tmp, &total);
   if (wave_id() == 0) {
@@ -449,7 +427,7 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
     atomicAdd(bad, static_cast<unsigned long long>(slots.bad));
     mail[2] = 1u;
   }
-  __syncthreads();  // (every word of the nodes has been read)
+  __syncthreads();
   if (!out || !children) return;
   store_tile(slots, s_words, g0, cnt, s_excl, before, total, out, children, child_cap);
 }
@@ -462,7 +440,7 @@ __global__ __launch_bounds__(kFmtThreads) void compact_kernel(
 // {children, slots without an exact form}. The second pass sums the groups before
 // its own and its group's tiles before its own.
 // What bounds them: 60 bytes a slot read twice and ~28 written; 0.99M slots take
-// 16 and 24 us, the call 54 where the one pass takes 45.
+// 15 and 22 us, the call 53 where the one pass takes 43.
 constexpr int32_t kCompactGroups = 2048;
 __host__ __device__ __forceinline__ int32_t tiles_per_group(int32_t tiles) {
   return (tiles + kCompactGroups - 1) / kCompactGroups;
@@ -470,7 +448,6 @@ __host__ __device__ __forceinline__ int32_t tiles_per_group(int32_t tiles) {
 __global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
     const OctNode* __restrict__ nodes, int64_t k_total, SegTables st, int32_t tiles,
     uint2* __restrict__ groups, uint32_t* __restrict__ tile_children) {
-  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
   __shared__ uint32_t s_tmp[2 * (kFmtThreads / 64)];
   const int32_t per = tiles_per_group(tiles);
   const int32_t t0 = static_cast<int32_t>(blockIdx.x) * per;
@@ -478,12 +455,8 @@ __global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
   for (int32_t t = t0; t < min(t0 + per, tiles); ++t) {
     const int64_t g0 = int64_t(t) * kFmtTile;
     const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
-    const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
-    const SegInfo info = st.of(seg0);
-    load_tile(nodes, g0, cnt, s_words);
-    __syncthreads();
     TileSlots slots;
-    slots.form(s_words, g0, cnt, st, seg0, info);
+    slots.form(nodes, g0, cnt, st);
     const uint32_t c = wave_sum(slots.children), b = wave_sum(slots.bad);
     if (lane_id() == 0) {
       s_tmp[2 * wave_id()] = c;
@@ -500,6 +473,7 @@ __global__ __launch_bounds__(kFmtThreads) void compact_count_kernel(
       tile_children[t] = n;
       sum.x += n;
     }
+    __syncthreads();
   }
   if (threadIdx.x == 0) groups[blockIdx.x] = sum;
 }
@@ -512,7 +486,7 @@ __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
     const uint2* __restrict__ groups, const uint32_t* __restrict__ tile_children,
     uint32_t* __restrict__ out, int32_t* __restrict__ children, int64_t child_cap,
     uint32_t* __restrict__ mail) {
-  __shared__ __attribute__((aligned(16))) int32_t s_words[kFmtTile * 15];
+  __shared__ uint32_t s_words[kFmtWords];
   __shared__ uint32_t s_tmp[kFmtThreads / 64];
   __shared__ uint32_t s_sum[3];  // children before the tile, all children, bad slots
   const int tid = threadIdx.x;
@@ -520,8 +494,6 @@ __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
   const int64_t g0 = int64_t(t) * kFmtTile;
   const int32_t cnt = static_cast<int32_t>(min(int64_t(kFmtTile), k_total - g0));
   if (tid < 3) s_sum[tid] = 0;
-  const int32_t seg0 = seg_of_slot(g0, st.oct_start, st.n_seg);
-  const SegInfo info = st.of(seg0);
   const int32_t per = tiles_per_group(tiles);
   const int32_t own = t / per, n_groups = (tiles + per - 1) / per;
   uint32_t before = 0, all = 0, bad = 0;
@@ -532,7 +504,8 @@ __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
     if (q < own) before += g.x;
   }
   for (int32_t q = own * per + tid; q < t; q += kFmtThreads) before += tile_children[q];
-  if (out) load_tile(nodes, g0, cnt, s_words);
+  TileSlots slots;
+  if (out) slots.form(nodes, g0, cnt, st);
   __syncthreads();
   before = wave_sum(before);
   all = wave_sum(all);
@@ -548,8 +521,6 @@ __global__ __launch_bounds__(kFmtThreads) void compact_write_kernel(
     mail[2] = s_sum[2];
   }
   if (!out || s_sum[2] != 0 || static_cast<int64_t>(s_sum[1]) > child_cap) return;
-  TileSlots slots;
-  slots.form(s_words, g0, cnt, st, seg0, info);
   uint32_t total;
   const uint32_t first = block_excl_scan<kFmtThreads>(slots.children, s_tmp, &total);
   store_tile(slots, s_words, g0, cnt, s_sum[0], first, total, out, children, child_cap);
