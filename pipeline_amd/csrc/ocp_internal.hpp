@@ -51,8 +51,7 @@ __device__ __forceinline__ bool stopped(const uint32_t* ctrl, uint32_t tag) {
 // show the time-out of a launch replayed from a caller's graph since.
 __device__ __forceinline__ void raise_timeout(uint32_t* ctrl, uint32_t tag) {
   ctrl[kCtrlTimeout] = timeout_mark(tag);
-  const uint64_t at = static_cast<uint64_t>(ctrl[kCtrlMailAt]) |
-                      (static_cast<uint64_t>(ctrl[kCtrlMailAt + 1]) << 32);
+  const uint64_t at = *reinterpret_cast<const uint64_t*>(ctrl + kCtrlMailAt);
   __hip_atomic_store(reinterpret_cast<uint32_t*>(at), timeout_mark(tag), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
